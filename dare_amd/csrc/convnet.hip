@@ -633,77 +633,178 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_sub(const uint16_t* __rest
 }
 
 // Weight gradient partials: P[c][tap][co][ci] = sum over the voxels of chunk c of
-// G[v][co] * X[v + off(tap)][ci]. Wave = one chunk of (z, y) rows for one 16x16 (co, ci)
-// block; A[co][voxel] = G, B[voxel][ci] = shifted X; 27 accumulators, one per tap.
-template <int CIN, int COUT>
+// G[v][co] * X[v + off(tap)][ci], a GEMM with K = voxels on v_mfma_f32_16x16x32_bf16. Both
+// operands must hold consecutive voxels per lane while the tensors are channels-last, so the
+// block stages 16-channel slices in LDS as they lie in memory ([voxel][16 channels], 32 bytes a
+// voxel) and reads fragments with the LDS transpose read (ds_read_b64_tr_b16): in a group of 16
+// lanes, lane s reads four channels of voxel s / 4 and receives channel s of the four voxels.
+// A tap's shift is then only another LDS address. K index kq * 4 + j of the first read and
+// 16 + kq * 4 + j of the second stand for voxel (kq, j) and 16 + (kq, j) of the step in both
+// operands, which keeps each read 512 contiguous bytes (no bank conflicts).
+//
+// Block = one 16 x 16 (co, ci) pair of a unit: 4 rows (one per wave) x XT voxels along x,
+// marching along z with a ring of three input planes; the next plane is loaded into registers
+// while this one is computed. A block takes units blockIdx.x, + gridDim.x, ... and keeps its 27
+// accumulators over all of them; its four waves are summed through LDS, so a chunk is a block.
+// What bounds it: 54 fragment reads feed 27 matrix instructions, so the LDS reads set the rate
+// of the inner loop (about half the matrix peak); at 64^3 the staging latency does. 16 -> 16
+// channels at 64^3: 219 -> 18 us (the earlier form read G and X as single 2-byte global loads).
+typedef short bf16x4s __attribute__((ext_vector_type(4)));
+
+__device__ inline bf16x8 lds_tr8(const uint16_t* p, int second) {
+    typedef __attribute__((address_space(3))) bf16x4s* lds_ptr;
+    const bf16x4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
+    const bf16x4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + second));
+    typedef short bf16x8s __attribute__((ext_vector_type(8)));
+    const bf16x8s v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+template <int CIN, int COUT, int XT>
 __global__ __launch_bounds__(kNetThreads) void k_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ G,
-                                                      int D, int H, int W, int rows_per_chunk, int nchunks,
+                                                      int D, int H, int W, int zb, int nxt, int nyt, int nunits,
                                                       float* __restrict__ P) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int chunk = blockIdx.x * 4 + wave;
-    if (chunk >= nchunks) return;
+    static_assert(XT % 32 == 0 && CIN % 8 == 0 && COUT % 16 == 0, "32-voxel K steps, 16-byte channel groups");
     constexpr int CB = CIN >= 16 ? CIN / 16 : 1;                // an 8-channel input is one half block
+    constexpr int RX = XT + 2;                                  // staged voxels of an input row
+    constexpr int kPlane = 6 * RX * 16;                         // elements of a staged input plane
+    constexpr int kStage = 3 * kPlane + 4 * XT * 16, kRed = 27 * 256 * 2;
+    constexpr int kLds = kStage > kRed ? kStage : kRed;         // the block reduction reuses the staging buffer
+    constexpr int NXP = (6 * RX * 2 + kNetThreads - 1) / kNetThreads;      // 16-byte loads per thread: input plane
+    constexpr int NGP = (4 * XT * 2) / kNetThreads;                        // ... and gradient rows
+    __shared__ __align__(16) uint16_t lds[kLds];
+    uint16_t* gl = lds + 3 * kPlane;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int cob = blockIdx.y / CB, cib = blockIdx.y % CB;
-    const int i = lane & 15, kq = lane >> 4;
-    const bool ci_ok = cib * 16 + i < CIN;
+    const int kq = lane >> 4, i = lane & 15;
+    const int frag = ((kq * 4 + (i >> 2)) * 16) + (i & 3) * 4;  // this lane's element offset in a fragment
     floatx4 acc[27];
 #pragma unroll
     for (int t = 0; t < 27; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const int rows = D * H;
-    const int r0 = chunk * rows_per_chunk;
-    const int r1 = (r0 + rows_per_chunk < rows) ? r0 + rows_per_chunk : rows;
-    for (int r = r0; r < r1; r++) {
-        const int z = r / H, y = r % H;
-        const long long vrow = static_cast<long long>(r) * W;
-        for (int xs = 0; xs < W; xs += 16) {
-            bf16x4 a;
+
+    for (int unit = blockIdx.x; unit < nunits; unit += gridDim.x) {
+        const int xt = unit % nxt, yt = (unit / nxt) % nyt, zt = unit / (nxt * nyt);
+        const int x0 = xt * XT, y0 = yt * 4;
+        const int z0 = zt * zb, z1 = (z0 + zb < D) ? z0 + zb : D;
+        // input plane z: rows y0 - 1 .. y0 + 4, voxels x0 - 1 .. x0 + XT, zero outside the box
+        auto load_x = [&](int z, uint4* r) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int xv = xs + kq * 4 + e;
-                a[e] = xv < W ? static_cast<short>(G[(vrow + xv) * COUT + cob * 16 + i]) : short(0);
+            for (int q = 0; q < NXP; q++) {
+                const int e = q * kNetThreads + tid;
+                const int half = e & 1, vox = e >> 1, row = vox / RX, xx = x0 - 1 + vox - row * RX, yy = y0 - 1 + row;
+                const bool ok = e < 6 * RX * 2 && z >= 0 && z < D && yy >= 0 && yy < H && xx >= 0 && xx < W &&
+                                cib * 16 + half * 8 < CIN;
+                r[q] = ok ? *reinterpret_cast<const uint4*>(X + ((static_cast<long long>(z) * H + yy) * W + xx) * CIN +
+                                                            cib * 16 + half * 8)
+                          : uint4{0u, 0u, 0u, 0u};
+            }
+        };
+        auto store_x = [&](int z, const uint4* r) {
+            uint16_t* p = lds + ((z + 3) % 3) * kPlane;
+#pragma unroll
+            for (int q = 0; q < NXP; q++) {
+                const int e = q * kNetThreads + tid;
+                if (e < 6 * RX * 2) *reinterpret_cast<uint4*>(p + e * 8) = r[q];
+            }
+        };
+        auto load_g = [&](int z, uint4* r) {
+#pragma unroll
+            for (int q = 0; q < NGP; q++) {
+                const int e = q * kNetThreads + tid;
+                const int half = e & 1, vox = e >> 1, row = vox / XT, xx = x0 + vox - row * XT, yy = y0 + row;
+                const bool ok = z < z1 && yy < H && xx < W;
+                r[q] = ok ? *reinterpret_cast<const uint4*>(G + ((static_cast<long long>(z) * H + yy) * W + xx) * COUT +
+                                                            cob * 16 + half * 8)
+                          : uint4{0u, 0u, 0u, 0u};
+            }
+        };
+        uint4 xr[NXP], gr[NGP], xa[NXP];
+        load_x(z0 - 1, xr);
+        load_x(z0, xa);
+        __syncthreads();                       // the previous unit's last step has read the buffers
+        store_x(z0 - 1, xr);
+        store_x(z0, xa);
+        load_x(z0 + 1, xr);
+        load_g(z0, gr);
+        for (int z = z0; z < z1; z++) {
+            store_x(z + 1, xr);                // the slot of plane z - 2, last read before the barrier below
+#pragma unroll
+            for (int q = 0; q < NGP; q++) *reinterpret_cast<uint4*>(gl + (q * kNetThreads + tid) * 8) = gr[q];
+            __syncthreads();
+            if (z + 1 < z1) {
+                load_x(z + 2, xr);
+                load_g(z + 1, gr);
             }
 #pragma unroll
-            for (int dz = -1; dz <= 1; dz++) {
-                const int zz = z + dz;
-                if (zz < 0 || zz >= D) continue;
+            for (int ks = 0; ks < XT / 32; ks++) {
+                const bf16x8 a = lds_tr8(gl + (wave * XT + ks * 32) * 16 + frag, 256);
 #pragma unroll
-                for (int dy = -1; dy <= 1; dy++) {
-                    const int yy = y + dy;
-                    if (yy < 0 || yy >= H) continue;
-                    const long long srow = (static_cast<long long>(zz) * H + yy) * W;
+                for (int dz = 0; dz < 3; dz++) {
+                    const uint16_t* pl = lds + ((z + 2 + dz) % 3) * kPlane;          // plane z - 1 + dz
 #pragma unroll
-                    for (int dx = -1; dx <= 1; dx++) {
-                        bf16x4 b;
+                    for (int dy = 0; dy < 3; dy++)
 #pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            const int xv = xs + kq * 4 + e;
-                            const int xx = xv + dx;
-                            const bool ok = ci_ok && xv < W && xx >= 0 && xx < W;
-                            b[e] = ok ? static_cast<short>(X[(srow + xx) * CIN + cib * 16 + i]) : short(0);
+                        for (int dx = 0; dx < 3; dx++) {
+                            const bf16x8 b = lds_tr8(pl + ((wave + dy) * RX + ks * 32 + dx) * 16 + frag, 256);
+                            const int tap = dz * 9 + dy * 3 + dx;
+                            acc[tap] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[tap], 0, 0, 0);
                         }
-                        const int tap = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1);
-                        acc[tap] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[tap], 0, 0, 0);
-                    }
                 }
             }
+            __syncthreads();
         }
     }
-    if (!ci_ok) return;
+    // the four waves' accumulators, added in wave order (each thread owns 27 x 4 / 4 sums)
+    float* red = reinterpret_cast<float*>(lds);
+    for (int w = 0; w < 4; w++) {
+        if (wave == w) {
 #pragma unroll
-    for (int t = 0; t < 27; t++)
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            P[((static_cast<long long>(chunk) * 27 + t) * COUT + cob * 16 + kq * 4 + e) * CIN + cib * 16 + i] = acc[t][e];
+            for (int t = 0; t < 27; t++) {
+                floatx4* p = reinterpret_cast<floatx4*>(red) + t * 64 + lane;
+                *p = w == 0 ? acc[t] : *p + acc[t];
+            }
+        }
+        __syncthreads();
+    }
+    // red[(t * 64 + l) * 4 + e] is row co = 4 (l / 16) + e, column ci = l % 16 of tap t
+    for (int q = tid; q < 27 * 256; q += kNetThreads) {
+        const int t = q >> 8, co = (q >> 4) & 15, ci = q & 15;
+        if (cib * 16 + ci < CIN)
+            P[((static_cast<long long>(blockIdx.x) * 27 + t) * COUT + cob * 16 + co) * CIN + cib * 16 + ci] =
+                red[(t * 64 + (co >> 2) * 16 + ci) * 4 + (co & 3)];
+    }
 }
 
-// grad[idx] = sum over chunks in chunk order (deterministic)
-__global__ __launch_bounds__(kNetThreads) void k_chunk_sum(const float* __restrict__ P, int nchunks, int n,
+// grad[idx] = sum over chunks, in a fixed order (deterministic): 64 entries per block, its 16
+// waves each sum a contiguous run of chunks in chunk order (eight loads in flight), the runs are
+// added in run order. One lane per entry over all chunks left 27 blocks waiting on one load at a
+// time: 100 us a layer on average, now 4.
+constexpr int kSumThreads = 1024;
+__global__ __launch_bounds__(kSumThreads) void k_chunk_sum(const float* __restrict__ P, int nchunks, int n,
                                                           float* __restrict__ grad) {
-    const int idx = blockIdx.x * kNetThreads + threadIdx.x;
-    if (idx >= n) return;
+    __shared__ float part[kSumThreads];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int idx = blockIdx.x * 64 + lane;
+    const int per = (nchunks + 15) / 16;
+    const int c0 = wave * per, c1 = (c0 + per < nchunks) ? c0 + per : nchunks;
     float s = 0.f;
-    for (int c = 0; c < nchunks; c++) s += P[static_cast<long long>(c) * n + idx];
-    grad[idx] = s;
+    if (idx < n) {
+        for (int c = c0; c < c1; c += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = c + u < c1 ? P[static_cast<long long>(c + u) * n + idx] : 0.f;
+#pragma unroll
+            for (int u = 0; u < 8; u++) s += v[u];
+        }
+    }
+    part[threadIdx.x] = s;
+    __syncthreads();
+    if (wave == 0 && idx < n) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < 16; w++) t += part[w * 64 + lane];
+        grad[idx] = t;
+    }
 }
 
 // ------------------------------------------------------------------------------ resampling
@@ -1272,18 +1373,30 @@ void conv_any(hipStream_t sm, int cin, int cout, bool relu, const uint16_t* X, c
 int wgrad_any(dare_convnet* net, hipStream_t sm, int layer, const uint16_t* X, const uint16_t* G) {
     const int cin = kDefs[layer].cin, cout = kDefs[layer].cout, level = kDefs[layer].level;
     const int D = net->dims[0] >> level, H = net->dims[1] >> level, W = net->dims[2] >> level;
-    const int rows = D * H;
     const int pairs = std::max(1, cin / 16) * (cout / 16);
-    long long cap = std::min<long long>(512, kWpartFloats / (27LL * cin * cout));
-    cap = std::min<long long>(cap, std::max(1, 4096 / pairs));
-    const int chunks0 = static_cast<int>(std::max<long long>(1, std::min<long long>(rows, cap)));
-    const int rpc = (rows + chunks0 - 1) / chunks0;
-    const int nchunks = (rows + rpc - 1) / rpc;
-    dim3 grid((nchunks + 3) / 4, pairs);
-#define DARE_WG_CASE(CI, CO)                                                                              \
-    if (cin == CI && cout == CO)                                                                          \
-        hipLaunchKernelGGL((k_wgrad<CI, CO>), grid, dim3(kNetThreads), 0, sm, X, G, D, H, W, rpc, nchunks, \
-                           net->wpart);
+    const int n = 27 * cin * cout;
+    // tile of 64 or 32 voxels along x; planes per unit so that about two blocks per CU result
+    // (one leaves the staging latency bare, more only adds partials), and no more blocks than
+    // the partials' buffer holds
+    const int xt = W > 32 ? 64 : 32;
+    const int nxt = (W + xt - 1) / xt, nyt = (H + 3) / 4;
+    const long long cols = static_cast<long long>(nxt) * nyt;
+    const long long want = std::max<long long>(1, 512 / pairs);
+    const long long nz = std::min<long long>(D, std::max<long long>(1, want / cols));
+    const int zb = static_cast<int>((D + nz - 1) / nz);
+    const int nunits = static_cast<int>(cols * ((D + zb - 1) / zb));
+    const int nchunks = static_cast<int>(
+        std::min<long long>(nunits, std::min<long long>(2 * want, std::max<long long>(1, kWpartFloats / n))));
+    const dim3 grid(nchunks, pairs);
+#define DARE_WG_CASE(CI, CO)                                                                                   \
+    if (cin == CI && cout == CO) {                                                                             \
+        if (xt == 64)                                                                                          \
+            hipLaunchKernelGGL((k_wgrad<CI, CO, 64>), grid, dim3(kNetThreads), 0, sm, X, G, D, H, W, zb, nxt,  \
+                               nyt, nunits, net->wpart);                                                       \
+        else                                                                                                   \
+            hipLaunchKernelGGL((k_wgrad<CI, CO, 32>), grid, dim3(kNetThreads), 0, sm, X, G, D, H, W, zb, nxt,  \
+                               nyt, nunits, net->wpart);                                                       \
+    }
     DARE_WG_CASE(kInChannels, 16)
     DARE_WG_CASE(16, 16)
     DARE_WG_CASE(16, 32)
@@ -1293,9 +1406,8 @@ int wgrad_any(dare_convnet* net, hipStream_t sm, int layer, const uint16_t* X, c
     DARE_WG_CASE(64, 32)
     DARE_WG_CASE(64, 64)
 #undef DARE_WG_CASE
-    const int n = 27 * cin * cout;
-    hipLaunchKernelGGL(k_chunk_sum, dim3((n + kNetThreads - 1) / kNetThreads), dim3(kNetThreads), 0, sm, net->wpart,
-                       nchunks, n, net->g + net->off[layer]);
+    hipLaunchKernelGGL(k_chunk_sum, dim3((n + 63) / 64), dim3(kSumThreads), 0, sm, net->wpart, nchunks, n,
+                       net->g + net->off[layer]);
     return DARE_OK;
 }
 

@@ -200,6 +200,41 @@ def test_backward_matches_oracle(ctx, rng):
     net.close()
 
 
+@pytest.mark.parametrize("box", [[4, 8, 36], [8, 20, 68], [4, 1092, 4], [12, 4, 132]])
+def test_weight_gradient_tiles_match_oracle(ctx, rng, box):
+    """Weight gradients where the tiling of k_wgrad has edges: x tiles with a remainder (36, 68,
+    132 against tiles of 64 and 32), rows that do not fill a tile, one-plane levels, and (1092
+    rows: 69 row tiles of the coarsest 64-channel layers against 64 blocks) blocks that take
+    more than one unit. The oracle's gradients from the device's own activations, so only the
+    FP32 sums of BF16 products differ: the bar is the data gradient's BF16 rounding, as in
+    test_backward_matches_oracle."""
+    import torch
+    net = WarmStartNet(ctx, box, in_channels=3, seed=7)
+    w = he_init(3, seed=7, out_scale=1.0)
+    net.set_params(w)
+    g = da.Grid.make(box, size=[1, 1, 1], ghost=2)
+    dev, _ = fields(rng, box)
+    net.pack(g, dev[0], dev[1], dev[2], 0.7)
+    net.forward()
+    xt = torch.from_numpy(rng.normal(size=int(np.prod(box)))).cuda()
+    net.loss(g, dev[2], xt)
+    net.backward()
+    ctx.synchronize()
+    ptr, _ = net.tensors()
+    x0 = d2h_bf16(ctx, ptr["x0"], box + [8])
+    W = cn.split(cn.bf16(w))
+    _, A = cn.forward(x0, W, exact=False)
+    dout = d2h_bf16(ctx, ptr["dout"], box + [16])[..., 0]
+    dW = cn.backward(dout, A, W, exact=False)
+    got = cn.split(net.grads().astype(np.float64))
+    for l in range(11):
+        e, a = dW[l], got[l]
+        if l == 10:                                   # only output channel 0 carries a gradient
+            e, a = e[:, :1], a[:, :1]
+        assert rel(a, e) <= 3e-2, (l, rel(a, e))
+    net.close()
+
+
 def test_training_reduces_loss(ctx, rng):
     """Adam on one fixed sample: the loss falls to a fraction of its start."""
     import torch
