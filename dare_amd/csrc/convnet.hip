@@ -642,13 +642,16 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_sub(const uint16_t* __rest
 // 16 + kq * 4 + j of the second stand for voxel (kq, j) and 16 + (kq, j) of the step in both
 // operands, which keeps each read 512 contiguous bytes (no bank conflicts).
 //
-// Block = one 16 x 16 (co, ci) pair of a unit: 4 rows (one per wave) x XT voxels along x,
-// marching along z with a ring of three input planes; the next plane is loaded into registers
-// while this one is computed. A block takes units blockIdx.x, + gridDim.x, ... and keeps its 27
-// accumulators over all of them; its four waves are summed through LDS, so a chunk is a block.
-// What bounds it: 54 fragment reads feed 27 matrix instructions, so the LDS reads set the rate
-// of the inner loop (about half the matrix peak); at 64^3 the staging latency does. 16 -> 16
-// channels at 64^3: 219 -> 18 us (the earlier form read G and X as single 2-byte global loads).
+// Block = one 16 x 16 (co, ci) pair of a unit: 4 rows x XT voxels along x, marching along z with
+// a ring of three input planes; the next plane is loaded into registers while this one is
+// computed. Each of the four waves owns seven of the 27 taps over all four rows, so no sum is
+// shared between waves: 28 accumulator registers instead of 108 and no block reduction, for
+// 14 % more fragment reads than a row per wave (which also left one block fewer per CU).
+// A block takes units blockIdx.x, + gridDim.x, ... and keeps its accumulators over all of them,
+// so a chunk is a block.
+// What bounds it: 64 fragment reads of 16 bytes a lane feed 56 matrix instructions, so the LDS
+// reads set the rate of the inner loop; at 64^3 the staging latency does. 16 -> 16 channels at
+// 64^3: 219 us (single 2-byte global loads) -> 16 (a row per wave) -> 11 us.
 typedef short bf16x4s __attribute__((ext_vector_type(4)));
 
 __device__ inline bf16x8 lds_tr8(const uint16_t* p, int second) {
@@ -668,19 +671,25 @@ __global__ __launch_bounds__(kNetThreads) void k_wgrad(const uint16_t* __restric
     constexpr int CB = CIN >= 16 ? CIN / 16 : 1;                // an 8-channel input is one half block
     constexpr int RX = XT + 2;                                  // staged voxels of an input row
     constexpr int kPlane = 6 * RX * 16;                         // elements of a staged input plane
-    constexpr int kStage = 3 * kPlane + 4 * XT * 16, kRed = 27 * 256 * 2;
-    constexpr int kLds = kStage > kRed ? kStage : kRed;         // the block reduction reuses the staging buffer
+    constexpr int kTaps = 7;                                    // taps 7 wave .. 7 wave + 6 (the last has 6)
     constexpr int NXP = (6 * RX * 2 + kNetThreads - 1) / kNetThreads;      // 16-byte loads per thread: input plane
     constexpr int NGP = (4 * XT * 2) / kNetThreads;                        // ... and gradient rows
-    __shared__ __align__(16) uint16_t lds[kLds];
+    __shared__ __align__(16) uint16_t lds[3 * kPlane + 4 * XT * 16];
     uint16_t* gl = lds + 3 * kPlane;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cob = blockIdx.y / CB, cib = blockIdx.y % CB;
     const int kq = lane >> 4, i = lane & 15;
     const int frag = ((kq * 4 + (i >> 2)) * 16) + (i & 3) * 4;  // this lane's element offset in a fragment
-    floatx4 acc[27];
+    floatx4 acc[kTaps];
 #pragma unroll
-    for (int t = 0; t < 27; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < kTaps; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    int tdz[kTaps], toff[kTaps];     // plane and in-plane offset of the wave's taps (a 28th repeats the 27th)
+#pragma unroll
+    for (int t = 0; t < kTaps; t++) {
+        const int tap = wave * kTaps + t < 27 ? wave * kTaps + t : 26;
+        tdz[t] = tap / 9;
+        toff[t] = ((tap / 3) % 3 * RX + tap % 3) * 16;
+    }
 
     for (int unit = blockIdx.x; unit < nunits; unit += gridDim.x) {
         const int xt = unit % nxt, yt = (unit / nxt) % nyt, zt = unit / (nxt * nyt);
@@ -735,56 +744,57 @@ __global__ __launch_bounds__(kNetThreads) void k_wgrad(const uint16_t* __restric
                 load_x(z + 2, xr);
                 load_g(z + 1, gr);
             }
+            const uint16_t* base[kTaps];
 #pragma unroll
-            for (int ks = 0; ks < XT / 32; ks++) {
-                const bf16x8 a = lds_tr8(gl + (wave * XT + ks * 32) * 16 + frag, 256);
+            for (int t = 0; t < kTaps; t++) base[t] = lds + ((z + 2 + tdz[t]) % 3) * kPlane + toff[t] + frag;
 #pragma unroll
-                for (int dz = 0; dz < 3; dz++) {
-                    const uint16_t* pl = lds + ((z + 2 + dz) % 3) * kPlane;          // plane z - 1 + dz
+            for (int row = 0; row < 4; row++)
 #pragma unroll
-                    for (int dy = 0; dy < 3; dy++)
+                for (int ks = 0; ks < XT / 32; ks++) {
+                    const bf16x8 a = lds_tr8(gl + (row * XT + ks * 32) * 16 + frag, 256);
 #pragma unroll
-                        for (int dx = 0; dx < 3; dx++) {
-                            const bf16x8 b = lds_tr8(pl + ((wave + dy) * RX + ks * 32 + dx) * 16 + frag, 256);
-                            const int tap = dz * 9 + dy * 3 + dx;
-                            acc[tap] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[tap], 0, 0, 0);
-                        }
+                    for (int t = 0; t < kTaps; t++) {
+                        const bf16x8 b = lds_tr8(base[t] + (row * RX + ks * 32) * 16, 256);
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
+                    }
                 }
-            }
             __syncthreads();
         }
     }
-    // the four waves' accumulators, added in wave order (each thread owns 27 x 4 / 4 sums)
-    float* red = reinterpret_cast<float*>(lds);
-    for (int w = 0; w < 4; w++) {
-        if (wave == w) {
+    if (cib * 16 + i >= CIN) return;
 #pragma unroll
-            for (int t = 0; t < 27; t++) {
-                floatx4* p = reinterpret_cast<floatx4*>(red) + t * 64 + lane;
-                *p = w == 0 ? acc[t] : *p + acc[t];
-            }
+    for (int t = 0; t < kTaps; t++) {
+        const int tap = wave * kTaps + t;
+        if (tap < 27) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                P[((static_cast<long long>(blockIdx.x) * 27 + tap) * COUT + cob * 16 + kq * 4 + e) * CIN + cib * 16 + i] =
+                    acc[t][e];
         }
-        __syncthreads();
-    }
-    // red[(t * 64 + l) * 4 + e] is row co = 4 (l / 16) + e, column ci = l % 16 of tap t
-    for (int q = tid; q < 27 * 256; q += kNetThreads) {
-        const int t = q >> 8, co = (q >> 4) & 15, ci = q & 15;
-        if (cib * 16 + ci < CIN)
-            P[((static_cast<long long>(blockIdx.x) * 27 + t) * COUT + cob * 16 + co) * CIN + cib * 16 + ci] =
-                red[(t * 64 + (co >> 2) * 16 + ci) * 4 + (co & 3)];
     }
 }
 
-// grad[idx] = sum over chunks, in a fixed order (deterministic): 64 entries per block, its 16
-// waves each sum a contiguous run of chunks in chunk order (eight loads in flight), the runs are
-// added in run order. One lane per entry over all chunks left 27 blocks waiting on one load at a
-// time: 100 us a layer on average, now 4.
-constexpr int kSumThreads = 1024;
-__global__ __launch_bounds__(kSumThreads) void k_chunk_sum(const float* __restrict__ P, int nchunks, int n,
-                                                          float* __restrict__ grad) {
+// grad[idx] = sum over chunks, in a fixed order (deterministic), for every layer whose partials
+// wait in the buffer (one launch for up to kSumLayers of them: 4 us each on their own): 64 entries
+// per block, its 16 waves each sum a contiguous run of chunks in chunk order (eight loads in
+// flight), the runs are added in run order. One lane per entry over all chunks left 27 blocks
+// waiting on one load at a time, 100 us a layer.
+constexpr int kSumThreads = 1024, kSumLayers = 4;
+struct ChunkSums {
+    const float* P[kSumLayers];
+    float* grad[kSumLayers];
+    int nchunks[kSumLayers], n[kSumLayers];
+    int block0[kSumLayers + 1];      // first block of each layer
+    int count;
+};
+__global__ __launch_bounds__(kSumThreads) void k_chunk_sum(ChunkSums S) {
     __shared__ float part[kSumThreads];
+    int l = 0;
+    while (l + 1 < S.count && static_cast<int>(blockIdx.x) >= S.block0[l + 1]) l++;
+    const float* __restrict__ P = S.P[l];
+    const int n = S.n[l], nchunks = S.nchunks[l];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int idx = blockIdx.x * 64 + lane;
+    const int idx = (static_cast<int>(blockIdx.x) - S.block0[l]) * 64 + lane;
     const int per = (nchunks + 15) / 16;
     const int c0 = wave * per, c1 = (c0 + per < nchunks) ? c0 + per : nchunks;
     float s = 0.f;
@@ -803,7 +813,7 @@ __global__ __launch_bounds__(kSumThreads) void k_chunk_sum(const float* __restri
         float t = 0.f;
 #pragma unroll
         for (int w = 0; w < 16; w++) t += part[w * 64 + lane];
-        grad[idx] = t;
+        S.grad[l][idx] = t;
     }
 }
 
@@ -1370,7 +1380,19 @@ void conv_any(hipStream_t sm, int cin, int cout, bool relu, const uint16_t* X, c
 #undef DARE_CONV_CASE
 }
 
-int wgrad_any(dare_convnet* net, hipStream_t sm, int layer, const uint16_t* X, const uint16_t* G) {
+// Partials of several layers share the buffer until k_chunk_sum runs over them.
+struct PendingSums {
+    ChunkSums S{};
+    long long used = 0;              // floats of the buffer in use
+    void flush(hipStream_t sm) {
+        if (S.count)
+            hipLaunchKernelGGL(k_chunk_sum, dim3(S.block0[S.count]), dim3(kSumThreads), 0, sm, S);
+        S = ChunkSums{};
+        used = 0;
+    }
+};
+
+void wgrad_any(dare_convnet* net, hipStream_t sm, PendingSums* sums, int layer, const uint16_t* X, const uint16_t* G) {
     const int cin = kDefs[layer].cin, cout = kDefs[layer].cout, level = kDefs[layer].level;
     const int D = net->dims[0] >> level, H = net->dims[1] >> level, W = net->dims[2] >> level;
     const int pairs = std::max(1, cin / 16) * (cout / 16);
@@ -1388,14 +1410,17 @@ int wgrad_any(dare_convnet* net, hipStream_t sm, int layer, const uint16_t* X, c
     const int nchunks = static_cast<int>(
         std::min<long long>(nunits, std::min<long long>(2 * want, std::max<long long>(1, kWpartFloats / n))));
     const dim3 grid(nchunks, pairs);
+    const long long need = static_cast<long long>(nchunks) * n;
+    if (sums->S.count == kSumLayers || sums->used + need > kWpartFloats) sums->flush(sm);
+    float* part = net->wpart + sums->used;
 #define DARE_WG_CASE(CI, CO)                                                                                   \
     if (cin == CI && cout == CO) {                                                                             \
         if (xt == 64)                                                                                          \
             hipLaunchKernelGGL((k_wgrad<CI, CO, 64>), grid, dim3(kNetThreads), 0, sm, X, G, D, H, W, zb, nxt,  \
-                               nyt, nunits, net->wpart);                                                       \
+                               nyt, nunits, part);                                                             \
         else                                                                                                   \
             hipLaunchKernelGGL((k_wgrad<CI, CO, 32>), grid, dim3(kNetThreads), 0, sm, X, G, D, H, W, zb, nxt,  \
-                               nyt, nunits, net->wpart);                                                       \
+                               nyt, nunits, part);                                                             \
     }
     DARE_WG_CASE(kInChannels, 16)
     DARE_WG_CASE(16, 16)
@@ -1406,9 +1431,14 @@ int wgrad_any(dare_convnet* net, hipStream_t sm, int layer, const uint16_t* X, c
     DARE_WG_CASE(64, 32)
     DARE_WG_CASE(64, 64)
 #undef DARE_WG_CASE
-    hipLaunchKernelGGL(k_chunk_sum, dim3((n + 63) / 64), dim3(kSumThreads), 0, sm, net->wpart, nchunks, n,
-                       net->g + net->off[layer]);
-    return DARE_OK;
+    ChunkSums& S = sums->S;
+    S.P[S.count] = part;
+    S.grad[S.count] = net->g + net->off[layer];
+    S.nchunks[S.count] = nchunks;
+    S.n[S.count] = n;
+    S.block0[S.count + 1] = S.block0[S.count] + (n + 63) / 64;
+    S.count++;
+    sums->used += need;
 }
 
 FieldGeo field_geo(const dare_grid* g, const int32_t* crop, int cf) {
@@ -1744,56 +1774,58 @@ int dare_conv_net_bwd(dare_ctx* ctx, dare_convnet* net) {
     const int* d = net->dims;
     const long long V0 = level_voxels(d, 0), V1 = level_voxels(d, 1), V2 = level_voxels(d, 2);
     const uint16_t* WB = net->wb;
+    PendingSums sums;
     const long long* o = net->off;
     // L11 (no ReLU): dd1 = conv_bwd(dout)
-    wgrad_any(net, sm, 10, net->d1, net->dout);
+    wgrad_any(net, sm, &sums, 10, net->d1, net->dout);
     conv_any(sm, 16, 16, false, net->dout, WB + o[10], net->t0a, d, 0);            // dd1
     hipLaunchKernelGGL(k_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->t0a, net->d1, net->t0b, V0 * 16);
     // L10: g10 = t0b
-    wgrad_any(net, sm, 9, net->s1, net->t0b);
+    wgrad_any(net, sm, &sums, 9, net->s1, net->t0b);
     conv_any(sm, 16, 16, false, net->t0b, WB + o[9], net->t0c, d, 0);              // ds1 (kept)
     hipLaunchKernelGGL(k_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->t0c, net->a9, net->t0a, V0 * 16);
     // L9: g9 = t0a (u1 = up(d2), read fused by the forward pass, materialized here)
     hipLaunchKernelGGL(k_up, dim3(ew_grid(V0 * 32)), dim3(kNetThreads), 0, sm, net->d2, net->u1, 32, d[0], d[1], d[2]);
-    wgrad_any(net, sm, 8, net->u1, net->t0a);
+    wgrad_any(net, sm, &sums, 8, net->u1, net->t0a);
     conv_any(sm, 16, 32, false, net->t0a, WB + o[8], net->t0w, d, 0);              // du1 (32 ch)
     hipLaunchKernelGGL(k_up_bwd_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->t0w, net->d2, net->h1a,
                        32, d[0] >> 1, d[1] >> 1, d[2] >> 1);                       // g8
     // L8
-    wgrad_any(net, sm, 7, net->s2, net->h1a);
+    wgrad_any(net, sm, &sums, 7, net->s2, net->h1a);
     conv_any(sm, 32, 32, false, net->h1a, WB + o[7], net->h1b, d, 1);              // ds2 (kept)
     hipLaunchKernelGGL(k_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->h1b, net->a7, net->h1c, V1 * 32);
     // L7: g7 = h1c (u2 = up(e3), as u1)
     hipLaunchKernelGGL(k_up, dim3(ew_grid(V1 * 64)), dim3(kNetThreads), 0, sm, net->e3, net->u2, 64, d[0] >> 1,
                        d[1] >> 1, d[2] >> 1);
-    wgrad_any(net, sm, 6, net->u2, net->h1c);
+    wgrad_any(net, sm, &sums, 6, net->u2, net->h1c);
     conv_any(sm, 32, 64, false, net->h1c, WB + o[6], net->h1w, d, 1);              // du2 (64 ch)
     hipLaunchKernelGGL(k_up_bwd_mask, dim3(ew_grid(V2 * 64)), dim3(kNetThreads), 0, sm, net->h1w, net->e3, net->q2a,
                        64, d[0] >> 2, d[1] >> 2, d[2] >> 2);                       // g6
     // L6
-    wgrad_any(net, sm, 5, net->a5, net->q2a);
+    wgrad_any(net, sm, &sums, 5, net->a5, net->q2a);
     conv_any(sm, 64, 64, false, net->q2a, WB + o[5], net->q2b, d, 2);              // da5
     hipLaunchKernelGGL(k_mask, dim3(ew_grid(V2 * 64)), dim3(kNetThreads), 0, sm, net->q2b, net->a5, net->q2a, V2 * 64);
     // L5: g5 = q2a
-    wgrad_any(net, sm, 4, net->p2, net->q2a);
+    wgrad_any(net, sm, &sums, 4, net->p2, net->q2a);
     conv_any(sm, 64, 32, false, net->q2a, WB + o[4], net->q2b, d, 2);              // dp2 (32 ch, quarter)
     hipLaunchKernelGGL(k_pool_bwd_add_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->q2b, net->h1b,
                        net->e2, net->h1a, 32, d[0] >> 1, d[1] >> 1, d[2] >> 1);     // g4
     // L4
-    wgrad_any(net, sm, 3, net->a3, net->h1a);
+    wgrad_any(net, sm, &sums, 3, net->a3, net->h1a);
     conv_any(sm, 32, 32, false, net->h1a, WB + o[3], net->h1c, d, 1);              // da3
     hipLaunchKernelGGL(k_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->h1c, net->a3, net->h1a, V1 * 32);
     // L3: g3 = h1a
-    wgrad_any(net, sm, 2, net->p1, net->h1a);
+    wgrad_any(net, sm, &sums, 2, net->p1, net->h1a);
     conv_any(sm, 32, 16, false, net->h1a, WB + o[2], net->h1c, d, 1);              // dp1 (16 ch, half)
     hipLaunchKernelGGL(k_pool_bwd_add_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->h1c, net->t0c,
                        net->e1, net->t0a, 16, d[0], d[1], d[2]);                   // g2
     // L2
-    wgrad_any(net, sm, 1, net->a1, net->t0a);
+    wgrad_any(net, sm, &sums, 1, net->a1, net->t0a);
     conv_any(sm, 16, 16, false, net->t0a, WB + o[1], net->t0b, d, 0);              // da1
     hipLaunchKernelGGL(k_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->t0b, net->a1, net->t0a, V0 * 16);
     // L1: g1 = t0a
-    wgrad_any(net, sm, 0, net->x0, net->t0a);
+    wgrad_any(net, sm, &sums, 0, net->x0, net->t0a);
+    sums.flush(sm);
     DARE_LAUNCH_CHECK();
     (void)V2;
     return DARE_OK;
