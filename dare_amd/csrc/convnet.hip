@@ -77,14 +77,27 @@ __device__ inline bf16x8 load8(const uint16_t* p, bool ok) {
     return __builtin_bit_cast(bf16x8, u);
 }
 
+// four BF16 gradients where the activations at y are positive, 0 elsewhere (ReLU backward)
+__device__ inline uint2 relu_mask(uint2 g, const uint16_t* y) {
+    const uint2 yv = *reinterpret_cast<const uint2*>(y);
+    auto pass = [](uint32_t h) { return bf2f(static_cast<uint16_t>(h)) > 0.f; };
+    uint2 o;
+    o.x = (pass(yv.x & 0xffffu) ? g.x & 0xffffu : 0u) | (pass(yv.x >> 16) ? g.x & 0xffff0000u : 0u);
+    o.y = (pass(yv.y & 0xffffu) ? g.y & 0xffffu : 0u) | (pass(yv.y >> 16) ? g.y & 0xffff0000u : 0u);
+    return o;
+}
+
 // Output-channel blocks of 16 per work-group (a group stages its slice of the weights).
 template <int COUT>
 constexpr int conv_nbb() { return COUT / 16 < 2 ? COUT / 16 : 2; }
 
 // Fusions of k_conv (MODE bits): kConvUp -- the input is the half-resolution tensor and the
 // conv reads its nearest-neighbour upsampling (staging fetches each voxel's parent); kConvAdd --
-// the epilogue also writes Y2 = bf16(Y + E) (the decoder's skip connection, as k_add).
-constexpr int kConvUp = 1, kConvAdd = 2;
+// the epilogue also writes Y2 = bf16(Y + E) (the decoder's skip connection, as k_add); kConvMask
+// -- the ReLU backward of the layer below: Y2 = Y where E > 0, else 0, and Y itself only if it is
+// not NULL (the skip gradients, which two consumers read). The mask as a pass of its own over the
+// written gradient took 3-8 us per layer at 64^3.
+constexpr int kConvUp = 1, kConvAdd = 2, kConvMask = 4;
 
 template <int CIN, int COUT, bool RELU, int OUT, int NSEG, int MODE = 0>
 __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Wt,
@@ -210,7 +223,8 @@ __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict
                 uint2 pk;
                 pk.x = static_cast<uint32_t>(b[0]) | (static_cast<uint32_t>(b[1]) << 16);
                 pk.y = static_cast<uint32_t>(b[2]) | (static_cast<uint32_t>(b[3]) << 16);
-                *reinterpret_cast<uint2*>(Y + at) = pk;
+                if (!(MODE & kConvMask) || Y) *reinterpret_cast<uint2*>(Y + at) = pk;
+                if constexpr ((MODE & kConvMask) != 0) *reinterpret_cast<uint2*>(Y2 + at) = relu_mask(pk, E + at);
                 if constexpr ((MODE & kConvAdd) != 0) {
                     const uint2 ev = *reinterpret_cast<const uint2*>(E + at);
                     const uint16_t e[4] = {static_cast<uint16_t>(ev.x & 0xffffu), static_cast<uint16_t>(ev.x >> 16),
@@ -380,7 +394,8 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_zm(const uint16_t* __restr
                     uint2 pk;
                     pk.x = static_cast<uint32_t>(b[0]) | (static_cast<uint32_t>(b[1]) << 16);
                     pk.y = static_cast<uint32_t>(b[2]) | (static_cast<uint32_t>(b[3]) << 16);
-                    *reinterpret_cast<uint2*>(Y + at) = pk;
+                    if (!(MODE & kConvMask) || Y) *reinterpret_cast<uint2*>(Y + at) = pk;
+                    if constexpr ((MODE & kConvMask) != 0) *reinterpret_cast<uint2*>(Y2 + at) = relu_mask(pk, E + at);
                     if constexpr ((MODE & kConvAdd) != 0) {
                         const uint2 ev = *reinterpret_cast<const uint2*>(E + at);
                         const uint16_t e[4] = {static_cast<uint16_t>(ev.x & 0xffffu), static_cast<uint16_t>(ev.x >> 16),
@@ -939,17 +954,6 @@ __global__ __launch_bounds__(kNetThreads) void k_add(const uint16_t* __restrict_
     }
 }
 
-__global__ __launch_bounds__(kNetThreads) void k_mask(const uint16_t* __restrict__ g, const uint16_t* __restrict__ y,
-                                                     uint16_t* __restrict__ out, long long n) {
-    DARE_EW8_LOOP(n / 8) {
-        const Bf8 gv = ld8(g, q), yv = ld8(y, q);
-        Bf8 o;
-#pragma unroll
-        for (int e = 0; e < 8; e++) o.h[e] = bf2f(yv.h[e]) > 0.f ? gv.h[e] : uint16_t(0);
-        st8(out, q, o);
-    }
-}
-
 // ------------------------------------------------------------------------------ solver side
 // Normalisation scales: s[0] = max|phi^n|, s[1] = max|phi^n - phi^{n-1}|,
 // s[2] = max|resid * resid_scale| over the cells of the box (block maxima, then one block);
@@ -1146,41 +1150,54 @@ __global__ __launch_bounds__(kNetThreads) void k_mse(FieldGeo F, const double* _
     }
 }
 
+// nblocks <= 1024 partials, sixteen per lane, all loads in flight at once (one thread adding them
+// one after the other waited out every load: 57 us)
 __global__ __launch_bounds__(64) void k_mse_finish(const double* __restrict__ part, int nblocks, long long n,
                                                   double* __restrict__ loss) {
-    if (threadIdx.x != 0) return;
+    double v[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) v[q] = q * 64 + static_cast<int>(threadIdx.x) < nblocks ? part[q * 64 + threadIdx.x] : 0.;
     double t = 0.;
-    for (int b = 0; b < nblocks; b++) t += part[b];
-    loss[0] = t / static_cast<double>(n);
+#pragma unroll
+    for (int q = 0; q < 16; q++) t += v[q];
+    t = wave_sum(t);
+    if (threadIdx.x == 0) loss[0] = t / static_cast<double>(n);
 }
 
 // ------------------------------------------------------------------------------ parameters
-// Adam (Kingma & Ba 2015) on the FP32 master weights of one layer, then the two BF16 copies:
-// forward [tap][co][ci] and data-backward [26 - tap][ci][co].
-__global__ __launch_bounds__(kNetThreads) void k_adam_cast(float* __restrict__ w, const float* __restrict__ g,
+// Adam (Kingma & Ba 2015) on the FP32 master weights, then the two BF16 copies: forward
+// [tap][co][ci] and data-backward [26 - tap][ci][co] of each layer. All layers in one launch
+// (eleven of 3 us each and their gaps otherwise).
+struct LayerTable {
+    int off[kLayers + 1], cin[kLayers], cout[kLayers];
+};
+__global__ __launch_bounds__(kNetThreads) void k_adam_cast(LayerTable L, float* __restrict__ w, const float* __restrict__ g,
                                                           float* __restrict__ m, float* __restrict__ v,
                                                           uint16_t* __restrict__ wf, uint16_t* __restrict__ wb,
-                                                          int cin, int cout, int update, float lr, float b1, float b2,
+                                                          int update, float lr, float b1, float b2,
                                                           float eps, float c1, float c2) {
-    const int n = 27 * cin * cout;
-    const int idx = blockIdx.x * kNetThreads + threadIdx.x;
-    if (idx >= n) return;
-    float wv = w[idx];
+    const int at = blockIdx.x * kNetThreads + threadIdx.x;
+    if (at >= L.off[kLayers]) return;
+    int l = 0;
+#pragma unroll
+    for (int q = 1; q < kLayers; q++) l = at >= L.off[q] ? q : l;
+    const int idx = at - L.off[l], cin = L.cin[l], cout = L.cout[l];
+    float wv = w[at];
     if (update) {
-        const float gv = g[idx];
-        const float mv = b1 * m[idx] + (1.f - b1) * gv;
-        const float vv = b2 * v[idx] + (1.f - b2) * gv * gv;
-        m[idx] = mv;
-        v[idx] = vv;
+        const float gv = g[at];
+        const float mv = b1 * m[at] + (1.f - b1) * gv;
+        const float vv = b2 * v[at] + (1.f - b2) * gv * gv;
+        m[at] = mv;
+        v[at] = vv;
         wv -= lr * (mv / c1) / (sqrtf(vv / c2) + eps);
-        w[idx] = wv;
+        w[at] = wv;
     }
     const int ci = idx % cin;
     const int co = (idx / cin) % cout;
     const int tap = idx / (cin * cout);
     const uint16_t h = f2bf(wv);
-    wf[idx] = h;
-    wb[((26 - tap) * cin + ci) * cout + co] = h;
+    wf[at] = h;
+    wb[L.off[l] + ((26 - tap) * cin + ci) * cout + co] = h;
 }
 
 inline unsigned ew_grid(long long n) {
@@ -1361,23 +1378,28 @@ void fold_sub_weights(hipStream_t sm, dare_convnet* net) {
     net->folded_stale = false;
 }
 
-// dispatch on (cin, cout) of the network's layers
-void conv_any(hipStream_t sm, int cin, int cout, bool relu, const uint16_t* X, const uint16_t* Wt, uint16_t* Y,
-              const int* d, int level) {
+// data gradient of a layer (no ReLU of its own), dispatch on (cin, cout) of the network's layers
+void conv_bwd(hipStream_t sm, int cin, int cout, const uint16_t* X, const uint16_t* Wt, uint16_t* Y, const int* d,
+              int level) {
 #define DARE_CONV_CASE(CI, CO)                                                     \
     if (cin == CI && cout == CO) {                                                 \
-        if (relu) conv<CI, CO, true, 0>(sm, X, Wt, Y, nullptr, d, level);          \
-        else conv<CI, CO, false, 0>(sm, X, Wt, Y, nullptr, d, level);              \
+        conv<CI, CO, false, 0>(sm, X, Wt, Y, nullptr, d, level);                   \
         return;                                                                    \
     }
-    DARE_CONV_CASE(16, 16)
     DARE_CONV_CASE(16, 32)
     DARE_CONV_CASE(32, 16)
-    DARE_CONV_CASE(32, 32)
     DARE_CONV_CASE(32, 64)
     DARE_CONV_CASE(64, 32)
-    DARE_CONV_CASE(64, 64)
 #undef DARE_CONV_CASE
+}
+
+// the same followed by the ReLU mask of the activations act below it, written to masked; raw
+// (may be NULL) receives the unmasked gradient
+void conv_bwd_mask(hipStream_t sm, int ch, const uint16_t* X, const uint16_t* Wt, uint16_t* raw, const uint16_t* act,
+                   uint16_t* masked, const int* d, int level) {
+    if (ch == 16) conv<16, 16, false, 0, kConvMask>(sm, X, Wt, raw, nullptr, d, level, act, masked);
+    else if (ch == 32) conv<32, 32, false, 0, kConvMask>(sm, X, Wt, raw, nullptr, d, level, act, masked);
+    else conv<64, 64, false, 0, kConvMask>(sm, X, Wt, raw, nullptr, d, level, act, masked);
 }
 
 // Partials of several layers share the buffer until k_chunk_sum runs over them.
@@ -1439,6 +1461,19 @@ void wgrad_any(dare_convnet* net, hipStream_t sm, PendingSums* sums, int layer, 
     S.block0[S.count + 1] = S.block0[S.count] + (n + 63) / 64;
     S.count++;
     sums->used += need;
+}
+
+void adam_cast(hipStream_t sm, dare_convnet* net, int update, float lr, float b1, float b2, float eps, float c1,
+               float c2) {
+    LayerTable L;
+    for (int l = 0; l < kLayers; l++) {
+        L.off[l] = static_cast<int>(net->off[l]);
+        L.cin[l] = kDefs[l].cin;
+        L.cout[l] = kDefs[l].cout;
+    }
+    L.off[kLayers] = static_cast<int>(net->nparams);
+    hipLaunchKernelGGL(k_adam_cast, dim3((L.off[kLayers] + kNetThreads - 1) / kNetThreads), dim3(kNetThreads), 0, sm, L,
+                       net->w, net->g, net->m, net->v, net->wf, net->wb, update, lr, b1, b2, eps, c1, c2);
 }
 
 FieldGeo field_geo(const dare_grid* g, const int32_t* crop, int cf) {
@@ -1591,13 +1626,7 @@ int dare_convnet_set_params(dare_ctx* ctx, dare_convnet* net, const float* host)
     DARE_HIP_TRY(hipMemcpy(net->m, z.data(), sizeof(float) * net->nparams, hipMemcpyHostToDevice));
     DARE_HIP_TRY(hipMemcpy(net->v, z.data(), sizeof(float) * net->nparams, hipMemcpyHostToDevice));
     net->adam_t = 0;
-    for (int l = 0; l < kLayers; l++) {
-        const int n = 27 * kDefs[l].cin * kDefs[l].cout;
-        hipLaunchKernelGGL(k_adam_cast, dim3((n + kNetThreads - 1) / kNetThreads), dim3(kNetThreads), 0, ctx->stream,
-                           net->w + net->off[l], net->g + net->off[l], net->m + net->off[l], net->v + net->off[l],
-                           net->wf + net->off[l], net->wb + net->off[l], kDefs[l].cin, kDefs[l].cout, 0, 0.f, 0.f, 0.f,
-                           0.f, 1.f, 1.f);
-    }
+    adam_cast(ctx->stream, net, 0, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
     net->folded_stale = true;
     DARE_LAUNCH_CHECK();
     return DARE_OK;
@@ -1778,53 +1807,47 @@ int dare_conv_net_bwd(dare_ctx* ctx, dare_convnet* net) {
     const long long* o = net->off;
     // L11 (no ReLU): dd1 = conv_bwd(dout)
     wgrad_any(net, sm, &sums, 10, net->d1, net->dout);
-    conv_any(sm, 16, 16, false, net->dout, WB + o[10], net->t0a, d, 0);            // dd1
-    hipLaunchKernelGGL(k_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->t0a, net->d1, net->t0b, V0 * 16);
+    conv_bwd_mask(sm, 16, net->dout, WB + o[10], nullptr, net->d1, net->t0b, d, 0);   // dd1, masked
     // L10: g10 = t0b
     wgrad_any(net, sm, &sums, 9, net->s1, net->t0b);
-    conv_any(sm, 16, 16, false, net->t0b, WB + o[9], net->t0c, d, 0);              // ds1 (kept)
-    hipLaunchKernelGGL(k_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->t0c, net->a9, net->t0a, V0 * 16);
+    conv_bwd_mask(sm, 16, net->t0b, WB + o[9], net->t0c, net->a9, net->t0a, d, 0);    // ds1 (t0c, kept)
     // L9: g9 = t0a (u1 = up(d2), read fused by the forward pass, materialized here)
     hipLaunchKernelGGL(k_up, dim3(ew_grid(V0 * 32)), dim3(kNetThreads), 0, sm, net->d2, net->u1, 32, d[0], d[1], d[2]);
     wgrad_any(net, sm, &sums, 8, net->u1, net->t0a);
-    conv_any(sm, 16, 32, false, net->t0a, WB + o[8], net->t0w, d, 0);              // du1 (32 ch)
+    conv_bwd(sm, 16, 32, net->t0a, WB + o[8], net->t0w, d, 0);              // du1 (32 ch)
     hipLaunchKernelGGL(k_up_bwd_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->t0w, net->d2, net->h1a,
                        32, d[0] >> 1, d[1] >> 1, d[2] >> 1);                       // g8
     // L8
     wgrad_any(net, sm, &sums, 7, net->s2, net->h1a);
-    conv_any(sm, 32, 32, false, net->h1a, WB + o[7], net->h1b, d, 1);              // ds2 (kept)
-    hipLaunchKernelGGL(k_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->h1b, net->a7, net->h1c, V1 * 32);
+    conv_bwd_mask(sm, 32, net->h1a, WB + o[7], net->h1b, net->a7, net->h1c, d, 1);    // ds2 (h1b, kept)
     // L7: g7 = h1c (u2 = up(e3), as u1)
     hipLaunchKernelGGL(k_up, dim3(ew_grid(V1 * 64)), dim3(kNetThreads), 0, sm, net->e3, net->u2, 64, d[0] >> 1,
                        d[1] >> 1, d[2] >> 1);
     wgrad_any(net, sm, &sums, 6, net->u2, net->h1c);
-    conv_any(sm, 32, 64, false, net->h1c, WB + o[6], net->h1w, d, 1);              // du2 (64 ch)
+    conv_bwd(sm, 32, 64, net->h1c, WB + o[6], net->h1w, d, 1);              // du2 (64 ch)
     hipLaunchKernelGGL(k_up_bwd_mask, dim3(ew_grid(V2 * 64)), dim3(kNetThreads), 0, sm, net->h1w, net->e3, net->q2a,
                        64, d[0] >> 2, d[1] >> 2, d[2] >> 2);                       // g6
     // L6
     wgrad_any(net, sm, &sums, 5, net->a5, net->q2a);
-    conv_any(sm, 64, 64, false, net->q2a, WB + o[5], net->q2b, d, 2);              // da5
-    hipLaunchKernelGGL(k_mask, dim3(ew_grid(V2 * 64)), dim3(kNetThreads), 0, sm, net->q2b, net->a5, net->q2a, V2 * 64);
-    // L5: g5 = q2a
-    wgrad_any(net, sm, &sums, 4, net->p2, net->q2a);
-    conv_any(sm, 64, 32, false, net->q2a, WB + o[4], net->q2b, d, 2);              // dp2 (32 ch, quarter)
-    hipLaunchKernelGGL(k_pool_bwd_add_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->q2b, net->h1b,
+    conv_bwd_mask(sm, 64, net->q2a, WB + o[5], nullptr, net->a5, net->q2b, d, 2);     // da5, masked
+    // L5: g5 = q2b
+    wgrad_any(net, sm, &sums, 4, net->p2, net->q2b);
+    conv_bwd(sm, 64, 32, net->q2b, WB + o[4], net->q2a, d, 2);              // dp2 (32 ch, quarter)
+    hipLaunchKernelGGL(k_pool_bwd_add_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->q2a, net->h1b,
                        net->e2, net->h1a, 32, d[0] >> 1, d[1] >> 1, d[2] >> 1);     // g4
     // L4
     wgrad_any(net, sm, &sums, 3, net->a3, net->h1a);
-    conv_any(sm, 32, 32, false, net->h1a, WB + o[3], net->h1c, d, 1);              // da3
-    hipLaunchKernelGGL(k_mask, dim3(ew_grid(V1 * 32)), dim3(kNetThreads), 0, sm, net->h1c, net->a3, net->h1a, V1 * 32);
-    // L3: g3 = h1a
-    wgrad_any(net, sm, &sums, 2, net->p1, net->h1a);
-    conv_any(sm, 32, 16, false, net->h1a, WB + o[2], net->h1c, d, 1);              // dp1 (16 ch, half)
-    hipLaunchKernelGGL(k_pool_bwd_add_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->h1c, net->t0c,
+    conv_bwd_mask(sm, 32, net->h1a, WB + o[3], nullptr, net->a3, net->h1c, d, 1);     // da3, masked
+    // L3: g3 = h1c
+    wgrad_any(net, sm, &sums, 2, net->p1, net->h1c);
+    conv_bwd(sm, 32, 16, net->h1c, WB + o[2], net->h1a, d, 1);              // dp1 (16 ch, half)
+    hipLaunchKernelGGL(k_pool_bwd_add_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->h1a, net->t0c,
                        net->e1, net->t0a, 16, d[0], d[1], d[2]);                   // g2
     // L2
     wgrad_any(net, sm, &sums, 1, net->a1, net->t0a);
-    conv_any(sm, 16, 16, false, net->t0a, WB + o[1], net->t0b, d, 0);              // da1
-    hipLaunchKernelGGL(k_mask, dim3(ew_grid(V0 * 16)), dim3(kNetThreads), 0, sm, net->t0b, net->a1, net->t0a, V0 * 16);
-    // L1: g1 = t0a
-    wgrad_any(net, sm, &sums, 0, net->x0, net->t0a);
+    conv_bwd_mask(sm, 16, net->t0a, WB + o[1], nullptr, net->a1, net->t0b, d, 0);     // da1, masked
+    // L1: g1 = t0b
+    wgrad_any(net, sm, &sums, 0, net->x0, net->t0b);
     sums.flush(sm);
     DARE_LAUNCH_CHECK();
     (void)V2;
@@ -1839,13 +1862,7 @@ int dare_conv_net_step(dare_ctx* ctx, dare_convnet* net, float lr, float beta1, 
     net->adam_t++;
     const float c1 = 1.f - std::pow(beta1, static_cast<float>(net->adam_t));
     const float c2 = 1.f - std::pow(beta2, static_cast<float>(net->adam_t));
-    for (int l = 0; l < kLayers; l++) {
-        const int n = 27 * kDefs[l].cin * kDefs[l].cout;
-        hipLaunchKernelGGL(k_adam_cast, dim3((n + kNetThreads - 1) / kNetThreads), dim3(kNetThreads), 0, ctx->stream,
-                           net->w + net->off[l], net->g + net->off[l], net->m + net->off[l], net->v + net->off[l],
-                           net->wf + net->off[l], net->wb + net->off[l], kDefs[l].cin, kDefs[l].cout, 1, lr, beta1,
-                           beta2, eps, c1, c2);
-    }
+    adam_cast(ctx->stream, net, 1, lr, beta1, beta2, eps, c1, c2);
     net->folded_stale = true;
     DARE_LAUNCH_CHECK();
     return DARE_OK;
