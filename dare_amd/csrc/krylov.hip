@@ -8,7 +8,7 @@
 //
 // Operators: a generic CSR traversal (grid-stride, one row per lane) and, for matrices
 // assembled from the 7-point structure, a tiled traversal of the slot-major diagonal view:
-// 64 (k) x 4 (j) x 16 (i) cells per work-group, the i-1/i/i+1 planes of x rolled through
+// up to 64 (k) x 4 (j) lanes x 16 (i) planes per work-group, the i-1/i/i+1 planes of x rolled through
 // registers, tiles ordered so that each XCD (blocks b = x mod 8) owns one contiguous slab.
 // Matrix values then stream fully coalesced and x is read from HBM about once per SpMV.
 #include <cmath>

@@ -16,7 +16,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kGridMax = 2048;      // work-groups of the grid-stride launches
-constexpr int kTileK = 64, kTileJ = 4, kTileI = 16;
+constexpr int kTileI = 16;          // planes per tile of the diagonal-view traversals
 constexpr int kXcd = 8;             // MI355X: 8 accelerator complex dies, blocks dealt round robin
 
 // Device-resident BiCGStab2 state (BiCGStab2.inl:180-196 scalars).
@@ -208,12 +208,23 @@ struct DiaOp {
     DiaView V;
     const VT* D;
     int tiles_k, tiles_j, tiles_i;
-    int tile_i;         // planes per tile (grown until the grid fits the reduction slots)
+    int lk_log2;        // lanes along k of a tile (16, 32 or 64); the other 256 / lanes go along j
+    int tile_i;         // planes per tile
     int per_xcd;        // tiles owned by each XCD (grid = kXcd * per_xcd)
-    int pair;           // cells per lane along k (2: tiles of 128 (k) x 4 (j), one component, n2 even)
+    int pair;           // cells per lane along k (2, or 4 for FP32: one component, n2 a multiple)
     bool sym = false;            // the view is exactly symmetric: the four-slot pair / quad traversals
 };
 
+// Tile of a work-group: 2^lk lanes along k (pair cells each) x 256 / 2^lk rows along j, marched
+// over tile_i planes. The lane split with the fewest idle lanes is taken (the widest on a tie):
+// at n2 = 64 the paired traversal fills 32 lanes, and 64 x 4 tiles left half of every wave idle.
+// tile_i starts at 16, which reads x about once, and is halved while the launch has too few
+// work-groups. A march is a chain of dependent loads, so small systems need them spread out:
+// 512 below a million rows (64^3: 15.2 us per sweep as 64 work-groups of 16 planes, 4.9 as 256,
+// 4.5 as 512). Above, a sweep is bound by the bytes in flight: one cell per lane needs four
+// work-groups per CU (145 x 128 x 121: 32.8 us as 640, 29.3 as 1216), two or four cells per lane
+// one (128^3: 24.4 us as 256, 25.8 as 1024, whose shorter marches read more of x twice).
+// tile_i grows past 16 only where the reduction slots would not hold the grid.
 template <typename VT>
 DiaOp<VT> make_dia(const DiaView& V, const VT* D, bool allow_pair = false) {
     DiaOp<VT> A;
@@ -221,17 +232,24 @@ DiaOp<VT> make_dia(const DiaView& V, const VT* D, bool allow_pair = false) {
     A.D = D;
     A.pair = (allow_pair && V.N == 1 && V.n[2] % 2 == 0) ? 2 : 1;
     if (allow_pair && std::is_same_v<VT, float> && V.N == 1 && V.n[2] % 4 == 0) A.pair = 4;
-    A.tiles_k = (V.n[2] + kTileK * A.pair - 1) / (kTileK * A.pair);
-    A.tiles_j = (V.n[1] + kTileJ - 1) / kTileJ;
-    A.tile_i = kTileI;
-    long long T = 0;
-    for (;;) {
-        A.tiles_i = (V.n[0] + A.tile_i - 1) / A.tile_i;
-        T = static_cast<long long>(A.tiles_k) * A.tiles_j * A.tiles_i;
-        if (kXcd * ((T + kXcd - 1) / kXcd) <= kReduceBlocks || A.tile_i >= V.n[0]) break;
-        A.tile_i *= 2;
+    long long best = 0;
+    for (int lk = 6; lk >= 4; lk--) {
+        const int lanes = 1 << lk, rows = kThreads >> lk;
+        const long long tk = (V.n[2] + lanes * A.pair - 1) / (lanes * A.pair), tj = (V.n[1] + rows - 1) / rows;
+        if (best == 0 || tk * tj < best) {
+            best = tk * tj;
+            A.lk_log2 = lk;
+            A.tiles_k = static_cast<int>(tk);
+            A.tiles_j = static_cast<int>(tj);
+        }
     }
-    A.per_xcd = static_cast<int>((T + kXcd - 1) / kXcd);
+    auto tiles = [&](int ti) { return best * ((V.n[0] + ti - 1) / ti); };
+    A.tile_i = kTileI;
+    const int want = V.nrows < (1LL << 20) ? 512 : A.pair == 1 ? 1024 : 256;
+    while (A.tile_i > 1 && tiles(A.tile_i) < want) A.tile_i /= 2;
+    while (kXcd * ((tiles(A.tile_i) + kXcd - 1) / kXcd) > kReduceBlocks && A.tile_i < V.n[0]) A.tile_i *= 2;
+    A.tiles_i = (V.n[0] + A.tile_i - 1) / A.tile_i;
+    A.per_xcd = static_cast<int>((tiles(A.tile_i) + kXcd - 1) / kXcd);
     return A;
 }
 
@@ -1052,8 +1070,9 @@ __global__ __launch_bounds__(kThreads) void k_apply_dia(DiaOp<VT> A, const XT* _
         const int t2 = tile / A.tiles_k;
         const int tj = t2 % A.tiles_j;
         const int ti = t2 / A.tiles_j;
-        const int k = (tk * kTileK + (threadIdx.x & 63)) * PAIR;
-        const int j = tj * kTileJ + (threadIdx.x >> 6);
+        const int lane_k = threadIdx.x & ((1 << A.lk_log2) - 1);
+        const int k = ((tk << A.lk_log2) + lane_k) * PAIR;
+        const int j = tj * (kThreads >> A.lk_log2) + (threadIdx.x >> A.lk_log2);
         if (k < A.V.n[2] && j < A.V.n[1]) {
             const int i0 = ti * A.tile_i;
             const int i1 = (i0 + A.tile_i < A.V.n[0]) ? i0 + A.tile_i : A.V.n[0];

@@ -1,0 +1,81 @@
+"""Operator sweeps and solves at the edges of the work-group tiles of the diagonal-view
+traversals (16, 32 or 64 lanes along k, one, two or four cells per lane, marches of 1 to 16
+planes) and of the CSR traversal, against the oracle.
+
+The tile shape follows from the extents: these straddle each lane split, leave partial tiles
+along k and j, and reach a march of every length from one plane (small grids) to sixteen."""
+import numpy as np
+import pytest
+
+import dare_amd as da
+import oracle as orc
+from conftest import bits_equal
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(5, 3, 16), (3, 17, 31), (2, 9, 32), (40, 5, 33), (9, 33, 64), (4, 4, 66), (2, 2, 96), (19, 6, 130),
+          (70, 20, 24), (37, 41, 43), (66, 34)]
+OPS = ["diff", "conv", "react"]
+
+
+def system(ctx, rng, shape, op):
+    import torch
+    ncomp = 2 if op == "react" else 1
+    dim = len(shape)
+    go = orc.grid(list(shape), size=[0.1 * m for m in shape], ghost=2, ncomp=ncomp)
+    cells = int(np.prod(shape))
+    pad = int(np.prod([m + 4 for m in shape])) * ncomp
+    kw = dict(dt=5e-3, bc_type=[1, 2, 1, 1, 2, 1][:2 * dim], bc_value=[0.3, 0.0, -1.0, 0.5, 0.0, 0.25][:2 * dim])
+    arr = {}
+    if op == "diff":
+        kw["diff"] = 0.4
+    elif op == "conv":
+        arr["diff_cell"] = rng.uniform(0.1, 0.9, size=pad)
+        kw["limiter"] = da.VANLEER
+        arr["vel"] = [rng.uniform(-1, 1, size=cells // shape[d] * (shape[d] + 1)) for d in range(dim)]
+    else:
+        kw["diff_comp"] = [0.2, 0.5]
+        k = rng.uniform(0.1, 10, size=(cells, 2))
+        arr["react"] = np.stack([-k[:, 0], k[:, 1], k[:, 0], -k[:, 1]], axis=1).ravel()
+    phi = rng.uniform(size=pad)
+    ref = orc.assemble(go, orc.terms(**kw, **arr), phi)
+    g = da.Grid.make(list(shape), size=[0.1 * m for m in shape], ghost=2, ncomp=ncomp)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    darr = {k: [dev(v) for v in a] if isinstance(a, list) else dev(a) for k, a in arr.items()}
+    t = da.Terms.make(**kw, **darr)
+    A = da.Csr(ctx)
+    da.build_structure(ctx, A, g, t)
+    b, x = dev(np.zeros(len(ref[3]))), dev(np.zeros(len(ref[3])))
+    da.fill_values(ctx, A, g, t, dev(phi), b, x)
+    ctx.synchronize()
+    return A, b, x, ref, (t, darr)
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_sweep_and_solves_on_tile_edges(ctx, rng, shape, op):
+    import torch
+    A, b, x0, (rp, col, val, rhs, ox0), keep = system(ctx, rng, shape, op)
+    n = len(rhs)
+    xs, ws = rng.normal(size=n), rng.normal(size=n)
+    y = torch.zeros_like(b)
+    if len(shape) < 3:                      # the CSR values are written on demand
+        A.download()
+    d = da.spmv_dot(ctx, A, torch.from_numpy(xs).cuda(), y, torch.from_numpy(ws).cuda())
+    exp = orc.spmv(rp, col, val, xs)
+    assert bits_equal(y.cpu().numpy(), exp)
+    assert abs(d - float(exp @ ws)) <= 1e-12 * float(np.abs(exp) @ np.abs(ws))
+    tol = 1e-12 * np.linalg.norm(rhs)
+    xo, ok, it, *_ = orc.bicgstab2(rp, col, val, rhs, ox0, tol, 300)
+    assert ok
+    x = x0.clone()
+    r = da.bicgstab2(ctx, A, b, x, tol=tol, tol_kind=0, max_it=300)
+    assert r["converged"] == 1 and abs(r["iterations"] - it) <= 1
+    assert abs(r["bnorm"] - np.linalg.norm(rhs)) <= 1e-13 * np.linalg.norm(rhs)
+    assert np.max(np.abs(x.cpu().numpy() - xo)) <= 1e-12 * np.max(np.abs(xo)) + tol
+    for precond in (0, 1):
+        x = x0.clone()
+        r = da.refine_mixed(ctx, A, b, x, tol=1e-10, tol_kind=1, inner_tol=1e-4, precond=precond)
+        assert r["converged"] == 1
+        assert np.linalg.norm(rhs - orc.spmv(rp, col, val, x.cpu().numpy())) <= 1e-10 * np.linalg.norm(rhs)
+    A.close()
