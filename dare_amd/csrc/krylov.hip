@@ -122,11 +122,21 @@ static_assert(sizeof(KState) <= 64 * sizeof(double), "pinned readback block too 
 // every operator application is A M^-1, the iterate y starts at zero and accumulates in y_buf
 // (or in x itself when x starts at zero), and x += M^-1 y at the end. The residual r stays the
 // residual of A x = b, so the stopping test keeps its meaning.
+struct Stop {                   // the stopping threshold: tol, or (relative) tol * ||b||
+    double tol;
+    bool relative;
+    double abs(double bnorm) const { return relative ? tol * bnorm : tol; }
+};
+struct Outcome {
+    int iters = 0, status = 0, hist_len = 0;
+    double rnorm = 0., bnorm = 0.;
+    bool converged = false;
+};
+
 template <typename VT, typename XT, bool NT>
-int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, double tol_abs, int max_it,
-                     double* hist, int hist_cap, int* hist_len, int* iters, double* rnorm, int* status,
-                     bool* converged, XT* work, int min_passes, bool x_zero, KState* st, ReduceWs ws,
-                     const MgHierarchy* mg = nullptr, XT* y_buf = nullptr) {
+int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, Stop stop, int max_it, double* hist,
+                     int hist_cap, Outcome* out, XT* work, int min_passes, bool x_zero, KState* st, ReduceWs ws,
+                     const MgHierarchy* mg, XT* y_buf) {
     const long long n = A.n;
     XT* r = work;
     XT* rh = r + n;
@@ -137,8 +147,7 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, do
     XT* t = w + n;
     const unsigned gr = grid_for(n);
     hipStream_t sm = ctx->stream;
-    *hist_len = 0;
-    *status = 0;
+    *out = Outcome{};
     XT* y = (mg && !x_zero) ? y_buf : x;       // the iterate the passes update
     const XT* rhv = x_zero ? b : rh;           // the shadow residual r0: b itself when x0 = 0
     auto pre = [&](const XT* in) -> const XT* { return mg ? mg_apply<VT, XT>(sm, *mg, in) : in; };
@@ -149,20 +158,21 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, do
         hipLaunchKernelGGL((k_init_zero<XT>), dim3(gr), dim3(kThreads), 0, sm, n, b, ws, st);
         launch_finish<2>(sm, ws, gr, st, TAIL_INIT, 0);
     } else {
-        A.launch(sm, x, EpiInit<XT, NT>{b, r, rh, u, v, w}, ws, st, TAIL_INIT, 0);     // (0)-(2)
+        A.launch(sm, x, EpiStart<XT, NT>{b, rh}, ws, st, TAIL_START, 0);     // (0)-(2)
         if (mg) hipLaunchKernelGGL((k_zero<XT>), dim3(gr), dim3(kThreads), 0, sm, n, y);
     }
     DARE_LAUNCH_CHECK();
     KState h;
     int rc = read_state(ctx, st, &h);
     if (rc) return rc;
+    out->bnorm = x_zero ? h.rnorm : std::sqrt(h.dots[1]);
+    const double tol_abs = stop.abs(out->bnorm);
     double conv = h.rnorm;
     if (conv < tol_abs) {
         if (!x_written) hipLaunchKernelGGL((k_zero<XT>), dim3(gr), dim3(kThreads), 0, sm, n, x);
         DARE_LAUNCH_CHECK();
-        *iters = 0;
-        *rnorm = conv;
-        *converged = true;
+        out->rnorm = conv;
+        out->converged = true;
         return DARE_OK;
     }
     int k = 1;
@@ -170,30 +180,36 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, do
     while (true) {
         if (k > max_it) break;
         if (h.next_status) {
-            *status = h.next_status;
+            out->status = h.next_status;
             break;
         }
-        // the first pass from a zero guess reads b for r and 0 for x, u (k_init_zero wrote none)
-        const bool first = x_zero && k == 1;
-        if (first) hipLaunchKernelGGL((k_upd_u<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, b, u, st);
-        else hipLaunchKernelGGL((k_upd_u<XT, NT>), dim3(gr), dim3(kThreads), 0, sm, n, r, u, st);
-        A.launch(sm, pre(u), EpiDot<XT, NT>{v, rhv}, ws, st, TAIL_GAMMA, 1);
-        if (first) hipLaunchKernelGGL((k_upd_rx<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, r, v, y, u, st, b);
-        else hipLaunchKernelGGL((k_upd_rx<XT, NT>), dim3(gr), dim3(kThreads), 0, sm, n, r, v, y, u, st, nullptr);
+        // the first pass starts from u = 0, so step 5 is u = r; r and u are read where the
+        // initialisation left r0
+        const bool first = k == 1;
+        const XT* ro = first ? rhv : r;
+        const XT* uo = first ? rhv : u;
+        if (!first) hipLaunchKernelGGL((k_comb<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, r, u, u, st);   // (5)
+        A.launch(sm, pre(uo), EpiDot<XT, NT>{v, rhv}, ws, st, TAIL_GAMMA, 1);                                       // (6), (7)
+        hipLaunchKernelGGL((k_comb<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, ro, v, r, st);               // (8)
+        A.launch(sm, pre(r), EpiDot<XT, NT>{s, rhv}, ws, st, TAIL_RHO, 1);                                          // (9), (11)
+        hipLaunchKernelGGL((k_comb<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, s, v, v, st);               // (12)
+        A.launch(sm, pre(v), EpiDot<XT, NT>{w, rhv}, ws, st, TAIL_GAMMA, 1);                                        // (13), (14)
+        hipLaunchKernelGGL((k_comb<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, s, w, s, st);                // (17)
+        if (mg) A.launch(sm, pre(s), EpiGcrP<XT, NT>{t, r, v, st, s}, ws, st, TAIL_GCR, 1);                         // (18)-(20)
+        else A.launch(sm, s, EpiGcrL<XT, NT>{t, r, v, st}, ws, st, TAIL_GCR, 1);
+        if (first && x_zero)
+            hipLaunchKernelGGL((k_pass_end<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, y, r, r, s, t, uo, u, v, w,
+                               rhv, ws, st);
+        else
+            hipLaunchKernelGGL((k_pass_end<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, y, r, r, s, t, uo, u, v,
+                               w, rhv, ws, st);
         x_written = true;
-        A.launch(sm, pre(r), EpiDot<XT, NT>{s, rhv}, ws, st, TAIL_RHO, 1);
-        hipLaunchKernelGGL((k_upd_v<XT, NT>), dim3(gr), dim3(kThreads), 0, sm, n, s, v, st);
-        A.launch(sm, pre(v), EpiDot<XT, NT>{w, rhv}, ws, st, TAIL_GAMMA, 1);
-        hipLaunchKernelGGL((k_upd_urs<XT, NT>), dim3(gr), dim3(kThreads), 0, sm, n, u, r, v, s, w, st);
-        if (mg) A.launch(sm, pre(s), EpiGcrP<XT, NT>{t, r, s}, ws, st, TAIL_GCR, 1);
-        else A.launch(sm, s, EpiGcr<XT, NT>{t, r}, ws, st, TAIL_GCR, 1);
-        hipLaunchKernelGGL((k_end<XT, NT>), dim3(gr), dim3(kThreads), 0, sm, n, y, r, s, t, u, v, w, rhv, ws, st);
         launch_finish<2>(sm, ws, gr, st, TAIL_END, 1);
         DARE_LAUNCH_CHECK();
         rc = read_state(ctx, st, &h);
         if (rc) return rc;
         if (h.status) {
-            *status = h.status;
+            out->status = h.status;
             if (h.status == 21) {
                 // tau == 0: true residual check (BiCGStab2.inl:514-536); preconditioned, the
                 // iterate is x + M^-1 y, formed in t (unused from here on)
@@ -204,24 +220,24 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, do
                                        static_cast<const XT*>(x_zero ? nullptr : x), z, t);
                     xt = t;
                 }
-                A.launch(sm, xt, EpiInit<XT, NT>{b, r, rh, u, v, w}, ws, st, TAIL_INIT, 0);
+                A.launch(sm, xt, EpiStart<XT, NT>{b, rh}, ws, st, TAIL_START, 0);
                 rc = read_state(ctx, st, &h);
                 if (rc) return rc;
                 conv = h.rnorm;
                 if (conv <= tol_abs) {
                     done_ok = true;
-                    *status = 0;
+                    out->status = 0;
                 }
                 if (mg) DARE_HIP_TRY(hipMemcpyAsync(x, t, sizeof(XT) * n, hipMemcpyDeviceToDevice, sm));
-                *iters = k;
-                *rnorm = conv;
-                *converged = done_ok;
+                out->iters = k;
+                out->rnorm = conv;
+                out->converged = done_ok;
                 return DARE_OK;
             }
             break;
         }
         conv = h.rnorm;
-        if (hist && *hist_len < hist_cap) hist[(*hist_len)++] = conv;
+        if (hist && out->hist_len < hist_cap) hist[out->hist_len++] = conv;
         if (conv <= tol_abs && k >= min_passes) break;   // reference: k > 1 (min_passes 2)
         ++k;
     }
@@ -232,43 +248,47 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, do
                            static_cast<const XT*>(x_zero ? nullptr : x), z, x);
         DARE_LAUNCH_CHECK();
     }
-    *iters = k;
-    *rnorm = conv;
-    *converged = done_ok || conv <= tol_abs;
+    out->iters = k;
+    out->rnorm = conv;
+    out->converged = done_ok || conv <= tol_abs;
     return DARE_OK;
 }
 
 // st / ws: the device scalars and reduction partials of this solve (the context's own, or the
 // allocation-free entry point's static scratch)
 template <typename VT, typename XT>
-int bicgstab2_run(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, double tol_abs, int max_it,
-                  double* hist, int hist_cap, int* hist_len, int* iters, double* rnorm, int* status,
-                  bool* converged, XT* work, int min_passes, bool x_zero, KState* st, ReduceWs ws,
+int bicgstab2_run(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, Stop stop, int max_it, double* hist,
+                  int hist_cap, Outcome* out, XT* work, int min_passes, bool x_zero, KState* st, ReduceWs ws,
                   const MgHierarchy* mg = nullptr, XT* y_buf = nullptr) {
     if (A.n >= kStreamRows)
-        return bicgstab2_run_nt<VT, XT, true>(ctx, A, b, x, tol_abs, max_it, hist, hist_cap, hist_len, iters, rnorm,
-                                              status, converged, work, min_passes, x_zero, st, ws, mg, y_buf);
-    return bicgstab2_run_nt<VT, XT, false>(ctx, A, b, x, tol_abs, max_it, hist, hist_cap, hist_len, iters, rnorm,
-                                           status, converged, work, min_passes, x_zero, st, ws, mg, y_buf);
+        return bicgstab2_run_nt<VT, XT, true>(ctx, A, b, x, stop, max_it, hist, hist_cap, out, work, min_passes, x_zero,
+                                              st, ws, mg, y_buf);
+    return bicgstab2_run_nt<VT, XT, false>(ctx, A, b, x, stop, max_it, hist, hist_cap, out, work, min_passes, x_zero,
+                                           st, ws, mg, y_buf);
 }
 
-static int dot_dev_on(dare_ctx* ctx, long long n, const double* a, const double* b, double* out, KState* st,
-                      ReduceWs ws) {
-    hipLaunchKernelGGL((k_dot<double>), dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream, n, a, b, ws, st);
-    launch_finish<1>(ctx->stream, ws, grid_for(n), st, TAIL_STORE, 0);
-    DARE_LAUNCH_CHECK();
-    KState h;
-    int rc = read_state(ctx, st, &h);
-    if (rc) return rc;
-    *out = h.dots[0];
-    return DARE_OK;
+static void fill_result(const Outcome& o, dare_solver_result* res) {
+    res->converged = o.converged ? 1 : 0;
+    res->iterations = o.iters;
+    res->status = o.status ? DARE_ERR_BREAKDOWN : 0;
+    res->refinements = 0;
+    res->residual = o.rnorm;
+    res->bnorm = o.bnorm;
+    res->history_len = o.hist_len;
 }
 
 static int dot_dev(dare_ctx* ctx, long long n, const double* a, const double* b, double* out) {
     Workspace W;
     int rc = ws_reserve(ctx, 0, &W);
     if (rc) return rc;
-    return dot_dev_on(ctx, n, a, b, out, W.st, ctx->ws);
+    hipLaunchKernelGGL((k_dot<double>), dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream, n, a, b, ctx->ws, W.st);
+    launch_finish<1>(ctx->stream, ctx->ws, grid_for(n), W.st, TAIL_STORE, 0);
+    DARE_LAUNCH_CHECK();
+    KState h;
+    rc = read_state(ctx, W.st, &h);
+    if (rc) return rc;
+    *out = h.dots[0];
+    return DARE_OK;
 }
 
 // ---- Jacobi right preconditioning (M = diag(A)). The method runs on A M^-1 with y = M x:
@@ -668,14 +688,18 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* A, const double* b, doub
     // + the preconditioned iterate (multigrid) or the scaled right-hand side (left Jacobi)
     int rc = ws_reserve(ctx, sizeof(double) * (use_mg || left ? 8 : 7) * n, &W);
     if (rc) return rc;
-    double bnorm2 = 0.;
-    rc = dot_dev(ctx, n, b, b, &bnorm2);
-    if (rc) return rc;
-    const double bnorm = std::sqrt(bnorm2);
-    const double tol_abs = p->tol_kind == 1 ? p->tol * bnorm : p->tol;
     SolveOp<double> op;
     rc = op64(ctx, A, true, &op, {b, x});
     if (rc) return rc;
+    Stop stop{p->tol, p->tol_kind == 1};
+    double bnorm = -1.;         // ||b|| comes out of the solve's first sweep, except where that reads a scaled b
+    if (left) {
+        double bnorm2 = 0.;
+        rc = dot_dev(ctx, n, b, b, &bnorm2);
+        if (rc) return rc;
+        bnorm = std::sqrt(bnorm2);
+        stop = Stop{stop.abs(bnorm), false};
+    }
     const bool pre = p->precond == 1;
     if (pre || left) {          // the scaled views are made from all seven slots
         rc = dia_ensure_full(const_cast<dare_csr*>(A), ctx->stream);
@@ -739,24 +763,17 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* A, const double* b, doub
         DARE_LAUNCH_CHECK();
         bs = bl;
     }
-    int iters = 0, status = 0, hl = 0;
-    double rn = 0.;
-    bool conv = false;
-    rc = bicgstab2_run<double, double>(ctx, op, bs, x, tol_abs, p->max_it, p->history, p->history_cap, &hl, &iters,
-                                       &rn, &status, &conv, static_cast<double*>(W.buf), 2, false, W.st, ctx->ws, mg,
+    Outcome o;
+    rc = bicgstab2_run<double, double>(ctx, op, bs, x, stop, p->max_it, p->history, p->history_cap, &o,
+                                       static_cast<double*>(W.buf), 2, false, W.st, ctx->ws, mg,
                                        static_cast<double*>(W.buf) + 7 * n);
     if (rc) return rc;
     if (pre) {
         hipLaunchKernelGGL(k_scale_by, dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream, n, x, A->dinv, 1);  // x = M^-1 y
         DARE_LAUNCH_CHECK();
     }
-    res->converged = conv ? 1 : 0;
-    res->iterations = iters;
-    res->status = status ? DARE_ERR_BREAKDOWN : 0;
-    res->refinements = 0;
-    res->residual = rn;
-    res->bnorm = bnorm;
-    res->history_len = hl;
+    if (left) o.bnorm = bnorm;
+    fill_result(o, res);
     return DARE_OK;
 }
 
@@ -784,31 +801,18 @@ int dare_bicgstab2_solve_noalloc(dare_ctx* ctx, const dare_csr* A, const double*
     // work vector and partial is written before it is read
     hipLaunchKernelGGL(k_clear_state, dim3(1), dim3(64), 0, ctx->stream, st);
     DARE_LAUNCH_CHECK();
-    double bnorm2 = 0.;
-    int rc = dot_dev_on(ctx, n, b, b, &bnorm2, st, ws);
-    if (rc) return rc;
-    const double bnorm = std::sqrt(bnorm2);
-    const double tol_abs = p->tol_kind == 1 ? p->tol * bnorm : p->tol;
     SolveOp<double> op;
-    rc = op64(ctx, A, true, &op, {b, x});
+    int rc = op64(ctx, A, true, &op, {b, x});
     if (rc) return rc;
     if (!op.dia) {
         rc = csr_ensure_values(const_cast<dare_csr*>(A), ctx->stream);
         if (rc) return rc;
     }
-    int iters = 0, status = 0, hl = 0;
-    double rn = 0.;
-    bool conv = false;
-    rc = bicgstab2_run<double, double>(ctx, op, b, x, tol_abs, p->max_it, p->history, p->history_cap, &hl, &iters,
-                                       &rn, &status, &conv, work, 2, false, st, ws);
+    Outcome o;
+    rc = bicgstab2_run<double, double>(ctx, op, b, x, Stop{p->tol, p->tol_kind == 1}, p->max_it, p->history,
+                                       p->history_cap, &o, work, 2, false, st, ws);
     if (rc) return rc;
-    res->converged = conv ? 1 : 0;
-    res->iterations = iters;
-    res->status = status ? DARE_ERR_BREAKDOWN : 0;
-    res->refinements = 0;
-    res->residual = rn;
-    res->bnorm = bnorm;
-    res->history_len = hl;
+    fill_result(o, res);
     return DARE_OK;
 }
 
@@ -952,25 +956,23 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
             break;
         }
         if (refine >= max_refine || total_it >= p->max_it) break;
-        int it = 0, ist = 0, dummy_len = 0;
-        double irn = 0.;
-        bool iconv = false;
         // an inner solve may stop after one pass once it meets its threshold when a pass costs
         // four V-cycles (multigrid); otherwise the second pass is cheaper than the extra
         // refinement (FP64 residual, correction, new inner start) that stopping early brings
-        rc = bicgstab2_run<float, float>(ctx, op32, r32, d32, inner_threshold(inner_tol, rn, tol_abs), inner_max,
-                                         nullptr, 0, &dummy_len, &it, &irn, &ist, &iconv, work, use_mg ? 1 : 2,
-                                         true, W.st, ctx->ws, mg);   // d32 = 0 to start
+        Outcome in;
+        rc = bicgstab2_run<float, float>(ctx, op32, r32, d32, Stop{inner_threshold(inner_tol, rn, tol_abs), false},
+                                         inner_max, nullptr, 0, &in, work, use_mg ? 1 : 2, true, W.st, ctx->ws,
+                                         mg);   // d32 = 0 to start
         if (rc) return rc;
-        total_it += it;
+        total_it += in.iters;
         if (pre)    // the inner solution is y = M d
             hipLaunchKernelGGL(k_add_correction_pre, dim3(gr), dim3(kThreads), 0, ctx->stream, n, x, d32, A->dinv);
         else
             hipLaunchKernelGGL(k_add_correction, dim3(gr), dim3(kThreads), 0, ctx->stream, n, x, d32);
         DARE_LAUNCH_CHECK();
         refine++;
-        if (ist && it <= 1) {
-            status = ist;
+        if (in.status && in.iters <= 1) {
+            status = in.status;
             break;
         }
     }

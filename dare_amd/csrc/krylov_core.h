@@ -23,10 +23,12 @@ constexpr int kXcd = 8;             // MI355X: 8 accelerator complex dies, block
 struct KState {
     double alpha, beta, gamma, rho0, rho1;
     double om1, om2, mu, nu, tau;
+    double alpha1;     // alpha of step 7, applied to x in the pass's last kernel
     double rnorm;      // ||r|| after the last update
     double dots[kMaxDots];
     int status;        // breakdown inside the pass (step number), 0 = none
     int next_status;   // breakdown in the prelude of the next pass (steps 3-4)
+    int x_due;         // step 10 (x += alpha1 u) has been reached and waits for the pass's last kernel
 };
 
 enum TailOp : int {
@@ -37,6 +39,7 @@ enum TailOp : int {
     TAIL_RHO = 4,       // rho1 = <r0, s>, beta, rho0 = rho1 (step 11)
     TAIL_GCR = 5,       // omega_1,2 (steps 19-23)
     TAIL_END = 6,       // ||r||, prelude of the next pass (steps 3-4)
+    TAIL_START = 7,     // TAIL_INIT from <r,r>, <b,b> (rh = r, so <rh,r> = <r,r>); dots[1] = <b,b>
 };
 
 __device__ void apply_tail(int op, KState* st, const double* d) {
@@ -44,8 +47,10 @@ __device__ void apply_tail(int op, KState* st, const double* d) {
     case TAIL_STORE:
         for (int j = 0; j < kMaxDots; j++) st->dots[j] = d[j];
         break;
+    case TAIL_START: st->dots[1] = d[1]; [[fallthrough]];
     case TAIL_INIT: {
         st->rnorm = sqrt(d[0]);
+        st->x_due = 0;
         st->alpha = 0.;
         st->rho0 = 1.;
         st->om1 = st->om2 = 1.;
@@ -56,7 +61,7 @@ __device__ void apply_tail(int op, KState* st, const double* d) {
             st->next_status = 3;
             break;
         }
-        st->rho1 = d[1];                                     // (4)
+        st->rho1 = op == TAIL_START ? d[0] : d[1];           // (4)
         st->beta = st->alpha * st->rho1 / st->rho0;
         st->rho0 = st->rho1;
         if (st->rho0 == 0.0) st->next_status = 4;
@@ -71,6 +76,8 @@ __device__ void apply_tail(int op, KState* st, const double* d) {
         st->alpha = st->rho0 / st->gamma;
         break;
     case TAIL_RHO:
+        st->alpha1 = st->alpha;
+        st->x_due = 1;
         st->rho1 = d[0];
         st->beta = st->alpha * st->rho1 / st->rho0;
         st->rho0 = st->rho1;
@@ -99,6 +106,7 @@ __device__ void apply_tail(int op, KState* st, const double* d) {
     }
     case TAIL_END: {
         st->rnorm = sqrt(d[0]);
+        st->x_due = 0;
         st->next_status = 0;
         st->rho0 = -st->om2 * st->rho0;
         if (st->rho0 == 0.0) {
@@ -312,26 +320,68 @@ struct EpiGcr {         // t = A s; <r,s>, <s,s>, <s,t>, <t,t>, <r,t>   (18)-(20
     }
 };
 
-// the same step when a right preconditioner sits between s and the operator: t = A (M^-1 s),
-// with s read from its own vector (the operand of the traversal is M^-1 s)
+// Epilogues that need a scalar of the device state read it once per work-item, in begin().
+template <class Epi>
+__device__ inline auto epi_begin(Epi& e, int) -> decltype(e.begin()) { return e.begin(); }
+template <class Epi>
+__device__ inline void epi_begin(Epi&, long) {}
+
+// r = b - A x into rh alone; <r,r>, <b,b>. The shadow residual never changes, so the first pass
+// reads it as r and as u (u = r - beta u with u = 0) and writes both vectors itself: nothing
+// else needs a value here, and ||b|| costs no sweep of its own.
 template <typename XT, bool NT = false>
-struct EpiGcrP {
+struct EpiStart {
+    static constexpr int NDOT = 2;
+    static constexpr bool kNT = NT;
+    const XT* b;
+    XT* rh;
+    __device__ double load(long long i) const { return static_cast<double>(b[i]); }
+    __device__ void operator()(long long i, double y, double, double bi, double* acc) const {
+        const XT ri = static_cast<XT>(bi - y);
+        put<NT>(rh + i, ri);
+        const double rd = static_cast<double>(ri);
+        acc[0] += rd * rd;
+        acc[1] += bi * bi;
+    }
+};
+
+// (16) and (18)-(20) in one: t = A s with r = r - alpha v formed here for the dots and again in
+// k_pass_end, never stored in between
+template <typename XT, bool NT = false>
+struct EpiGcrL {
     static constexpr int NDOT = 5;
     static constexpr bool kNT = NT;
     XT* t;
     const XT* r;
-    const XT* s;
-    __device__ double load(long long i) const { return static_cast<double>(r[i]); }
-    __device__ void operator()(long long i, double y, double, double rd, double* acc) const {
+    const XT* v;
+    const KState* st;
+    double alpha = 0.;
+    __device__ void begin() { alpha = st->alpha; }
+    __device__ double load(long long i) const {
+        return static_cast<double>(static_cast<XT>(static_cast<double>(r[i]) - alpha * static_cast<double>(v[i])));
+    }
+    __device__ void operator()(long long i, double y, double sc, double rd, double* acc) const {
         const XT ti = static_cast<XT>(y);
         put<NT>(t + i, ti);
         const double td = static_cast<double>(ti);
-        const double sc = static_cast<double>(s[i]);
         acc[0] += rd * sc;
         acc[1] += sc * sc;
         acc[2] += sc * td;
         acc[3] += td * td;
         acc[4] += rd * td;
+    }
+};
+
+// the same step when a right preconditioner sits between s and the operator: t = A (M^-1 s),
+// with s read from its own vector (the operand of the traversal is M^-1 s)
+template <typename XT, bool NT = false>
+struct EpiGcrP : EpiGcrL<XT, NT> {
+    const XT* s;
+    __device__ EpiGcrP() = default;
+    __host__ __device__ EpiGcrP(XT* t_, const XT* r_, const XT* v_, const KState* st_, const XT* s_)
+        : EpiGcrL<XT, NT>{t_, r_, v_, st_}, s(s_) {}
+    __device__ void operator()(long long i, double y, double, double rd, double* acc) const {
+        EpiGcrL<XT, NT>::operator()(i, y, static_cast<double>(s[i]), rd, acc);
     }
 };
 
@@ -503,6 +553,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
     for (int j = 0; j < Epi::NDOT; j++) acc[j] = 0.;
     const bool run = !(check_status && st->status);
     if (run) {
+        epi_begin(epi, 0);
         const int lane = threadIdx.x % kCsrWaveRows, wv = threadIdx.x / kCsrWaveRows;
         double* prod = s_prod[wv];
         const long long ntiles = (A.n + kCsrWaveRows - 1) / kCsrWaveRows;
@@ -1066,6 +1117,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_dia(DiaOp<VT> A, const XT* _
     const int tile = static_cast<int>(blockIdx.x % kXcd) * A.per_xcd + static_cast<int>(blockIdx.x / kXcd);
     const int ntiles = A.tiles_k * A.tiles_j * A.tiles_i;
     if (run && tile < ntiles) {
+        epi_begin(epi, 0);
         const int tk = tile % A.tiles_k;
         const int t2 = tile / A.tiles_k;
         const int tj = t2 % A.tiles_j;
@@ -1103,134 +1155,58 @@ constexpr int kU = 4;
          base_ += (long long)gridDim.x * (kThreads * kU))
 #define DARE_IDX(u) (base_ + (long long)(u) * kThreads + threadIdx.x)
 
-// FIRST: the first pass from a zero guess (k_init_zero), where r = b and u = 0 were never
-// written: r is b itself, u reads as 0 (the same arithmetic, r - beta * 0).
-template <typename XT, bool NT, bool FIRST = false>
-__global__ __launch_bounds__(kThreads) void k_upd_u(long long n, const XT* __restrict__ r, XT* __restrict__ u,
-                                                    const KState* __restrict__ st) {
+// Steps 5, 8, 12 and 17: out = a - c b with c = beta or alpha. (out may be a or b.)
+template <typename XT, bool NT, bool ALPHA>
+__global__ __launch_bounds__(kThreads) void k_comb(long long n, const XT* a, const XT* b, XT* out,
+                                                   const KState* __restrict__ st) {
     if (st->status) return;
-    const double beta = st->beta;
+    const double c = ALPHA ? st->alpha : st->beta;
     DARE_CHUNK_LOOP(n) {
-        double rv[kU], uv[kU];
+        double av[kU], bv[kU];
 #pragma unroll
         for (int q = 0; q < kU; q++) {
             const long long i = DARE_IDX(q) < n ? DARE_IDX(q) : 0;
-            rv[q] = static_cast<double>(r[i]);
-            uv[q] = FIRST ? 0. : static_cast<double>(u[i]);
+            av[q] = static_cast<double>(a[i]);
+            bv[q] = static_cast<double>(b[i]);
         }
 #pragma unroll
         for (int q = 0; q < kU; q++)
-            if (DARE_IDX(q) < n) put<NT>(u + DARE_IDX(q), static_cast<XT>(rv[q] - beta * uv[q]));   // (5)
+            if (DARE_IDX(q) < n) put<NT>(out + DARE_IDX(q), static_cast<XT>(av[q] - c * bv[q]));
     }
 }
 
-// FIRST: the first pass from a zero guess: the old r is b (read from b0) and the old x is 0,
-// both written here for the first time -- also when the pass has already broken down, so the
-// solve then returns x = 0, r = b as the zero-guess initialisation leaves them.
-template <typename XT, bool NT, bool FIRST = false>
-__global__ __launch_bounds__(kThreads) void k_upd_rx(long long n, XT* __restrict__ r, const XT* __restrict__ v,
-                                                     XT* __restrict__ x, const XT* __restrict__ u,
-                                                     const KState* __restrict__ st, const XT* __restrict__ b0 = nullptr) {
-    if (st->status) {
-        if constexpr (FIRST) {
-            for (long long i = blockIdx.x * (long long)kThreads + threadIdx.x; i < n; i += (long long)gridDim.x * kThreads) {
-                put<NT>(r + i, b0[i]);
-                put<NT>(x + i, XT(0));
-            }
-        }
-        return;
-    }
-    const double a = st->alpha;
-    DARE_CHUNK_LOOP(n) {
-        double rv[kU], vv[kU], xv[kU], uv[kU];
-#pragma unroll
-        for (int q = 0; q < kU; q++) {
-            const long long i = DARE_IDX(q) < n ? DARE_IDX(q) : 0;
-            rv[q] = static_cast<double>(FIRST ? b0[i] : r[i]);
-            vv[q] = static_cast<double>(v[i]);
-            xv[q] = FIRST ? 0. : static_cast<double>(x[i]);
-            uv[q] = static_cast<double>(u[i]);
-        }
-#pragma unroll
-        for (int q = 0; q < kU; q++) {
-            const long long i = DARE_IDX(q);
-            if (i < n) {
-                put<NT>(r + i, static_cast<XT>(rv[q] - a * vv[q]));                                // (8)
-                put<NT>(x + i, static_cast<XT>(1. * xv[q] + a * uv[q]));                           // (10)
-            }
-        }
-    }
-}
-
-template <typename XT, bool NT>
-__global__ __launch_bounds__(kThreads) void k_upd_v(long long n, const XT* __restrict__ s, XT* __restrict__ v,
-                                                    const KState* __restrict__ st) {
-    if (st->status) return;
-    const double beta = st->beta;
-    DARE_CHUNK_LOOP(n) {
-        double sv[kU], vv[kU];
-#pragma unroll
-        for (int q = 0; q < kU; q++) {
-            const long long i = DARE_IDX(q) < n ? DARE_IDX(q) : 0;
-            sv[q] = static_cast<double>(s[i]);
-            vv[q] = static_cast<double>(v[i]);
-        }
-#pragma unroll
-        for (int q = 0; q < kU; q++)
-            if (DARE_IDX(q) < n) put<NT>(v + DARE_IDX(q), static_cast<XT>(sv[q] - beta * vv[q]));   // (12)
-    }
-}
-
-template <typename XT, bool NT>
-__global__ __launch_bounds__(kThreads) void k_upd_urs(long long n, XT* __restrict__ u, XT* __restrict__ r,
-                                                      const XT* __restrict__ v, XT* __restrict__ s,
-                                                      const XT* __restrict__ w, const KState* __restrict__ st) {
-    if (st->status) return;
-    const double a = st->alpha, beta = st->beta;
-    DARE_CHUNK_LOOP(n) {
-        double uv[kU], rv[kU], vv[kU], sv[kU], wv[kU];
-#pragma unroll
-        for (int q = 0; q < kU; q++) {
-            const long long i = DARE_IDX(q) < n ? DARE_IDX(q) : 0;
-            uv[q] = static_cast<double>(u[i]);
-            rv[q] = static_cast<double>(r[i]);
-            vv[q] = static_cast<double>(v[i]);
-            sv[q] = static_cast<double>(s[i]);
-            wv[q] = static_cast<double>(w[i]);
-        }
-#pragma unroll
-        for (int q = 0; q < kU; q++) {
-            const long long i = DARE_IDX(q);
-            if (i < n) {
-                put<NT>(u + i, static_cast<XT>(rv[q] - beta * uv[q]));                             // (15)
-                put<NT>(r + i, static_cast<XT>(rv[q] - a * vv[q]));                                // (16)
-                put<NT>(s + i, static_cast<XT>(sv[q] - a * wv[q]));                                // (17)
-            }
-        }
-    }
-}
-
-// x += om1 r + om2 s; x += alpha u; r -= om1 s + om2 t; u -= om1 v + om2 w; <r,r>, <rh,r>
-template <typename XT, bool NT>
-__global__ __launch_bounds__(kThreads) void k_end(long long n, XT* __restrict__ x, XT* __restrict__ r,
-                                                  const XT* __restrict__ s, const XT* __restrict__ t,
-                                                  XT* __restrict__ u, const XT* __restrict__ v,
-                                                  const XT* __restrict__ w, const XT* __restrict__ rh, ReduceWs ws,
-                                                  KState* st) {
+// The pass's last kernel: every update of x, r and u that no operator application of the pass
+// waits for, from the vectors as the applications left them.
+//   (15) u' = r - beta u    (16) r' = r - alpha v    (10) x' = x + alpha1 u
+//   x = x' + om1 r' + om2 s + alpha u'; r = r' - om1 s - om2 t; u = u' - om1 v - om2 w;
+//   <r,r>, <rh,r>
+// Steps 10, 15 and 16 took 64 B/row of their own (FP64) and r', u' were written only to be read
+// back here: a pass moves 416 B/row instead of 472, with the same rounding at every step
+// (256^3 FP64: steps 8, 10 and 15-17 took 135 + 184 us, steps 8 and 17 alone 65 + 65; t's sweep
+// reads one vector more, 210 -> 212 us; this kernel 272 -> 256).
+// ro, uo: r and u before the pass's last updates (the shadow residual in a first pass, which
+// reads u = r); XZERO: x was never written and counts as 0. A breakdown after step 10 leaves
+// x = x + alpha1 u, as the reference's order of the updates does.
+template <typename XT, bool NT, bool XZERO>
+__global__ __launch_bounds__(kThreads) void k_pass_end(long long n, XT* __restrict__ x, const XT* ro, XT* r,
+                                                       const XT* __restrict__ s, const XT* __restrict__ t, const XT* uo,
+                                                       XT* u, const XT* __restrict__ v, const XT* __restrict__ w,
+                                                       const XT* rh, ReduceWs ws, KState* st) {
     double acc[2] = {0., 0.};
     const bool run = st->status == 0;
+    const double a1 = st->alpha1;
     if (run) {
-        const double o1 = st->om1, o2 = st->om2, a = st->alpha;
+        const double o1 = st->om1, o2 = st->om2, a = st->alpha, beta = st->beta;
         DARE_CHUNK_LOOP(n) {
             double xv[kU], rv[kU], sv[kU], tv[kU], uv[kU], vv[kU], wv[kU], hv[kU];
 #pragma unroll
             for (int q = 0; q < kU; q++) {
                 const long long i = DARE_IDX(q) < n ? DARE_IDX(q) : 0;
-                xv[q] = static_cast<double>(x[i]);
-                rv[q] = static_cast<double>(r[i]);
+                xv[q] = XZERO ? 0. : static_cast<double>(x[i]);
+                rv[q] = static_cast<double>(ro[i]);
                 sv[q] = static_cast<double>(s[i]);
                 tv[q] = static_cast<double>(t[i]);
-                uv[q] = static_cast<double>(u[i]);
+                uv[q] = static_cast<double>(uo[i]);
                 vv[q] = static_cast<double>(v[i]);
                 wv[q] = static_cast<double>(w[i]);
                 hv[q] = static_cast<double>(rh[i]);
@@ -1239,18 +1215,27 @@ __global__ __launch_bounds__(kThreads) void k_end(long long n, XT* __restrict__ 
             for (int q = 0; q < kU; q++) {
                 const long long i = DARE_IDX(q);
                 if (i < n) {
-                    double xi = 1. * xv[q] + o1 * rv[q] + o2 * sv[q];                           // (24)
-                    xi = 1. * xi + a * uv[q];
+                    const double x1 = static_cast<double>(static_cast<XT>(1. * xv[q] + a1 * uv[q]));      // (10)
+                    const double u1 = static_cast<double>(static_cast<XT>(rv[q] - beta * uv[q]));         // (15)
+                    const double r1 = static_cast<double>(static_cast<XT>(rv[q] - a * vv[q]));            // (16)
+                    double xi = 1. * x1 + o1 * r1 + o2 * sv[q];                                           // (24)
+                    xi = 1. * xi + a * u1;
                     put<NT>(x + i, static_cast<XT>(xi));
-                    const XT rn = static_cast<XT>(1. * rv[q] + (-o1) * sv[q] + (-o2) * tv[q]);  // (25)
+                    const XT rn = static_cast<XT>(1. * r1 + (-o1) * sv[q] + (-o2) * tv[q]);               // (25)
                     put<NT>(r + i, rn);
-                    put<NT>(u + i, static_cast<XT>(1. * uv[q] + (-o1) * vv[q] + (-o2) * wv[q]));
+                    put<NT>(u + i, static_cast<XT>(1. * u1 + (-o1) * vv[q] + (-o2) * wv[q]));
                     const double rd = static_cast<double>(rn);
                     acc[0] += rd * rd;
                     acc[1] += hv[q] * rd;
                 }
             }
         }
+    } else if (st->x_due || XZERO) {
+        const double c = st->x_due ? a1 : 0.;
+        for (long long i = blockIdx.x * (long long)kThreads + threadIdx.x; i < n; i += (long long)gridDim.x * kThreads)
+            put<NT>(x + i, c == 0. ? (XZERO ? XT(0) : x[i])
+                                   : static_cast<XT>((XZERO ? 0. : 1. * static_cast<double>(x[i])) +
+                                                     c * static_cast<double>(uo[i])));
     }
     grid_reduce<2>(acc, ws, st, run ? TAIL_END : TAIL_NONE);
 }
@@ -1276,10 +1261,9 @@ __global__ __launch_bounds__(kThreads) void k_dot(long long n, const XT* __restr
 
 // Initialisation (0)-(2) for a zero initial guess: A x0 is +0 in every row, so r = b - A x0 = b
 // bit for bit, and <r,r>, <rh,r> go to the reduction as EpiInit's do. Nothing is written: the
-// first pass reads b where it would read r and 0 where it would read x or u
-// (k_upd_u / k_upd_rx <..., FIRST>), and writes them. rh = r0 is never written again, so the
-// caller reads b itself as rh (b stays untouched during the solve); v and w are written before
-// they are read (EpiInit).
+// first pass reads b where it would read r or u and 0 where it would read x, and writes them.
+// rh = r0 is never written again, so the caller reads b itself as rh (b stays untouched during
+// the solve); v and w are written before they are read.
 template <typename XT>
 __global__ __launch_bounds__(kThreads) void k_init_zero(long long n, const XT* __restrict__ b, ReduceWs ws, KState* st) {
     double acc[2] = {0., 0.};

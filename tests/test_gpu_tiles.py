@@ -79,3 +79,24 @@ def test_sweep_and_solves_on_tile_edges(ctx, rng, shape, op):
         assert r["converged"] == 1
         assert np.linalg.norm(rhs - orc.spmv(rp, col, val, x.cpu().numpy())) <= 1e-10 * np.linalg.norm(rhs)
     A.close()
+
+
+@pytest.mark.parametrize("n", [1, 257])
+def test_breakdown_after_the_first_x_update_keeps_it(ctx, n):
+    """A multiple of the identity breaks the method down in its first pass after step 10 (r = 0,
+    so the second gamma is 0): x has then moved to the solution, as in the oracle's order of the
+    updates -- in the FP64 solve, and in the zero-guess FP32 solve inside the refinement."""
+    import torch
+    rp, col, val = np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32), np.full(n, 2.0)
+    A = da.Csr(ctx)
+    da.upload_host_csr(ctx, A, rp, col, val)
+    b = np.arange(1, n + 1, dtype=np.float64)
+    xo, ok, it, res, _ = orc.bicgstab2(rp, col, val, b, np.zeros(n), 1e-30, 10)
+    x = torch.zeros(n, dtype=torch.float64, device="cuda")
+    r = da.bicgstab2(ctx, A, torch.from_numpy(b).cuda(), x, tol=1e-30, tol_kind=0, max_it=10)
+    assert r["status"] == da.DARE_ERR_BREAKDOWN and not ok
+    assert bits_equal(x.cpu().numpy(), xo) and np.array_equal(xo, b / 2)
+    x.zero_()
+    r = da.refine_mixed(ctx, A, torch.from_numpy(b).cuda(), x, tol=0.0, tol_kind=0, max_refine=1)
+    assert np.array_equal(x.cpu().numpy(), b / 2)
+    A.close()
