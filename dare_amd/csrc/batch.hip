@@ -120,7 +120,7 @@ __global__ __launch_bounds__(kThreads) void kb_apply(const BSys* __restrict__ sy
         if (k < S.V.n[2] && j < S.V.n[1]) {
             const int i0 = ti * S.tile_i;
             const int i1 = (i0 + S.tile_i < S.V.n[0]) ? i0 + S.tile_i : S.V.n[0];
-            dia_column<NC, VT, XT, Epi>(S.V, dia_of<VT>(S), x + S.row0, S.row0, k, j, i0, i1, epi, acc);
+            dia_column<NC, VT>(S.V, dia_of<VT>(S), x + S.row0, S.row0, k, j, i0, i1, epi, acc);
         }
         block_partials_at<Epi::NDOT>(acc, partial, pstride, S.op_slot0 + item.local);
         __syncthreads();

@@ -57,6 +57,7 @@ struct dare_ctx {
     dare_hip::ReduceWs ws{nullptr, nullptr};
     double* dot_out = nullptr;     // device results of dare_dot
     double* host_pinned = nullptr; // 64 doubles of pinned host memory for scalar readback
+    unsigned long long read_seq = 0;   // sequence number of the last scalar readback
     int num_cu = 256;
     void* solve_buf = nullptr;     // Krylov work vectors, grown on demand
     size_t solve_bytes = 0;

@@ -89,11 +89,12 @@ int dare_ctx_create(int32_t device, dare_ctx** out) {
     if (hipMalloc(&c->ws.partial, sizeof(double) * kReduceBlocks * kMaxDots) != hipSuccess ||
         hipMalloc(&c->ws.count, sizeof(unsigned int) * 64) != hipSuccess ||
         hipMalloc(&c->dot_out, sizeof(double) * 64) != hipSuccess ||
-        hipHostMalloc(&c->host_pinned, sizeof(double) * 64, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc(&c->host_pinned, sizeof(double) * 64, hipHostMallocCoherent) != hipSuccess) {
         set_error("context allocation failed");
         delete c;
         return DARE_ERR_OOM;
     }
+    for (int i = 0; i < 64; i++) c->host_pinned[i] = 0.;   // no sequence number yet
     // counters start at zero; every reduction's last block resets its counter to zero
     DARE_HIP_TRY(hipMemset(c->ws.count, 0, sizeof(unsigned int) * 64));
     DARE_HIP_TRY(hipDeviceSynchronize());

@@ -1,9 +1,10 @@
 // Krylov kernels and the BiCGStab(2) driver for gfx950.
 //
-// BiCGStab2::Solve (MatrixSystem/BiCGStab2.inl:167-582) is restated as nine fused launches per
-// pass. All method scalars (alpha, beta, gamma, rho, omega, mu, nu, tau) live in device memory
-// and are updated by the one-work-group finish kernel of each reduction, so the host reads
-// back only one small status block per pass (the convergence test). Reductions are
+// BiCGStab2::Solve (MatrixSystem/BiCGStab2.inl:167-582) is restated as nine launches per pass and
+// a one-work-group finish kernel after each of its five reductions; below 4 M rows as five
+// launches and one finish (k_step_*, k_step_end). All method scalars (alpha, beta, gamma, rho,
+// omega, mu, nu, tau) live in device memory and are updated there, so the host reads back only
+// one small status block per pass (the convergence test). Reductions are
 // deterministic: fixed grid, fixed per-thread order, block partials summed in block order.
 //
 // Operators: a generic CSR traversal (grid-stride, one row per lane) and, for matrices
@@ -33,7 +34,8 @@ struct SolveOp {
     long long n;
 
     template <typename XT, class Epi>
-    void launch(hipStream_t sm, const XT* x, const Epi& epi, ReduceWs ws, KState* st, int tail, int check) const {
+    void launch(hipStream_t sm, const XT* x, const Epi& epi, ReduceWs ws, KState* st, int tail, int check,
+                Publish pub = {}) const {
         unsigned grid;
         if (dia) {
             grid = static_cast<unsigned>(kXcd * d.per_xcd);   // <= kReduceBlocks
@@ -64,7 +66,32 @@ struct SolveOp {
             hipLaunchKernelGGL((k_apply_csr<VT, XT, Epi>), dim3(grid), dim3(kThreads), 0, sm, csr, x, epi, ws,
                                st, tail, check);
         }
-        if (tail >= 0) launch_finish<Epi::NDOT>(sm, ws, grid, st, tail, check);
+        if (tail >= 0) launch_finish<Epi::NDOT>(sm, ws, grid, st, tail, check, pub);
+    }
+
+    unsigned grid() const { return dia ? static_cast<unsigned>(kXcd * d.per_xcd) : grid_rows(n); }
+
+    // one fused step (k_step_dia / k_step_csr), the traversals as in launch
+    template <bool GCR, typename XT>
+    void step(hipStream_t sm, const StepVecs<XT>& S, const StepRed& R) const {
+        const dim3 g(grid()), b(kThreads);
+        if (!dia) {
+            hipLaunchKernelGGL((k_step_csr<VT, XT, GCR>), g, b, 0, sm, csr, S, R);
+        } else if (d.V.N == 2) {
+            hipLaunchKernelGGL((k_step_dia<2, VT, XT, GCR, 1, false>), g, b, 0, sm, d, S, R);
+        } else if (d.pair == 4) {
+            if constexpr (std::is_same_v<VT, float>) {
+                if (d.sym) hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 4, true>), g, b, 0, sm, d, S, R);
+                else hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 4, false>), g, b, 0, sm, d, S, R);
+            }
+        } else if (d.pair == 2 && d.sym) {
+            if constexpr (std::is_same_v<VT, double>)
+                hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 2, true>), g, b, 0, sm, d, S, R);
+        } else if (d.pair == 2) {
+            hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 2, false>), g, b, 0, sm, d, S, R);
+        } else {
+            hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 1, false>), g, b, 0, sm, d, S, R);
+        }
     }
 };
 
@@ -84,7 +111,7 @@ struct Workspace {
 
 static int ws_reserve(dare_ctx* ctx, size_t bytes, Workspace* out) {
     if (!ctx->solve_state) {
-        if (hipMalloc(&ctx->solve_state, sizeof(KState)) != hipSuccess) {
+        if (hipMalloc(&ctx->solve_state, sizeof(KState) * kStates) != hipSuccess) {
             hipGetLastError();
             set_error("solver state allocation failed");
             return DARE_ERR_OOM;
@@ -107,14 +134,34 @@ static int ws_reserve(dare_ctx* ctx, size_t bytes, Workspace* out) {
     return DARE_OK;
 }
 
-static int read_state(dare_ctx* ctx, KState* dev, KState* host) {
-    DARE_HIP_TRY(hipMemcpyAsync(ctx->host_pinned, dev, sizeof(KState), hipMemcpyDeviceToHost, ctx->stream));
-    DARE_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    std::memcpy(host, ctx->host_pinned, sizeof(KState));
-    return DARE_OK;
+// The next readback of this context: its pinned block and a new sequence number for the finish
+// kernel that fills it.
+static Publish publish(dare_ctx* ctx) {
+    return Publish{reinterpret_cast<HostState*>(ctx->host_pinned), ++ctx->read_seq};
 }
 
-static_assert(sizeof(KState) <= 64 * sizeof(double), "pinned readback block too small");
+// Waits until the finish kernel launched with pub has published the state, and copies it. The
+// kernel's store reaches the host before the stream would be reported idle, and no copy is queued
+// for it. The stream is asked now and then, so that a failed launch or a stream under capture ends
+// in an error instead of a wait for good.
+static int wait_state(dare_ctx* ctx, const Publish& pub, KState* host) {
+    auto here = [&] { return __atomic_load_n(&pub.host->seq, __ATOMIC_ACQUIRE) == pub.seq; };
+    for (unsigned spins = 1; !here(); spins++) {
+        __builtin_ia32_pause();
+        if (spins % 2048) continue;
+        if (hipStreamQuery(ctx->stream) == hipErrorNotReady) {
+            (void)hipGetLastError();      // not an error of the launches that follow
+            continue;
+        }
+        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        if (e == hipSuccess && here()) break;
+        (void)hipGetLastError();
+        set_error(std::string("the solver's scalars did not arrive: ") + hipGetErrorString(e));
+        return DARE_ERR_HIP;
+    }
+    std::memcpy(host, &pub.host->k, sizeof(KState));
+    return DARE_OK;
+}
 
 // Host-driven BiCGStab2 over device-resident scalars; XT is the type of every vector, NT the
 // choice of non-temporal stores (vectors larger than the caches).
@@ -138,6 +185,8 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, St
                      int hist_cap, Outcome* out, XT* work, int min_passes, bool x_zero, KState* st, ReduceWs ws,
                      const MgHierarchy* mg, XT* y_buf) {
     const long long n = A.n;
+    // work vectors; of the fused steps rr, uu and vv hold the operands (r, u and v cannot be
+    // written where neighbouring rows still read them), and r, u, v also serve as w, t and s
     XT* r = work;
     XT* rh = r + n;
     XT* u = rh + n;
@@ -145,6 +194,8 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, St
     XT* s = v + n;
     XT* w = s + n;
     XT* t = w + n;
+    XT *rr = w, *uu = t, *vv = t + n;
+    const bool fused = !NT && !mg && n < kFusedRows;
     const unsigned gr = grid_for(n);
     hipStream_t sm = ctx->stream;
     *out = Outcome{};
@@ -154,16 +205,17 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, St
     // x = 0: no operator sweep for r = b - A x, and no vector written before the first pass
     // (which writes x and r); a solve that ends before it zeroes x itself (x_written)
     bool x_written = !x_zero;
+    Publish pub = publish(ctx);
     if (x_zero) {
         hipLaunchKernelGGL((k_init_zero<XT>), dim3(gr), dim3(kThreads), 0, sm, n, b, ws, st);
-        launch_finish<2>(sm, ws, gr, st, TAIL_INIT, 0);
+        launch_finish<2>(sm, ws, gr, st, TAIL_INIT, 0, pub);
     } else {
-        A.launch(sm, x, EpiStart<XT, NT>{b, rh}, ws, st, TAIL_START, 0);     // (0)-(2)
+        A.launch(sm, x, EpiStart<XT, NT>{b, rh}, ws, st, TAIL_START, 0, pub);     // (0)-(2)
         if (mg) hipLaunchKernelGGL((k_zero<XT>), dim3(gr), dim3(kThreads), 0, sm, n, y);
     }
     DARE_LAUNCH_CHECK();
     KState h;
-    int rc = read_state(ctx, st, &h);
+    int rc = wait_state(ctx, pub, &h);
     if (rc) return rc;
     out->bnorm = x_zero ? h.rnorm : std::sqrt(h.dots[1]);
     const double tol_abs = stop.abs(out->bnorm);
@@ -188,25 +240,44 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, St
         const bool first = k == 1;
         const XT* ro = first ? rhv : r;
         const XT* uo = first ? rhv : u;
-        if (!first) hipLaunchKernelGGL((k_comb<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, r, u, u, st);   // (5)
-        A.launch(sm, pre(uo), EpiDot<XT, NT>{v, rhv}, ws, st, TAIL_GAMMA, 1);                                       // (6), (7)
-        hipLaunchKernelGGL((k_comb<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, ro, v, r, st);               // (8)
-        A.launch(sm, pre(r), EpiDot<XT, NT>{s, rhv}, ws, st, TAIL_RHO, 1);                                          // (9), (11)
-        hipLaunchKernelGGL((k_comb<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, s, v, v, st);               // (12)
-        A.launch(sm, pre(v), EpiDot<XT, NT>{w, rhv}, ws, st, TAIL_GAMMA, 1);                                        // (13), (14)
-        hipLaunchKernelGGL((k_comb<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, s, w, s, st);                // (17)
-        if (mg) A.launch(sm, pre(s), EpiGcrP<XT, NT>{t, r, v, st, s}, ws, st, TAIL_GCR, 1);                         // (18)-(20)
-        else A.launch(sm, s, EpiGcrL<XT, NT>{t, r, v, st}, ws, st, TAIL_GCR, 1);
-        if (first && x_zero)
-            hipLaunchKernelGGL((k_pass_end<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, y, r, r, s, t, uo, u, v, w,
-                               rhv, ws, st);
-        else
-            hipLaunchKernelGGL((k_pass_end<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, y, r, r, s, t, uo, u, v,
-                               w, rhv, ws, st);
+        pub = publish(ctx);
+        if (fused) {
+            double *p0 = ws.partial, *p1 = ws.partial + 2 * kReduceBlocks;     // two dots, five dots
+            const unsigned g = A.grid(), ge = gr < kFusedEndBlocks ? gr : kFusedEndBlocks;
+            A.template step<false>(sm, StepVecs<XT>{ro, uo, uu, v, rhv, nullptr},
+                                   StepRed{nullptr, 0, p0, st, nullptr, TAIL_NONE, 0});                   // (5)-(7)
+            A.template step<false>(sm, StepVecs<XT>{ro, v, rr, s, rhv, nullptr},
+                                   StepRed{p0, g, p1, st, st + 1, TAIL_GAMMA, 1});                        // (8), (9), (11)
+            A.template step<false>(sm, StepVecs<XT>{s, v, vv, r, rhv, nullptr},
+                                   StepRed{p1, g, p0, st + 1, st + 2, TAIL_RHO, 0});                      // (12)-(14)
+            A.template step<true>(sm, StepVecs<XT>{s, r, v, u, rr, vv},
+                                  StepRed{p0, g, p1, st + 2, st + 3, TAIL_GAMMA, 1});                     // (17)-(20)
+            const EndVecs<XT> E{y, rr, v, u, uu, vv, r, rhv, r, u};
+            const StepRed R{p1, g, p0, st + 3, st + 4, TAIL_GCR, 0};
+            if (first && x_zero) hipLaunchKernelGGL((k_step_end<XT, true>), dim3(ge), dim3(kThreads), 0, sm, n, E, R);
+            else hipLaunchKernelGGL((k_step_end<XT, false>), dim3(ge), dim3(kThreads), 0, sm, n, E, R);
+            launch_finish<2>(sm, ws, ge, st, TAIL_END, 1, pub, st + 4);
+        } else {
+            if (!first) hipLaunchKernelGGL((k_comb<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, r, u, u, st);   // (5)
+            A.launch(sm, pre(uo), EpiDot<XT, NT>{v, rhv}, ws, st, TAIL_GAMMA, 1);                                       // (6), (7)
+            hipLaunchKernelGGL((k_comb<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, ro, v, r, st);               // (8)
+            A.launch(sm, pre(r), EpiDot<XT, NT>{s, rhv}, ws, st, TAIL_RHO, 1);                                          // (9), (11)
+            hipLaunchKernelGGL((k_comb<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n, s, v, v, st);               // (12)
+            A.launch(sm, pre(v), EpiDot<XT, NT>{w, rhv}, ws, st, TAIL_GAMMA, 1);                                        // (13), (14)
+            hipLaunchKernelGGL((k_comb<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n, s, w, s, st);                // (17)
+            if (mg) A.launch(sm, pre(s), EpiGcrP<XT, NT>{t, r, v, st, s}, ws, st, TAIL_GCR, 1);                         // (18)-(20)
+            else A.launch(sm, s, EpiGcrL<XT, NT>{t, r, v, st}, ws, st, TAIL_GCR, 1);
+            if (first && x_zero)
+                hipLaunchKernelGGL((k_pass_end<XT, NT, true>), dim3(gr), dim3(kThreads), 0, sm, n,
+                                   EndVecs<XT>{y, r, s, t, uo, v, w, rhv, r, u}, ws, st);
+            else
+                hipLaunchKernelGGL((k_pass_end<XT, NT, false>), dim3(gr), dim3(kThreads), 0, sm, n,
+                                   EndVecs<XT>{y, r, s, t, uo, v, w, rhv, r, u}, ws, st);
+            launch_finish<2>(sm, ws, gr, st, TAIL_END, 1, pub);
+        }
         x_written = true;
-        launch_finish<2>(sm, ws, gr, st, TAIL_END, 1);
         DARE_LAUNCH_CHECK();
-        rc = read_state(ctx, st, &h);
+        rc = wait_state(ctx, pub, &h);
         if (rc) return rc;
         if (h.status) {
             out->status = h.status;
@@ -220,8 +291,9 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, St
                                        static_cast<const XT*>(x_zero ? nullptr : x), z, t);
                     xt = t;
                 }
-                A.launch(sm, xt, EpiStart<XT, NT>{b, rh}, ws, st, TAIL_START, 0);
-                rc = read_state(ctx, st, &h);
+                pub = publish(ctx);
+                A.launch(sm, xt, EpiStart<XT, NT>{b, rh}, ws, st, TAIL_START, 0, pub);
+                rc = wait_state(ctx, pub, &h);
                 if (rc) return rc;
                 conv = h.rnorm;
                 if (conv <= tol_abs) {
@@ -282,10 +354,11 @@ static int dot_dev(dare_ctx* ctx, long long n, const double* a, const double* b,
     int rc = ws_reserve(ctx, 0, &W);
     if (rc) return rc;
     hipLaunchKernelGGL((k_dot<double>), dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream, n, a, b, ctx->ws, W.st);
-    launch_finish<1>(ctx->stream, ctx->ws, grid_for(n), W.st, TAIL_STORE, 0);
+    const Publish pub = publish(ctx);
+    launch_finish<1>(ctx->stream, ctx->ws, grid_for(n), W.st, TAIL_STORE, 0, pub);
     DARE_LAUNCH_CHECK();
     KState h;
-    rc = read_state(ctx, W.st, &h);
+    rc = wait_state(ctx, pub, &h);
     if (rc) return rc;
     *out = h.dots[0];
     return DARE_OK;
@@ -506,7 +579,7 @@ static int op64(dare_ctx* ctx, const dare_csr* A, bool allow_dia, SolveOp<double
 }  // namespace dare_hip
 
 // ---- static scratch of the allocation-free solve (dare_bicgstab2_solve_noalloc) -------------
-// Seven FP64 work vectors of at most kNoAllocMaxRows rows, the reduction partials and the
+// The FP64 work vectors of a pass for at most kNoAllocMaxRows rows, the reduction partials and the
 // device scalar block. Each device that loads this library holds its own copy until the
 // process ends. Host code never passes `scratch` itself to a kernel: its address on a device
 // comes from hipGetSymbolAddress (noalloc_scratch_init, run by dare_ctx_create with that
@@ -514,12 +587,12 @@ static int op64(dare_ctx* ctx, const dare_csr* A, bool allow_dia, SolveOp<double
 namespace dare_hip {
 namespace {
 constexpr long long kNoAllocMaxRows = 1LL << 18;                                   // 262,144 rows (64^3)
-constexpr long long kScratchVec = 7 * kNoAllocMaxRows;                            // doubles
+constexpr long long kScratchVec = kPassVecs * kNoAllocMaxRows;                    // doubles
 constexpr long long kScratchPartial = static_cast<long long>(kReduceBlocks) * kMaxDots;
-constexpr long long kScratchState = 64;                                           // KState slot
+constexpr long long kScratchState = 256;                                          // KState slots
 constexpr long long kScratchCount = 32;                                           // ReduceWs::count slot
 constexpr long long kScratchDoubles = kScratchVec + kScratchPartial + kScratchState + kScratchCount;
-static_assert(sizeof(KState) <= kScratchState * sizeof(double), "scratch state slot too small");
+static_assert(kStates * sizeof(KState) <= kScratchState * sizeof(double), "scratch state slots too small");
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double* g_scratch[kMaxDevices] = {};
@@ -607,12 +680,13 @@ int dare_residual(dare_ctx* ctx, const dare_csr* A, const double* b, const doubl
         if (rc) return rc;
     }
     hipLaunchKernelGGL(k_clear_state, dim3(1), dim3(64), 0, ctx->stream, W.st);
-    if (A->nrows >= kStreamRows) op.launch(ctx->stream, x, EpiResid64<true>{b, r}, ctx->ws, W.st, TAIL_STORE, 0);
-    else op.launch(ctx->stream, x, EpiResid64<false>{b, r}, ctx->ws, W.st, TAIL_STORE, 0);
+    const Publish pub = norm_host ? publish(ctx) : Publish{};
+    if (A->nrows >= kStreamRows) op.launch(ctx->stream, x, EpiResid64<true>{b, r}, ctx->ws, W.st, TAIL_STORE, 0, pub);
+    else op.launch(ctx->stream, x, EpiResid64<false>{b, r}, ctx->ws, W.st, TAIL_STORE, 0, pub);
     DARE_LAUNCH_CHECK();
     if (norm_host) {
         KState h;
-        rc = read_state(ctx, W.st, &h);
+        rc = wait_state(ctx, pub, &h);
         if (rc) return rc;
         *norm_host = std::sqrt(h.dots[0]);
     }
@@ -634,12 +708,14 @@ int dare_spmv_dot(dare_ctx* ctx, const dare_csr* A, const double* x, double* y, 
     SolveOp<double> op;
     rc = op64(ctx, A, true, &op, {x, y, w});
     if (rc) return rc;
-    if (A->nrows >= kStreamRows) op.launch(ctx->stream, x, EpiDot<double, true>{y, w}, ctx->ws, W.st, TAIL_STORE, 1);
-    else op.launch(ctx->stream, x, EpiDot<double, false>{y, w}, ctx->ws, W.st, TAIL_STORE, 1);
+    const Publish pub = out_host ? publish(ctx) : Publish{};
+    if (A->nrows >= kStreamRows)
+        op.launch(ctx->stream, x, EpiDot<double, true>{y, w}, ctx->ws, W.st, TAIL_STORE, 1, pub);
+    else op.launch(ctx->stream, x, EpiDot<double, false>{y, w}, ctx->ws, W.st, TAIL_STORE, 1, pub);
     DARE_LAUNCH_CHECK();
     if (out_host) {
         KState h;
-        rc = read_state(ctx, W.st, &h);
+        rc = wait_state(ctx, pub, &h);
         if (rc) return rc;
         *out_host = h.dots[0];
     }
@@ -686,7 +762,7 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* A, const double* b, doub
     const bool left = p->precond == DARE_PRECOND_JACOBI_LEFT;
     Workspace W;
     // + the preconditioned iterate (multigrid) or the scaled right-hand side (left Jacobi)
-    int rc = ws_reserve(ctx, sizeof(double) * (use_mg || left ? 8 : 7) * n, &W);
+    int rc = ws_reserve(ctx, sizeof(double) * (kPassVecs + (use_mg || left ? 1 : 0)) * n, &W);
     if (rc) return rc;
     SolveOp<double> op;
     rc = op64(ctx, A, true, &op, {b, x});
@@ -757,7 +833,7 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* A, const double* b, doub
                                A->val, A->dinv, Am->dia_pre);
             op.csr.val = Am->dia_pre;
         }
-        double* bl = static_cast<double*>(W.buf) + 7 * n;
+        double* bl = static_cast<double*>(W.buf) + kPassVecs * n;
         DARE_HIP_TRY(hipMemcpyAsync(bl, b, sizeof(double) * n, hipMemcpyDeviceToDevice, ctx->stream));
         hipLaunchKernelGGL(k_scale_by, dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream, n, bl, A->dinv, 1);
         DARE_LAUNCH_CHECK();
@@ -766,7 +842,7 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* A, const double* b, doub
     Outcome o;
     rc = bicgstab2_run<double, double>(ctx, op, bs, x, stop, p->max_it, p->history, p->history_cap, &o,
                                        static_cast<double*>(W.buf), 2, false, W.st, ctx->ws, mg,
-                                       static_cast<double*>(W.buf) + 7 * n);
+                                       static_cast<double*>(W.buf) + kPassVecs * n);
     if (rc) return rc;
     if (pre) {
         hipLaunchKernelGGL(k_scale_by, dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream, n, x, A->dinv, 1);  // x = M^-1 y
@@ -908,11 +984,11 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
         if (mrc) return mrc;
     }
     Workspace W;
-    // 7 FP32 work vectors + FP32 residual + FP32 correction
-    int rc = ws_reserve(ctx, sizeof(float) * 9 * n, &W);
+    // the FP32 work vectors + FP32 residual + FP32 correction
+    int rc = ws_reserve(ctx, sizeof(float) * (kPassVecs + 2) * n, &W);
     if (rc) return rc;
     float* work = static_cast<float*>(W.buf);
-    float* r32 = work + 7 * n;
+    float* r32 = work + kPassVecs * n;
     float* d32 = r32 + n;
     // ||b|| comes out of the first residual sweep (EpiResidB), which reads b anyway
     double bnorm = 0., tol_abs = 0.;
@@ -933,17 +1009,18 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
     const double inner_tol = p->inner_tol > 0. ? p->inner_tol : 1e-4;
     while (true) {
         const bool first = refine == 0;
+        const Publish pub = publish(ctx);
         if (first && n >= kStreamRows)
-            op.launch(ctx->stream, x, EpiResidB<true>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0);
+            op.launch(ctx->stream, x, EpiResidB<true>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0, pub);
         else if (first)
-            op.launch(ctx->stream, x, EpiResidB<false>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0);
+            op.launch(ctx->stream, x, EpiResidB<false>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0, pub);
         else if (n >= kStreamRows)
-            op.launch(ctx->stream, x, EpiResid<true>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0);
+            op.launch(ctx->stream, x, EpiResid<true>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0, pub);
         else
-            op.launch(ctx->stream, x, EpiResid<false>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0);   // r = b - A x
+            op.launch(ctx->stream, x, EpiResid<false>{b, r32}, ctx->ws, W.st, TAIL_STORE, 0, pub);   // r = b - A x
         DARE_LAUNCH_CHECK();
         KState h;
-        rc = read_state(ctx, W.st, &h);
+        rc = wait_state(ctx, pub, &h);
         if (rc) return rc;
         if (first) {
             bnorm = std::sqrt(h.dots[1]);

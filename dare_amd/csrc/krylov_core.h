@@ -152,12 +152,36 @@ __device__ inline void block_partials(double (&acc)[NDOT], ReduceWs ws) {
     block_partials_at<NDOT>(acc, ws.partial, kReduceBlocks, blockIdx.x);
 }
 
+// The scalars as the host reads them: pinned memory the finish kernel writes itself (seq last,
+// released to the system), so that a readback is neither a copy on the stream nor a stream
+// synchronisation. The host waits for its sequence number (wait_state).
+struct HostState {
+    KState k;
+    unsigned long long seq;
+};
+static_assert(sizeof(HostState) <= 64 * sizeof(double), "pinned readback block too small");
+
+__device__ inline void publish_state(HostState* host, const KState& k, unsigned long long seq) {
+    host->k = k;
+    __threadfence_system();
+    __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 constexpr int kFinishThreads = 1024;
 
+// sin / sout: the state before and after the tail (the same where no other kernel reads sin);
+// host != NULL: the new state is published to the host under seq
 template <int NDOT>
-__global__ __launch_bounds__(kFinishThreads) void k_finish(ReduceWs ws, unsigned nblocks, KState* st, int tail,
-                                                           int check_status) {
-    if (check_status && st->status) return;       // the pass has broken down: keep its state
+__global__ __launch_bounds__(kFinishThreads) void k_finish(ReduceWs ws, unsigned nblocks, const KState* sin, KState* sout,
+                                                           int tail, int check_status, HostState* host,
+                                                           unsigned long long seq) {
+    if (check_status && sin->status) {            // the pass has broken down: keep its state
+        if (threadIdx.x == 0) {
+            if (sout != sin) *sout = *sin;
+            if (host) publish_state(host, *sin, seq);
+        }
+        return;
+    }
     __shared__ double red[kMaxDots][kFinishThreads / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     double tot[NDOT];
@@ -187,7 +211,9 @@ __global__ __launch_bounds__(kFinishThreads) void k_finish(ReduceWs ws, unsigned
     if (threadIdx.x == 0) {
         double d[kMaxDots];
         for (int j = 0; j < kMaxDots; j++) d[j] = j < NDOT ? tot[j] : 0.;
-        apply_tail(tail, st, d);
+        if (sout != sin) *sout = *sin;
+        apply_tail(tail, sout, d);
+        if (host) publish_state(host, *sout, seq);
     }
 }
 
@@ -197,9 +223,17 @@ __device__ inline void grid_reduce(double (&acc)[NDOT], ReduceWs ws, KState*, in
     block_partials<NDOT>(acc, ws);
 }
 
+// Where a finish kernel publishes the state, if at all.
+struct Publish {
+    HostState* host = nullptr;
+    unsigned long long seq = 0;
+};
+
 template <int NDOT>
-inline void launch_finish(hipStream_t sm, ReduceWs ws, unsigned nblocks, KState* st, int tail, int check) {
-    hipLaunchKernelGGL((k_finish<NDOT>), dim3(1), dim3(kFinishThreads), 0, sm, ws, nblocks, st, tail, check);
+inline void launch_finish(hipStream_t sm, ReduceWs ws, unsigned nblocks, KState* st, int tail, int check,
+                          Publish pub = {}, const KState* sin = nullptr) {
+    hipLaunchKernelGGL((k_finish<NDOT>), dim3(1), dim3(kFinishThreads), 0, sm, ws, nblocks, sin ? sin : st, st, tail,
+                       check, pub.host, pub.seq);
 }
 
 // ------------------------------------------------------------------------------ operators
@@ -494,6 +528,43 @@ __device__ __forceinline__ void epi_quad(const EpiInit<XT, NT>& e, long long i, 
     }
 }
 
+// ------------------------------------------------------------------------------ operands
+// What a traversal multiplies: a vector, or the combination a - c b formed where it is read
+// (rounded to the vector type, as the vector it stands for would hold it). 1, 2 or 4 entries.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <typename XT>
+struct Comb {
+    const XT* a;
+    const XT* b;
+    double c;
+    __device__ XT of(XT av, XT bv) const {
+        return static_cast<XT>(static_cast<double>(av) - c * static_cast<double>(bv));
+    }
+};
+template <typename XT>
+__device__ __forceinline__ XT src1(const XT* x, long long i) { return x[i]; }
+template <typename XT>
+__device__ __forceinline__ XT src1(const Comb<XT>& x, long long i) { return x.of(x.a[i], x.b[i]); }
+template <typename XT>
+__device__ __forceinline__ void src2(const XT* x, long long i, double* o) {      // i even, x 2-element aligned
+    typedef XT x2 __attribute__((ext_vector_type(2)));
+    const x2 v = *reinterpret_cast<const x2*>(x + i);
+    o[0] = static_cast<double>(v.x);
+    o[1] = static_cast<double>(v.y);
+}
+template <typename XT>
+__device__ __forceinline__ void src2(const Comb<XT>& x, long long i, double* o) {
+    typedef XT x2 __attribute__((ext_vector_type(2)));
+    const x2 a = *reinterpret_cast<const x2*>(x.a + i), b = *reinterpret_cast<const x2*>(x.b + i);
+    o[0] = static_cast<double>(x.of(a.x, b.x));
+    o[1] = static_cast<double>(x.of(a.y, b.y));
+}
+__device__ __forceinline__ f32x4 src4(const float* x, long long i) { return *reinterpret_cast<const f32x4*>(x + i); }
+__device__ __forceinline__ f32x4 src4(const Comb<float>& x, long long i) {
+    const f32x4 a = src4(x.a, i), b = src4(x.b, i);
+    return f32x4{x.of(a.x, b.x), x.of(a.y, b.y), x.of(a.z, b.z), x.of(a.w, b.w)};
+}
+
 // ------------------------------------------------------------------------------ traversals
 // Generic CSR, one wave per 64 consecutive rows. The wave walks its rows' run of the CSR
 // arrays -- one contiguous range -- with coalesced loads (lane l takes entries l, l + 64, ...),
@@ -544,16 +615,10 @@ __device__ inline void csr_tile_cv(const CsrOp<VT>& A, const CsrTileRp& R, int l
     }
 }
 
-template <typename VT, typename XT, class Epi>
-__global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* __restrict__ x, Epi epi, ReduceWs ws,
-                                                       KState* st, int tail, int check_status) {
+template <typename VT, class Src, class Epi>
+__device__ inline void csr_sweep(const CsrOp<VT>& A, const Src x, const Epi& epi, double* acc) {
     __shared__ double s_prod[kCsrWaves][kCsrWaveNnz];
-    double acc[Epi::NDOT];
-#pragma unroll
-    for (int j = 0; j < Epi::NDOT; j++) acc[j] = 0.;
-    const bool run = !(check_status && st->status);
-    if (run) {
-        epi_begin(epi, 0);
+    {
         const int lane = threadIdx.x % kCsrWaveRows, wv = threadIdx.x / kCsrWaveRows;
         double* prod = s_prod[wv];
         const long long ntiles = (A.n + kCsrWaveRows - 1) / kCsrWaveRows;
@@ -575,7 +640,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
             const long long i = tile * kCsrWaveRows + lane;
             const bool own = i < A.n;
             const long long ic = own ? i : A.n - 1;      // a valid address for every lane
-            const double xi = static_cast<double>(x[ic]);
+            const double xi = static_cast<double>(src1(x, ic));
             const double pre = epi.load(ic);
             const int nnz = R0.E - R0.B, b = R0.b - R0.B, e = R0.e - R0.B;
             const bool staged = nnz <= kCsrWaveNnz;
@@ -591,7 +656,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
                 if (nnz > 0) {
                     double xv[8];
 #pragma unroll
-                    for (int u = 0; u < 8; u++) xv[u] = static_cast<double>(x[c[u]]);
+                    for (int u = 0; u < 8; u++) xv[u] = static_cast<double>(src1(x, c[u]));
 #pragma unroll
                     for (int u = 0; u < 8; u++) prod[u * kCsrWaveRows + lane] = v[u] * xv[u];
                 }
@@ -607,7 +672,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
                 wave_lds_sync();   // the slice is rewritten by the wave's next tile
             } else {
                 for (int k = R0.B + b; k < R0.B + e; k++)
-                    s += static_cast<double>(A.val[k]) * static_cast<double>(x[A.col[k]]);
+                    s += static_cast<double>(A.val[k]) * static_cast<double>(src1(x, A.col[k]));
             }
             if (own) epi(i, s, xi, pre, acc);
             R0 = R1;
@@ -618,6 +683,19 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
                 v[u] = vn[u];
             }
         }
+    }
+}
+
+template <typename VT, typename XT, class Epi>
+__global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* __restrict__ x, Epi epi, ReduceWs ws,
+                                                       KState* st, int tail, int check_status) {
+    double acc[Epi::NDOT];
+#pragma unroll
+    for (int j = 0; j < Epi::NDOT; j++) acc[j] = 0.;
+    const bool run = !(check_status && st->status);
+    if (run) {
+        epi_begin(epi, 0);
+        csr_sweep<VT>(A, x, epi, acc);
     }
     if (tail >= 0) grid_reduce<Epi::NDOT>(acc, ws, st, run ? tail : TAIL_NONE);
 }
@@ -631,8 +709,8 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
 // dia_column runs one (j, k) column of a tile over the planes i0 <= i < i1 with the i-1/i/i+1
 // values of x rolled through registers. x and D belong to one system; row0 is that system's
 // first row in the epilogue's vectors (0 for a single system).
-template <int NC, typename VT, typename XT, class Epi>
-__device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, const XT* __restrict__ x,
+template <int NC, typename VT, class Src, class Epi>
+__device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, const Src x,
                                   long long row0, int k, int j, int i0, int i1, const Epi& epi, double* acc) {
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
@@ -653,8 +731,8 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
         const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            xc[c] = static_cast<double>(x[node * NC + c]);
-            xp[c] = static_cast<double>(x[nprev * NC + c]);
+            xc[c] = static_cast<double>(src1(x, node * NC + c));
+            xp[c] = static_cast<double>(src1(x, nprev * NC + c));
         }
     }
     for (int i = i0; i < i1; i++) {
@@ -666,12 +744,7 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
             // the two component rows of a cell are adjacent (row = 2 node + c, nrows even, the
             // arrays start on 2-element boundaries): one 2-wide load per slot and per x entry
             typedef VT v2 __attribute__((ext_vector_type(2)));
-            typedef XT x2 __attribute__((ext_vector_type(2)));
-            auto ldx = [&](long long nd, double* o) {
-                const x2 v = *reinterpret_cast<const x2*>(x + nd * 2);
-                o[0] = static_cast<double>(v.x);
-                o[1] = static_cast<double>(v.y);
-            };
+            auto ldx = [&](long long nd, double* o) { src2(x, nd * 2, o); };
             ldx(nnext, xn);
             ldx(node + dS, xs);
             ldx(node + dN, xnn);
@@ -695,11 +768,11 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
 #pragma unroll
             for (int c = 0; c < NC; c++) {
                 const long long row = node * NC + c;
-                xn[c] = static_cast<double>(x[nnext * NC + c]);
-                xs[c] = static_cast<double>(x[(node + dS) * NC + c]);
-                xnn[c] = static_cast<double>(x[(node + dN) * NC + c]);
-                xb[c] = static_cast<double>(x[(node + dB) * NC + c]);
-                xt[c] = static_cast<double>(x[(node + dT) * NC + c]);
+                xn[c] = static_cast<double>(src1(x, nnext * NC + c));
+                xs[c] = static_cast<double>(src1(x, (node + dS) * NC + c));
+                xnn[c] = static_cast<double>(src1(x, (node + dN) * NC + c));
+                xb[c] = static_cast<double>(src1(x, (node + dB) * NC + c));
+                xt[c] = static_cast<double>(src1(x, (node + dT) * NC + c));
 #pragma unroll
                 for (int sl = 0; sl < 7; sl++) {
                     if constexpr (Epi::kNT) dv[c][sl] = static_cast<double>(ld_nt(D + sl * nr + row));
@@ -742,8 +815,8 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
 // the top neighbour of cell k and the bottom neighbour of cell k+1 are the pair itself; only
 // k-1 (cell k) and k+2 (cell k+1) are single loads. Each cell's sum keeps the order of
 // dia_column, so y is bit-identical; the per-lane dot accumulation order differs.
-template <typename VT, typename XT, class Epi>
-__device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ D, const XT* __restrict__ x,
+template <typename VT, class Src, class Epi>
+__device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ D, const Src x,
                                        int k, int j, int i0, int i1, const Epi& epi, double* acc) {
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
@@ -761,20 +834,20 @@ __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ 
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
         const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
-        xc0 = static_cast<double>(x[node]);
-        xc1 = static_cast<double>(x[node + 1]);
-        xp0 = static_cast<double>(x[nprev]);
-        xp1 = static_cast<double>(x[nprev + 1]);
+        xc0 = static_cast<double>(src1(x, node));
+        xc1 = static_cast<double>(src1(x, node + 1));
+        xp0 = static_cast<double>(src1(x, nprev));
+        xp1 = static_cast<double>(src1(x, nprev + 1));
     }
     for (int i = i0; i < i1; i++) {
         const bool hasW = !(i == 0 && V.rm_lo[0]);
         const bool hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
         const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
-        const double xn0 = static_cast<double>(x[nnext]), xn1 = static_cast<double>(x[nnext + 1]);
-        const double xs0 = static_cast<double>(x[node + dS]), xs1 = static_cast<double>(x[node + dS + 1]);
-        const double xq0 = static_cast<double>(x[node + dN]), xq1 = static_cast<double>(x[node + dN + 1]);
-        const double xb = static_cast<double>(x[node + dB]);
-        const double xt = static_cast<double>(x[node + 1 + dT]);
+        const double xn0 = static_cast<double>(src1(x, nnext)), xn1 = static_cast<double>(src1(x, nnext + 1));
+        const double xs0 = static_cast<double>(src1(x, node + dS)), xs1 = static_cast<double>(src1(x, node + dS + 1));
+        const double xq0 = static_cast<double>(src1(x, node + dN)), xq1 = static_cast<double>(src1(x, node + dN + 1));
+        const double xb = static_cast<double>(src1(x, node + dB));
+        const double xt = static_cast<double>(src1(x, node + 1 + dT));
         double d0[7], d1[7];
 #pragma unroll
         for (int sl = 0; sl < 7; sl++) {
@@ -819,8 +892,8 @@ __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ 
 // bit-identical. The east neighbour's W is the next plane's own W: it is loaded once and kept
 // in registers. S and B are read again as partners of the rows south and below (from the
 // caches), so they carry no non-temporal hint; C and the east W do.
-template <typename VT, typename XT, class Epi>
-__device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restrict__ D, const XT* __restrict__ x,
+template <typename VT, class Src, class Epi>
+__device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restrict__ D, const Src x,
                                            int k, int j, int i0, int i1, const Epi& epi, double* acc) {
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
@@ -846,10 +919,10 @@ __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restric
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
         const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
-        xc0 = static_cast<double>(x[node]);
-        xc1 = static_cast<double>(x[node + 1]);
-        xp0 = static_cast<double>(x[nprev]);
-        xp1 = static_cast<double>(x[nprev + 1]);
+        xc0 = static_cast<double>(src1(x, node));
+        xc1 = static_cast<double>(src1(x, node + 1));
+        xp0 = static_cast<double>(src1(x, nprev));
+        xp1 = static_cast<double>(src1(x, nprev + 1));
     }
     double w0 = ldnt(DW + node), w1 = ldnt(DW + node + 1);
     for (int i = i0; i < i1; i++) {
@@ -858,11 +931,11 @@ __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restric
         // a following plane of this tile is always node + sI (i < n0 - 1 there), so the east
         // W loaded here is that plane's own W
         const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
-        const double xn0 = static_cast<double>(x[nnext]), xn1 = static_cast<double>(x[nnext + 1]);
-        const double xs0 = static_cast<double>(x[node + dS]), xs1 = static_cast<double>(x[node + dS + 1]);
-        const double xq0 = static_cast<double>(x[node + dN]), xq1 = static_cast<double>(x[node + dN + 1]);
-        const double xb = static_cast<double>(x[node + dB]);
-        const double xt = static_cast<double>(x[node + 1 + dT]);
+        const double xn0 = static_cast<double>(src1(x, nnext)), xn1 = static_cast<double>(src1(x, nnext + 1));
+        const double xs0 = static_cast<double>(src1(x, node + dS)), xs1 = static_cast<double>(src1(x, node + dS + 1));
+        const double xq0 = static_cast<double>(src1(x, node + dN)), xq1 = static_cast<double>(src1(x, node + dN + 1));
+        const double xb = static_cast<double>(src1(x, node + dB));
+        const double xt = static_cast<double>(src1(x, node + 1 + dT));
         const double sv0 = static_cast<double>(DS[node]), sv1 = static_cast<double>(DS[node + 1]);
         const double bv0 = static_cast<double>(DB[node]), bv1 = static_cast<double>(DB[node + 1]);
         const double cv0 = ldnt(DC + node), cv1 = ldnt(DC + node + 1);
@@ -902,8 +975,8 @@ __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restric
 // float4 and a wave moves 1 KB per memory instruction. The products and sums are FP32 (the
 // precision of the inner iterations; the slot order of each row is dia_column's), the dot
 // accumulators stay FP64. Rows k..k+3 with k a multiple of 4 and n2 % 4 == 0.
-template <class Epi>
-__device__ inline void dia_column_quad(const DiaView& V, const float* __restrict__ D, const float* __restrict__ x,
+template <class Src, class Epi>
+__device__ inline void dia_column_quad(const DiaView& V, const float* __restrict__ D, const Src x,
                                        int k, int j, int i0, int i1, const Epi& epi, double* acc) {
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
@@ -916,7 +989,7 @@ __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict
     const long long dN = !hasN ? 0 : (j == n1 - 1) ? -(long long)(n1 - 1) * sJ : sJ;
     const long long dB = !hasB ? 0 : (k == 0) ? (long long)(n2 - 1) : -1;            // from cell k
     const long long dT = !hasT ? 0 : (k + 3 == n2 - 1) ? -(long long)(n2 - 1) : 1;   // from cell k+3
-    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef f32x4 f4;
     auto ld4 = [](const float* p) { return *reinterpret_cast<const f4*>(p); };
     auto ld4nt = [](const float* p) {
         if constexpr (Epi::kNT) return __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
@@ -927,15 +1000,15 @@ __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
         const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
-        xc = ld4(x + node);
-        xp = ld4(x + nprev);
+        xc = src4(x, node);
+        xp = src4(x, nprev);
     }
     for (int i = i0; i < i1; i++) {
         const bool hasW = !(i == 0 && V.rm_lo[0]);
         const bool hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
         const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
-        const f4 xn = ld4(x + nnext), xs = ld4(x + node + dS), xq = ld4(x + node + dN);
-        const float xb = x[node + dB], xt = x[node + 3 + dT];
+        const f4 xn = src4(x, nnext), xs = src4(x, node + dS), xq = src4(x, node + dN);
+        const float xb = src1(x, node + dB), xt = src1(x, node + 3 + dT);
         f4 d[7];
 #pragma unroll
         for (int sl = 0; sl < 7; sl++) d[sl] = ld4nt(D + sl * nr + node);
@@ -973,8 +1046,8 @@ __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict
 // floats and the arithmetic is that of dia_column_quad, so the results are bit-identical. The
 // W, S and B slots are read twice (as a row's own and as its neighbour's partner), the second
 // time from the caches, so they carry no non-temporal hint.
-template <class Epi>
-__device__ inline void dia_column_quad_sym(const DiaView& V, const float* __restrict__ D, const float* __restrict__ x,
+template <class Src, class Epi>
+__device__ inline void dia_column_quad_sym(const DiaView& V, const float* __restrict__ D, const Src x,
                                            int k, int j, int i0, int i1, const Epi& epi, double* acc) {
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
@@ -987,7 +1060,7 @@ __device__ inline void dia_column_quad_sym(const DiaView& V, const float* __rest
     const long long dN = !hasN ? 0 : (j == n1 - 1) ? -(long long)(n1 - 1) * sJ : sJ;
     const long long dB = !hasB ? 0 : (k == 0) ? (long long)(n2 - 1) : -1;
     const long long dT = !hasT ? 0 : (k + 3 == n2 - 1) ? -(long long)(n2 - 1) : 1;
-    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef f32x4 f4;
     auto ld4 = [](const float* p) { return *reinterpret_cast<const f4*>(p); };
     auto ld4nt = [](const float* p) {
         if constexpr (Epi::kNT) return __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
@@ -1009,11 +1082,11 @@ __device__ inline void dia_column_quad_sym(const DiaView& V, const float* __rest
         P.hasW = !(i == 0 && V.rm_lo[0]);
         P.hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
         const long long nnext = !P.hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
-        P.xn = ld4(x + nnext);
-        P.xs = ld4(x + node + dS);
-        P.xq = ld4(x + node + dN);
-        P.xb = x[node + dB];
-        P.xt = x[node + 3 + dT];
+        P.xn = src4(x, nnext);
+        P.xs = src4(x, node + dS);
+        P.xq = src4(x, node + dN);
+        P.xb = src1(x, node + dB);
+        P.xt = src1(x, node + 3 + dT);
         P.cW = ld4(DW + node);
         P.cS = ld4(DS + node);
         P.cB = ld4(DB + node);
@@ -1029,8 +1102,8 @@ __device__ inline void dia_column_quad_sym(const DiaView& V, const float* __rest
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
         const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
-        xc = ld4(x + node);
-        xp = ld4(x + nprev);
+        xc = src4(x, node);
+        xp = src4(x, nprev);
     }
     Plane cur;
     load(i0, node, cur);
@@ -1105,8 +1178,37 @@ __global__ __launch_bounds__(kThreads) void k_dia_asym(DiaView V, const VT* __re
 
 __global__ void k_set_int(int* __restrict__ p, int v) { p[0] = v; }
 
-// PAIR: cells per lane along k (1, 2, or 4 for FP32); SYM (pairs and quads): the symmetric
-// traversal, a separate instantiation so that the seven-slot one keeps its own register count
+// One work-group's tile of the view. PAIR: cells per lane along k (1, 2, or 4 for FP32); SYM
+// (pairs and quads): the symmetric traversal.
+template <int NC, int PAIR, bool SYM, typename VT, class Src, class Epi>
+__device__ inline void dia_tile(const DiaOp<VT>& A, const Src x, const Epi& epi, double* acc) {
+    const int tile = static_cast<int>(blockIdx.x % kXcd) * A.per_xcd + static_cast<int>(blockIdx.x / kXcd);
+    if (tile >= A.tiles_k * A.tiles_j * A.tiles_i) return;
+    const int tk = tile % A.tiles_k;
+    const int t2 = tile / A.tiles_k;
+    const int tj = t2 % A.tiles_j;
+    const int ti = t2 / A.tiles_j;
+    const int lane_k = threadIdx.x & ((1 << A.lk_log2) - 1);
+    const int k = ((tk << A.lk_log2) + lane_k) * PAIR;
+    const int j = tj * (kThreads >> A.lk_log2) + (threadIdx.x >> A.lk_log2);
+    if (k >= A.V.n[2] || j >= A.V.n[1]) return;
+    const int i0 = ti * A.tile_i;
+    const int i1 = (i0 + A.tile_i < A.V.n[0]) ? i0 + A.tile_i : A.V.n[0];
+    if constexpr (PAIR == 4) {
+        static_assert(std::is_same_v<VT, float>, "quad traversal is FP32");
+        if constexpr (SYM) dia_column_quad_sym(A.V, A.D, x, k, j, i0, i1, epi, acc);
+        else dia_column_quad(A.V, A.D, x, k, j, i0, i1, epi, acc);
+    } else if constexpr (PAIR == 2 && SYM) {
+        dia_column_pair_sym<VT>(A.V, A.D, x, k, j, i0, i1, epi, acc);
+    } else if constexpr (PAIR == 2) {
+        dia_column_pair<VT>(A.V, A.D, x, k, j, i0, i1, epi, acc);
+    } else {
+        dia_column<NC, VT>(A.V, A.D, x, 0, k, j, i0, i1, epi, acc);
+    }
+}
+
+// the symmetric traversal is a separate instantiation so that the seven-slot one keeps its own
+// register count
 template <int NC, typename VT, typename XT, class Epi, int PAIR = 1, bool SYM = false>
 __global__ __launch_bounds__(kThreads) void k_apply_dia(DiaOp<VT> A, const XT* __restrict__ x, Epi epi, ReduceWs ws,
                                                        KState* st, int tail, int check_status) {
@@ -1114,34 +1216,151 @@ __global__ __launch_bounds__(kThreads) void k_apply_dia(DiaOp<VT> A, const XT* _
 #pragma unroll
     for (int j = 0; j < Epi::NDOT; j++) acc[j] = 0.;
     const bool run = !(check_status && st->status);
-    const int tile = static_cast<int>(blockIdx.x % kXcd) * A.per_xcd + static_cast<int>(blockIdx.x / kXcd);
-    const int ntiles = A.tiles_k * A.tiles_j * A.tiles_i;
-    if (run && tile < ntiles) {
+    if (run) {
         epi_begin(epi, 0);
-        const int tk = tile % A.tiles_k;
-        const int t2 = tile / A.tiles_k;
-        const int tj = t2 % A.tiles_j;
-        const int ti = t2 / A.tiles_j;
-        const int lane_k = threadIdx.x & ((1 << A.lk_log2) - 1);
-        const int k = ((tk << A.lk_log2) + lane_k) * PAIR;
-        const int j = tj * (kThreads >> A.lk_log2) + (threadIdx.x >> A.lk_log2);
-        if (k < A.V.n[2] && j < A.V.n[1]) {
-            const int i0 = ti * A.tile_i;
-            const int i1 = (i0 + A.tile_i < A.V.n[0]) ? i0 + A.tile_i : A.V.n[0];
-            if constexpr (PAIR == 4) {
-                static_assert(std::is_same_v<VT, float> && std::is_same_v<XT, float>, "quad traversal is FP32");
-                if constexpr (SYM) dia_column_quad_sym<Epi>(A.V, A.D, x, k, j, i0, i1, epi, acc);
-                else dia_column_quad<Epi>(A.V, A.D, x, k, j, i0, i1, epi, acc);
-            } else if constexpr (PAIR == 2 && SYM) {
-                dia_column_pair_sym<VT, XT, Epi>(A.V, A.D, x, k, j, i0, i1, epi, acc);
-            } else if constexpr (PAIR == 2) {
-                dia_column_pair<VT, XT, Epi>(A.V, A.D, x, k, j, i0, i1, epi, acc);
-            } else {
-                dia_column<NC, VT, XT, Epi>(A.V, A.D, x, 0, k, j, i0, i1, epi, acc);
-            }
-        }
+        dia_tile<NC, PAIR, SYM>(A, x, epi, acc);
     }
     if (tail >= 0) grid_reduce<Epi::NDOT>(acc, ws, st, run ? tail : TAIL_NONE);
+}
+
+// ------------------------------------------------------------------------------ fused steps
+// Passes below kFusedRows: five launches and a finish instead of thirteen. Each operator
+// application forms its operand a - c b where it reads it (steps 5, 8, 12, 17) and writes it out
+// once; and each kernel sums the previous one's partials itself and applies the scalar update
+// (every work-group alike; the first one stores the new state for the next kernel, which reads
+// another slot), so the four finish kernels between them are gone. A small kernel is a few
+// microseconds of latency whatever it does: the 64^3 implicit step went from 233 to 172 us (with
+// the readback through pinned memory), a 160 x 120 two-component one from 200 to 123. At 128^3
+// the two forms are level (a step 37.9 us; update, sweep and finish 9.0 + 24.3 + 4.5), and above
+// 4 M rows the sweep's streaming form is not given up. The vector operations round as the
+// separate kernels do.
+template <typename XT>
+struct StepVecs {
+    const XT *a, *b;     // the operand is a - c b
+    XT* xo;              // where it goes
+    XT* y;               // A times it
+    const XT* w;         // <y, w>; for step 18: r before step 16
+    const XT* v;         // step 18: v
+};
+struct StepRed {
+    const double* pin;   // partials of the previous kernel, dot-major with stride kReduceBlocks
+    unsigned npin;
+    double* pout;
+    const KState* sin;
+    KState* sout;
+    int tail;            // TAIL_NONE: no partials to sum, the state is sin
+    int alpha;           // c = alpha, else beta
+};
+
+// The state at this kernel's start, the same in every work-group: sin after the tail with the
+// sums of pin. st: one per work-group, in LDS. Ends with a barrier; true unless broken down.
+template <int NIN>
+__device__ inline bool step_state(const StepRed& R, KState* st) {
+    __shared__ double red[NIN][kThreads / 64];
+    if (R.tail != TAIL_NONE) {
+        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        double s[NIN];
+#pragma unroll
+        for (int j = 0; j < NIN; j++) s[j] = 0.;
+        for (unsigned b0 = 0; b0 < R.npin; b0 += 4 * kThreads) {
+            double v[NIN][4];
+#pragma unroll
+            for (int j = 0; j < NIN; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const unsigned b = b0 + q * kThreads + threadIdx.x;
+                    v[j][q] = b < R.npin ? R.pin[j * kReduceBlocks + b] : 0.;
+                }
+#pragma unroll
+            for (int j = 0; j < NIN; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) s[j] += v[j][q];
+        }
+#pragma unroll
+        for (int j = 0; j < NIN; j++) {
+            const double t = wave_sum(s[j]);
+            if (lane == 0) red[j][wid] = t;
+        }
+    }
+    KState k = *R.sin;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (R.tail != TAIL_NONE && !k.status) {
+            double d[kMaxDots] = {};
+            for (int j = 0; j < NIN; j++)
+                for (int w = 0; w < kThreads / 64; w++) d[j] += red[j][w];
+            apply_tail(R.tail, &k, d);
+        }
+        *st = k;
+        if (blockIdx.x == 0 && R.sout) *R.sout = k;
+    }
+    __syncthreads();
+    return st->status == 0;
+}
+
+template <typename XT>
+struct EpiStepDot {      // the operand and out = A p; <out, w>
+    static constexpr int NDOT = 1;
+    static constexpr bool kNT = false;
+    XT* xo;
+    XT* out;
+    const XT* w;
+    __device__ double load(long long i) const { return static_cast<double>(w[i]); }
+    __device__ void operator()(long long i, double y, double xc, double wi, double* acc) const {
+        const XT yi = static_cast<XT>(y);
+        xo[i] = static_cast<XT>(xc);
+        out[i] = yi;
+        acc[0] += static_cast<double>(yi) * wi;
+    }
+};
+template <typename XT>
+struct EpiStepGcr {      // the operand s, t = A s, and step 18's five dots with r - alpha v
+    static constexpr int NDOT = 5;
+    static constexpr bool kNT = false;
+    XT* xo;
+    XT* t;
+    const XT* r;
+    const XT* v;
+    double alpha;
+    __device__ double load(long long i) const {
+        return static_cast<double>(static_cast<XT>(static_cast<double>(r[i]) - alpha * static_cast<double>(v[i])));
+    }
+    __device__ void operator()(long long i, double y, double sc, double rd, double* acc) const {
+        const XT ti = static_cast<XT>(y);
+        xo[i] = static_cast<XT>(sc);
+        t[i] = ti;
+        const double td = static_cast<double>(ti);
+        acc[0] += rd * sc;
+        acc[1] += sc * sc;
+        acc[2] += sc * td;
+        acc[3] += td * td;
+        acc[4] += rd * td;
+    }
+};
+
+// GCR: steps 17-20, else one of steps 5-7, 8-11 (its two parts) or 12-14; APPLY runs the sweep
+// over the work-group's rows
+template <bool GCR, typename XT, class Apply>
+__device__ inline void step_body(const StepVecs<XT>& S, const StepRed& R, Apply&& apply) {
+    __shared__ KState st;
+    constexpr int NDOT = GCR ? 5 : 1;
+    double acc[NDOT] = {};
+    if (step_state<1>(R, &st)) {
+        const Comb<XT> x{S.a, S.b, R.alpha ? st.alpha : st.beta};
+        if constexpr (GCR) apply(x, EpiStepGcr<XT>{S.xo, S.y, S.w, S.v, st.alpha}, acc);
+        else apply(x, EpiStepDot<XT>{S.xo, S.y, S.w}, acc);
+    }
+    block_partials_at<NDOT>(acc, R.pout, kReduceBlocks, blockIdx.x);
+}
+template <int NC, typename VT, typename XT, bool GCR, int PAIR, bool SYM>
+__global__ __launch_bounds__(kThreads) void k_step_dia(DiaOp<VT> A, StepVecs<XT> S, StepRed R) {
+    step_body<GCR>(S, R, [&](const Comb<XT>& x, const auto& epi, double* acc) {
+        dia_tile<NC, PAIR, SYM>(A, x, epi, acc);
+    });
+}
+template <typename VT, typename XT, bool GCR>
+__global__ __launch_bounds__(kThreads) void k_step_csr(CsrOp<VT> A, StepVecs<XT> S, StepRed R) {
+    step_body<GCR>(S, R, [&](const Comb<XT>& x, const auto& epi, double* acc) { csr_sweep<VT>(A, x, epi, acc); });
 }
 
 // ------------------------------------------------------------------------------ vector updates
@@ -1187,13 +1406,17 @@ __global__ __launch_bounds__(kThreads) void k_comb(long long n, const XT* a, con
 // ro, uo: r and u before the pass's last updates (the shadow residual in a first pass, which
 // reads u = r); XZERO: x was never written and counts as 0. A breakdown after step 10 leaves
 // x = x + alpha1 u, as the reference's order of the updates does.
+template <typename XT>
+struct EndVecs {
+    XT* x;
+    const XT *ro, *s, *t, *uo, *v, *w, *rh;
+    XT *r, *u;           // written: r may be ro or w, u may be uo or t
+};
 template <typename XT, bool NT, bool XZERO>
-__global__ __launch_bounds__(kThreads) void k_pass_end(long long n, XT* __restrict__ x, const XT* ro, XT* r,
-                                                       const XT* __restrict__ s, const XT* __restrict__ t, const XT* uo,
-                                                       XT* u, const XT* __restrict__ v, const XT* __restrict__ w,
-                                                       const XT* rh, ReduceWs ws, KState* st) {
-    double acc[2] = {0., 0.};
-    const bool run = st->status == 0;
+__device__ inline void pass_end(long long n, const EndVecs<XT>& E, const KState* st, bool run, double (&acc)[2]) {
+    XT* x = E.x;
+    const XT *ro = E.ro, *s = E.s, *t = E.t, *uo = E.uo, *v = E.v, *w = E.w, *rh = E.rh;
+    XT *r = E.r, *u = E.u;
     const double a1 = st->alpha1;
     if (run) {
         const double o1 = st->om1, o2 = st->om2, a = st->alpha, beta = st->beta;
@@ -1237,7 +1460,23 @@ __global__ __launch_bounds__(kThreads) void k_pass_end(long long n, XT* __restri
                                    : static_cast<XT>((XZERO ? 0. : 1. * static_cast<double>(x[i])) +
                                                      c * static_cast<double>(uo[i])));
     }
-    grid_reduce<2>(acc, ws, st, run ? TAIL_END : TAIL_NONE);
+}
+
+template <typename XT, bool NT, bool XZERO>
+__global__ __launch_bounds__(kThreads) void k_pass_end(long long n, EndVecs<XT> E, ReduceWs ws, KState* st) {
+    double acc[2] = {0., 0.};
+    pass_end<XT, NT, XZERO>(n, E, st, st->status == 0, acc);
+    block_partials<2>(acc, ws);
+}
+
+// the same as the last of the fused steps: the scalars of step 19 from the partials first
+template <typename XT, bool XZERO>
+__global__ __launch_bounds__(kThreads) void k_step_end(long long n, EndVecs<XT> E, StepRed R) {
+    __shared__ KState st;
+    double acc[2] = {0., 0.};
+    const bool run = step_state<5>(R, &st);
+    pass_end<XT, false, XZERO>(n, E, &st, run, acc);
+    block_partials_at<2>(acc, R.pout, kReduceBlocks, blockIdx.x);
 }
 
 template <typename XT>
@@ -1312,6 +1551,12 @@ __global__ void k_clear_state(KState* st) {
         st->next_status = 0;
     }
 }
+
+// Rows below which a solve runs the fused steps (figures there).
+constexpr long long kFusedRows = kStreamRows;
+constexpr unsigned kFusedEndBlocks = 512;    // k_step_end: every work-group sums all of step 18's partials
+constexpr int kStates = 5;                   // state slots of a solve, one per kernel of a fused pass
+constexpr int kPassVecs = 8;                 // work vectors of a pass (seven without the fused steps)
 
 inline unsigned grid_rows(long long n) {      // CSR traversal: kThreads rows (one per wave and 64 rows) per block and sweep
     long long g = (n + kThreads - 1) / kThreads;

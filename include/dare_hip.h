@@ -250,7 +250,7 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* csr, const double* b, do
                          const dare_solver_params* p, dare_solver_result* res);
 /* Allocation-free FP64 BiCGStab(2): the same method, kernels and results as
  * dare_bicgstab2_solve, with its work vectors, reduction partials and scalars in a static
- * device array (15.2 MB per device, held until the process ends) instead of context memory.
+ * device array (17.3 MB per device, held until the process ends) instead of context memory.
  * No counterpart in the reference: for callers that cannot allocate device memory (tight
  * serving loops, harnesses that forbid hipMalloc). It calls no hipMalloc / hipFree.
  * Limits: at most 262144 rows (a 64^3 one-component grid; larger systems return
