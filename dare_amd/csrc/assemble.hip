@@ -56,11 +56,12 @@ __device__ inline double lim_psi(int id, double r) {
         const double m = (1. < r) ? 1. : r;
         return (0. < m) ? m : 0.;
     }
-    case DARE_LIMITER_VANLEER: {
-        if (isnan(r)) return 0.;
-        if (isinf(r)) return r > 0. ? 2. : 0.;
+    case DARE_LIMITER_VANLEER: {     // branch-free: the special cases are selected over the quotient
         const double a = fabs(r);
-        return (r + a) / (1. + a);
+        double q = (r + a) / (1. + a);
+        asm volatile("" : "+v"(q));   // keeps the division unconditional (not sunk into a branch)
+        const double psi = isinf(r) ? (r > 0. ? 2. : 0.) : q;
+        return isnan(r) ? 0. : psi;
     }
     default: return 0.;
     }
@@ -97,7 +98,7 @@ constexpr int kPosOfSlot[7] = {1, 3, 5, 0, 6, 4, 2};
 // DIM = 0 takes the dimension from G at run time; DIM = 3 (the diagonal-view fill) lets every
 // per-axis loop unroll, so the per-position arrays live in registers.
 // FEAT: the terms the instantiation may meet (kFeat* bits); a cleared bit drops that term's
-// code (the host dispatches the diagonal-view fill of operators without them to FEAT = 0).
+// code (the host picks the diagonal-view fill's smallest mask that covers the operator).
 enum { kFeatConv = 1, kFeatDiffCell = 2, kFeatSource = 4, kFeatCross = 8, kFeatFixed = 16, kFeatAll = 31 };
 template <int MODE, bool SORT, int DIM = 0, int FEAT = kFeatAll>
 __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, long long node,
@@ -179,20 +180,16 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
                 const double u[2] = {T.vel[d][fi], T.vel[d][fi + T.fs[d][d]]};
                 double nb[2], cc[2], fr[2];
                 const long long s = G.sl[d] * N;
+                // the five cells of the axis, loaded whatever the signs of u (loads behind a branch
+                // on u waited one for the other); both ghost layers exist (make_terms)
+                double p[5];
+#pragma unroll
+                for (int m = 0; m < 5; m++) p[m] = T.phi[lp * N + c + (m - 2) * s];
+#pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const bool up = u[h] >= 0.;
                     const double vp = up ? 1. : 0., vn = up ? 0. : 1.;
-                    const double* base = T.phi + (lp + (h ? 0 : -G.sl[d])) * N + c;   // cell L
-                    double pUU, pU, pD;
-                    if (up) {
-                        pUU = base[-s];
-                        pU = base[0];
-                        pD = base[s];
-                    } else {
-                        pUU = base[2 * s];
-                        pU = base[s];
-                        pD = base[0];
-                    }
+                    const double pUU = up ? p[h] : p[h + 3], pU = up ? p[h + 1] : p[h + 2], pD = up ? p[h + 2] : p[h + 1];
                     const double r = (pU - pUU) / (pD - pU);
                     const double psi = lim_psi(T.conv_limiter, r);
                     if (h == 0) {
@@ -431,46 +428,54 @@ __global__ __launch_bounds__(256) void k_fill_values(Geo G, Terms T, long long n
     if (x0) x0[row] = x;
 }
 
-// Diagonal-view fill (3-D): one lane per cell, lanes along k, no column sort. Writes the slot
-// values (coalesced, slot-major), rhs and x0. The CSR values are materialized from the slots
-// only when a CSR consumer asks for them (k_materialize_csr, same sort and merge). HALF (an
-// operator symmetric by construction): only W, S, B, C are written; E, N, T equal the W, S, B
-// of the east, north and top neighbours, bit for bit (k_dia_mirror writes them on demand).
+// Diagonal-view fill (3-D): one lane per row, lanes along the rows of a (i, j) line, no column
+// sort. Writes the slot values (coalesced, slot-major), rhs and x0. The CSR values are
+// materialized from the slots only when a CSR consumer asks for them (k_materialize_csr, same
+// sort and merge). HALF (an operator symmetric by construction): only W, S, B, C are written; E,
+// N, T equal the W, S, B of the east, north and top neighbours, bit for bit (k_dia_mirror writes
+// them on demand).
+// With every term's code the kernel is bound by issue (arguments spilled to lanes, branches
+// around absent terms), hence one instantiation per common operator, before and after: cell
+// diffusivity and source, 256^3, W, S, B, C only 552 -> 366 us; TVD convection, 128^3 96 -> 75;
+// two components with a reaction, 16^3 to 64^3 cells 10.3 -> 6.7 each (a lane per cell looped over
+// its two rows before).
 template <bool NT, bool F32, int FEAT, bool HALF>
 __global__ __launch_bounds__(256) void k_fill_dia(Geo G, Terms T, double* __restrict__ dia, float* __restrict__ dia32,
                                                   int slots, double* __restrict__ rhs, double* __restrict__ x0) {
-    const int k = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int N = (FEAT & kFeatCross) ? G.N : (HALF ? 1 : G.N);
+    const int kc = blockIdx.x * 64 + (threadIdx.x & 63);            // k * N + component
     const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
     const int i = blockIdx.z;
-    if (k >= G.n[2] || j >= G.n[1]) return;
+    if (kc >= G.n[2] * N || j >= G.n[1]) return;
+    const int k = N == 1 ? kc : kc / N, c = kc - k * N;
     const int q[3] = {i, j, k};
     const long long node = (static_cast<long long>(i) * G.n[1] + j) * G.n[2] + k;
-    const long long nrows = G.ncell_int * G.N;
-    for (int c = 0; c < G.N; c++) {
-        const long long row = node * G.N + c;
-        double slotv[kDiaSlots];
-        double r = 0., x = 0.;
-        row_entries<kRowValues, false, 3, FEAT>(G, T, q, c, node, nullptr, nullptr, &r, &x, slotv);
-        if constexpr (HALF) {                           // W, S, B, C
+    const long long nrows = G.ncell_int * N;
+    const long long row = node * N + c;
+    double slotv[kDiaSlots];
+    double r = 0., x = 0.;
+    row_entries<kRowValues, false, 3, FEAT>(G, T, q, c, node, nullptr, nullptr, &r, &x, slotv);
+    if constexpr (HALF) {                           // W, S, B, C
 #pragma unroll
-            for (int sl = 0; sl < 4; sl++) put<NT>(dia + sl * nrows + row, slotv[sl]);
-            if constexpr (F32)
+        for (int sl = 0; sl < 4; sl++) put<NT>(dia + sl * nrows + row, slotv[sl]);
+        if constexpr (F32)
 #pragma unroll
-                for (int sl = 0; sl < 4; sl++) put<NT>(dia32 + sl * nrows + row, static_cast<float>(slotv[sl]));
-        } else if constexpr ((FEAT & kFeatCross) == 0) {      // seven slots
+            for (int sl = 0; sl < 4; sl++) put<NT>(dia32 + sl * nrows + row, static_cast<float>(slotv[sl]));
+    } else {
 #pragma unroll
-            for (int sl = 0; sl < 7; sl++) put<NT>(dia + sl * nrows + row, slotv[sl]);
-            if constexpr (F32)
+        for (int sl = 0; sl < 7; sl++) put<NT>(dia + sl * nrows + row, slotv[sl]);
+        if constexpr (F32)
 #pragma unroll
-                for (int sl = 0; sl < 7; sl++) put<NT>(dia32 + sl * nrows + row, static_cast<float>(slotv[sl]));
-        } else {
-            for (int sl = 0; sl < slots; sl++) put<NT>(dia + sl * nrows + row, slotv[sl]);
-            if constexpr (F32)
-                for (int sl = 0; sl < slots; sl++) put<NT>(dia32 + sl * nrows + row, static_cast<float>(slotv[sl]));
+            for (int sl = 0; sl < 7; sl++) put<NT>(dia32 + sl * nrows + row, static_cast<float>(slotv[sl]));
+        if constexpr ((FEAT & kFeatCross) != 0) {
+            if (slots == 8) {
+                put<NT>(dia + 7 * nrows + row, slotv[7]);
+                if constexpr (F32) put<NT>(dia32 + 7 * nrows + row, static_cast<float>(slotv[7]));
+            }
         }
-        put<NT>(rhs + row, r);
-        if (x0) put<NT>(x0 + row, x);
     }
+    put<NT>(rhs + row, r);
+    if (x0) put<NT>(x0 + row, x);
 }
 
 // E, N, T of every row of a one-component view from the W, S, B slots of its east, north and
@@ -789,15 +794,17 @@ int dare_csr_fill_values(dare_ctx* ctx, dare_csr* A, const dare_grid* g, const d
     for (int f = 0; f < 6; f++)
         DARE_CHECK_ARG(T.bc_type[f] == A->bc_type[f], "boundary edits differ from the structure's");
     if (A->has_dia) {
-        const dim3 grid(ceil_div(G.n[2], 64), ceil_div(G.n[1], 4), G.n[0]);
+        const dim3 grid(ceil_div(static_cast<long long>(G.n[2]) * G.N, 64), ceil_div(G.n[1], 4), G.n[0]);
         const int slots = A->cross ? 8 : 7;
         // the FP32 copy rides along once a mixed solve has used this matrix
         const bool f32 = A->dia32_mode && A->dia32 && A->cap_dia32 >= static_cast<int64_t>(slots) * nrows;
         const bool nt = A->nrows >= kStreamRows;
-        // operators with only DDT, constant / per-component diffusion and Dirichlet / Neumann
-        // edits take the instantiation without the other terms' code
-        bool plain = T.conv_limiter < 0 && !T.diff_cell && !T.source && !T.cross;
-        for (int f = 0; f < 6; f++) plain = plain && T.bc_type[f] != DARE_BC_FIXED;
+        // the terms of this operator beyond DDT, constant / per-component diffusion and
+        // Dirichlet / Neumann edits; the instantiation is the first whose mask covers them
+        int feat = (T.conv_limiter >= 0 ? kFeatConv : 0) | (T.diff_cell ? kFeatDiffCell : 0) |
+                   (T.source ? kFeatSource : 0) | (T.cross ? kFeatCross : 0);
+        for (int f = 0; f < 6; f++)
+            if (T.bc_type[f] == DARE_BC_FIXED) feat |= kFeatFixed;
         // Symmetric by construction: a face coefficient is A_d * (dnr_d * D_f) in both rows it
         // couples (with the signs exchanged twice), and the per-cell harmonic mean takes its two
         // diffusivities in face order (low cell first) from either side. Not claimed for fixed
@@ -815,12 +822,18 @@ int dare_csr_fill_values(dare_ctx* ctx, dare_csr* A, const dare_grid* g, const d
                           (!f32 || G.n[2] % 4 == 0);
         auto launch = [&](auto ntc, auto f32c, auto halfc) {
             constexpr bool NTV = decltype(ntc)::value, F32V = decltype(f32c)::value, HV = decltype(halfc)::value;
-            if (plain)
-                hipLaunchKernelGGL((k_fill_dia<NTV, F32V, 0, HV>), grid, dim3(256), 0, ctx->stream, G, T, A->dia,
-                                   F32V ? A->dia32 : nullptr, slots, rhs, x0);
-            else
-                hipLaunchKernelGGL((k_fill_dia<NTV, F32V, kFeatAll, HV>), grid, dim3(256), 0, ctx->stream, G, T,
-                                   A->dia, F32V ? A->dia32 : nullptr, slots, rhs, x0);
+            auto run = [&](auto fc) {
+                hipLaunchKernelGGL((k_fill_dia<NTV, F32V, decltype(fc)::value, HV>), grid, dim3(256), 0, ctx->stream, G,
+                                   T, A->dia, F32V ? A->dia32 : nullptr, slots, rhs, x0);
+            };
+            constexpr int kVar = kFeatDiffCell | kFeatSource;
+            if (feat == 0) run(std::integral_constant<int, 0>{});
+            else if ((feat & ~kVar) == 0) run(std::integral_constant<int, kVar>{});
+            else if constexpr (!HV) {       // a symmetric operator has none of the other terms
+                if (feat == kFeatConv) run(std::integral_constant<int, kFeatConv>{});
+                else if (feat == kFeatCross) run(std::integral_constant<int, kFeatCross>{});
+                else run(std::integral_constant<int, kFeatAll>{});
+            }
         };
         using Yes = std::true_type;
         using No = std::false_type;
