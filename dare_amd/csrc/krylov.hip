@@ -47,6 +47,9 @@ struct SolveOp {
                     if (d.sym)
                         hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4, true>), dim3(grid), dim3(kThreads), 0, sm, d,
                                            x, epi, ws, st, tail, check);
+                    else if (d.unit_c)
+                        hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4, false, true>), dim3(grid), dim3(kThreads), 0,
+                                           sm, d, x, epi, ws, st, tail, check);
                     else
                         hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4>), dim3(grid), dim3(kThreads), 0, sm, d, x,
                                            epi, ws, st, tail, check);
@@ -374,24 +377,34 @@ __global__ __launch_bounds__(kThreads) void k_dinv(long long n, const double* __
         dinv[i] = 1.0 / diag[i];
 }
 
-// out[s][r] = D[s][r] * dinv[column of slot s in row r]; a removed entry holds 0 and stays 0
-template <typename OT>
+// out[s][r] = D[s][r] * dinv[column of slot s in row r]; a removed entry holds 0 and stays 0.
+// SYM: the view's E, N, T were left out by a symmetric fill (dare_csr::ent_lazy) and are read as
+// the W, S, B of the east, north and top neighbours, so neither the fill nor a mirror pass has to
+// write them (256^3: the fill 40 bytes a row instead of 64, this kernel 316 -> 200 us).
+// skip_c: slot C is left out. In FP32 it is 1 in every row: a (1 / a) in FP64 is 1 to one unit
+// in the last place, whatever a (a zero, infinite or NaN diagonal never meets the stopping test
+// either way: the other coefficients of its column are then not finite, or A x is not).
+template <typename OT, bool SYM>
 __global__ __launch_bounds__(kThreads) void k_dia_colscale(DiaView V, const double* __restrict__ D,
-                                                           const double* __restrict__ dinv, OT* __restrict__ out) {
+                                                           const double* __restrict__ dinv, OT* __restrict__ out,
+                                                           int skip_c) {
+    // one lane per row, 64 along the rows of a (i, j) line x 4 lines (a grid-stride loop over the
+    // rows spent as long on the 64-bit divisions of their coordinates as on the memory: 286 us)
     const long long nr = V.nrows;
-    const int N = V.N;
+    const int N = SYM ? 1 : V.N;
     const long long sI = static_cast<long long>(V.n[1]) * V.n[2], sJ = V.n[2];
-    for (long long r = blockIdx.x * (long long)kThreads + threadIdx.x; r < nr; r += (long long)gridDim.x * kThreads) {
-        const long long node = r / N;
-        const int c = static_cast<int>(r % N);
-        const int k = static_cast<int>(node % V.n[2]);
-        const int j = static_cast<int>((node / V.n[2]) % V.n[1]);
-        const int i = static_cast<int>(node / sI);
+    const int kc = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (kc >= V.n[2] * N || j >= V.n[1]) return;
+    const int k = N == 1 ? kc : kc / N, c = kc - k * N;
+    for (int i = blockIdx.z; i < V.n[0]; i += gridDim.z) {
+        const long long node = (static_cast<long long>(i) * V.n[1] + j) * V.n[2] + k, r = node * N + c;
         const int pos[3] = {i, j, k};
         const long long stride[3] = {sI, sJ, 1};
         long long nb[7];
+        bool hi_gone[3];
         // slots 0 W, 1 S, 2 B, 3 C, 4 T, 5 N, 6 E: low neighbour of axis d is slot d, high is 6 - d
         nb[3] = node;
+#pragma unroll
         for (int d = 0; d < 3; d++) {
             const int n = V.n[d];
             long long lo = node - stride[d], hi = node + stride[d];
@@ -399,19 +412,35 @@ __global__ __launch_bounds__(kThreads) void k_dia_colscale(DiaView V, const doub
             if (pos[d] == n - 1) hi = V.per[d] ? node - static_cast<long long>(n - 1) * stride[d] : node;
             nb[d] = lo;
             nb[6 - d] = hi;
+            hi_gone[d] = pos[d] == n - 1 && V.rm_hi[d];
         }
         double dv[8], sc[8];
 #pragma unroll
         for (int sl = 0; sl < 7; sl++) {
-            dv[sl] = D[sl * nr + r];
+            if (SYM && sl > 3) dv[sl] = D[(6 - sl) * nr + nb[sl]];
+            else dv[sl] = D[sl * nr + r];
             sc[sl] = dinv[nb[sl] * N + c];
+        }
+        if constexpr (SYM) {
+#pragma unroll
+            for (int sl = 4; sl < 7; sl++) dv[sl] = hi_gone[6 - sl] ? 0. : dv[sl];
         }
         dv[7] = (N == 2 && V.cross) ? D[7 * nr + r] : 0.;
         sc[7] = (N == 2 && V.cross) ? dinv[node * N + (1 - c)] : 0.;
 #pragma unroll
-        for (int sl = 0; sl < 7; sl++) out[sl * nr + r] = static_cast<OT>(dv[sl] * sc[sl]);
+        for (int sl = 0; sl < 7; sl++)
+            if (sl != 3 || !skip_c) out[sl * nr + r] = static_cast<OT>(dv[sl] * sc[sl]);
         if (N == 2 && V.cross) out[7 * nr + r] = static_cast<OT>(dv[7] * sc[7]);
     }
+}
+template <typename OT>
+void launch_colscale(hipStream_t sm, const dare_csr* A, OT* out, bool skip_c = false) {
+    const DiaView& V = A->dia_view;
+    const dim3 g(ceil_div(static_cast<long long>(V.n[2]) * V.N, 64), ceil_div(V.n[1], 4), V.n[0]), b(kThreads);
+    if (A->ent_lazy)
+        hipLaunchKernelGGL((k_dia_colscale<OT, true>), g, b, 0, sm, A->dia_view, A->dia, A->dinv, out, skip_c);
+    else
+        hipLaunchKernelGGL((k_dia_colscale<OT, false>), g, b, 0, sm, A->dia_view, A->dia, A->dinv, out, skip_c);
 }
 
 // 1 / diag(A) from the CSR rows (columns ascending, duplicates merged); a row without a
@@ -777,7 +806,7 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* A, const double* b, doub
         stop = Stop{stop.abs(bnorm), false};
     }
     const bool pre = p->precond == 1;
-    if (pre || left) {          // the scaled views are made from all seven slots
+    if (left) {                 // the row scaling reads all seven slots
         rc = dia_ensure_full(const_cast<dare_csr*>(A), ctx->stream);
         if (rc) return rc;
     }
@@ -798,8 +827,7 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* A, const double* b, doub
             const int slots = A->dia_view.cross ? 8 : 7;
             rc = grow_buffer(&Am->dia_pre, &Am->cap_dia_pre, static_cast<int64_t>(slots) * n, "preconditioned view");
             if (rc) return rc;
-            hipLaunchKernelGGL((k_dia_colscale<double>), dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream,
-                               A->dia_view, A->dia, A->dinv, Am->dia_pre);
+            launch_colscale<double>(ctx->stream, A, Am->dia_pre);
             op.d = make_dia<double>(A->dia_view, Am->dia_pre, true);
         } else {                  // generic CSR: scaled copy of the values
             rc = grow_buffer(&Am->dia_pre, &Am->cap_dia_pre, A->nnz, "preconditioned values");
@@ -904,8 +932,9 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
     DARE_CHECK_ARG(p->precond >= 0 && p->precond <= 2, "precond must be 0 (none), 1 (Jacobi) or 2 (multigrid)");
     const bool pre = p->precond == 1;
     const bool use_mg = p->precond == DARE_PRECOND_MG;
+    bool unit_c = false;
     if (A->has_dia && kXcd * make_dia<double>(A->dia_view, A->dia).per_xcd <= kReduceBlocks) {
-        if (pre || use_mg) {    // the scaled FP32 view and the multigrid levels read all seven slots
+        if (use_mg) {           // the multigrid levels read all seven slots
             const int erc = dia_ensure_full(A, ctx->stream);
             if (erc) return erc;
         }
@@ -926,8 +955,10 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
         if (pre) {       // FP32 copy of A M^-1 (the inner solves run right-preconditioned)
             int prc = jacobi_setup(ctx, A);
             if (prc) return prc;
-            hipLaunchKernelGGL((k_dia_colscale<float>), dim3(grid_for(n)), dim3(kThreads), 0, ctx->stream,
-                               A->dia_view, A->dia, A->dinv, A->dia32);
+            // the streaming quad traversal takes C as 1
+            op32.d = make_dia<float>(A->dia_view, A->dia32, true);
+            unit_c = op32.d.pair == 4 && n >= kStreamRows;
+            launch_colscale<float>(ctx->stream, A, A->dia32, unit_c);
             A->dia32_fresh = 0;
         } else {
             // written by the last fill when it already ran in FP32 mode, converted here otherwise;
@@ -939,6 +970,7 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
             A->dia32_mode = 1;
         }
         op32.d = make_dia<float>(A->dia_view, A->dia32, true);
+        op32.d.unit_c = unit_c;
         op32.dia = kXcd * op32.d.per_xcd <= kReduceBlocks;
         if (op32.dia && op32.d.pair == 4 && !pre && A->sym_traversal) {
             // the FP32 copy of an exactly symmetric FP64 view is exactly symmetric (Jacobi
@@ -948,7 +980,7 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
             if (src) return src;
             op32.d.sym = A->sym64 == 1;
         }
-        if (!op32.d.sym) {      // the seven-slot FP32 traversal
+        if (!op32.d.sym && !pre) {      // the seven-slot FP32 traversal of the view as filled
             const int erc = dia_ensure_full(A, ctx->stream);
             if (erc) return erc;
         }

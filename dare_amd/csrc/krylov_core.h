@@ -255,6 +255,7 @@ struct DiaOp {
     int per_xcd;        // tiles owned by each XCD (grid = kXcd * per_xcd)
     int pair;           // cells per lane along k (2, or 4 for FP32: one component, n2 a multiple)
     bool sym = false;            // the view is exactly symmetric: the four-slot pair / quad traversals
+    bool unit_c = false;         // every C coefficient is 1 and not stored (FP32 quads, column-scaled view)
 };
 
 // Tile of a work-group: 2^lk lanes along k (pair cells each) x 256 / 2^lk rows along j, marched
@@ -975,7 +976,8 @@ __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restric
 // float4 and a wave moves 1 KB per memory instruction. The products and sums are FP32 (the
 // precision of the inner iterations; the slot order of each row is dia_column's), the dot
 // accumulators stay FP64. Rows k..k+3 with k a multiple of 4 and n2 % 4 == 0.
-template <class Src, class Epi>
+// UNIT: the C slot is 1 in every row and not read (36 instead of 40 bytes a row).
+template <bool UNIT, class Src, class Epi>
 __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict__ D, const Src x,
                                        int k, int j, int i0, int i1, const Epi& epi, double* acc) {
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
@@ -1011,7 +1013,8 @@ __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict
         const float xb = src1(x, node + dB), xt = src1(x, node + 3 + dT);
         f4 d[7];
 #pragma unroll
-        for (int sl = 0; sl < 7; sl++) d[sl] = ld4nt(D + sl * nr + node);
+        for (int sl = 0; sl < 7; sl++)
+            if (!(UNIT && sl == 3)) d[sl] = ld4nt(D + sl * nr + node);
         const double p0 = epi.load(node), p1 = epi.load(node + 1), p2 = epi.load(node + 2), p3 = epi.load(node + 3);
         const float xcv[4] = {xc.x, xc.y, xc.z, xc.w}, xpv[4] = {xp.x, xp.y, xp.z, xp.w};
         const float xsv[4] = {xs.x, xs.y, xs.z, xs.w}, xqv[4] = {xq.x, xq.y, xq.z, xq.w};
@@ -1025,7 +1028,7 @@ __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict
             s += hasS ? dv(1) * xsv[m] : 0.f;
             if (m == 0) s += hasB ? dv(2) * xb : 0.f;
             else s += dv(2) * xcv[m - 1];
-            s += dv(3) * xcv[m];
+            s += UNIT ? xcv[m] : dv(3) * xcv[m];
             if (m == 3) s += hasT ? dv(4) * xt : 0.f;
             else s += dv(4) * xcv[m + 1];
             s += hasN ? dv(5) * xqv[m] : 0.f;
@@ -1180,7 +1183,7 @@ __global__ void k_set_int(int* __restrict__ p, int v) { p[0] = v; }
 
 // One work-group's tile of the view. PAIR: cells per lane along k (1, 2, or 4 for FP32); SYM
 // (pairs and quads): the symmetric traversal.
-template <int NC, int PAIR, bool SYM, typename VT, class Src, class Epi>
+template <int NC, int PAIR, bool SYM, bool UNIT = false, typename VT, class Src, class Epi>
 __device__ inline void dia_tile(const DiaOp<VT>& A, const Src x, const Epi& epi, double* acc) {
     const int tile = static_cast<int>(blockIdx.x % kXcd) * A.per_xcd + static_cast<int>(blockIdx.x / kXcd);
     if (tile >= A.tiles_k * A.tiles_j * A.tiles_i) return;
@@ -1197,7 +1200,7 @@ __device__ inline void dia_tile(const DiaOp<VT>& A, const Src x, const Epi& epi,
     if constexpr (PAIR == 4) {
         static_assert(std::is_same_v<VT, float>, "quad traversal is FP32");
         if constexpr (SYM) dia_column_quad_sym(A.V, A.D, x, k, j, i0, i1, epi, acc);
-        else dia_column_quad(A.V, A.D, x, k, j, i0, i1, epi, acc);
+        else dia_column_quad<UNIT>(A.V, A.D, x, k, j, i0, i1, epi, acc);
     } else if constexpr (PAIR == 2 && SYM) {
         dia_column_pair_sym<VT>(A.V, A.D, x, k, j, i0, i1, epi, acc);
     } else if constexpr (PAIR == 2) {
@@ -1209,7 +1212,7 @@ __device__ inline void dia_tile(const DiaOp<VT>& A, const Src x, const Epi& epi,
 
 // the symmetric traversal is a separate instantiation so that the seven-slot one keeps its own
 // register count
-template <int NC, typename VT, typename XT, class Epi, int PAIR = 1, bool SYM = false>
+template <int NC, typename VT, typename XT, class Epi, int PAIR = 1, bool SYM = false, bool UNIT = false>
 __global__ __launch_bounds__(kThreads) void k_apply_dia(DiaOp<VT> A, const XT* __restrict__ x, Epi epi, ReduceWs ws,
                                                        KState* st, int tail, int check_status) {
     double acc[Epi::NDOT];
@@ -1218,7 +1221,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_dia(DiaOp<VT> A, const XT* _
     const bool run = !(check_status && st->status);
     if (run) {
         epi_begin(epi, 0);
-        dia_tile<NC, PAIR, SYM>(A, x, epi, acc);
+        dia_tile<NC, PAIR, SYM, UNIT>(A, x, epi, acc);
     }
     if (tail >= 0) grid_reduce<Epi::NDOT>(acc, ws, st, run ? tail : TAIL_NONE);
 }

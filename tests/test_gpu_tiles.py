@@ -100,3 +100,37 @@ def test_breakdown_after_the_first_x_update_keeps_it(ctx, n):
     r = da.refine_mixed(ctx, A, torch.from_numpy(b).cuda(), x, tol=0.0, tol_kind=0, max_refine=1)
     assert np.array_equal(x.cpu().numpy(), b / 2)
     A.close()
+
+
+def test_jacobi_scaled_views_of_half_and_full_fills_agree(ctx, rng):
+    """4 M rows, where the FP32 column-scaled view's C slot is taken as 1 and not stored: the view
+    scaled from a fill that left E, N, T out and the one scaled from all seven slots give the same
+    mixed and FP64 Jacobi solves bit for bit, to a true residual below the tolerance."""
+    import torch
+    n = [128, 128, 256]
+    g = da.Grid.make(n, ghost=2)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(11)
+    D = torch.rand(g.num_padded, generator=gen, dtype=torch.float64, device="cuda") + 0.1
+    phi = torch.rand(g.num_padded, generator=gen, dtype=torch.float64, device="cuda")
+    t = da.Terms.make(dt=2e-5, diff_cell=D, bc_type=[1, 2, 1, 1, 2, 1], bc_value=[0.3, 0, -1.0, 0.5, 0, 0.25])
+    got = {}
+    for half in (True, False):
+        A = da.Csr(ctx)
+        da.build_structure(ctx, A, g, t)
+        da.set_symmetric_traversal(A, half)
+        b = torch.zeros(g.num_cells, dtype=torch.float64, device="cuda")
+        x = torch.zeros_like(b)
+        for mixed in (True, False):
+            da.fill_values(ctx, A, g, t, phi, b, x)
+            if mixed:
+                r = da.refine_mixed(ctx, A, b, x, tol=1e-10, precond=1)
+            else:
+                r = da.bicgstab2(ctx, A, b, x, tol=1e-10, tol_kind=1, precond=1)
+            assert r["converged"] == 1
+            y = torch.zeros_like(x)
+            assert da.residual(ctx, A, b, x, y, norm=True) <= 1.01e-10 * float(b.norm())
+            got[half, mixed] = (x.cpu().numpy().copy(), r["iterations"])
+        A.close()
+    for mixed in (True, False):
+        assert bits_equal(got[True, mixed][0], got[False, mixed][0]) and got[True, mixed][1] == got[False, mixed][1]
