@@ -25,25 +25,44 @@ static FaceGeo make_face_geo(const Geo& G) {
     return F;
 }
 
-// Launch shape: x along axis dim-1 (64 lanes), y along axis dim-2, z along axis dim-3.
+// Launch shape of the kernels for any dimension and component count: one lane per (cell,
+// component), x along axis dim-1 with the components innermost, y along axis dim-2, z along axis
+// dim-3; 64 x 4 lanes, or 32 x 8 or 16 x 16 where that saves an eighth of the work-groups (for
+// 5 % fewer, the shorter rows of writes cost more: the case below 83 us instead of 77).
+// A lane per cell that looped over its N components made every access of a wave N doubles apart:
+// three components on 97 x 131 x 115 cells, gradient and divergence 119 us a pair with the ghost
+// fill, now 77 (a contiguous run of tiles per die instead of tiles in order: 82, the face arrays'
+// writes then go to eight places at once).
 struct Launch {
     dim3 grid, block;
 };
 
 static Launch cell_launch(const Geo& G) {
     Launch L;
-    L.block = dim3(64, G.dim >= 2 ? 4 : 1, 1);
     const int ax_x = G.dim - 1, ax_y = G.dim - 2, ax_z = G.dim - 3;
-    L.grid = dim3(ceil_div(G.n[ax_x], 64), ax_y >= 0 ? ceil_div(G.n[ax_y], 4) : 1, ax_z >= 0 ? G.n[ax_z] : 1);
+    const long long nx = static_cast<long long>(G.n[ax_x]) * G.N;
+    if (ax_y < 0) {
+        L.block = dim3(64);
+        L.grid = dim3(ceil_div(nx, 64));
+        return L;
+    }
+    unsigned lanes = 64;
+    const auto tiles = [&](unsigned l) { return static_cast<long long>(ceil_div(nx, l)) * ceil_div(G.n[ax_y], 256 / l); };
+    for (unsigned l = 32; l >= 16; l /= 2)
+        if (8 * tiles(l) <= 7 * tiles(lanes)) lanes = l;
+    L.block = dim3(lanes, 256 / lanes);
+    L.grid = dim3(ceil_div(nx, lanes), ceil_div(G.n[ax_y], 256 / lanes), ax_z >= 0 ? G.n[ax_z] : 1);
     return L;
 }
 
 template <int DIM>
-__device__ inline bool cell_coord(const Geo& G, int q[3]) {
+__device__ inline bool cell_coord(const Geo& G, int q[3], int& c) {
     q[0] = q[1] = q[2] = 0;
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    q[DIM - 1] = a;
-    if (a >= G.n[DIM - 1]) return false;
+    const unsigned a = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned N = static_cast<unsigned>(G.N), k = N == 1 ? a : a / N;
+    c = static_cast<int>(a - k * N);
+    q[DIM - 1] = static_cast<int>(k);
+    if (k >= static_cast<unsigned>(G.n[DIM - 1])) return false;
     if (DIM >= 2) {
         const int b = blockIdx.y * blockDim.y + threadIdx.y;
         if (b >= G.n[DIM - 2]) return false;
@@ -99,76 +118,73 @@ __device__ inline double limiter(int id, double r) {
     }
 }
 
-// TVD face value between cells L and L+1 along a stride s (TVD_Cartesian.inl:133-157).
-// base points at component c of cell L.
-__device__ inline double tvd_face(const double* __restrict__ base, long long s, int lim, double u) {
+// Face value between L and L+1 given the four cells a = L-1, b = L, c = L+1, d = L+2
+// (TVD_Cartesian.inl:133-157), times the face velocity.
+__device__ inline double tvd_flux4(double a, double b, double c, double d, int lim, double u) {
     double pUU, pU, pD;
     if (u >= 0.) {
-        pUU = base[-s];
-        pU = base[0];
-        pD = base[s];
+        pUU = a;
+        pU = b;
+        pD = c;
     } else {
-        pUU = base[2 * s];
-        pU = base[s];
-        pD = base[0];
+        pUU = d;
+        pU = c;
+        pD = b;
     }
     const double r = (pU - pUU) / (pD - pU);
     const double psi = limiter(lim, r);
-    return pU + (psi * 0.5) * (pD - pU);
+    return (pU + (psi * 0.5) * (pD - pU)) * u;
 }
 
 // ------------------------------------------------------------------------------ ghost fill
 struct GhostSlabs {
     long long start[7];      // prefix offsets of the 6 slabs (W,E,S,N,B,T)
-    int other[6][2];         // the two non-normal axes per slab (or -1)
     int mode[6];
     double value[6];
 };
 
-template <int DIM>
-__global__ void k_ghost_fill(Geo G, GhostSlabs S, double* __restrict__ phi) {
-    const long long t = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= S.start[2 * DIM]) return;
+// One lane per ghost value (slab by slab, components innermost); I: 32-bit indices where they hold
+// the count, whose divisions by the extents are a fraction of the 64-bit ones (2-D 128 x 128
+// periodic 3.5 -> 3.1 us, three components on 97 x 131 x 115 cells 7.5 -> 6.3).
+template <int DIM, typename I>
+__global__ __launch_bounds__(256) void k_ghost_fill(Geo G, GhostSlabs S, double* __restrict__ phi) {
+    I r = static_cast<I>(blockIdx.x) * 256 + threadIdx.x;
+    if (r >= static_cast<I>(S.start[2 * DIM] * G.N)) return;
+    const I N = static_cast<I>(G.N);
+    int c = 0;
+    if (G.N > 1) {
+        const I t = r / N;
+        c = static_cast<int>(r - t * N);
+        r = t;
+    }
     int f = 0;
-    while (f < 2 * DIM - 1 && t >= S.start[f + 1]) f++;
-    if (S.mode[f] == DARE_GHOST_LEAVE) return;
-    long long r = t - S.start[f];
+#pragma unroll
+    for (int e = 1; e < 2 * DIM; e++) f = r >= static_cast<I>(S.start[e]) ? e : f;
+    const int mode = S.mode[f];
+    if (mode == DARE_GHOST_LEAVE) return;
+    r -= static_cast<I>(S.start[f]);
     const int d = f / 2;
     const bool low = (f % 2) == 0;
     int p[3] = {0, 0, 0};       // padded index
     // decompose r over (layer, other axes) with the last other axis fastest
-    int o1 = S.other[f][0], o2 = S.other[f][1];
-    int i2 = 0, i1 = 0;
-    if (o2 >= 0) {
-        i2 = static_cast<int>(r % G.n[o2]);
-        r /= G.n[o2];
-    }
-    if (o1 >= 0) {
-        i1 = static_cast<int>(r % G.n[o1]);
-        r /= G.n[o1];
+#pragma unroll
+    for (int e = DIM - 1; e >= 0; e--) {
+        if (e == d) continue;
+        const I n = static_cast<I>(G.n[e]), t = r / n;
+        p[e] = static_cast<int>(r - t * n) + G.g;
+        r = t;
     }
     const int l = static_cast<int>(r) + 1;   // ghost layer 1..g
-    if (o1 >= 0) p[o1] = i1 + G.g;
-    if (o2 >= 0) p[o2] = i2 + G.g;
-    p[d] = low ? G.g - l : G.g + G.n[d] - 1 + l;
-    int src[3] = {p[0], p[1], p[2]};
-    if (S.mode[f] == DARE_GHOST_PERIODIC) src[d] = G.g + (low ? G.n[d] - l : l - 1);
-    else src[d] = G.g + (low ? l - 1 : G.n[d] - l);
-    long long od = 0, os = 0;
-    for (int e = 0; e < DIM; e++) {
-        od += G.sl[e] * p[e];
-        os += G.sl[e] * src[e];
-    }
-    for (int c = 0; c < G.N; c++) {
-        const double s = phi[os * G.N + c];
-        double v;
-        switch (S.mode[f]) {
-        case DARE_GHOST_DIRICHLET: v = 2. * S.value[f] - s; break;
-        case DARE_GHOST_CONSTANT: v = S.value[f]; break;
-        default: v = s; break;
-        }
-        phi[od * G.N + c] = v;
-    }
+    const int n = G.n[d];
+    const int to = low ? G.g - l : G.g + n - 1 + l;
+    const int from = mode == DARE_GHOST_PERIODIC ? G.g + (low ? n - l : l - 1) : G.g + (low ? l - 1 : n - l);
+    long long o = 0;
+#pragma unroll
+    for (int e = 0; e < DIM; e++) o += G.sl[e] * p[e];
+    double* line = phi + o * G.N + c;
+    const long long sd = G.sl[d] * G.N;
+    const double s = line[from * sd];
+    line[to * sd] = mode == DARE_GHOST_DIRICHLET ? 2. * S.value[f] - s : mode == DARE_GHOST_CONSTANT ? S.value[f] : s;
 }
 
 // --------------------------------------------------------------------------- face gradient
@@ -177,22 +193,24 @@ template <int DIM>
 __global__ __launch_bounds__(256) void k_grad_faces(Geo G, FaceGeo F, const double* __restrict__ phi,
                                                     double* __restrict__ f0, double* __restrict__ f1,
                                                     double* __restrict__ f2) {
-    int q[3];
-    if (!cell_coord<DIM>(G, q)) return;
+    int q[3], c;
+    if (!cell_coord<DIM>(G, q, c)) return;
     double* out[3] = {f0, f1, f2};
-    const long long lp = pad_ord<DIM>(G, q);
     const int N = G.N;
+    const double* b = phi + pad_ord<DIM>(G, q) * N + c;
+    const double pc = b[0];
+    double lo[DIM], hi[DIM];
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
         const long long s = G.sl[d] * N;
-        const long long fo = face_ord<DIM>(F, d, q) * N;
-        const bool last = q[d] == G.n[d] - 1;
-        for (int c = 0; c < N; c++) {
-            const double* b = phi + lp * N + c;
-            const double pc = b[0];
-            out[d][fo + c] = (pc - b[-s]) * G.dnr[d];
-            if (last) out[d][fo + F.fs[d][d] * N + c] = (b[s] - pc) * G.dnr[d];
-        }
+        lo[d] = b[-s];
+        hi[d] = b[q[d] == G.n[d] - 1 ? s : 0];
+    }
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+        double* o = out[d] + face_ord<DIM>(F, d, q) * N + c;
+        o[0] = (pc - lo[d]) * G.dnr[d];
+        if (q[d] == G.n[d] - 1) o[F.fs[d][d] * N] = (hi[d] - pc) * G.dnr[d];
     }
 }
 
@@ -206,8 +224,8 @@ __global__ __launch_bounds__(256) void k_interp_faces(Geo G, FaceGeo F, const do
                                                       const double* __restrict__ u1, const double* __restrict__ u2,
                                                       double* __restrict__ f0, double* __restrict__ f1,
                                                       double* __restrict__ f2) {
-    int q[3];
-    if (!cell_coord<DIM>(G, q)) return;
+    int q[3], c;
+    if (!cell_coord<DIM>(G, q, c)) return;
     const double* in[3] = {u0, u1, u2};
     double* out[3] = {f0, f1, f2};
     const long long lp = pad_ord<DIM>(G, q);
@@ -234,23 +252,25 @@ __global__ __launch_bounds__(256) void k_div_faces(Geo G, FaceGeo F, const doubl
                                                    const double* __restrict__ f1,
                                                    const double* __restrict__ f2,
                                                    double* __restrict__ out) {
-    int q[3];
-    if (!cell_coord<DIM>(G, q)) return;
+    int q[3], c;
+    if (!cell_coord<DIM>(G, q, c)) return;
     const double* in[3] = {f0, f1, f2};
-    const long long lp = pad_ord<DIM>(G, q);
     const int N = G.N;
-    for (int c = 0; c < N; c++) {
-        double v = 0.;
+    double lo[DIM], hi[DIM];
 #pragma unroll
-        for (int d = 0; d < DIM; d++) {
-            const long long fo = face_ord<DIM>(F, d, q) * N + c;
-            const double lo = in[d][fo], hi = in[d][fo + F.fs[d][d] * N];
-            if (d == 0) v = G.A[0] * hi;
-            else v += G.A[d] * hi;
-            v -= G.A[d] * lo;
-        }
-        out[lp * N + c] = v;
+    for (int d = 0; d < DIM; d++) {
+        const double* f = in[d] + face_ord<DIM>(F, d, q) * N + c;
+        lo[d] = f[0];
+        hi[d] = f[F.fs[d][d] * N];
     }
+    double v = G.A[0] * hi[0];
+    v -= G.A[0] * lo[0];
+#pragma unroll
+    for (int d = 1; d < DIM; d++) {
+        v += G.A[d] * hi[d];
+        v -= G.A[d] * lo[d];
+    }
+    out[pad_ord<DIM>(G, q) * N + c] = v;
 }
 
 // -------------------------------------------------------------------------- TVD face flux
@@ -260,24 +280,26 @@ __global__ __launch_bounds__(256) void k_tvd_flux(Geo G, FaceGeo F, int lim, con
                                                   const double* __restrict__ u1,
                                                   const double* __restrict__ u2, double* __restrict__ f0,
                                                   double* __restrict__ f1, double* __restrict__ f2) {
-    int q[3];
-    if (!cell_coord<DIM>(G, q)) return;
+    int q[3], c;
+    if (!cell_coord<DIM>(G, q, c)) return;
     const double* vel[3] = {u0, u1, u2};
     double* out[3] = {f0, f1, f2};
-    const long long lp = pad_ord<DIM>(G, q);
     const int N = G.N;
+    const double* b = phi + pad_ord<DIM>(G, q) * N + c;
+    double p[DIM][5], ulo[DIM], uhi[DIM];       // every load first: the five cells of each axis
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-        const long long s = G.sl[d] * N;
-        const long long fi = face_ord<DIM>(F, d, q);
-        const double ulo = vel[d][fi];
-        const bool last = q[d] == G.n[d] - 1;
-        const double uhi = last ? vel[d][fi + F.fs[d][d]] : 0.;
-        for (int c = 0; c < N; c++) {
-            const double* b = phi + lp * N + c;
-            out[d][fi * N + c] = tvd_face(b - s, s, lim, ulo) * ulo;
-            if (last) out[d][(fi + F.fs[d][d]) * N + c] = tvd_face(b, s, lim, uhi) * uhi;
-        }
+        const long long s = G.sl[d] * N, fi = face_ord<DIM>(F, d, q);
+#pragma unroll
+        for (int m = 0; m < 5; m++) p[d][m] = b[(m - 2) * s];
+        ulo[d] = vel[d][fi];
+        uhi[d] = vel[d][q[d] == G.n[d] - 1 ? fi + F.fs[d][d] : fi];
+    }
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+        double* o = out[d] + face_ord<DIM>(F, d, q) * N + c;
+        o[0] = tvd_flux4(p[d][0], p[d][1], p[d][2], p[d][3], lim, ulo[d]);
+        if (q[d] == G.n[d] - 1) o[F.fs[d][d] * N] = tvd_flux4(p[d][1], p[d][2], p[d][3], p[d][4], lim, uhi[d]);
     }
 }
 
@@ -290,111 +312,34 @@ __global__ __launch_bounds__(256) void k_tvd_step(Geo G, FaceGeo F, int lim, con
                                                   const double* __restrict__ u1,
                                                   const double* __restrict__ u2, double fac,
                                                   double* __restrict__ phi_out) {
-    int q[3];
-    if (!cell_coord<DIM>(G, q)) return;
+    int q[3], c;
+    if (!cell_coord<DIM>(G, q, c)) return;
     const double* vel[3] = {u0, u1, u2};
-    const long long lp = pad_ord<DIM>(G, q);
     const int N = G.N;
-    double ulo[3], uhi[3];
+    const long long at = pad_ord<DIM>(G, q) * N + c;
+    const double* b = phi + at;
+    double p[DIM][5], ulo[DIM], uhi[DIM];
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-        const long long fi = face_ord<DIM>(F, d, q);
+        const long long s = G.sl[d] * N, fi = face_ord<DIM>(F, d, q);
+#pragma unroll
+        for (int m = 0; m < 5; m++) p[d][m] = b[(m - 2) * s];
         ulo[d] = vel[d][fi];
         uhi[d] = vel[d][fi + F.fs[d][d]];
     }
-    for (int c = 0; c < N; c++) {
-        const double* b = phi + lp * N + c;
-        double v = 0.;
+    double v = 0.;
 #pragma unroll
-        for (int d = 0; d < DIM; d++) {
-            const long long s = G.sl[d] * N;
-            const double flo = tvd_face(b - s, s, lim, ulo[d]) * ulo[d];
-            const double fhi = tvd_face(b, s, lim, uhi[d]) * uhi[d];
-            if (d == 0) v = G.A[0] * fhi;
-            else v += G.A[d] * fhi;
-            v -= G.A[d] * flo;
-        }
-        phi_out[lp * N + c] = b[0] - fac * v;
+    for (int d = 0; d < DIM; d++) {
+        const double flo = tvd_flux4(p[d][0], p[d][1], p[d][2], p[d][3], lim, ulo[d]);
+        const double fhi = tvd_flux4(p[d][1], p[d][2], p[d][3], p[d][4], lim, uhi[d]);
+        if (d == 0) v = G.A[0] * fhi;
+        else v += G.A[d] * fhi;
+        v -= G.A[d] * flo;
     }
-}
-
-// Face value between L and L+1 given the four cells a = L-1, b = L, c = L+1, d = L+2
-// (same selection and arithmetic as tvd_face), times the face velocity.
-__device__ inline double tvd_flux4(double a, double b, double c, double d, int lim, double u) {
-    double pUU, pU, pD;
-    if (u >= 0.) {
-        pUU = a;
-        pU = b;
-        pD = c;
-    } else {
-        pUU = d;
-        pU = c;
-        pD = b;
-    }
-    const double r = (pU - pUU) / (pD - pU);
-    const double psi = limiter(lim, r);
-    return (pU + (psi * 0.5) * (pD - pU)) * u;
+    phi_out[at] = p[0][2] - fac * v;
 }
 
 constexpr int kStepTileK = 64, kStepTileJ = 4, kStepXcd = 8, kStepMinPlanes = 8;
-
-// One x-march of a 64 (k) x 4 (j) column over the planes [i0, i1): the planes i-2..i+2 of phi
-// stay in registers and the x-face flux at (i, i+1) is carried to the next plane as its low
-// face. NT streams the x-face velocities in and the result out with the non-temporal hint.
-template <bool NT>
-__device__ __forceinline__ void tvd_march3(const Geo& G, int lim, const double* __restrict__ phi,
-                                           const double* __restrict__ ux, const double* __restrict__ uy,
-                                           const double* __restrict__ uz, double fac, double* __restrict__ out,
-                                           int k, int j, int i0, int i1) {
-    const int n1 = G.n[1], n2 = G.n[2];
-    const long long sI = G.sl[0], sJ = G.sl[1];
-    long long lp = (static_cast<long long>(i0 + G.g) * G.np[1] + (j + G.g)) * G.np[2] + (k + G.g);
-    // face arrays: x (n0+1, n1, n2), y (n0, n1+1, n2), z (n0, n1, n2+1)
-    const long long fxs = static_cast<long long>(n1) * n2;
-    long long fx = static_cast<long long>(i0) * fxs + static_cast<long long>(j) * n2 + k;
-    long long fy = (static_cast<long long>(i0) * (n1 + 1) + j) * n2 + k;
-    const long long fys = static_cast<long long>(n1 + 1) * n2;
-    long long fz = (static_cast<long long>(i0) * n1 + j) * (n2 + 1) + k;
-    const long long fzs = static_cast<long long>(n1) * (n2 + 1);
-    double pm2 = phi[lp - 2 * sI], pm1 = phi[lp - sI], p0 = phi[lp], pp1 = phi[lp + sI];
-    double f_lo = tvd_flux4(pm2, pm1, p0, pp1, lim, ux[fx]);
-    const double A0 = G.A[0], A1 = G.A[1], A2 = G.A[2];
-    for (int i = i0; i < i1; i++) {
-        // every load of the plane first: x (i+2 and the face velocity), y (cells j-2..j+2),
-        // z (cells k-2..k+2); the scheduling barrier keeps them ahead of the divisions
-        const double pp2 = phi[lp + 2 * sI];
-        double u_hi;
-        if constexpr (NT) u_hi = ld_nt(ux + fx + fxs);
-        else u_hi = ux[fx + fxs];
-        const double ym2 = phi[lp - 2 * sJ], ym1 = phi[lp - sJ], yp1 = phi[lp + sJ], yp2 = phi[lp + 2 * sJ];
-        const double vy_lo = uy[fy], vy_hi = uy[fy + n2];
-        const double zm2 = phi[lp - 2], zm1 = phi[lp - 1], zp1 = phi[lp + 1], zp2 = phi[lp + 2];
-        const double wz_lo = uz[fz], wz_hi = uz[fz + 1];
-        __builtin_amdgcn_sched_barrier(0);
-        const double f_hi = tvd_flux4(pm1, p0, pp1, pp2, lim, u_hi);
-        const double gy_lo = tvd_flux4(ym2, ym1, p0, yp1, lim, vy_lo);
-        const double gy_hi = tvd_flux4(ym1, p0, yp1, yp2, lim, vy_hi);
-        const double hz_lo = tvd_flux4(zm2, zm1, p0, zp1, lim, wz_lo);
-        const double hz_hi = tvd_flux4(zm1, p0, zp1, zp2, lim, wz_hi);
-        double v = A0 * f_hi;
-        v -= A0 * f_lo;
-        v += A1 * gy_hi;
-        v -= A1 * gy_lo;
-        v += A2 * hz_hi;
-        v -= A2 * hz_lo;
-        put<NT>(out + lp, p0 - fac * v);
-        // roll
-        pm2 = pm1;
-        pm1 = p0;
-        p0 = pp1;
-        pp1 = pp2;
-        f_lo = f_hi;
-        lp += sI;
-        fx += fxs;
-        fy += fys;
-        fz += fzs;
-    }
-}
 
 // Walks logical block L's column-plane range [L*chunk, (L+1)*chunk) (columns of 64 PW (k) x 4
 // (j) cells ordered k-tile fastest, planes along i; lane l takes cells PW l .. PW l + PW - 1 of
@@ -418,15 +363,20 @@ __device__ __forceinline__ void march_columns(const Geo& G, int tiles_k, long lo
     }
 }
 
-// LDS-staged march of one full 64 (k) x TJ (j) tile (all 64 TJ threads active, so the block can
-// synchronise). Plane i of phi is staged with two ghost rows and columns (rows j0-2..j0+TJ+1,
-// columns k0-2..k0+65), each y and z face flux of the plane is computed once, by one lane, and
-// shared through LDS (the face between rows j-1 and j by the lane of cell j; the top face row
-// by the last wave; the right face column by lanes 0..TJ-1 of wave 0), and every cell combines
-// its six fluxes in the order of tvd_march3. Each flux has the same four cells and velocity as
-// there, so the result is bit-identical with about (3 + 2/TJ) / 5 of the flux evaluations and
-// five loads per cell and plane instead of fourteen. The x faces stay in registers as in
-// tvd_march3. Waves 0, 1 stage the two ghost rows below the tile, waves 2, 3 the two above.
+// LDS-staged march of a 64 (k) x TJ (j) tile over the planes [i0, i1) (all 64 TJ threads active,
+// so the block can synchronise). The planes i-2..i+2 of phi at a cell stay in registers and the
+// x-face flux at (i, i+1) is carried to the next plane as its low face. Plane i of phi is staged
+// with two ghost rows and columns (rows j0-2..j0+TJ+1, columns k0-2..k0+65), each y and z face
+// flux of the plane is computed once, by one lane, and shared through LDS (the face between rows
+// j-1 and j by the lane of cell j; the top face row by the last wave; the right face column by
+// lanes 0..TJ-1 of wave 0): (3 + 2/TJ) fluxes and five loads per cell and plane instead of five
+// and fourteen. Waves 0, 1 stage the two ghost rows below the tile, waves 2, 3 the two above. NT
+// streams the x-face velocities in and the result out with the non-temporal hint.
+// In a tile cut by the grid's edge the lanes past the last cell take the coordinates of the
+// nearest ghost cell (of phi) or face: the first two of them stage the high ghost layers and
+// compute the last faces like any other lane, and none of them stores. (Such tiles used to march
+// without LDS, five fluxes and fourteen loads per cell: 150 x 161 x 173, a third of whose tiles
+// are cut, 57.5 -> 54.3 us.)
 constexpr int kTvdRow = 68;   // staged row: 2 + 64 + 2 doubles
 template <bool NT, int TJ>
 __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const double* __restrict__ phi,
@@ -435,29 +385,36 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
                                                int k0, int j0, int i0, int i1, double* T, double* Fy, double* Fz) {
     static_assert(TJ >= 4 && TJ <= 16, "ghost rows are staged by waves 0..3, ghost columns by wave 1");
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int k = k0 + lane, j = j0 + w;
     const int n1 = G.n[1], n2 = G.n[2];
+    const bool own = k0 + lane < n2 && j0 + w < n1;
+    // this lane's cell of phi (ghost layers n, n + 1 at most), its x face and its low y, z faces
+    const auto upto = [](int v, int most) { return v < most ? v : most; };
+    const int k = upto(k0 + lane, n2 + 1), j = upto(j0 + w, n1 + 1);
+    const int kx = upto(k0 + lane, n2 - 1), jx = upto(j0 + w, n1 - 1);
+    const int jy = upto(j0 + w, n1), kz = upto(k0 + lane, n2);
     const long long sI = G.sl[0], sJ = G.sl[1];
     long long lp = (static_cast<long long>(i0 + G.g) * G.np[1] + (j + G.g)) * G.np[2] + (k + G.g);
     const long long fxs = static_cast<long long>(n1) * n2;
-    long long fx = static_cast<long long>(i0) * fxs + static_cast<long long>(j) * n2 + k;
-    long long fy = (static_cast<long long>(i0) * (n1 + 1) + j) * n2 + k;
+    long long fx = static_cast<long long>(i0) * fxs + static_cast<long long>(jx) * n2 + kx;
+    long long fy = (static_cast<long long>(i0) * (n1 + 1) + jy) * n2 + kx;
     const long long fys = static_cast<long long>(n1 + 1) * n2;
-    long long fz = (static_cast<long long>(i0) * n1 + j) * (n2 + 1) + k;
+    long long fz = (static_cast<long long>(i0) * n1 + jx) * (n2 + 1) + kz;
     const long long fzs = static_cast<long long>(n1) * (n2 + 1);
     // ghost row staged by waves 0..3: j0-2, j0-1, j0+TJ, j0+TJ+1 (staged rows 0, 1, TJ+2, TJ+3)
     const bool hload = w < 4;
     const int hj = w < 2 ? w - 2 : TJ + w - 2;                  // tile-relative row
-    const long long hoff = static_cast<long long>(hj - w) * sJ;
+    const long long hoff = static_cast<long long>(upto(j0 + hj, n1 + 1) - j) * sJ;
     const int hrow = hj + 2;
     // ghost columns (wave 1, lanes 0..4 TJ-1): rows j0..j0+TJ-1 x columns k0-2, k0-1, k0+64, k0+65
     const int gr = lane >> 2, gq = lane & 3;
     const int gdk = gq < 2 ? gq - 2 : 62 + gq;                  // -2, -1, 64, 65
-    const long long goff = static_cast<long long>(gr - w) * sJ + (gdk - lane);   // from this lane's cell
+    const long long goff = static_cast<long long>(upto(j0 + gr, n1 + 1) - j) * sJ + (upto(k0 + gdk, n2 + 1) - k);
     const int gslot = (2 + gr) * kTvdRow + (gdk + 2);
     const bool gload = w == 1 && lane < 4 * TJ;
-    // right face column (wave 0, lanes 0..TJ-1): row j0+lane, face k0+64
-    const long long zx_off = (static_cast<long long>(lane) - w) * (n2 + 1) + (64 - lane);
+    // top face row (last wave): face j0 + TJ; right face column (wave 0, lanes 0..TJ-1): row
+    // j0 + lane, face k0 + 64; both only meet cells of a tile that is full along their axis
+    const long long ty_off = static_cast<long long>(upto(j0 + TJ, n1) - jy) * n2;
+    const long long zx_off = static_cast<long long>(upto(j0 + lane, n1 - 1) - jx) * (n2 + 1) + (upto(k0 + 64, n2) - kz);
     double pm2 = phi[lp - 2 * sI], pm1 = phi[lp - sI], p0 = phi[lp], pp1 = phi[lp + sI];
     double f_lo = tvd_flux4(pm2, pm1, p0, pp1, lim, ux[fx]);
     const double A0 = G.A[0], A1 = G.A[1], A2 = G.A[2];
@@ -469,7 +426,7 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
         else u_hi = ux[fx + fxs];
         const double hal = hload ? phi[lp + hoff] : 0.;
         const double vy = uy[fy], wz = uz[fz];
-        const double vyt = w == TJ - 1 ? uy[fy + n2] : 0.;
+        const double vyt = w == TJ - 1 ? uy[fy + ty_off] : 0.;
         const double wzr = (w == 0 && lane < TJ) ? uz[fz + zx_off] : 0.;
         const double gv = gload ? phi[lp + goff] : 0.;
         Trow[0] = p0;
@@ -500,7 +457,7 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
         v -= A1 * gy_lo;
         v += A2 * hz_hi;
         v -= A2 * hz_lo;
-        put<NT>(out + lp, p0 - fac * v);
+        if (own) put<NT>(out + lp, p0 - fac * v);
         pm2 = pm1;
         pm1 = p0;
         p0 = pp1;
@@ -515,9 +472,8 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
 
 // 3-D, one component, persistent and balanced TVD step over 64 (k) x kStepTvdJ (j) tiles.
 // Logical block L takes the column-plane range [L*chunk, (L+1)*chunk) (the walk of
-// march_columns); a piece of a full tile marches with the LDS-staged form, a piece of an edge
-// tile (k or j extent cut by the grid) with the register form, each lane on its own. The
-// limiter is a template parameter so that each instantiation carries only its own branch.
+// march_columns). The limiter is a template parameter so that each instantiation carries only its
+// own branch.
 constexpr int kStepTvdJ = 8;
 template <bool NT, int LIM>
 __global__ __launch_bounds__(64 * kStepTvdJ) void k_tvd_step3(Geo G, const double* __restrict__ phi,
@@ -539,12 +495,7 @@ __global__ __launch_bounds__(64 * kStepTvdJ) void k_tvd_step3(Geo G, const doubl
         const int i1 = (cend - c < n0 - i0) ? i0 + static_cast<int>(cend - c) : n0;
         const int k0 = static_cast<int>(col % tiles_k) * kStepTileK;
         const int j0 = static_cast<int>(col / tiles_k) * kStepTvdJ;
-        if (k0 + kStepTileK <= G.n[2] && j0 + kStepTvdJ <= G.n[1]) {      // block-uniform
-            tvd_march3_lds<NT, kStepTvdJ>(G, LIM, phi, ux, uy, uz, fac, out, k0, j0, i0, i1, T, Fy, Fz);
-        } else {
-            const int k = k0 + (threadIdx.x & 63), j = j0 + (threadIdx.x >> 6);
-            if (k < G.n[2] && j < G.n[1]) tvd_march3<NT>(G, LIM, phi, ux, uy, uz, fac, out, k, j, i0, i1);
-        }
+        tvd_march3_lds<NT, kStepTvdJ>(G, LIM, phi, ux, uy, uz, fac, out, k0, j0, i0, i1, T, Fy, Fz);
         c += i1 - i0;
     }
 }
@@ -732,14 +683,20 @@ __global__ __launch_bounds__(256) void k_stream_probe(const dvec2* __restrict__ 
 
 template <int DIM>
 __global__ __launch_bounds__(256) void k_copy_to_field(Geo G, const double* __restrict__ x, double* __restrict__ phi) {
-    int q[3];
-    if (!cell_coord<DIM>(G, q)) return;
+    int q[3], c;
+    if (!cell_coord<DIM>(G, q, c)) return;
     long long nd = 0;
 #pragma unroll
     for (int d = 0; d < DIM; d++) nd += G.si[d] * q[d];
-    const long long lp = pad_ord<DIM>(G, q);
-    for (int c = 0; c < G.N; c++) phi[lp * G.N + c] = x[nd * G.N + c];
+    phi[pad_ord<DIM>(G, q) * G.N + c] = x[nd * G.N + c];
 }
+
+// Cells from which the 3-D one-component stencils march along i in persistent work-groups. Below,
+// a launch of one lane per cell is over before a march of eight planes (its shortest): TVD van
+// Leer 24^3 10.6 us marched, 4.6 not; 64^3 14.6 and 6.7; 96^3 22.8 and 17.5; level at 1.3 M cells;
+// 150 x 161 x 173 50 and 66. Gradient 64^3 6.9 and 4.7, divergence level below 1 M, 8.6 and 11.0 at
+// 1.3 M.
+constexpr long long kMarchCells = 1LL << 20;
 
 // Balanced persistent schedule of the 3-D marching kernels: as many 256-thread blocks as stay
 // resident at once (per_cu, queried once per kernel), each with at least kStepMinPlanes planes.
@@ -887,27 +844,27 @@ int dare_ghost_fill(dare_ctx* ctx, const dare_grid* g, const int32_t* mode6, con
         S.value[f] = value6 ? value6[f] : 0.;
         DARE_CHECK_ARG(S.mode[f] >= 0 && S.mode[f] <= DARE_GHOST_CONSTANT, "invalid ghost mode");
         DARE_CHECK_ARG(!(S.mode[f] == DARE_GHOST_PERIODIC && !G.per[d]), "periodic ghost fill on a non-periodic axis");
-        int k = 0;
-        S.other[f][0] = S.other[f][1] = -1;
         long long cnt = 0;
         if (f < 2 * G.dim) {
             cnt = G.g;
             for (int e = 0; e < G.dim; e++)
-                if (e != d) {
-                    S.other[f][k++] = e;
-                    cnt *= G.n[e];
-                }
+                if (e != d) cnt *= G.n[e];
         }
         S.start[f + 1] = S.start[f] + cnt;
     }
-    const long long total = S.start[2 * G.dim];
+    const long long total = S.start[2 * G.dim] * G.N;
     if (total == 0) return DARE_OK;
     const dim3 grid(ceil_div(total, 256)), block(256);
-    switch (G.dim) {
-    case 1: hipLaunchKernelGGL(k_ghost_fill<1>, grid, block, 0, ctx->stream, G, S, phi); break;
-    case 2: hipLaunchKernelGGL(k_ghost_fill<2>, grid, block, 0, ctx->stream, G, S, phi); break;
-    default: hipLaunchKernelGGL(k_ghost_fill<3>, grid, block, 0, ctx->stream, G, S, phi); break;
-    }
+    const auto launch = [&](auto index) {
+        using I = decltype(index);
+        switch (G.dim) {
+        case 1: hipLaunchKernelGGL((k_ghost_fill<1, I>), grid, block, 0, ctx->stream, G, S, phi); break;
+        case 2: hipLaunchKernelGGL((k_ghost_fill<2, I>), grid, block, 0, ctx->stream, G, S, phi); break;
+        default: hipLaunchKernelGGL((k_ghost_fill<3, I>), grid, block, 0, ctx->stream, G, S, phi); break;
+        }
+    };
+    if (total < (1LL << 31)) launch(0u);
+    else launch(0ULL);
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }
@@ -921,7 +878,7 @@ int dare_grad_faces(dare_ctx* ctx, const dare_grid* g, const double* phi, double
     DARE_CHECK_ARG(G.g >= 1, "face gradient needs >= 1 ghost layer");
     DARE_CHECK_ARG(G.dim < 2 || fy, "fy is NULL");
     DARE_CHECK_ARG(G.dim < 3 || fz, "fz is NULL");
-    if (G.dim == 3 && G.N == 1) {
+    if (G.dim == 3 && G.N == 1 && G.ncell_int >= kMarchCells) {
         if (G.ncell_int >= kStreamRows) launch_grad3<true>(ctx, G, phi, fx, fy, fz);
         else launch_grad3<false>(ctx, G, phi, fx, fy, fz);
         DARE_LAUNCH_CHECK();
@@ -960,7 +917,7 @@ int dare_div_faces(dare_ctx* ctx, const dare_grid* g, const double* fx, const do
     if (rc) return rc;
     DARE_CHECK_ARG(G.dim < 2 || fy, "fy is NULL");
     DARE_CHECK_ARG(G.dim < 3 || fz, "fz is NULL");
-    if (G.dim == 3 && G.N == 1) {
+    if (G.dim == 3 && G.N == 1 && G.ncell_int >= kMarchCells) {
         if (G.ncell_int >= kStreamRows) launch_div3<true>(ctx, G, fx, fy, fz, out);
         else launch_div3<false>(ctx, G, fx, fy, fz, out);
         DARE_LAUNCH_CHECK();
@@ -1005,7 +962,7 @@ int dare_tvd_explicit_step(dare_ctx* ctx, const dare_grid* g, int32_t limiter, c
     const FaceGeo F = make_face_geo(G);
     const Launch L = cell_launch(G);
     const double fac = dt / G.V;
-    if (G.dim == 3 && G.N == 1) {
+    if (G.dim == 3 && G.N == 1 && G.ncell_int >= kMarchCells) {
         if (G.ncell_int >= kStreamRows) launch_step3_lim<true>(ctx, G, limiter, phi, ux, uy, uz, fac, phi_out);
         else launch_step3_lim<false>(ctx, G, limiter, phi, ux, uy, uz, fac, phi_out);
         DARE_LAUNCH_CHECK();
