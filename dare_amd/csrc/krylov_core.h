@@ -301,28 +301,6 @@ DiaOp<VT> make_dia(const DiaView& V, const VT* D, bool allow_pair = false) {
 // operator() gets y = (A x)_i, xc = x_i and the loaded operands, stores results and adds to
 // the per-thread dot accumulators.
 template <typename XT, bool NT = false>
-// r = b - A x; rh = r; u = 0; <r,r>, <rh,r>   (BiCGStab2.inl:265-273). The reference also sets
-// v = w = 0; here both are written (by the SpMVs of steps 6 and 13) before the first pass reads
-// them, so those two zero sweeps are left out. v and w are kept in the member list for the
-// batched solver's call sites.
-struct EpiInit {
-    static constexpr int NDOT = 2;
-    static constexpr bool kNT = NT;
-    const XT* b;
-    XT *r, *rh, *u, *v, *w;
-    __device__ double load(long long i) const { return static_cast<double>(b[i]); }
-    __device__ void operator()(long long i, double y, double, double bi, double* acc) const {
-        const XT ri = static_cast<XT>(bi - y);
-        put<NT>(r + i, ri);
-        put<NT>(rh + i, ri);
-        put<NT>(u + i, XT(0));
-        const double rd = static_cast<double>(ri);
-        acc[0] += rd * rd;
-        acc[1] += rd * rd;
-    }
-};
-
-template <typename XT, bool NT = false>
 struct EpiDot {         // out = A p; <out, w>                   (6)-(7), (9)+(11), (13)-(14)
     static constexpr int NDOT = 1;
     static constexpr bool kNT = NT;
@@ -336,30 +314,16 @@ struct EpiDot {         // out = A p; <out, w>                   (6)-(7), (9)+(1
     }
 };
 
-template <typename XT, bool NT = false>
-struct EpiGcr {         // t = A s; <r,s>, <s,s>, <s,t>, <t,t>, <r,t>   (18)-(20)
-    static constexpr int NDOT = 5;
-    static constexpr bool kNT = NT;
-    XT* t;
-    const XT* r;
-    __device__ double load(long long i) const { return static_cast<double>(r[i]); }
-    __device__ void operator()(long long i, double y, double sc, double rd, double* acc) const {
-        const XT ti = static_cast<XT>(y);
-        put<NT>(t + i, ti);
-        const double td = static_cast<double>(ti);
-        acc[0] += rd * sc;
-        acc[1] += sc * sc;
-        acc[2] += sc * td;
-        acc[3] += td * td;
-        acc[4] += rd * td;
-    }
-};
-
 // Epilogues that need a scalar of the device state read it once per work-item, in begin().
 template <class Epi>
 __device__ inline auto epi_begin(Epi& e, int) -> decltype(e.begin()) { return e.begin(); }
 template <class Epi>
 __device__ inline void epi_begin(Epi&, long) {}
+// the same where the state is not the epilogue's own (the batched solver's, one per system)
+template <class Epi>
+__device__ inline auto epi_begin(Epi& e, const KState& k, int) -> decltype(e.begin(k)) { return e.begin(k); }
+template <class Epi>
+__device__ inline void epi_begin(Epi&, const KState&, long) {}
 
 // r = b - A x into rh alone; <r,r>, <b,b>. The shadow residual never changes, so the first pass
 // reads it as r and as u (u = r - beta u with u = 0) and writes both vectors itself: nothing
@@ -391,7 +355,8 @@ struct EpiGcrL {
     const XT* v;
     const KState* st;
     double alpha = 0.;
-    __device__ void begin() { alpha = st->alpha; }
+    __device__ void begin() { begin(*st); }
+    __device__ void begin(const KState& k) { alpha = k.alpha; }
     __device__ double load(long long i) const {
         return static_cast<double>(static_cast<XT>(static_cast<double>(r[i]) - alpha * static_cast<double>(v[i])));
     }
@@ -474,61 +439,21 @@ struct EpiStore {
     }
 };
 
-// The epilogue of a lane's two adjacent rows i, i+1 (paired traversal): by default two calls,
-// whose single stores land next to each other and merge into one wide store; EpiInit writes
-// three vectors per row, so its pair form orders the stores vector by vector for the same
-// effect. The dot accumulators see row i, then row i+1, as with two calls.
+// The epilogue of a lane's two adjacent rows i, i+1 (paired traversal): two calls, whose single
+// stores land next to each other and merge into one wide store.
 template <class Epi>
 __device__ __forceinline__ void epi_pair(const Epi& e, long long i, double y0, double y1, double x0, double x1,
                                          double p0, double p1, double* acc) {
     e(i, y0, x0, p0, acc);
     e(i + 1, y1, x1, p1, acc);
 }
-template <typename XT, bool NT>
-__device__ __forceinline__ void epi_pair(const EpiInit<XT, NT>& e, long long i, double y0, double y1, double,
-                                         double, double b0, double b1, double* acc) {
-    const XT r0 = static_cast<XT>(b0 - y0), r1 = static_cast<XT>(b1 - y1);
-    put<NT>(e.r + i, r0);
-    put<NT>(e.r + i + 1, r1);
-    put<NT>(e.rh + i, r0);
-    put<NT>(e.rh + i + 1, r1);
-    put<NT>(e.u + i, XT(0));
-    put<NT>(e.u + i + 1, XT(0));
-    const double d0 = static_cast<double>(r0), d1 = static_cast<double>(r1);
-    acc[0] += d0 * d0;
-    acc[1] += d0 * d0;
-    acc[0] += d1 * d1;
-    acc[1] += d1 * d1;
-}
-
-// The epilogue of four adjacent rows (the FP32 quad traversal): four calls, or for EpiInit the
-// stores ordered vector by vector, as epi_pair.
+// The epilogue of four adjacent rows (the FP32 quad traversal): four calls.
 template <class Epi>
 __device__ __forceinline__ void epi_quad(const Epi& e, long long i, const double* y, const double* xc,
                                          const double* pre, double* acc) {
 #pragma unroll
     for (int m = 0; m < 4; m++) e(i + m, y[m], xc[m], pre[m], acc);
 }
-template <typename XT, bool NT>
-__device__ __forceinline__ void epi_quad(const EpiInit<XT, NT>& e, long long i, const double* y, const double*,
-                                         const double* b, double* acc) {
-    XT r[4];
-#pragma unroll
-    for (int m = 0; m < 4; m++) r[m] = static_cast<XT>(b[m] - y[m]);
-#pragma unroll
-    for (int m = 0; m < 4; m++) put<NT>(e.r + i + m, r[m]);
-#pragma unroll
-    for (int m = 0; m < 4; m++) put<NT>(e.rh + i + m, r[m]);
-#pragma unroll
-    for (int m = 0; m < 4; m++) put<NT>(e.u + i + m, XT(0));
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-        const double dd = static_cast<double>(r[m]);
-        acc[0] += dd * dd;
-        acc[1] += dd * dd;
-    }
-}
-
 // ------------------------------------------------------------------------------ operands
 // What a traversal multiplies: a vector, or the combination a - c b formed where it is read
 // (rounded to the vector type, as the vector it stands for would hold it). 1, 2 or 4 entries.
@@ -710,9 +635,11 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
 // dia_column runs one (j, k) column of a tile over the planes i0 <= i < i1 with the i-1/i/i+1
 // values of x rolled through registers. x and D belong to one system; row0 is that system's
 // first row in the epilogue's vectors (0 for a single system).
-template <int NC, typename VT, class Src, class Epi>
+// COPY: each slot value is also written to D32 in FP32 (every row is visited once per sweep).
+template <int NC, typename VT, bool COPY = false, class Src, class Epi>
 __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, const Src x,
-                                  long long row0, int k, int j, int i0, int i1, const Epi& epi, double* acc) {
+                                  long long row0, int k, int j, int i0, int i1, const Epi& epi, double* acc,
+                                  float* __restrict__ D32 = nullptr) {
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
     const long long nr = V.nrows;
@@ -740,7 +667,8 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
         const bool hasW = !(i == 0 && V.rm_lo[0]);
         const bool hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
         const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
-        double xn[NC], xs[NC], xnn[NC], xb[NC], xt[NC], dv[NC][8], pre[NC];
+        double xn[NC], xs[NC], xnn[NC], xb[NC], xt[NC], pre[NC];
+        VT dv[NC][8];      // converted where they are used: FP32 slots take half the registers
         if constexpr (NC == 2) {
             // the two component rows of a cell are adjacent (row = 2 node + c, nrows even, the
             // arrays start on 2-element boundaries): one 2-wide load per slot and per x entry
@@ -760,8 +688,13 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
                     if constexpr (Epi::kNT) d = __builtin_nontemporal_load(p);
                     else d = *p;
                 }
-                dv[0][sl] = static_cast<double>(d.x);
-                dv[1][sl] = static_cast<double>(d.y);
+                dv[0][sl] = d.x;
+                dv[1][sl] = d.y;
+                if constexpr (COPY) {
+                    typedef float f2 __attribute__((ext_vector_type(2)));
+                    if (sl < nsl)
+                        *reinterpret_cast<f2*>(D32 + sl * nr + node * 2) = f2{static_cast<float>(d.x), static_cast<float>(d.y)};
+                }
             }
 #pragma unroll
             for (int c = 0; c < NC; c++) pre[c] = epi.load(row0 + node * NC + c);
@@ -776,10 +709,11 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
                 xt[c] = static_cast<double>(src1(x, (node + dT) * NC + c));
 #pragma unroll
                 for (int sl = 0; sl < 7; sl++) {
-                    if constexpr (Epi::kNT) dv[c][sl] = static_cast<double>(ld_nt(D + sl * nr + row));
-                    else dv[c][sl] = static_cast<double>(D[sl * nr + row]);
+                    if constexpr (Epi::kNT) dv[c][sl] = ld_nt(D + sl * nr + row);
+                    else dv[c][sl] = D[sl * nr + row];
+                    if constexpr (COPY) D32[sl * nr + row] = static_cast<float>(dv[c][sl]);
                 }
-                dv[c][7] = 0.;
+                dv[c][7] = VT(0);
                 pre[c] = epi.load(row0 + row);
             }
         }
@@ -787,16 +721,17 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
         // invariant code motion promotes a store out of a one-trip loop and drops its
         // non-temporal hint on the way)
         auto row_out = [&](const int c) {
+            const auto d = [&](int sl) { return static_cast<double>(dv[c][sl]); };
             double s = 0.;
-            s += hasW ? dv[c][0] * xp[c] : 0.;
-            s += hasS ? dv[c][1] * xs[c] : 0.;
-            s += hasB ? dv[c][2] * xb[c] : 0.;
-            if (NC == 2 && V.cross && c == 1) s += dv[c][7] * xc[0];
-            s += dv[c][3] * xc[c];
-            if (NC == 2 && V.cross && c == 0) s += dv[c][7] * xc[NC - 1];
-            s += hasT ? dv[c][4] * xt[c] : 0.;
-            s += hasN ? dv[c][5] * xnn[c] : 0.;
-            s += hasE ? dv[c][6] * xn[c] : 0.;
+            s += hasW ? d(0) * xp[c] : 0.;
+            s += hasS ? d(1) * xs[c] : 0.;
+            s += hasB ? d(2) * xb[c] : 0.;
+            if (NC == 2 && V.cross && c == 1) s += d(7) * xc[0];
+            s += d(3) * xc[c];
+            if (NC == 2 && V.cross && c == 0) s += d(7) * xc[NC - 1];
+            s += hasT ? d(4) * xt[c] : 0.;
+            s += hasN ? d(5) * xnn[c] : 0.;
+            s += hasE ? d(6) * xn[c] : 0.;
             epi(row0 + node * NC + c, s, xc[c], pre[c], acc);
         };
         row_out(0);
@@ -1502,7 +1437,7 @@ __global__ __launch_bounds__(kThreads) void k_dot(long long n, const XT* __restr
 }
 
 // Initialisation (0)-(2) for a zero initial guess: A x0 is +0 in every row, so r = b - A x0 = b
-// bit for bit, and <r,r>, <rh,r> go to the reduction as EpiInit's do. Nothing is written: the
+// bit for bit, and <r,r>, <rh,r> go to the reduction. Nothing is written: the
 // first pass reads b where it would read r or u and 0 where it would read x, and writes them.
 // rh = r0 is never written again, so the caller reads b itself as rh (b stays untouched during
 // the solve); v and w are written before they are read.
