@@ -455,6 +455,26 @@ __device__ __forceinline__ void epi_quad(const Epi& e, long long i, const double
     for (int m = 0; m < 4; m++) e(i + m, y[m], xc[m], pre[m], acc);
 }
 // ------------------------------------------------------------------------------ operands
+// Element offsets within one system's slot or vector. Where a sweep does not stream from memory
+// they are 32 bits, also in bytes (kDiaRows; only a grid most of whose rows are identities fits
+// more rows under the 2^31 entries of a matrix, and is applied from its CSR values): a load then
+// takes a scalar base and one register of offset instead of a 64-bit address per access, which
+// gives the fused steps a wave more per SIMD (128^3, seven slots: 37.9 -> 31.1 us). The streaming
+// sweeps keep 64 bits: with eight waves per SIMD instead of six the symmetric pairs evict the
+// partner slots they are about to read again (256^3: 179 -> 192 us). So does the five-dot sweep of
+// step 18, which reads two vectors more (128^3: 33.5 us, with 32 bits 40.2).
+constexpr long long kDiaRows = 1LL << 29;
+template <class Epi>
+using SweepIndex = std::conditional_t<Epi::kNT || Epi::NDOT == 5, long long, unsigned>;
+template <typename T>
+__device__ __forceinline__ const T* at_off(const T* base, unsigned e) {
+    return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + e * static_cast<unsigned>(sizeof(T)));
+}
+template <typename T>
+__device__ __forceinline__ const T* at_off(const T* base, long long e) { return base + e; }
+template <typename T>
+__device__ __forceinline__ const T* at_off(const T* base, int e) { return base + e; }      // CSR columns
+
 // What a traversal multiplies: a vector, or the combination a - c b formed where it is read
 // (rounded to the vector type, as the vector it stands for would hold it). 1, 2 or 4 entries.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -467,26 +487,29 @@ struct Comb {
         return static_cast<XT>(static_cast<double>(av) - c * static_cast<double>(bv));
     }
 };
-template <typename XT>
-__device__ __forceinline__ XT src1(const XT* x, long long i) { return x[i]; }
-template <typename XT>
-__device__ __forceinline__ XT src1(const Comb<XT>& x, long long i) { return x.of(x.a[i], x.b[i]); }
-template <typename XT>
-__device__ __forceinline__ void src2(const XT* x, long long i, double* o) {      // i even, x 2-element aligned
+template <typename XT, typename Ix>
+__device__ __forceinline__ XT src1(const XT* x, Ix i) { return *at_off(x, i); }
+template <typename XT, typename Ix>
+__device__ __forceinline__ XT src1(const Comb<XT>& x, Ix i) { return x.of(*at_off(x.a, i), *at_off(x.b, i)); }
+template <typename XT, typename Ix>
+__device__ __forceinline__ void src2(const XT* x, Ix i, double* o) {      // i even, x 2-element aligned
     typedef XT x2 __attribute__((ext_vector_type(2)));
-    const x2 v = *reinterpret_cast<const x2*>(x + i);
+    const x2 v = *reinterpret_cast<const x2*>(at_off(x, i));
     o[0] = static_cast<double>(v.x);
     o[1] = static_cast<double>(v.y);
 }
-template <typename XT>
-__device__ __forceinline__ void src2(const Comb<XT>& x, long long i, double* o) {
+template <typename XT, typename Ix>
+__device__ __forceinline__ void src2(const Comb<XT>& x, Ix i, double* o) {
     typedef XT x2 __attribute__((ext_vector_type(2)));
-    const x2 a = *reinterpret_cast<const x2*>(x.a + i), b = *reinterpret_cast<const x2*>(x.b + i);
+    const x2 a = *reinterpret_cast<const x2*>(at_off(x.a, i)),
+             b = *reinterpret_cast<const x2*>(at_off(x.b, i));
     o[0] = static_cast<double>(x.of(a.x, b.x));
     o[1] = static_cast<double>(x.of(a.y, b.y));
 }
-__device__ __forceinline__ f32x4 src4(const float* x, long long i) { return *reinterpret_cast<const f32x4*>(x + i); }
-__device__ __forceinline__ f32x4 src4(const Comb<float>& x, long long i) {
+template <typename Ix>
+__device__ __forceinline__ f32x4 src4(const float* x, Ix i) { return *reinterpret_cast<const f32x4*>(at_off(x, i)); }
+template <typename Ix>
+__device__ __forceinline__ f32x4 src4(const Comb<float>& x, Ix i) {
     const f32x4 a = src4(x.a, i), b = src4(x.b, i);
     return f32x4{x.of(a.x, b.x), x.of(a.y, b.y), x.of(a.z, b.z), x.of(a.w, b.w)};
 }
@@ -640,23 +663,24 @@ template <int NC, typename VT, bool COPY = false, class Src, class Epi>
 __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, const Src x,
                                   long long row0, int k, int j, int i0, int i1, const Epi& epi, double* acc,
                                   float* __restrict__ D32 = nullptr) {
+    using Ix = SweepIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
-    const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
+    const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
     // j and k neighbours: presence (boundary edits) and wrap
     const bool hasS = !(j == 0 && V.rm_lo[1]);
     const bool hasN = !(j == n1 - 1 && V.rm_hi[1] && !(j == 0 && V.rm_lo[1]));
     const bool hasB = !(k == 0 && V.rm_lo[2]);
     const bool hasT = !(k == n2 - 1 && V.rm_hi[2] && !(k == 0 && V.rm_lo[2]));
-    const long long dS = !hasS ? 0 : (j == 0) ? (long long)(n1 - 1) * sJ : -sJ;
-    const long long dN = !hasN ? 0 : (j == n1 - 1) ? -(long long)(n1 - 1) * sJ : sJ;
-    const long long dB = !hasB ? 0 : (k == 0) ? (long long)(n2 - 1) : -1;
-    const long long dT = !hasT ? 0 : (k == n2 - 1) ? -(long long)(n2 - 1) : 1;
-    long long node = (static_cast<long long>(i0) * n1 + j) * n2 + k;
+    const Ix dS = !hasS ? 0 : (j == 0) ? (n1 - 1) * sJ : 0 - sJ;
+    const Ix dN = !hasN ? 0 : (j == n1 - 1) ? 0 - (n1 - 1) * sJ : sJ;
+    const Ix dB = !hasB ? 0 : (k == 0) ? sJ - one : 0 - one;
+    const Ix dT = !hasT ? 0 : (k == n2 - 1) ? one - sJ : one;
+    Ix node = (static_cast<Ix>(i0) * n1 + j) * n2 + k;
     double xp[NC], xc[NC];
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
-        const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
+        const Ix nprev = !need ? node : (i0 == 0) ? node + (n0 - 1) * sI : node - sI;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             xc[c] = static_cast<double>(src1(x, node * NC + c));
@@ -666,14 +690,14 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
     for (int i = i0; i < i1; i++) {
         const bool hasW = !(i == 0 && V.rm_lo[0]);
         const bool hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
-        const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
+        const Ix nnext = !hasE ? node : (i == n0 - 1) ? node - (n0 - 1) * sI : node + sI;
         double xn[NC], xs[NC], xnn[NC], xb[NC], xt[NC], pre[NC];
         VT dv[NC][8];      // converted where they are used: FP32 slots take half the registers
         if constexpr (NC == 2) {
             // the two component rows of a cell are adjacent (row = 2 node + c, nrows even, the
             // arrays start on 2-element boundaries): one 2-wide load per slot and per x entry
             typedef VT v2 __attribute__((ext_vector_type(2)));
-            auto ldx = [&](long long nd, double* o) { src2(x, nd * 2, o); };
+            auto ldx = [&](Ix nd, double* o) { src2(x, nd * 2, o); };
             ldx(nnext, xn);
             ldx(node + dS, xs);
             ldx(node + dN, xnn);
@@ -684,7 +708,7 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
             for (int sl = 0; sl < 8; sl++) {
                 v2 d = v2{VT(0), VT(0)};
                 if (sl < nsl) {
-                    const v2* p = reinterpret_cast<const v2*>(D + sl * nr + node * 2);
+                    const v2* p = reinterpret_cast<const v2*>(at_off(D + sl * nr, node * 2));
                     if constexpr (Epi::kNT) d = __builtin_nontemporal_load(p);
                     else d = *p;
                 }
@@ -701,7 +725,7 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
         } else {
 #pragma unroll
             for (int c = 0; c < NC; c++) {
-                const long long row = node * NC + c;
+                const Ix row = node * NC + c;
                 xn[c] = static_cast<double>(src1(x, nnext * NC + c));
                 xs[c] = static_cast<double>(src1(x, (node + dS) * NC + c));
                 xnn[c] = static_cast<double>(src1(x, (node + dN) * NC + c));
@@ -709,8 +733,8 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
                 xt[c] = static_cast<double>(src1(x, (node + dT) * NC + c));
 #pragma unroll
                 for (int sl = 0; sl < 7; sl++) {
-                    if constexpr (Epi::kNT) dv[c][sl] = ld_nt(D + sl * nr + row);
-                    else dv[c][sl] = D[sl * nr + row];
+                    if constexpr (Epi::kNT) dv[c][sl] = ld_nt(at_off(D + sl * nr, row));
+                    else dv[c][sl] = *at_off(D + sl * nr, row);
                     if constexpr (COPY) D32[sl * nr + row] = static_cast<float>(dv[c][sl]);
                 }
                 dv[c][7] = VT(0);
@@ -754,22 +778,23 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
 template <typename VT, class Src, class Epi>
 __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ D, const Src x,
                                        int k, int j, int i0, int i1, const Epi& epi, double* acc) {
+    using Ix = SweepIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
-    const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
+    const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
     const bool hasS = !(j == 0 && V.rm_lo[1]);
     const bool hasN = !(j == n1 - 1 && V.rm_hi[1] && !(j == 0 && V.rm_lo[1]));
     const bool hasB = !(k == 0 && V.rm_lo[2]);               // cell k   (its top is cell k+1)
     const bool hasT = !(k + 1 == n2 - 1 && V.rm_hi[2]);      // cell k+1 (its bottom is cell k; n2 >= 2)
-    const long long dS = !hasS ? 0 : (j == 0) ? (long long)(n1 - 1) * sJ : -sJ;
-    const long long dN = !hasN ? 0 : (j == n1 - 1) ? -(long long)(n1 - 1) * sJ : sJ;
-    const long long dB = !hasB ? 0 : (k == 0) ? (long long)(n2 - 1) : -1;            // from cell k
-    const long long dT = !hasT ? 0 : (k + 1 == n2 - 1) ? -(long long)(n2 - 1) : 1;   // from cell k+1
-    long long node = (static_cast<long long>(i0) * n1 + j) * n2 + k;
+    const Ix dS = !hasS ? 0 : (j == 0) ? (n1 - 1) * sJ : 0 - sJ;
+    const Ix dN = !hasN ? 0 : (j == n1 - 1) ? 0 - (n1 - 1) * sJ : sJ;
+    const Ix dB = !hasB ? 0 : (k == 0) ? sJ - one : 0 - one;            // from cell k
+    const Ix dT = !hasT ? 0 : (k + 1 == n2 - 1) ? one - sJ : one;   // from cell k+1
+    Ix node = (static_cast<Ix>(i0) * n1 + j) * n2 + k;
     double xp0, xp1, xc0, xc1;
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
-        const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
+        const Ix nprev = !need ? node : (i0 == 0) ? node + (n0 - 1) * sI : node - sI;
         xc0 = static_cast<double>(src1(x, node));
         xc1 = static_cast<double>(src1(x, node + 1));
         xp0 = static_cast<double>(src1(x, nprev));
@@ -778,7 +803,7 @@ __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ 
     for (int i = i0; i < i1; i++) {
         const bool hasW = !(i == 0 && V.rm_lo[0]);
         const bool hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
-        const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
+        const Ix nnext = !hasE ? node : (i == n0 - 1) ? node - (n0 - 1) * sI : node + sI;
         const double xn0 = static_cast<double>(src1(x, nnext)), xn1 = static_cast<double>(src1(x, nnext + 1));
         const double xs0 = static_cast<double>(src1(x, node + dS)), xs1 = static_cast<double>(src1(x, node + dS + 1));
         const double xq0 = static_cast<double>(src1(x, node + dN)), xq1 = static_cast<double>(src1(x, node + dN + 1));
@@ -788,11 +813,11 @@ __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ 
 #pragma unroll
         for (int sl = 0; sl < 7; sl++) {
             if constexpr (Epi::kNT) {
-                d0[sl] = static_cast<double>(ld_nt(D + sl * nr + node));
-                d1[sl] = static_cast<double>(ld_nt(D + sl * nr + node + 1));
+                d0[sl] = static_cast<double>(ld_nt(at_off(D + sl * nr, node)));
+                d1[sl] = static_cast<double>(ld_nt(at_off(D + sl * nr, node) + 1));
             } else {
-                d0[sl] = static_cast<double>(D[sl * nr + node]);
-                d1[sl] = static_cast<double>(D[sl * nr + node + 1]);
+                d0[sl] = static_cast<double>(*at_off(D + sl * nr, node));
+                d1[sl] = static_cast<double>(at_off(D + sl * nr, node)[1]);
             }
         }
         const double pre0 = epi.load(node), pre1 = epi.load(node + 1);
@@ -831,17 +856,18 @@ __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ 
 template <typename VT, class Src, class Epi>
 __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restrict__ D, const Src x,
                                            int k, int j, int i0, int i1, const Epi& epi, double* acc) {
+    using Ix = SweepIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
-    const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
+    const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
     const bool hasS = !(j == 0 && V.rm_lo[1]);
     const bool hasN = !(j == n1 - 1 && V.rm_hi[1] && !(j == 0 && V.rm_lo[1]));
     const bool hasB = !(k == 0 && V.rm_lo[2]);
     const bool hasT = !(k + 1 == n2 - 1 && V.rm_hi[2]);
-    const long long dS = !hasS ? 0 : (j == 0) ? (long long)(n1 - 1) * sJ : -sJ;
-    const long long dN = !hasN ? 0 : (j == n1 - 1) ? -(long long)(n1 - 1) * sJ : sJ;
-    const long long dB = !hasB ? 0 : (k == 0) ? (long long)(n2 - 1) : -1;
-    const long long dT = !hasT ? 0 : (k + 1 == n2 - 1) ? -(long long)(n2 - 1) : 1;
+    const Ix dS = !hasS ? 0 : (j == 0) ? (n1 - 1) * sJ : 0 - sJ;
+    const Ix dN = !hasN ? 0 : (j == n1 - 1) ? 0 - (n1 - 1) * sJ : sJ;
+    const Ix dB = !hasB ? 0 : (k == 0) ? sJ - one : 0 - one;
+    const Ix dT = !hasT ? 0 : (k + 1 == n2 - 1) ? one - sJ : one;
     const VT* DW = D;
     const VT* DS = D + nr;
     const VT* DB = D + 2 * nr;
@@ -850,34 +876,34 @@ __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restric
         if constexpr (Epi::kNT) return static_cast<double>(ld_nt(p));
         else return static_cast<double>(*p);
     };
-    long long node = (static_cast<long long>(i0) * n1 + j) * n2 + k;
+    Ix node = (static_cast<Ix>(i0) * n1 + j) * n2 + k;
     double xp0, xp1, xc0, xc1;
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
-        const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
+        const Ix nprev = !need ? node : (i0 == 0) ? node + (n0 - 1) * sI : node - sI;
         xc0 = static_cast<double>(src1(x, node));
         xc1 = static_cast<double>(src1(x, node + 1));
         xp0 = static_cast<double>(src1(x, nprev));
         xp1 = static_cast<double>(src1(x, nprev + 1));
     }
-    double w0 = ldnt(DW + node), w1 = ldnt(DW + node + 1);
+    double w0 = ldnt(at_off(DW, node)), w1 = ldnt(at_off(DW, node) + 1);
     for (int i = i0; i < i1; i++) {
         const bool hasW = !(i == 0 && V.rm_lo[0]);
         const bool hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
         // a following plane of this tile is always node + sI (i < n0 - 1 there), so the east
         // W loaded here is that plane's own W
-        const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
+        const Ix nnext = !hasE ? node : (i == n0 - 1) ? node - (n0 - 1) * sI : node + sI;
         const double xn0 = static_cast<double>(src1(x, nnext)), xn1 = static_cast<double>(src1(x, nnext + 1));
         const double xs0 = static_cast<double>(src1(x, node + dS)), xs1 = static_cast<double>(src1(x, node + dS + 1));
         const double xq0 = static_cast<double>(src1(x, node + dN)), xq1 = static_cast<double>(src1(x, node + dN + 1));
         const double xb = static_cast<double>(src1(x, node + dB));
         const double xt = static_cast<double>(src1(x, node + 1 + dT));
-        const double sv0 = static_cast<double>(DS[node]), sv1 = static_cast<double>(DS[node + 1]);
-        const double bv0 = static_cast<double>(DB[node]), bv1 = static_cast<double>(DB[node + 1]);
-        const double cv0 = ldnt(DC + node), cv1 = ldnt(DC + node + 1);
-        const double ev0 = ldnt(DW + nnext), ev1 = ldnt(DW + nnext + 1);        // W of the east neighbour
-        const double nv0 = static_cast<double>(DS[node + dN]), nv1 = static_cast<double>(DS[node + dN + 1]);
-        const double tv1 = static_cast<double>(DB[node + 1 + dT]);              // B of cell k+1's top neighbour
+        const double sv0 = static_cast<double>(*at_off(DS, node)), sv1 = static_cast<double>(*at_off(DS, node + 1));
+        const double bv0 = static_cast<double>(*at_off(DB, node)), bv1 = static_cast<double>(*at_off(DB, node + 1));
+        const double cv0 = ldnt(at_off(DC, node)), cv1 = ldnt(at_off(DC, node) + 1);
+        const double ev0 = ldnt(at_off(DW, nnext)), ev1 = ldnt(at_off(DW, nnext) + 1);        // W of the east neighbour
+        const double nv0 = static_cast<double>(*at_off(DS, node + dN)), nv1 = static_cast<double>(*at_off(DS, node + dN + 1));
+        const double tv1 = static_cast<double>(*at_off(DB, node + 1 + dT));              // B of cell k+1's top neighbour
         const double pre0 = epi.load(node), pre1 = epi.load(node + 1);
         double s0 = 0.;
         s0 += hasW ? w0 * xp0 : 0.;
@@ -915,41 +941,42 @@ __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restric
 template <bool UNIT, class Src, class Epi>
 __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict__ D, const Src x,
                                        int k, int j, int i0, int i1, const Epi& epi, double* acc) {
+    using Ix = SweepIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
-    const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
+    const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
     const bool hasS = !(j == 0 && V.rm_lo[1]);
     const bool hasN = !(j == n1 - 1 && V.rm_hi[1] && !(j == 0 && V.rm_lo[1]));
     const bool hasB = !(k == 0 && V.rm_lo[2]);               // cell k   (its top is cell k+1)
     const bool hasT = !(k + 3 == n2 - 1 && V.rm_hi[2]);      // cell k+3 (n2 >= 4)
-    const long long dS = !hasS ? 0 : (j == 0) ? (long long)(n1 - 1) * sJ : -sJ;
-    const long long dN = !hasN ? 0 : (j == n1 - 1) ? -(long long)(n1 - 1) * sJ : sJ;
-    const long long dB = !hasB ? 0 : (k == 0) ? (long long)(n2 - 1) : -1;            // from cell k
-    const long long dT = !hasT ? 0 : (k + 3 == n2 - 1) ? -(long long)(n2 - 1) : 1;   // from cell k+3
+    const Ix dS = !hasS ? 0 : (j == 0) ? (n1 - 1) * sJ : 0 - sJ;
+    const Ix dN = !hasN ? 0 : (j == n1 - 1) ? 0 - (n1 - 1) * sJ : sJ;
+    const Ix dB = !hasB ? 0 : (k == 0) ? sJ - one : 0 - one;            // from cell k
+    const Ix dT = !hasT ? 0 : (k + 3 == n2 - 1) ? one - sJ : one;   // from cell k+3
     typedef f32x4 f4;
     auto ld4 = [](const float* p) { return *reinterpret_cast<const f4*>(p); };
     auto ld4nt = [](const float* p) {
         if constexpr (Epi::kNT) return __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
         else return *reinterpret_cast<const f4*>(p);
     };
-    long long node = (static_cast<long long>(i0) * n1 + j) * n2 + k;
+    Ix node = (static_cast<Ix>(i0) * n1 + j) * n2 + k;
     f4 xp, xc;
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
-        const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
+        const Ix nprev = !need ? node : (i0 == 0) ? node + (n0 - 1) * sI : node - sI;
         xc = src4(x, node);
         xp = src4(x, nprev);
     }
     for (int i = i0; i < i1; i++) {
         const bool hasW = !(i == 0 && V.rm_lo[0]);
         const bool hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
-        const long long nnext = !hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
+        const Ix nnext = !hasE ? node : (i == n0 - 1) ? node - (n0 - 1) * sI : node + sI;
         const f4 xn = src4(x, nnext), xs = src4(x, node + dS), xq = src4(x, node + dN);
         const float xb = src1(x, node + dB), xt = src1(x, node + 3 + dT);
         f4 d[7];
 #pragma unroll
         for (int sl = 0; sl < 7; sl++)
-            if (!(UNIT && sl == 3)) d[sl] = ld4nt(D + sl * nr + node);
+            if (!(UNIT && sl == 3)) d[sl] = ld4nt(at_off(D + sl * nr, node));
         const double p0 = epi.load(node), p1 = epi.load(node + 1), p2 = epi.load(node + 2), p3 = epi.load(node + 3);
         const float xcv[4] = {xc.x, xc.y, xc.z, xc.w}, xpv[4] = {xp.x, xp.y, xp.z, xp.w};
         const float xsv[4] = {xs.x, xs.y, xs.z, xs.w}, xqv[4] = {xq.x, xq.y, xq.z, xq.w};
@@ -987,17 +1014,18 @@ __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict
 template <class Src, class Epi>
 __device__ inline void dia_column_quad_sym(const DiaView& V, const float* __restrict__ D, const Src x,
                                            int k, int j, int i0, int i1, const Epi& epi, double* acc) {
+    using Ix = SweepIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
-    const long long sI = static_cast<long long>(n1) * n2, sJ = n2;
+    const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
     const bool hasS = !(j == 0 && V.rm_lo[1]);
     const bool hasN = !(j == n1 - 1 && V.rm_hi[1] && !(j == 0 && V.rm_lo[1]));
     const bool hasB = !(k == 0 && V.rm_lo[2]);
     const bool hasT = !(k + 3 == n2 - 1 && V.rm_hi[2]);
-    const long long dS = !hasS ? 0 : (j == 0) ? (long long)(n1 - 1) * sJ : -sJ;
-    const long long dN = !hasN ? 0 : (j == n1 - 1) ? -(long long)(n1 - 1) * sJ : sJ;
-    const long long dB = !hasB ? 0 : (k == 0) ? (long long)(n2 - 1) : -1;
-    const long long dT = !hasT ? 0 : (k + 3 == n2 - 1) ? -(long long)(n2 - 1) : 1;
+    const Ix dS = !hasS ? 0 : (j == 0) ? (n1 - 1) * sJ : 0 - sJ;
+    const Ix dN = !hasN ? 0 : (j == n1 - 1) ? 0 - (n1 - 1) * sJ : sJ;
+    const Ix dB = !hasB ? 0 : (k == 0) ? sJ - one : 0 - one;
+    const Ix dT = !hasT ? 0 : (k + 3 == n2 - 1) ? one - sJ : one;
     typedef f32x4 f4;
     auto ld4 = [](const float* p) { return *reinterpret_cast<const f4*>(p); };
     auto ld4nt = [](const float* p) {
@@ -1016,30 +1044,30 @@ __device__ inline void dia_column_quad_sym(const DiaView& V, const float* __rest
         double pre[4];
         bool hasW, hasE;
     };
-    auto load = [&](int i, long long node, Plane& P) {
+    auto load = [&](int i, Ix node, Plane& P) {
         P.hasW = !(i == 0 && V.rm_lo[0]);
         P.hasE = !(i == n0 - 1 && V.rm_hi[0] && !(i == 0 && V.rm_lo[0]));
-        const long long nnext = !P.hasE ? node : (i == n0 - 1) ? node - (long long)(n0 - 1) * sI : node + sI;
+        const Ix nnext = !P.hasE ? node : (i == n0 - 1) ? node - (n0 - 1) * sI : node + sI;
         P.xn = src4(x, nnext);
         P.xs = src4(x, node + dS);
         P.xq = src4(x, node + dN);
         P.xb = src1(x, node + dB);
         P.xt = src1(x, node + 3 + dT);
-        P.cW = ld4(DW + node);
-        P.cS = ld4(DS + node);
-        P.cB = ld4(DB + node);
-        P.cC = ld4nt(DC + node);
-        P.cN = ld4(DS + node + dN);          // S of the north neighbour (unused without it)
-        P.cE = ld4(DW + nnext);              // W of the east neighbour
-        P.cT3 = DB[node + 3 + dT];           // B of the top neighbour of cell k + 3
+        P.cW = ld4(at_off(DW, node));
+        P.cS = ld4(at_off(DS, node));
+        P.cB = ld4(at_off(DB, node));
+        P.cC = ld4nt(at_off(DC, node));
+        P.cN = ld4(at_off(DS, node + dN));          // S of the north neighbour (unused without it)
+        P.cE = ld4(at_off(DW, nnext));              // W of the east neighbour
+        P.cT3 = *at_off(DB, node + 3 + dT);           // B of the top neighbour of cell k + 3
 #pragma unroll
         for (int m = 0; m < 4; m++) P.pre[m] = epi.load(node + m);
     };
-    long long node = (static_cast<long long>(i0) * n1 + j) * n2 + k;
+    Ix node = (static_cast<Ix>(i0) * n1 + j) * n2 + k;
     f4 xp, xc;
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
-        const long long nprev = !need ? node : (i0 == 0) ? node + (long long)(n0 - 1) * sI : node - sI;
+        const Ix nprev = !need ? node : (i0 == 0) ? node + (n0 - 1) * sI : node - sI;
         xc = src4(x, node);
         xp = src4(x, nprev);
     }

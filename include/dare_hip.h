@@ -275,7 +275,7 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* csr, const double* b,
  * x + offset to dare_csr_fill_values). */
 typedef struct dare_batch dare_batch;
 typedef struct {
-    int32_t tile_k;   /* lanes along k per work-group: 16, 32, 64, or 0 = by each system's nz */
+    int32_t tile_k;   /* lanes along k per work-group: 16, 32, 64, or 0 = by each system's extents */
     int32_t tile_i;   /* planes per tile */
     int32_t grid;     /* work-groups of the persistent launches (multiple of 8) */
     int32_t order;    /* work list: 0 system-major, 1 XCD slabs, 2 XCD slabs largest first */
