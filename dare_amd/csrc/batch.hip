@@ -469,6 +469,7 @@ struct dare_batch {
     std::vector<dare_csr*> sys;
     std::vector<long long> row0;       // nsys + 1
     long long rows = 0;
+    bool wide = false;                 // a system has more than kWideRows rows
     hipStream_t stream = nullptr;      // private stream: graph capture needs a non-null stream
     hipEvent_t ev_in = nullptr, ev_out = nullptr, ev_t0 = nullptr, ev_t1 = nullptr;
     dare_batch_config cfg{};
@@ -634,8 +635,13 @@ int refresh_tables(dare_batch* B) {
 
 template <int NC, typename VT, typename XT, bool COPY = false, class Epi>
 void launch_op(dare_batch* B, const XT* x, const Epi& epi, int outer_mask, int check, const XT* x_first = nullptr) {
-    hipLaunchKernelGGL((kb_apply<NC, VT, XT, Epi, COPY>), dim3(B->cfg.grid), dim3(kThreads), 0, B->stream, B->d_sys,
-                       B->d_op, B->n_op, x, x_first, epi, B->partial, B->pstride, B->ctl, outer_mask, check);
+    const auto launch = [&](auto e) {
+        hipLaunchKernelGGL((kb_apply<NC, VT, XT, decltype(e), COPY>), dim3(B->cfg.grid), dim3(kThreads), 0, B->stream,
+                           B->d_sys, B->d_op, B->n_op, x, x_first, e, B->partial, B->pstride, B->ctl, outer_mask,
+                           check);
+    };
+    if (B->wide) launch(Wide<Epi>{epi});
+    else launch(epi);
 }
 
 template <typename XT, int OP>
@@ -842,7 +848,6 @@ int dare_batch_create(dare_ctx* ctx, int32_t nsys, dare_csr* const* systems, dar
         DARE_CHECK_ARG(systems[s]->stencil_structured && systems[s]->has_dia && systems[s]->dia,
                        "batch systems must be 3-D structured operators with a diagonal view "
                        "(dare_csr_build_structure on a 3-D grid with 1 or 2 components)");
-        DARE_CHECK_ARG(systems[s]->nrows <= kDiaRows, "a batch system may have at most 2^29 rows");
         if (N < 0) N = systems[s]->dia_view.N;
         DARE_CHECK_ARG(systems[s]->dia_view.N == N, "all systems of a batch need the same number of components");
     }
@@ -863,6 +868,7 @@ int dare_batch_create(dare_ctx* ctx, int32_t nsys, dare_csr* const* systems, dar
     B->row0[0] = 0;
     for (int s = 0; s < nsys; s++) B->row0[s + 1] = B->row0[s] + systems[s]->dia_view.nrows;
     B->rows = B->row0[nsys];
+    for (int s = 0; s < nsys; s++) B->wide |= systems[s]->nrows > kWideRows;
     B->h_sys.resize(nsys);
     auto fail = [&](int rc) {
         dare_batch_destroy(B);

@@ -587,7 +587,7 @@ static int op64(dare_ctx* ctx, const dare_csr* A, bool allow_dia, SolveOp<double
     op.dia = allow_dia && A->has_dia;
     if (op.dia) {
         op.d = make_dia<double>(A->dia_view, A->dia, true);
-        op.dia = kXcd * op.d.per_xcd <= kReduceBlocks && A->nrows <= kDiaRows;   // else the CSR traversal
+        op.dia = kXcd * op.d.per_xcd <= kReduceBlocks;   // else the CSR traversal
     }
     if (op.dia && op.d.pair == 2 && A->sym_traversal) {
         const int rc = sym64_prepare(ctx, const_cast<dare_csr*>(A));
@@ -933,7 +933,7 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
     const bool pre = p->precond == 1;
     const bool use_mg = p->precond == DARE_PRECOND_MG;
     bool unit_c = false;
-    if (A->has_dia && n <= kDiaRows && kXcd * make_dia<double>(A->dia_view, A->dia).per_xcd <= kReduceBlocks) {
+    if (A->has_dia && kXcd * make_dia<double>(A->dia_view, A->dia).per_xcd <= kReduceBlocks) {
         if (use_mg) {           // the multigrid levels read all seven slots
             const int erc = dia_ensure_full(A, ctx->stream);
             if (erc) return erc;

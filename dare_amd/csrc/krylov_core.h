@@ -456,16 +456,26 @@ __device__ __forceinline__ void epi_quad(const Epi& e, long long i, const double
 }
 // ------------------------------------------------------------------------------ operands
 // Element offsets within one system's slot or vector. Where a sweep does not stream from memory
-// they are 32 bits, also in bytes (kDiaRows; only a grid most of whose rows are identities fits
-// more rows under the 2^31 entries of a matrix, and is applied from its CSR values): a load then
-// takes a scalar base and one register of offset instead of a 64-bit address per access, which
-// gives the fused steps a wave more per SIMD (128^3, seven slots: 37.9 -> 31.1 us). The streaming
-// sweeps keep 64 bits: with eight waves per SIMD instead of six the symmetric pairs evict the
-// partner slots they are about to read again (256^3: 179 -> 192 us). So does the five-dot sweep of
-// step 18, which reads two vectors more (128^3: 33.5 us, with 32 bits 40.2).
-constexpr long long kDiaRows = 1LL << 29;
+// they are 32 bits, also in bytes (so up to kWideRows rows): a load then takes a scalar base and
+// one register of offset instead of a 64-bit address per access, which gives the fused steps a
+// wave more per SIMD (128^3, seven slots: 37.9 -> 31.1 us). The streaming sweeps, every single
+// solver's from kStreamRows rows on, keep 64 bits: with eight waves per SIMD instead of six the
+// symmetric pairs evict the partner slots they are about to read again (256^3: 179 -> 192 us). So
+// does the five-dot sweep of step 18, which reads two vectors more (128^3: 33.5 us, with 32 bits
+// 40.2), and a batch with a system of more rows than kWideRows (Wide).
+constexpr long long kWideRows = 1LL << 29;
 template <class Epi>
-using SweepIndex = std::conditional_t<Epi::kNT || Epi::NDOT == 5, long long, unsigned>;
+struct Wide : Epi {};
+template <class Epi>
+struct SweepIndexOf {
+    using type = std::conditional_t<Epi::kNT || Epi::NDOT == 5, long long, unsigned>;
+};
+template <class Epi>
+struct SweepIndexOf<Wide<Epi>> {
+    using type = long long;
+};
+template <class Epi>
+using SweepIndex = typename SweepIndexOf<Epi>::type;
 template <typename T>
 __device__ __forceinline__ const T* at_off(const T* base, unsigned e) {
     return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + e * static_cast<unsigned>(sizeof(T)));
