@@ -541,11 +541,17 @@ int mg_prepare(dare_ctx* ctx, dare_csr* A, const SolveOp<VT>& op, const VT* D0, 
         set_error("the multigrid preconditioner needs a device-assembled 3-D operator (diagonal view)");
         return DARE_ERR_UNSUPPORTED;
     }
-    const int erc = dia_ensure_full(A, ctx->stream);     // the levels read all seven slots
-    if (erc) return erc;
+    // an exactly symmetric view (sym64_prepare's rule; not checked on the device for this alone)
+    // is read without its E, N, T slots
+    const bool sym = A->sym_traversal && A->dia_view.N == 1 && !A->dia_view.cross &&
+                     (A->sym64 == 1 || (A->sym64 < 0 && A->sym_fill));
+    if (!sym) {
+        const int erc = dia_ensure_full(A, ctx->stream);
+        if (erc) return erc;
+    }
     if (!A->mg) A->mg = new MgHierarchy();
     MgHierarchy* H = static_cast<MgHierarchy*>(A->mg);
-    const int rc = mg_setup<VT, XT>(ctx, H, A->dia_view, D0);
+    const int rc = mg_setup<VT, XT>(ctx, H, A->dia_view, D0, sym);
     *out = H;
     return rc;
 }
@@ -934,10 +940,6 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
     const bool use_mg = p->precond == DARE_PRECOND_MG;
     bool unit_c = false;
     if (A->has_dia && kXcd * make_dia<double>(A->dia_view, A->dia).per_xcd <= kReduceBlocks) {
-        if (use_mg) {           // the multigrid levels read all seven slots
-            const int erc = dia_ensure_full(A, ctx->stream);
-            if (erc) return erc;
-        }
         const int slots = A->dia_view.cross ? 8 : 7;
         const int64_t need = static_cast<int64_t>(slots) * n;
         if (A->cap_dia32 < need) {

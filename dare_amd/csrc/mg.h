@@ -20,11 +20,12 @@
 //   rc = P^T t (the sum over each aggregate, in a fixed order)      zc = coarse cycle of rc
 //   z  = z0 + P zc                                                  out = z + W (r - A z)
 // Each level runs as two kernels: k_mg_down forms rc straight from r (z0 and t are formed per
-// cell and never stored; the eight cells of an aggregate sit in one wave and are summed across
-// lanes) and k_mg_up forms out with z evaluated at each neighbour on the fly. The coarsest
-// level (at most 1024 rows) runs its sweeps inside one work-group. Work is dealt so that each
-// XCD (blocks b = x mod 8) owns one contiguous eighth of a level, keeping the neighbour planes
-// of a row in that XCD's L2.
+// cell and never stored; the eight cells of an aggregate sit in two lanes) and k_mg_up forms out
+// with z evaluated at each neighbour on the fly. The coarsest level (at most 1024 rows) runs its
+// sweeps inside one work-group (taking the level above it into that work-group as well cost 38 us
+// against 15 for the three launches at 19 x 16 x 16). Work is dealt so that each XCD (blocks b =
+// x mod 8) owns one contiguous eighth of a level, keeping the neighbour planes of a row in that
+// XCD's L2.
 #pragma once
 
 namespace dare_hip {
@@ -53,6 +54,7 @@ struct MgHierarchy {
     void* fine = nullptr;      // fine level: W (VT) and the cycle result (XT)
     size_t fine_bytes = 0;
     const void* D0 = nullptr;  // fine-level slots (VT) of the last set-up
+    bool sym = false;          // ... which were exactly symmetric: E, N, T are not read
     double omega = 0.8;
     int coarse_sweeps = 12;
 };
@@ -85,11 +87,6 @@ __device__ inline void mg_cell(const DiaView& V, long long row, int p[3]) {
     p[1] = static_cast<int>((row / V.n[2]) % V.n[1]);
     p[0] = static_cast<int>(row / (static_cast<long long>(V.n[1]) * V.n[2]));
 }
-// aggregate (coarse row) of fine cell q
-__device__ inline long long mg_agg(const DiaView& Vc, const int q[3]) {
-    return (static_cast<long long>(q[0] / 2) * Vc.n[1] + q[1] / 2) * Vc.n[2] + q[2] / 2;
-}
-
 // this lane's rows of an n-row level: XCD x (blocks b = x mod 8) owns rows [n x / 8, n (x+1) / 8)
 struct MgSlab {
     long long first, end, step;
@@ -104,45 +101,6 @@ __device__ inline MgSlab mg_slab(long long n) {
     return S;
 }
 
-// coarse slots and W of level l+1 from the slots of level l (one lane per coarse row)
-template <typename VT, typename CT>
-__global__ __launch_bounds__(kThreads) void k_mg_coarsen(DiaView Vf, const VT* __restrict__ Df, DiaView Vc,
-                                                        CT* __restrict__ Dc, CT* __restrict__ Wc, double beta,
-                                                        double omega) {
-    const long long nrf = Vf.nrows, nrc = Vc.nrows;
-    const MgSlab S = mg_slab(nrc);
-    for (long long row = S.first; row < S.end; row += S.step) {
-        int agg[3];
-        mg_cell(Vc, row, agg);
-        double excess = 0., cpl[7] = {0., 0., 0., 0., 0., 0., 0.};
-        for (int di = 0; di < 2; di++)
-            for (int dj = 0; dj < 2; dj++)
-                for (int dk = 0; dk < 2; dk++) {
-                    const int p[3] = {2 * agg[0] + di, 2 * agg[1] + dj, 2 * agg[2] + dk};
-                    if (p[0] >= Vf.n[0] || p[1] >= Vf.n[1] || p[2] >= Vf.n[2]) continue;
-                    const long long frow = mg_row(Vf, p);
-                    excess += static_cast<double>(Df[3 * nrf + frow]);
-                    for (int s = 0; s < 7; s++) {
-                        if (s == 3) continue;
-                        int q[3];
-                        if (!mg_nb(Vf, p, s, q)) continue;                 // removed boundary entry (0)
-                        const double a = static_cast<double>(Df[s * nrf + frow]);
-                        excess += a;
-                        const int d = s < 3 ? s : 6 - s;
-                        if (q[d] / 2 != agg[d]) cpl[s] += beta * a;        // coupling to a neighbour aggregate
-                    }
-                }
-        double c = excess;
-        for (int s = 0; s < 7; s++)
-            if (s != 3) {
-                c -= cpl[s];
-                Dc[s * nrc + row] = static_cast<CT>(cpl[s]);
-            }
-        Dc[3 * nrc + row] = static_cast<CT>(c);
-        Wc[row] = static_cast<CT>(omega / c);
-    }
-}
-
 // W = omega / C of the fine level
 template <typename VT>
 __global__ __launch_bounds__(kThreads) void k_mg_weight(long long n, const VT* __restrict__ C, VT* __restrict__ W,
@@ -151,150 +109,295 @@ __global__ __launch_bounds__(kThreads) void k_mg_weight(long long n, const VT* _
     for (long long i = S.first; i < S.end; i += S.step) W[i] = static_cast<VT>(omega / static_cast<double>(C[i]));
 }
 
-// Fine cells of a level in wave-sized bricks of 16 (k) x 2 (j) x 2 (i) cells: lane l of brick
-// (I, J, G) holds cell (2I + (l >> 5 & 1), 2J + (l >> 4 & 1), 16 G + (l & 15)), so the 2x2x2
-// cells of one aggregate sit in lanes that differ in bits 0, 4 and 5. Bricks are dealt so that
-// XCD x (blocks b = x mod 8) owns one contiguous eighth of them.
-struct MgBricks {
-    int ng;                    // bricks along k
+// ---- the level kernels. One lane holds the four cells (2 i x 2 j at one k) of an aggregate's
+// half; the lane of the other k is its neighbour in the wave, so an aggregate's sum is three adds
+// in the lane and one exchange. A wave is 2^lk lanes along k times 64 >> lk pairs of rows along j
+// on one pair of planes, and XCD x (blocks b = x mod 8) owns one contiguous eighth of the tiles.
+// What bounds the fine level is the slots' and vectors' bytes; before, with a lane per cell, 28
+// (up) and 21 (down) loads a cell in runs of 16 k cells kept it above that. Here a run is up to 64
+// cells, the four cells share their neighbours, and the seven values of zc serve all four (18 and
+// 16 loads a cell). 145 x 128 x 121, FP64, four slots: down 28.8 -> 25.7 us, up 34.3 -> 27.5 (seven slots and 64-bit
+// rows: down 35, up 38).
+struct MgTiles {
+    int lk;                    // log2 of the lanes along k
+    unsigned tk, tj;           // tiles along k and along j
     long long total;
 };
-inline MgBricks mg_bricks(const DiaView& V) {
-    MgBricks B;
-    B.ng = (V.n[2] + 15) / 16;
-    B.total = static_cast<long long>((V.n[0] + 1) / 2) * ((V.n[1] + 1) / 2) * B.ng;
-    return B;
+inline MgTiles mg_tiles(const DiaView& V) {
+    // the longest run whose padding of the k extent is within 1/8 of the least, at least a pair
+    const auto padded = [&](int lk) { return (static_cast<long long>(V.n[2]) + (1 << lk) - 1) >> lk << lk; };
+    MgTiles T;
+    T.lk = 6;
+    while (T.lk > 4 && (V.n[2] <= 1 << (T.lk - 1) || 8 * padded(T.lk) > 9 * padded(4))) T.lk--;
+    while (T.lk > 1 && V.n[2] <= 1 << (T.lk - 1)) T.lk--;
+    const int rows = 64 >> T.lk;
+    T.tk = static_cast<unsigned>(padded(T.lk) >> T.lk);
+    T.tj = static_cast<unsigned>(((V.n[1] + 1) / 2 + rows - 1) / rows);
+    T.total = static_cast<long long>(T.tk) * T.tj * ((V.n[0] + 1) / 2);
+    return T;
 }
-inline unsigned mg_brick_grid(const MgBricks& B) {   // four bricks (waves) per work-group, a multiple of kXcd
-    long long g = (B.total + 3) / 4;
-    if (g > 65536) g = 65536;                         // one brick per wave up to 256^3
-    g = (g + kXcd - 1) / kXcd * kXcd;
-    return static_cast<unsigned>(g);
+inline unsigned mg_tile_grid(const MgTiles& T) {      // one wave per work-group, a multiple of kXcd
+    const long long g = T.total < (1LL << 20) ? T.total : (1LL << 20);
+    return static_cast<unsigned>((g + kXcd - 1) / kXcd * kXcd);
 }
-struct MgBrickIter {
+struct MgTileIter {
     long long first, end, step;
 };
-__device__ inline MgBrickIter mg_brick_iter(const MgBricks& B) {
+__device__ inline MgTileIter mg_tile_iter(const MgTiles& T) {
     const int xcd = static_cast<int>(blockIdx.x % kXcd);
-    MgBrickIter it;
-    it.first = B.total * xcd / kXcd + static_cast<long long>(blockIdx.x / kXcd) * 4 + threadIdx.x / 64;
-    it.end = B.total * (xcd + 1) / kXcd;
-    it.step = static_cast<long long>(gridDim.x / kXcd) * 4;
+    MgTileIter it;
+    it.first = T.total * xcd / kXcd + blockIdx.x / kXcd;
+    it.end = T.total * (xcd + 1) / kXcd;
+    it.step = gridDim.x / kXcd;
     return it;
 }
-// this lane's cell of brick w; false when it lies outside the level
-__device__ inline bool mg_brick_cell(const DiaView& V, const MgBricks& B, long long w, int p[3]) {
+
+// Rows, in 32 bits, that a lane reads: its cells c[a][b] (plane 2I + a, row 2J + b) and their
+// neighbours. A neighbour that the boundary edit removed (mg_nb) counts as the cell itself: its
+// slot holds 0, so the term it feeds is +0.0 and every load can be issued unconditionally. Cells
+// outside the level (an odd extent's last pair, lanes beyond the tile's end) stand on a valid cell
+// and are dropped by the caller.
+struct MgQuad {
+    unsigned c[2][2], loI[2], hiI[2], loJ[2], hiJ[2];
+    unsigned dlo, dhi;         // to the neighbours along k, added mod 2^32
+    bool in, i1, j1;           // the lane's cells 0, its second plane and its second row exist
+    unsigned gone;             // axes (bit d) whose removed higher neighbour the last cell would have
+    int I[3];                  // aggregate
+    int lo[3], hi[3];          // aggregate coordinate of the neighbours along each axis
+};
+__device__ inline MgQuad mg_quad(const DiaView& V, const MgTiles& T, long long w) {
+    MgQuad q;
     const int lane = threadIdx.x % 64;
-    const unsigned nj = static_cast<unsigned>((V.n[1] + 1) / 2);
-    const unsigned wu = static_cast<unsigned>(w);     // bricks < 2^32 (mg_setup)
-    const unsigned ij = wu / static_cast<unsigned>(B.ng);
-    p[0] = 2 * static_cast<int>(ij / nj) + ((lane >> 5) & 1);
-    p[1] = 2 * static_cast<int>(ij % nj) + ((lane >> 4) & 1);
-    p[2] = 16 * static_cast<int>(wu - ij * static_cast<unsigned>(B.ng)) + (lane & 15);
-    return p[0] < V.n[0] && p[1] < V.n[1] && p[2] < V.n[2];
-}
-
-// Row of the neighbour of cell p through slot s, or the cell's own row when the boundary edit
-// removed that neighbour: its slot holds 0, so the term it feeds is +0.0 and every load can
-// be issued unconditionally (all of a cell's loads in flight together).
-__device__ inline long long mg_nb_row(const DiaView& V, const int p[3], int s, long long self, int q[3]) {
-    if (!mg_nb(V, p, s, q)) {
-        q[0] = p[0];
-        q[1] = p[1];
-        q[2] = p[2];
-        return self;
+    const unsigned wu = static_cast<unsigned>(w);     // tiles < 2^32 (mg_setup)
+    const unsigned ij = wu / T.tk;
+    const unsigned ti = ij / T.tj;
+    int p[3] = {2 * static_cast<int>(ti), static_cast<int>(ij - ti * T.tj) * (64 >> T.lk) + (lane >> T.lk),
+                static_cast<int>(wu - ij * T.tk) << T.lk | (lane & ((1 << T.lk) - 1))};
+    p[1] *= 2;
+    q.in = p[1] < V.n[1] && p[2] < V.n[2];
+    p[1] = p[1] < V.n[1] ? p[1] : 0;
+    p[2] = p[2] < V.n[2] ? p[2] : V.n[2] - 1;
+    q.i1 = p[0] + 1 < V.n[0];
+    q.j1 = p[1] + 1 < V.n[1];
+    const unsigned stride[3] = {static_cast<unsigned>(V.n[1]) * static_cast<unsigned>(V.n[2]),
+                                static_cast<unsigned>(V.n[2]), 1u};
+    const int last[3] = {p[0] + (q.i1 ? 1 : 0), p[1] + (q.j1 ? 1 : 0), p[2]};
+    unsigned dlo[3], dhi[3];   // from the first cell of the axis
+    q.gone = 0u;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int n = V.n[d];
+        const bool lo_gone = p[d] == 0 && V.rm_lo[d];
+        const bool hi_gone = last[d] == n - 1 && V.rm_hi[d] && !(last[d] == 0 && V.rm_lo[d]);
+        const int lo = lo_gone ? p[d] : p[d] == 0 ? n - 1 : p[d] - 1;
+        const int hi = hi_gone ? last[d] : last[d] == n - 1 ? 0 : last[d] + 1;
+        q.gone |= static_cast<unsigned>(hi_gone) << d;
+        dlo[d] = static_cast<unsigned>(lo - p[d]) * stride[d];
+        dhi[d] = static_cast<unsigned>(hi - p[d]) * stride[d];
+        q.I[d] = p[d] >> 1;
+        q.lo[d] = lo >> 1;
+        q.hi[d] = hi >> 1;
     }
-    return mg_row(V, q);
+    const unsigned c0 = p[0] * stride[0] + p[1] * stride[1] + p[2];
+    const unsigned si = q.i1 ? stride[0] : 0u, sj = q.j1 ? stride[1] : 0u;
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+#pragma unroll
+        for (int b = 0; b < 2; b++) q.c[a][b] = c0 + (a ? si : 0u) + (b ? sj : 0u);
+        q.loI[a] = c0 + dlo[0] + (a ? sj : 0u);
+        q.hiI[a] = c0 + dhi[0] + (a ? sj : 0u);
+        q.loJ[a] = c0 + dlo[1] + (a ? si : 0u);
+        q.hiJ[a] = c0 + dhi[1] + (a ? si : 0u);
+    }
+    q.dlo = dlo[2];
+    q.dhi = dhi[2];
+    return q;
 }
 
-// rc = P^T (r - A W r) (PRE) or P^T r: one lane per fine cell, the aggregate's eight values
-// summed across lanes in a fixed order
-template <bool PRE, typename DT, typename XT, typename CT>
-__global__ __launch_bounds__(kThreads) void k_mg_down(DiaView Vf, MgBricks Bf, const DT* __restrict__ Df,
-                                                     const DT* __restrict__ Wf, const XT* __restrict__ r, DiaView Vc,
-                                                     CT* __restrict__ rc) {
-    const long long nrf = Vf.nrows;
-    const MgBrickIter it = mg_brick_iter(Bf);
-    for (long long w = it.first; w < it.end; w += it.step) {
-        int p[3];
-        const bool in = mg_brick_cell(Vf, Bf, w, p);
-        if (!in) {                    // a valid cell for the loads; the lane's value is dropped
-            p[0] = p[0] < Vf.n[0] ? p[0] : Vf.n[0] - 1;
-            p[1] = p[1] < Vf.n[1] ? p[1] : Vf.n[1] - 1;
-            p[2] = p[2] < Vf.n[2] ? p[2] : Vf.n[2] - 1;
-        }
-        const long long frow = mg_row(Vf, p);
-        double t = static_cast<double>(r[frow]);
-        if (PRE) {
-            long long nb[7];
-            double a[7], wn[7], rn[7];
+// The slots of a lane's four cells. SYM: the view is exactly symmetric, and its E, N, T slots,
+// which a fill may have left out, are read as the W, S, B slots of the neighbours.
+template <bool SYM, typename Ix, typename DT>
+__device__ inline void mg_slots(const DT* __restrict__ D, long long nr, const MgQuad& q, DT a[2][2][7]) {
+    const auto at = [&](int s, unsigned row) { return *at_off(D + s * nr, static_cast<Ix>(row)); };
 #pragma unroll
-            for (int s = 0; s < 7; s++) {
-                int q[3];
-                nb[s] = s == 3 ? frow : mg_nb_row(Vf, p, s, frow, q);
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int s = 0; s < (SYM ? 4 : 7); s++) a[i][j][s] = at(s, q.c[i][j]);
+    if constexpr (SYM) {
+        const DT z = static_cast<DT>(0);
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const DT e = at(0, q.hiI[m]), n = at(1, q.hiJ[m]);
+            a[1][m][6] = q.gone & 1u ? z : e;
+            a[0][m][6] = q.i1 ? a[1][m][0] : a[1][m][6];
+            a[m][1][5] = q.gone & 2u ? z : n;
+            a[m][0][5] = q.j1 ? a[m][1][1] : a[m][1][5];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const DT t = at(2, q.c[m][j] + q.dhi);
+                a[m][j][4] = q.gone & 4u ? z : t;
             }
-#pragma unroll
-            for (int s = 0; s < 7; s++) {
-                a[s] = static_cast<double>(Df[s * nrf + frow]);
-                wn[s] = static_cast<double>(Wf[nb[s]]);
-                rn[s] = static_cast<double>(r[nb[s]]);
-            }
-            double y = a[3] * (wn[3] * rn[3]);
-#pragma unroll
-            for (int s = 0; s < 7; s++)
-                if (s != 3) y += a[s] * (wn[s] * rn[s]);
-            t -= y;
-        }
-        if (!in) t = 0.;
-        t += __shfl_xor(t, 1);
-        t += __shfl_xor(t, 16);
-        t += __shfl_xor(t, 32);
-        const int lane = threadIdx.x % 64;
-        if (in && (lane & 0x31) == 0) {
-            const int ag[3] = {p[0] / 2, p[1] / 2, p[2] / 2};
-            rc[mg_row(Vc, ag)] = static_cast<CT>(t);
         }
     }
 }
 
-// out = z + W (r - A z) with z = [W r] + P zc evaluated at each neighbour: one lane per row
-template <bool PRE, typename DT, typename XT, typename CT>
-__global__ __launch_bounds__(kThreads) void k_mg_up(DiaView Vf, MgBricks Bf, const DT* __restrict__ Df,
-                                                   const DT* __restrict__ Wf, const XT* __restrict__ r, DiaView Vc,
-                                                   const CT* __restrict__ zc, XT* __restrict__ out) {
-    const long long nrf = Vf.nrows;
-    const MgBrickIter it = mg_brick_iter(Bf);
+// The value at a row of the operand, by what of(row, aggregate's part) gives, at the lane's cells
+// and their neighbours; y(i, j) is then the row's product, in the order C W S B T N E.
+struct MgPoints {
+    double c[2][2], loI[2], hiI[2], loJ[2], hiJ[2], loK[2][2], hiK[2][2];
+    bool i1, j1;
+    template <typename DT>
+    __device__ double product(const DT a[2][2][7], int i, int j) const {
+        const auto f = [&](int s) { return static_cast<double>(a[i][j][s]); };
+        double y = f(3) * c[i][j];
+        y += f(0) * (i ? c[0][j] : loI[j]);
+        y += f(1) * (j ? c[i][0] : loJ[i]);
+        y += f(2) * loK[i][j];
+        y += f(4) * hiK[i][j];
+        y += f(5) * (j == 0 && j1 ? c[i][1] : hiJ[i]);
+        y += f(6) * (i == 0 && i1 ? c[1][j] : hiI[j]);
+        return y;
+    }
+};
+// of(row, n): n is 0 for the lane's own aggregate, 1..6 for its W S B T N E neighbour
+template <class F>
+__device__ inline MgPoints mg_points(const MgQuad& q, const F& of) {
+    MgPoints z;
+    z.i1 = q.i1;
+    z.j1 = q.j1;
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            z.c[m][j] = of(q.c[m][j], 0);
+            z.loK[m][j] = of(q.c[m][j] + q.dlo, 3);
+            z.hiK[m][j] = of(q.c[m][j] + q.dhi, 4);
+        }
+        z.loI[m] = of(q.loI[m], 1);
+        z.hiI[m] = of(q.hiI[m], 6);
+        z.loJ[m] = of(q.loJ[m], 2);
+        z.hiJ[m] = of(q.hiJ[m], 5);
+    }
+    return z;
+}
+
+// coarse slots and W of level l+1 from the slots of level l. On a symmetric view they are
+// symmetric too: a face's coefficients are summed in the same order from both sides.
+template <bool SYM, typename Ix, typename VT, typename CT>
+__global__ __launch_bounds__(64) void k_mg_coarsen(DiaView Vf, MgTiles Tf, const VT* __restrict__ Df, DiaView Vc,
+                                                  CT* __restrict__ Dc, CT* __restrict__ Wc, double beta, double omega) {
+    const long long nrf = Vf.nrows, nrc = Vc.nrows;
+    const MgTileIter it = mg_tile_iter(Tf);
     for (long long w = it.first; w < it.end; w += it.step) {
-        int p[3];
-        if (!mg_brick_cell(Vf, Bf, w, p)) continue;
-        const long long row = mg_row(Vf, p);
-        long long nb[7], ag[7];
+        const MgQuad q = mg_quad(Vf, Tf, w);
+        VT a[2][2][7];
+        mg_slots<SYM, Ix>(Df, nrf, q, a);
+        double excess = 0., cpl[7] = {0., 0., 0., 0., 0., 0., 0.};
 #pragma unroll
-        for (int s = 0; s < 7; s++) {
-            int q[3];
-            nb[s] = s == 3 ? row : mg_nb_row(Vf, p, s, row, q);
-            ag[s] = s == 3 ? mg_agg(Vc, p) : mg_agg(Vc, q);
-        }
-        double a[7], wn[7], rn[7], zn[7];
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int s = 0; s < 7; s++) {
-            a[s] = static_cast<double>(Df[s * nrf + row]);
-            wn[s] = PRE ? static_cast<double>(Wf[nb[s]]) : 0.;
-            rn[s] = PRE ? static_cast<double>(r[nb[s]]) : 0.;
-            zn[s] = static_cast<double>(zc[ag[s]]);
-        }
-        const double wr = static_cast<double>(Wf[row]), rr = static_cast<double>(r[row]);
-        const double zi = (PRE ? wn[3] * rn[3] : 0.) + zn[3];
-        double y = a[3] * zi;
+            for (int j = 0; j < 2; j++) {
+                if (!q.in || (i && !q.i1) || (j && !q.j1)) continue;
+                const bool out[7] = {i == 0 && q.lo[0] != q.I[0], j == 0 && q.lo[1] != q.I[1], q.lo[2] != q.I[2], false,
+                                     q.hi[2] != q.I[2], (j || !q.j1) && q.hi[1] != q.I[1],
+                                     (i || !q.i1) && q.hi[0] != q.I[0]};
+                excess += static_cast<double>(a[i][j][3]);
+#pragma unroll
+                for (int s = 0; s < 7; s++) {
+                    if (s == 3) continue;
+                    const double v = static_cast<double>(a[i][j][s]);
+                    excess += v;
+                    if (out[s]) cpl[s] += beta * v;            // coupling to a neighbour aggregate
+                }
+            }
+        excess += __shfl_xor(excess, 1);
+        double c = excess;
 #pragma unroll
         for (int s = 0; s < 7; s++)
-            if (s != 3) y += a[s] * ((PRE ? wn[s] * rn[s] : 0.) + zn[s]);
-        out[row] = static_cast<XT>(zi + wr * (rr - y));
+            if (s != 3) {
+                cpl[s] += __shfl_xor(cpl[s], 1);
+                c -= cpl[s];
+            }
+        if (q.in && (threadIdx.x & 1) == 0) {
+            const long long row = mg_row(Vc, q.I);
+#pragma unroll
+            for (int s = 0; s < 7; s++) Dc[s * nrc + row] = static_cast<CT>(s == 3 ? c : cpl[s]);
+            Wc[row] = static_cast<CT>(omega / c);
+        }
+    }
+}
+
+// rc = P^T (r - A W r), an aggregate's eight values summed in a fixed order
+template <bool SYM, typename Ix, typename DT, typename XT, typename CT>
+__global__ __launch_bounds__(64) void k_mg_down(DiaView Vf, MgTiles Tf, const DT* __restrict__ Df,
+                                               const DT* __restrict__ Wf, const XT* __restrict__ r, DiaView Vc,
+                                               CT* __restrict__ rc) {
+    const MgTileIter it = mg_tile_iter(Tf);
+    for (long long w = it.first; w < it.end; w += it.step) {
+        const MgQuad q = mg_quad(Vf, Tf, w);
+        DT a[2][2][7];
+        mg_slots<SYM, Ix>(Df, Vf.nrows, q, a);
+        const MgPoints z = mg_points(q, [&](unsigned row, int) {
+            return static_cast<double>(*at_off(Wf, static_cast<Ix>(row))) *
+                   static_cast<double>(*at_off(r, static_cast<Ix>(row)));
+        });
+        double t = 0.;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const double d = static_cast<double>(*at_off(r, static_cast<Ix>(q.c[i][j]))) - z.product(a, i, j);
+                if (q.in && (!i || q.i1) && (!j || q.j1)) t += d;
+            }
+        t += __shfl_xor(t, 1);
+        if (q.in && (threadIdx.x & 1) == 0) rc[mg_row(Vc, q.I)] = static_cast<CT>(t);
+    }
+}
+
+// out = z + W (r - A z) with z = W r + P zc evaluated at each neighbour
+template <bool SYM, typename Ix, typename DT, typename XT, typename CT>
+__global__ __launch_bounds__(64) void k_mg_up(DiaView Vf, MgTiles Tf, const DT* __restrict__ Df,
+                                             const DT* __restrict__ Wf, const XT* __restrict__ r, DiaView Vc,
+                                             const CT* __restrict__ zc, XT* __restrict__ out) {
+    const MgTileIter it = mg_tile_iter(Tf);
+    for (long long w = it.first; w < it.end; w += it.step) {
+        const MgQuad q = mg_quad(Vf, Tf, w);
+        DT a[2][2][7];
+        mg_slots<SYM, Ix>(Df, Vf.nrows, q, a);
+        const unsigned stride[3] = {static_cast<unsigned>(Vc.n[1]) * static_cast<unsigned>(Vc.n[2]),
+                                    static_cast<unsigned>(Vc.n[2]), 1u};
+        const unsigned own = q.I[0] * stride[0] + q.I[1] * stride[1] + q.I[2];
+        double zn[7];
+        zn[0] = static_cast<double>(*at_off(zc, static_cast<Ix>(own)));
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const unsigned lo = own + static_cast<unsigned>(q.lo[d] - q.I[d]) * stride[d];
+            const unsigned hi = own + static_cast<unsigned>(q.hi[d] - q.I[d]) * stride[d];
+            zn[1 + d] = static_cast<double>(*at_off(zc, static_cast<Ix>(lo)));
+            zn[6 - d] = static_cast<double>(*at_off(zc, static_cast<Ix>(hi)));
+        }
+        const MgPoints z = mg_points(q, [&](unsigned row, int n) {
+            return static_cast<double>(*at_off(Wf, static_cast<Ix>(row))) *
+                       static_cast<double>(*at_off(r, static_cast<Ix>(row))) +
+                   zn[n];
+        });
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const double wr = static_cast<double>(*at_off(Wf, static_cast<Ix>(q.c[i][j])));
+                const double rr = static_cast<double>(*at_off(r, static_cast<Ix>(q.c[i][j])));
+                const double o = z.c[i][j] + wr * (rr - z.product(a, i, j));
+                if (q.in && (!i || q.i1) && (!j || q.j1)) out[q.c[i][j]] = static_cast<XT>(o);
+            }
     }
 }
 
 // the coarsest level: z = W r, then sweeps - 1 damped-Jacobi sweeps, all in one work-group
-// (rows <= 1024) with z held in LDS
+// (rows <= 1024) with z held in LDS. A chain of sweeps bounds it: the seven reads of a row go out
+// together, a removed neighbour's as the row itself times 0 (640 rows: 7.2 -> 5.6 us).
 template <typename CT>
 __global__ __launch_bounds__(1024) void k_mg_coarsest(DiaView V, const CT* __restrict__ D, const CT* __restrict__ W,
                                                      const CT* __restrict__ r, CT* __restrict__ z, int sweeps) {
@@ -302,15 +405,16 @@ __global__ __launch_bounds__(1024) void k_mg_coarsest(DiaView V, const CT* __res
     const long long nr = V.nrows;
     const int row = threadIdx.x;
     CT a[7] = {0, 0, 0, 0, 0, 0, 0};
-    int nb[7] = {-1, -1, -1, -1, -1, -1, -1};
+    int nb[7] = {row, row, row, row, row, row, row};
     CT rv = 0, wv = 0;
     if (row < nr) {
         int p[3];
         mg_cell(V, row, p);
+#pragma unroll
         for (int s = 0; s < 7; s++) {
             a[s] = D[s * nr + row];
             int q[3];
-            nb[s] = s == 3 ? row : mg_nb(V, p, s, q) ? static_cast<int>(mg_row(V, q)) : -1;
+            if (s != 3 && mg_nb(V, p, s, q)) nb[s] = static_cast<int>(mg_row(V, q));
         }
         rv = r[row];
         wv = W[row];
@@ -321,9 +425,11 @@ __global__ __launch_bounds__(1024) void k_mg_coarsest(DiaView V, const CT* __res
     CT* nxt = zb;
     for (int it = 1; it < sweeps; it++) {
         if (row < nr) {
-            CT y = 0;
-            for (int s = 0; s < 7; s++)
-                if (nb[s] >= 0) y += a[s] * cur[nb[s]];
+            CT v[7], y = 0;
+#pragma unroll
+            for (int s = 0; s < 7; s++) v[s] = cur[nb[s]];
+#pragma unroll
+            for (int s = 0; s < 7; s++) y += a[s] * v[s];
             nxt[row] = cur[row] + wv * (rv - y);
         }
         __syncthreads();
@@ -348,10 +454,19 @@ inline unsigned mg_grid(long long n) {   // a multiple of kXcd (mg_slab)
     return static_cast<unsigned>(g);
 }
 
+// f(symmetric view?, type of the row offsets) for a level
+template <class F>
+void mg_level(bool sym, long long rows, const F& f) {
+    if (sym && rows > kWideRows) f(std::true_type{}, 0LL);
+    else if (sym) f(std::true_type{}, 0u);
+    else if (rows > kWideRows) f(std::false_type{}, 0LL);
+    else f(std::false_type{}, 0u);
+}
+
 // Builds (or refreshes) the hierarchy of a one-component 3-D diagonal view whose level-0 slots
 // D0 are of type VT; XT is the vector type of the solve and of the coarse levels.
 template <typename VT, typename XT>
-int mg_setup(dare_ctx* ctx, MgHierarchy* H, const DiaView& V0, const VT* D0) {
+int mg_setup(dare_ctx* ctx, MgHierarchy* H, const DiaView& V0, const VT* D0, bool sym) {
     using CT = XT;
     if (V0.N != 1 || V0.cross) {
         set_error("the multigrid preconditioner needs a one-component operator without cross entries");
@@ -375,7 +490,7 @@ int mg_setup(dare_ctx* ctx, MgHierarchy* H, const DiaView& V0, const VT* D0) {
         set_error("multigrid needs a grid that coarsens (at least two cells along an axis) to at most 1024 rows");
         return DARE_ERR_UNSUPPORTED;
     }
-    if (mg_bricks(V0).total >= (1LL << 32)) {
+    if (mg_tiles(V0).total >= (1LL << 32)) {
         set_error("grid too large for the multigrid preconditioner");
         return DARE_ERR_UNSUPPORTED;
     }
@@ -420,16 +535,24 @@ int mg_setup(dare_ctx* ctx, MgHierarchy* H, const DiaView& V0, const VT* D0) {
     lv[0].W = H->fine;
     lv[0].z = static_cast<char*>(H->fine) + sizeof(VT) * V0.nrows;
     H->nlev = nlev;
+    H->sym = sym;
     H->D0 = D0;
     for (int l = 0; l < nlev; l++) H->lev[l] = lv[l];
     hipLaunchKernelGGL((k_mg_weight<VT>), dim3(mg_grid(V0.nrows)), dim3(kThreads), 0, ctx->stream, V0.nrows,
                        D0 + 3 * V0.nrows, mg_ptr<VT>(lv[0].W), H->omega);
-    hipLaunchKernelGGL((k_mg_coarsen<VT, CT>), dim3(mg_grid(lv[1].rows)), dim3(kThreads), 0, ctx->stream, V0, D0,
-                       lv[1].V, mg_ptr<CT>(lv[1].D), mg_ptr<CT>(lv[1].W), 0.5, H->omega);
-    for (int l = 2; l < nlev; l++)
-        hipLaunchKernelGGL((k_mg_coarsen<CT, CT>), dim3(mg_grid(lv[l].rows)), dim3(kThreads), 0, ctx->stream,
-                           lv[l - 1].V, static_cast<const CT*>(lv[l - 1].D), lv[l].V, mg_ptr<CT>(lv[l].D),
-                           mg_ptr<CT>(lv[l].W), 0.5, H->omega);
+    // every level's kernels by the view's symmetry and the width of its row offsets
+    for (int l = 0; l + 1 < nlev; l++)
+        mg_level(sym, lv[l].rows, [&](auto sc, auto ix) {
+            const MgTiles T = mg_tiles(lv[l].V);
+            const auto run = [&](const auto* D) {
+                using DT = std::remove_const_t<std::remove_pointer_t<decltype(D)>>;
+                hipLaunchKernelGGL((k_mg_coarsen<decltype(sc)::value, decltype(ix), DT, CT>), dim3(mg_tile_grid(T)),
+                                   dim3(64), 0, ctx->stream, lv[l].V, T, D, lv[l + 1].V, mg_ptr<CT>(lv[l + 1].D),
+                                   mg_ptr<CT>(lv[l + 1].W), 0.5, H->omega);
+            };
+            if (l == 0) run(D0);
+            else run(static_cast<const CT*>(lv[l].D));
+        });
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }
@@ -444,32 +567,33 @@ XT* mg_apply(hipStream_t sm, const MgHierarchy& H, const XT* r) {
     const int L = H.nlev - 1;
     const MgLevel& F = H.lev[0];
     const VT* W0 = static_cast<const VT*>(F.W);
-    const MgBricks B0 = mg_bricks(F.V);
-    hipLaunchKernelGGL((k_mg_down<true, VT, XT, CT>), dim3(mg_brick_grid(B0)), dim3(kThreads), 0, sm, F.V, B0, D0,
-                       W0, r, H.lev[1].V, mg_ptr<CT>(H.lev[1].r));
-    for (int l = 1; l < L; l++) {
+    // restriction from level l to l + 1, and correction of level l by l + 1
+    const auto down = [&](int l, auto sc, auto ix, const auto* D, const auto* W, const XT* rl) {
+        using DT = std::remove_const_t<std::remove_pointer_t<decltype(D)>>;
+        const MgTiles T = mg_tiles(H.lev[l].V);
+        hipLaunchKernelGGL((k_mg_down<decltype(sc)::value, decltype(ix), DT, XT, CT>), dim3(mg_tile_grid(T)), dim3(64),
+                           0, sm, H.lev[l].V, T, D, W, rl, H.lev[l + 1].V, mg_ptr<CT>(H.lev[l + 1].r));
+    };
+    const auto up = [&](int l, auto sc, auto ix, const auto* D, const auto* W, const XT* rl) {
+        using DT = std::remove_const_t<std::remove_pointer_t<decltype(D)>>;
+        const MgTiles T = mg_tiles(H.lev[l].V);
+        hipLaunchKernelGGL((k_mg_up<decltype(sc)::value, decltype(ix), DT, XT, CT>), dim3(mg_tile_grid(T)), dim3(64), 0,
+                           sm, H.lev[l].V, T, D, W, rl, H.lev[l + 1].V, static_cast<const CT*>(H.lev[l + 1].z),
+                           mg_ptr<XT>(H.lev[l].z));
+    };
+    const auto level = [&](int l, const auto& step) {
         const MgLevel& A = H.lev[l];
-        const MgLevel& C = H.lev[l + 1];
-        const MgBricks B = mg_bricks(A.V);
-        hipLaunchKernelGGL((k_mg_down<true, CT, CT, CT>), dim3(mg_brick_grid(B)), dim3(kThreads), 0, sm, A.V, B,
-                           static_cast<const CT*>(A.D), static_cast<const CT*>(A.W), static_cast<const CT*>(A.r), C.V,
-                           mg_ptr<CT>(C.r));
-    }
+        mg_level(H.sym, A.rows, [&](auto sc, auto ix) {
+            if (l == 0) step(l, sc, ix, D0, W0, r);
+            else step(l, sc, ix, static_cast<const CT*>(A.D), static_cast<const CT*>(A.W), static_cast<const CT*>(A.r));
+        });
+    };
     const MgLevel& Z = H.lev[L];
+    for (int l = 0; l < L; l++) level(l, down);
     hipLaunchKernelGGL((k_mg_coarsest<CT>), dim3(1), dim3(1024), 0, sm, Z.V, static_cast<const CT*>(Z.D),
                        static_cast<const CT*>(Z.W), static_cast<const CT*>(Z.r), mg_ptr<CT>(Z.z), H.coarse_sweeps);
-    for (int l = L - 1; l >= 1; l--) {
-        const MgLevel& A = H.lev[l];
-        const MgLevel& C = H.lev[l + 1];
-        const MgBricks B = mg_bricks(A.V);
-        hipLaunchKernelGGL((k_mg_up<true, CT, CT, CT>), dim3(mg_brick_grid(B)), dim3(kThreads), 0, sm, A.V, B,
-                           static_cast<const CT*>(A.D), static_cast<const CT*>(A.W), static_cast<const CT*>(A.r), C.V,
-                           static_cast<const CT*>(C.z), mg_ptr<CT>(A.z));
-    }
-    XT* z = mg_ptr<XT>(F.z);
-    hipLaunchKernelGGL((k_mg_up<true, VT, XT, CT>), dim3(mg_brick_grid(B0)), dim3(kThreads), 0, sm, F.V, B0, D0, W0,
-                       r, H.lev[1].V, static_cast<const CT*>(H.lev[1].z), z);
-    return z;
+    for (int l = L - 1; l >= 0; l--) level(l, up);
+    return mg_ptr<XT>(F.z);
 }
 
 }  // namespace
