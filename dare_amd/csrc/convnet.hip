@@ -108,8 +108,7 @@ __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict
     // slice of the input, the block stages in LDS the input it needs -- (16 NSEG + 2) x 6 x 3
     // voxels, zero outside the box -- as [half][voxel] (16 bytes = 8 channels per voxel), and
     // its weights as [half][tap][co] (16 bytes each). Every MFMA then reads both operands from
-    // LDS: a staged input value feeds up to 27 taps x NBB instructions. All global loads of a
-    // stage are issued before it is written, in batches of eight per thread.
+    // LDS: a staged input value feeds up to 27 taps x NBB instructions.
     // K = 32 is two taps x 16 channels (the 28th tap is zero).
     constexpr int SX = 16 * NSEG + 2, SY = 6, NV = SX * SY * 3;
     // the two channel halves are NVS pieces apart, a multiple of 256 bytes: lanes 0-15 and
@@ -131,37 +130,43 @@ __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict
     for (int s = 0; s < NSEG; s++)
 #pragma unroll
         for (int nb = 0; nb < NBB; nb++) acc[s][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int cc = 0; cc < CIN / 16; cc++) {
-        for (int b0 = 0; b0 < NPIECE; b0 += 8 * kNetThreads) {
-            uint4 u[8];
+    // a slice's pieces, all in flight together, and while the slice before is multiplied (in
+    // batches of eight and after its barrier they bounded the block: 16^3, 64 to 64 channels,
+    // 12.1 -> 10.0 us)
+    constexpr int RPS = (NPIECE + kNetThreads - 1) / kNetThreads;
+    uint4 u[RPS];
+    auto load_slice = [&](int cc) {
 #pragma unroll
-            for (int r = 0; r < 8; r++) {
-                const int t = b0 + r * kNetThreads + threadIdx.x;
-                u[r] = uint4{0u, 0u, 0u, 0u};
-                if (t < 2 * NV) {        // input piece (voxel, half), half fastest
-                    const int v = t >> 1, h = t & 1;
-                    const int xl = v % SX, yl = (v / SX) % SY, zl = v / (SX * SY);
-                    const int gx = x0 - 1 + xl, gy = y0 - 1 + yl, gz = z - 1 + zl;
-                    if (gx >= 0 && gx < W && gy >= 0 && gy < H && gz >= 0 && gz < D) {
-                        const long long src = (MODE & kConvUp)
-                            ? (static_cast<long long>(gz >> 1) * (H >> 1) + (gy >> 1)) * (W >> 1) + (gx >> 1)
-                            : (static_cast<long long>(gz) * H + gy) * W + gx;
-                        u[r] = *reinterpret_cast<const uint4*>(X + src * CIN + 16 * cc + 8 * h);
-                    }
-                } else if (t < NPIECE) { // weight piece (half, tap, co), co fastest
-                    const int w = t - 2 * NV;
-                    const int co = w % (16 * NBB), tap = (w / (16 * NBB)) % 27, h = w / (16 * NBB * 27);
-                    u[r] = *reinterpret_cast<const uint4*>(
-                        Wt + (static_cast<long long>(tap) * COUT + grp * 16 * NBB + co) * CIN + 16 * cc + 8 * h);
+        for (int r = 0; r < RPS; r++) {
+            const int t = r * kNetThreads + threadIdx.x;
+            u[r] = uint4{0u, 0u, 0u, 0u};
+            if (t < 2 * NV) {        // input piece (voxel, half), half fastest
+                const int v = t >> 1, h = t & 1;
+                const int xl = v % SX, yl = (v / SX) % SY, zl = v / (SX * SY);
+                const int gx = x0 - 1 + xl, gy = y0 - 1 + yl, gz = z - 1 + zl;
+                if (gx >= 0 && gx < W && gy >= 0 && gy < H && gz >= 0 && gz < D) {
+                    const long long src = (MODE & kConvUp)
+                        ? (static_cast<long long>(gz >> 1) * (H >> 1) + (gy >> 1)) * (W >> 1) + (gx >> 1)
+                        : (static_cast<long long>(gz) * H + gy) * W + gx;
+                    u[r] = *reinterpret_cast<const uint4*>(X + src * CIN + 16 * cc + 8 * h);
                 }
-            }
-#pragma unroll
-            for (int r = 0; r < 8; r++) {
-                const int t = b0 + r * kNetThreads + threadIdx.x;
-                if (t < 2 * NV) stage[(t & 1) * NVS + (t >> 1)] = u[r];
-                else if (t < NPIECE) wl[t - 2 * NV] = u[r];
+            } else if (t < NPIECE) { // weight piece (half, tap, co), co fastest
+                const int w = t - 2 * NV;
+                const int co = w % (16 * NBB), tap = (w / (16 * NBB)) % 27, h = w / (16 * NBB * 27);
+                u[r] = *reinterpret_cast<const uint4*>(
+                    Wt + (static_cast<long long>(tap) * COUT + grp * 16 * NBB + co) * CIN + 16 * cc + 8 * h);
             }
         }
+    };
+    load_slice(0);
+    for (int cc = 0; cc < CIN / 16; cc++) {
+#pragma unroll
+        for (int r = 0; r < RPS; r++) {
+            const int t = r * kNetThreads + threadIdx.x;
+            if (t < 2 * NV) stage[(t & 1) * NVS + (t >> 1)] = u[r];
+            else if (t < NPIECE) wl[t - 2 * NV] = u[r];
+        }
+        if (cc + 1 < CIN / 16) load_slice(cc + 1);
         __syncthreads();
         if (y < H) {                           // wave-uniform; every wave reaches both barriers
             // operands of step c + 1 are read from LDS before the MFMAs of step c
@@ -313,6 +318,8 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_zm(const uint16_t* __restr
     // 2 (q % 14) + 1; lane (i, kq) holds output channel grp 16 + i, tap 2 (q % 14) + kq / 2,
     // channels 8 (2 (q / 14) + kq % 2) .. +7 (zero for the 28th tap)
     bf16x8 wr[WREG ? NSTEP : 1];
+    constexpr int RWP = (NWP + kNetThreads - 1) / kNetThreads;
+    uint4 wu[RWP];
     if constexpr (WREG) {
 #pragma unroll
         for (int q = 0; q < NSTEP; q++) {
@@ -321,18 +328,29 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_zm(const uint16_t* __restr
             wr[q] = load8(Wt + (static_cast<long long>(tap) * COUT + grp * 16 + i) * CIN + 8 * p8, tap < 27);
         }
     } else {
-        for (int t = threadIdx.x; t < NWP; t += kNetThreads) {
+#pragma unroll
+        for (int r = 0; r < RWP; r++) {
+            const int t = r * kNetThreads + threadIdx.x;
             const int co = t % 16, tap = (t / 16) % 27, p8 = t / (16 * 27);
-            wl[t] = *reinterpret_cast<const uint4*>(Wt + (static_cast<long long>(tap) * COUT + grp * 16 + co) * CIN +
-                                                    8 * p8);
+            wu[r] = uint4{0u, 0u, 0u, 0u};
+            if (t < NWP)
+                wu[r] = *reinterpret_cast<const uint4*>(
+                    Wt + (static_cast<long long>(tap) * COUT + grp * 16 + co) * CIN + 8 * p8);
         }
     }
-    // the first three planes (z0-1, z0, z0+1 -> slots by plane mod 3)
+    // the first three planes (z0-1, z0, z0+1 -> slots by plane mod 3), all loaded before the first
+    // is written: a march of a few planes is otherwise bounded by waiting out one load after the
+    // other (64^3, 16 to 16 channels, two planes a block: 11.0 -> 10.3 us)
     {
-        uint4 u[RPL];
-        for (int q = -1; q <= 1; q++) {
-            load_plane(z0 + q, u);
-            store_plane((z0 + q + 3) % 3, u);
+        uint4 u[3][RPL];
+#pragma unroll
+        for (int q = 0; q < 3; q++) load_plane(z0 - 1 + q, u[q]);
+#pragma unroll
+        for (int q = 0; q < 3; q++) store_plane((z0 + q + 2) % 3, u[q]);
+        if constexpr (!WREG) {
+#pragma unroll
+            for (int r = 0; r < RWP; r++)
+                if (r * kNetThreads + static_cast<int>(threadIdx.x) < NWP) wl[r * kNetThreads + threadIdx.x] = wu[r];
         }
     }
     __syncthreads();
@@ -520,11 +538,11 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_sub(const uint16_t* __rest
         }
     };
     {
-        uint4 u[RPL];
-        for (int q = 0; q < 2; q++) {                            // coarse planes k0 - 1 + rz, k0 + rz
-            load_plane(k0 - 1 + rz + q, u);
-            store_plane(k0 - 1 + rz + q, u);
-        }
+        uint4 u[2][RPL];                                         // coarse planes k0 - 1 + rz, k0 + rz
+#pragma unroll
+        for (int q = 0; q < 2; q++) load_plane(k0 - 1 + rz + q, u[q]);
+#pragma unroll
+        for (int q = 0; q < 2; q++) store_plane(k0 - 1 + rz + q, u[q]);
     }
     __syncthreads();
     // E of output plane z = 2k + rz (the skip operand), loaded before the MFMAs that precede
@@ -1021,17 +1039,6 @@ __global__ __launch_bounds__(kNetThreads) void k_scales(FieldGeo F, const double
     }
 }
 
-// one wave per scale: lanes stride over the block maxima, then a wave maximum (max is exact in
-// any order)
-__global__ __launch_bounds__(192) void k_scales_finish(const double* __restrict__ part, int nblocks, double* __restrict__ s) {
-    const int which = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double m = 0.;
-    for (int b = lane; b < nblocks; b += 64) m = fmax(m, part[which * 1024 + b]);
-    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_down(m, off));
-    // floors keep the channels finite when a field is flat (first step of a trajectory)
-    if (lane == 0) s[which] = fmax(m, 1e-300);
-}
-
 // x0[v][c]: c0 = phi^n / s0, c1 = (phi^n - phi^{n-1}) / s1, c2 = resid * resid_scale / s2,
 // c3.. = (extra_e - offset_e) * scale_e (static fields), the rest 0.
 struct Extras {
@@ -1040,36 +1047,79 @@ struct Extras {
     int n;
 };
 
+// The scales are the maxima over k_scales' nblocks <= 1024 block maxima (exact in any order):
+// every block forms them itself, and block 0 leaves them in s (a kernel of one block between the
+// two took 5.7 us). Then a lane per voxel, all of a field's loads in flight: bytes bound it
+// (128^3 to 64^3 voxels: 11.1 and 5.7 -> 13.5 us).
 template <int CF>
 __global__ __launch_bounds__(kNetThreads) void k_pack(FieldGeo F, const double* __restrict__ phi,
                                                      const double* __restrict__ phim, const double* __restrict__ resid,
-                                                     double resid_scale, Extras ex, const double* __restrict__ s,
-                                                     uint16_t* __restrict__ x0) {
+                                                     double resid_scale, Extras ex, const double* __restrict__ part,
+                                                     int nblocks, double* __restrict__ s, uint16_t* __restrict__ x0) {
+    __shared__ double red[3][kNetThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double sc[3], pt[3][4];
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int b = u * kNetThreads + threadIdx.x;
+            pt[m][u] = part[m * 1024 + (b < nblocks ? b : 0)];
+        }
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        sc[m] = fmax(fmax(fmax(0., pt[m][0]), pt[m][1]), fmax(pt[m][2], pt[m][3]));
+        for (int off = 32; off > 0; off >>= 1) sc[m] = fmax(sc[m], __shfl_xor(sc[m], off));
+        if (lane == 0) red[m][wave] = sc[m];
+    }
+    __syncthreads();
+    // floors keep the channels finite when a field is flat (first step of a trajectory)
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        for (int w = 0; w < kNetThreads / 64; w++) sc[m] = fmax(sc[m], red[m][w]);
+        sc[m] = fmax(sc[m], 1e-300);
+        if (blockIdx.x == 0 && threadIdx.x == 0) s[m] = sc[m];
+    }
     // channel values of a voxel: their mean over its CF^3 cells (CF = 1: the cell's values)
     const long long n = static_cast<long long>(F.c0) * F.c1 * F.c2;
-    const double i0 = 1. / s[0], i1 = 1. / s[1], i2 = 1. / s[2];
-    const double avg = 1. / (CF * CF * CF);
+    const double i0 = 1. / sc[0], i1 = 1. / sc[1], i2 = 1. / sc[2];
+    constexpr int NC = CF * CF * CF;
+    const double avg = 1. / NC;
     for (long long q = blockIdx.x * (long long)kNetThreads + threadIdx.x; q < n; q += (long long)gridDim.x * kNetThreads) {
         int z, y, x;
         box_zyx(q, F.c1, F.c2, z, y, x);
         double acc[kInChannels];
+#pragma unroll
         for (int c = 0; c < kInChannels; c++) acc[c] = 0.;
-        for (int a = 0; a < CF; a++)
-            for (int b = 0; b < CF; b++)
-                for (int d = 0; d < CF; d++) {
-                    const int zz = CF * z + a, yy = CF * y + b, xx = CF * x + d;
-                    const long long pi = pad_index(F, zz, yy, xx);
-                    const double p = phi[pi];
-                    acc[0] += p * i0;
-                    acc[1] += (p - phim[pi]) * i1;
-                    acc[2] += resid[row_index(F, zz, yy, xx)] * resid_scale * i2;
-                    for (int c = 3; c < kInChannels; c++) {
-                        const int e = c - 3;
-                        if (e < ex.n) acc[c] += (ex.f[e][pi] - ex.offset[e]) * ex.scale[e];
-                    }
-                }
+        long long pi[NC];
+        double p[NC], pm[NC], rs[NC];
+#pragma unroll
+        for (int e = 0; e < NC; e++) {
+            const int zz = CF * z + e / (CF * CF), yy = CF * y + e / CF % CF, xx = CF * x + e % CF;
+            pi[e] = pad_index(F, zz, yy, xx);
+            p[e] = phi[pi[e]];
+            pm[e] = phim[pi[e]];
+            rs[e] = resid[row_index(F, zz, yy, xx)];
+        }
+#pragma unroll
+        for (int e = 0; e < NC; e++) {
+            acc[0] += p[e] * i0;
+            acc[1] += (p[e] - pm[e]) * i1;
+            acc[2] += rs[e] * resid_scale * i2;
+        }
+#pragma unroll
+        for (int c = 3; c < kInChannels; c++) {
+            if (c - 3 >= ex.n) break;
+            double f[NC];
+#pragma unroll
+            for (int e = 0; e < NC; e++) f[e] = ex.f[c - 3][pi[e]];
+#pragma unroll
+            for (int e = 0; e < NC; e++) acc[c] += (f[e] - ex.offset[c - 3]) * ex.scale[c - 3];
+        }
         uint16_t ch[kInChannels];
+#pragma unroll
         for (int c = 0; c < kInChannels; c++) ch[c] = f2bf(static_cast<float>(acc[c] * avg));
+#pragma unroll
         for (int c = 0; c < kInChannels; c++) x0[q * kInChannels + c] = ch[c];
     }
 }
@@ -1078,37 +1128,55 @@ __global__ __launch_bounds__(kNetThreads) void k_pack(FieldGeo F, const double* 
 // whose residual the network saw). CF = 2: out is read at the cell through the trilinear
 // interpolation of the voxel values (cell centres: weights 3/4 and 1/4 of the two nearest
 // voxels per axis, the nearest one repeated at the box faces).
+// A lane holds a voxel's CF^3 cells, which share the 27 values around it (a lane per cell read
+// eight values a cell with their indices: 128^3, 12.2 -> 8.7 us).
 template <int CF>
 __global__ __launch_bounds__(kNetThreads) void k_unpack(FieldGeo F, const double* __restrict__ base,
                                                        const float* __restrict__ out, const double* __restrict__ s,
                                                        double* __restrict__ xg) {
-    const long long n = static_cast<long long>(F.n0) * F.n1 * F.n2;
+    const long long n = static_cast<long long>(F.c0) * F.c1 * F.c2;
     const double s2 = s[2];
     for (long long q = blockIdx.x * (long long)kNetThreads + threadIdx.x; q < n; q += (long long)gridDim.x * kNetThreads) {
         int z, y, x;
-        box_zyx(q, F.n1, F.n2, z, y, x);
-        const long long r = row_index(F, z, y, x);
-        double o;
-        if (CF == 1) {
-            o = static_cast<double>(out[q]);
+        box_zyx(q, F.c1, F.c2, z, y, x);
+        if constexpr (CF == 1) {
+            const long long r = row_index(F, z, y, x);
+            xg[r] = base[r] + s2 * static_cast<double>(out[q]);
         } else {
             const int p[3] = {z, y, x}, nc[3] = {F.c0, F.c1, F.c2};
-            int v0[3], v1[3];
+            long long at[3][3];                // the voxel before, the voxel, the one after, per axis
+            const long long st[3] = {static_cast<long long>(F.c1) * F.c2, F.c2, 1};
+#pragma unroll
             for (int d = 0; d < 3; d++) {
-                v0[d] = p[d] >> 1;
-                const int other = v0[d] + ((p[d] & 1) ? 1 : -1);
-                v1[d] = other < 0 ? 0 : (other >= nc[d] ? nc[d] - 1 : other);
+                at[d][0] = st[d] * (p[d] > 0 ? p[d] - 1 : 0);
+                at[d][1] = st[d] * p[d];
+                at[d][2] = st[d] * (p[d] + 1 < nc[d] ? p[d] + 1 : nc[d] - 1);
             }
-            o = 0.;
-            for (int a = 0; a < 2; a++)
-                for (int b = 0; b < 2; b++)
-                    for (int c = 0; c < 2; c++) {
-                        const double w = (a ? 0.25 : 0.75) * (b ? 0.25 : 0.75) * (c ? 0.25 : 0.75);
-                        const long long vz = a ? v1[0] : v0[0], vy = b ? v1[1] : v0[1], vx = c ? v1[2] : v0[2];
-                        o += w * static_cast<double>(out[(vz * F.c1 + vy) * F.c2 + vx]);
-                    }
+            double v[3][3][3], b[8];
+            long long r[8];
+#pragma unroll
+            for (int a = 0; a < 3; a++)
+#pragma unroll
+                for (int e = 0; e < 3; e++)
+#pragma unroll
+                    for (int c = 0; c < 3; c++)
+                        v[a][e][c] = static_cast<double>(out[at[0][a] + at[1][e] + at[2][c]]);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                r[e] = row_index(F, 2 * z + (e >> 2), 2 * y + (e >> 1 & 1), 2 * x + (e & 1));
+                b[e] = base[r[e]];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                double o = 0.;
+#pragma unroll
+                for (int t = 0; t < 8; t++) {  // t: the further voxel along z (4), y (2), x (1)
+                    const double w = (t & 4 ? 0.25 : 0.75) * (t & 2 ? 0.25 : 0.75) * (t & 1 ? 0.25 : 0.75);
+                    o += w * v[t & 4 ? (e & 4 ? 2 : 0) : 1][t & 2 ? (e & 2 ? 2 : 0) : 1][t & 1 ? (e & 1 ? 2 : 0) : 1];
+                }
+                xg[r[e]] = b[e] + s2 * o;
+            }
         }
-        xg[r] = base[r] + s2 * o;
     }
 }
 
@@ -1668,13 +1736,12 @@ int dare_convnet_pack(dare_ctx* ctx, dare_convnet* net, const dare_grid* g, cons
     const unsigned gs = std::min<unsigned>(ew_grid(n), 1024);
     hipLaunchKernelGGL(k_scales, dim3(gs), dim3(kNetThreads), 0, ctx->stream, F, phi, phi_prev, resid, resid_scale,
                        net->part);
-    hipLaunchKernelGGL(k_scales_finish, dim3(1), dim3(192), 0, ctx->stream, net->part, static_cast<int>(gs), net->scales);
     if (net->cf == 2)
         hipLaunchKernelGGL(k_pack<2>, dim3(ew_grid(nv)), dim3(kNetThreads), 0, ctx->stream, F, phi, phi_prev, resid,
-                           resid_scale, ex, net->scales, net->x0);
+                           resid_scale, ex, net->part, static_cast<int>(gs), net->scales, net->x0);
     else
         hipLaunchKernelGGL(k_pack<1>, dim3(ew_grid(nv)), dim3(kNetThreads), 0, ctx->stream, F, phi, phi_prev, resid,
-                           resid_scale, ex, net->scales, net->x0);
+                           resid_scale, ex, net->part, static_cast<int>(gs), net->scales, net->x0);
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }
@@ -1735,7 +1802,7 @@ int dare_convnet_unpack(dare_ctx* ctx, dare_convnet* net, const dare_grid* g, co
                    "box differs from the one of the last forward pass");
     const long long n = static_cast<long long>(F.n0) * F.n1 * F.n2;
     if (net->cf == 2)
-        hipLaunchKernelGGL(k_unpack<2>, dim3(ew_grid(n)), dim3(kNetThreads), 0, ctx->stream, F, base, net->out,
+        hipLaunchKernelGGL(k_unpack<2>, dim3(ew_grid(n / 8)), dim3(kNetThreads), 0, ctx->stream, F, base, net->out,
                            net->scales, x_guess);
     else
         hipLaunchKernelGGL(k_unpack<1>, dim3(ew_grid(n)), dim3(kNetThreads), 0, ctx->stream, F, base, net->out,
