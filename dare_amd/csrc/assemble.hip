@@ -67,44 +67,42 @@ __device__ inline double lim_psi(int id, double r) {
     }
 }
 
-// Column of neighbor position pos (0 = centre, 1..6 = W,E,S,N,B,T) with the periodic wrap of
-// MapIndexToOrdinalGlobalInternal(ind, true) (CartesianRepresentation.inl:418-450).
-__device__ inline long long nb_col(const Geo& G, const int q[3], int pos) {
-    int p[3] = {q[0], q[1], q[2]};
-    if (pos > 0) {
-        const int d = (pos - 1) / 2;
-        p[d] += (pos & 1) ? -1 : 1;
-    }
-    long long o = 0;
-    for (int d = 0; d < G.dim; d++) {
-        int v = p[d];
-        if (G.any_periodic) {
-            if (v < 0) v = G.n[d] + v;
-            else if (v >= G.n[d]) v = v - G.n[d];
-        }
-        o += G.si[d] * v;
-    }
-    return o;
+// Column (component 0, in cells) of neighbor position pos (0 = centre, 1..6 = W,E,S,N,B,T) of
+// cell `node` at q, with the periodic wrap of MapIndexToOrdinalGlobalInternal(ind, true)
+// (CartesianRepresentation.inl:418-450).
+__device__ inline int nb_col(const Geo& G, const int q[3], int node, int pos) {
+    if (pos == 0) return node;
+    const int d = (pos - 1) / 2, n = G.n[d], si = static_cast<int>(G.si[d]);
+    if (pos & 1) return node + (G.any_periodic && q[d] == 0 ? n - 1 : -1) * si;
+    return node + (G.any_periodic && q[d] == n - 1 ? 1 - n : 1) * si;
 }
 
-// Builds the (unsorted) entries of one row in Finalize order: explicit cross entry first, then
-// W,S,B,C,T,N,E for set positions. Then stable-sorts by column and merges duplicates.
+// The entries of one row: explicit cross entry first, then W,S,B,C,T,N,E for set positions (the
+// Finalize order), stable-sorted by column, equal columns merged. emit(j, column, value) receives
+// entry j; returns their number. An entry's place is the number of lower columns among the first
+// of each column, by compares of all pairs: a sort of arrays indexed at run time kept them, and
+// with them the positions' values, in scratch memory (two components, 160 x 120 cells: 21.7
+// -> 5.5 us a fill; the structure of 128^3: 315 -> 72 us).
 // MODE 0: structure only; 1: evaluate the functor; 2: values taken from the diagonal-view
 // slots (slot_in) written earlier by mode 1. SORT = false stops after the values (the
 // diagonal-view fill needs no column order).
 enum { kRowStructure = 0, kRowValues = 1, kRowFromSlots = 2 };
 constexpr int kPosOfSlot[7] = {1, 3, 5, 0, 6, 4, 2};
 
-// DIM = 0 takes the dimension from G at run time; DIM = 3 (the diagonal-view fill) lets every
-// per-axis loop unroll, so the per-position arrays live in registers.
+// DIM = 0 takes the dimension from G at run time. Every per-axis loop unrolls, so the per-position
+// arrays live in registers.
 // FEAT: the terms the instantiation may meet (kFeat* bits); a cleared bit drops that term's
 // code (the host picks the diagonal-view fill's smallest mask that covers the operator).
 enum { kFeatConv = 1, kFeatDiffCell = 2, kFeatSource = 4, kFeatCross = 8, kFeatFixed = 16, kFeatAll = 31 };
-template <int MODE, bool SORT, int DIM = 0, int FEAT = kFeatAll>
-__device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, long long node,
-                           int* cols, double* vals, double* rhs_out, double* x0_out,
-                           double* slotv = nullptr, const double* slot_in = nullptr) {
+struct NoEmit {
+    __device__ void operator()(int, int, double) const {}
+};
+template <int MODE, bool SORT, int DIM = 0, int FEAT = kFeatAll, class Emit = NoEmit>
+__device__ __forceinline__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, long long node,
+                           double* rhs_out, double* x0_out, double* slotv = nullptr,
+                           const double* slot_in = nullptr, const Emit& emit = Emit()) {
     constexpr bool VALUES = MODE == kRowValues;
+    constexpr int kD = DIM ? DIM : 3;
     const int dim = DIM ? DIM : G.dim;
     double nbv[7] = {0., 0., 0., 0., 0., 0., 0.};
     double rhs = 0.;
@@ -112,7 +110,8 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
     double cross = 0.;
     const bool has_cross = (FEAT & kFeatCross) && T.cross != 0;
     long long lp = 0;
-    for (int d = 0; d < dim; d++) lp += G.sl[d] * (q[d] + G.g);
+#pragma unroll
+    for (int d = 0; d < kD && (DIM || d < dim); d++) lp += G.sl[d] * (q[d] + G.g);
     const int N = G.N;
 
     // a cell on a DARE_BC_FIXED face (the first axis that has one, low face first) is an
@@ -125,7 +124,8 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
     const bool fixed = fixed_face >= 0;
     // boundary faces hit by an edit (they only depend on the structure)
     int bc_face[3] = {-1, -1, -1};
-    for (int d = 0; d < dim; d++) {
+#pragma unroll
+    for (int d = 0; d < kD && (DIM || d < dim); d++) {
         if (q[d] == 0 && T.bc_type[2 * d] != 0) bc_face[d] = 2 * d;
         else if (q[d] == G.n[d] - 1 && T.bc_type[2 * d + 1] != 0) bc_face[d] = 2 * d + 1;
         // position bc_face + 1, written with constant indices
@@ -144,7 +144,8 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
         }
         {   // mb -= div(D_f * grad(mb))
             double o[7] = {0., 0., 0., 0., 0., 0., 0.};
-            for (int d = 0; d < dim; d++) {
+#pragma unroll
+            for (int d = 0; d < kD && (DIM || d < dim); d++) {
                 double Df[2];
                 for (int h = 0; h < 2; h++) {
                     if ((FEAT & kFeatDiffCell) && T.diff_cell) {
@@ -168,15 +169,18 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
             }
             // the scheme weight of the implicit level (s_c *= coef_td); the gradient's face
             // right-hand sides are 0, so the explicit levels add nothing here
-            for (int pos = 0; pos < 2 * dim + 1; pos++) nbv[pos] += (o[pos] * T.div_w[0]) * -1.;
+#pragma unroll
+            for (int pos = 0; pos < 2 * kD + 1 && (DIM || pos < 2 * dim + 1); pos++) nbv[pos] += (o[pos] * T.div_w[0]) * -1.;
             rhs += 0. * -1.;
         }
         if ((FEAT & kFeatConv) && T.conv_limiter >= 0) {   // mb += div(tvd * phi)
             double o[7] = {0., 0., 0., 0., 0., 0., 0.};
             double orhs = 0., frd[3] = {0., 0., 0.};
-            for (int d = 0; d < dim; d++) {
+#pragma unroll
+            for (int d = 0; d < kD && (DIM || d < dim); d++) {
                 long long fi = 0;
-                for (int e = 0; e < dim; e++) fi += T.fs[d][e] * q[e];
+#pragma unroll
+                for (int e = 0; e < kD && (DIM || e < dim); e++) fi += T.fs[d][e] * q[e];
                 const double u[2] = {T.vel[d][fi], T.vel[d][fi + T.fs[d][d]]};
                 double nb[2], cc[2], fr[2];
                 const long long s = G.sl[d] * N;
@@ -213,8 +217,10 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
             // time scheme (Divergence_Cartesian.inl:183-204): coefficients times w0, the face
             // right-hand sides once more per explicit level t, weighted by w_t
             for (int t = 1; t < T.div_nt; t++)
-                for (int d = 0; d < dim; d++) orhs += T.div_w[t] * G.A[d] * frd[d];
-            for (int pos = 0; pos < 2 * dim + 1; pos++) nbv[pos] += o[pos] * T.div_w[0];
+#pragma unroll
+                for (int d = 0; d < kD && (DIM || d < dim); d++) orhs += T.div_w[t] * G.A[d] * frd[d];
+#pragma unroll
+            for (int pos = 0; pos < 2 * kD + 1 && (DIM || pos < 2 * dim + 1); pos++) nbv[pos] += o[pos] * T.div_w[0];
             rhs += orhs;
         }
         if ((FEAT & kFeatSource) && T.source) rhs += G.V * T.source[lp * N + c];
@@ -223,7 +229,8 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
             nbv[0] -= G.V * R[c * 2 + c];
             cross = -(G.V * R[c * 2 + (1 - c)]);
         }
-        for (int d = 0; d < dim; d++) {                  // boundary edits
+#pragma unroll
+        for (int d = 0; d < kD && (DIM || d < dim); d++) {                  // boundary edits
             const int f = bc_face[d];
             if (f < 0) continue;
             const double nbf = (f == 2 * d) ? nbv[2 * d + 1] : nbv[2 * d + 2];   // nbv[f + 1]
@@ -256,60 +263,58 @@ __device__ int row_entries(const Geo& G, const Terms& T, const int q[3], int c, 
     }
     if (!SORT) return 0;
 
-    // Finalize order, then stable sort by column + merge of equal columns
-    long long kc[kMaxEntries];
+    // cross, W, S, B, C, T, N, E
+    int kc[kMaxEntries];
     double kv[kMaxEntries];
-    int k = 0;
-    if (has_cross && !fixed) {
-        kc[k] = node * N + (1 - c);
-        kv[k] = cross;
-        k++;
-    }
-    const int order[7] = {1, 3, 5, 0, 6, 4, 2};
-    for (int j = 0; j < 7; j++) {
-        const int pos = order[j];
-        if (pos > 2 * dim || removed[pos]) continue;
-        kc[k] = nb_col(G, q, pos) * N + c;
-        kv[k] = nbv[pos];
-        k++;
-    }
-    for (int i = 1; i < k; i++) {                          // insertion sort (stable)
-        const long long ck = kc[i];
-        const double cv = kv[i];
-        int j = i - 1;
-        while (j >= 0 && kc[j] > ck) {
-            kc[j + 1] = kc[j];
-            kv[j + 1] = kv[j];
-            j--;
-        }
-        kc[j + 1] = ck;
-        kv[j + 1] = cv;
+    bool on[kMaxEntries], lead[kMaxEntries];
+    kc[0] = static_cast<int>(node) * N + (1 - c);
+    kv[0] = cross;
+    on[0] = has_cross && !fixed;
+#pragma unroll
+    for (int sl = 0; sl < 7; sl++) {
+        const int pos = kPosOfSlot[sl];
+        on[sl + 1] = pos <= 2 * dim && !removed[pos];
+        kc[sl + 1] = pos <= 2 * kD ? nb_col(G, q, static_cast<int>(node), pos) * N + c : 0;
+        kv[sl + 1] = nbv[pos];
     }
     int w = 0;
-    for (int i = 0; i < k; i++) {
-        if (w > 0 && kc[w - 1] == kc[i]) {
-            kv[w - 1] += kv[i];
-        } else {
-            kc[w] = kc[i];
-            kv[w] = kv[i];
-            w++;
-        }
+#pragma unroll
+    for (int e = 0; e < kMaxEntries; e++) {
+        lead[e] = on[e];
+#pragma unroll
+        for (int f = 0; f < e; f++) lead[e] = lead[e] && !(on[f] && kc[f] == kc[e]);
+        w += lead[e] ? 1 : 0;
     }
-    for (int i = 0; i < w; i++) {
-        if (cols) cols[i] = static_cast<int>(kc[i]);
-        if (MODE != kRowStructure) vals[i] = kv[i];
+    if constexpr (!std::is_same_v<Emit, NoEmit>) {
+#pragma unroll
+        for (int e = 0; e < kMaxEntries; e++) {
+            int at = 0;
+            double v = kv[e];
+#pragma unroll
+            for (int f = 0; f < kMaxEntries; f++) {
+                at += lead[f] && kc[f] < kc[e] ? 1 : 0;
+                if (f > e && on[f] && kc[f] == kc[e]) v += kv[f];
+            }
+            if (lead[e]) emit(at, kc[e], v);
+        }
     }
     return w;
 }
 
+// rows and cells fit 31 bits (make_geo)
 __device__ inline void row_to_cell(const Geo& G, long long row, int q[3], int* c, long long* node) {
-    *c = static_cast<int>(row % G.N);
-    long long nd = row / G.N;
+    const unsigned r = static_cast<unsigned>(row), N = static_cast<unsigned>(G.N);
+    unsigned nd = r / N;
+    *c = static_cast<int>(r - nd * N);
     *node = nd;
     q[0] = q[1] = q[2] = 0;
-    for (int d = 0; d < G.dim; d++) {
-        q[d] = static_cast<int>(nd / G.si[d]);
-        nd -= static_cast<long long>(q[d]) * G.si[d];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        if (d >= G.dim) break;
+        const unsigned si = static_cast<unsigned>(G.si[d]);
+        const unsigned v = nd / si;
+        q[d] = static_cast<int>(v);
+        nd -= v * si;
     }
 }
 
@@ -321,8 +326,7 @@ __device__ inline int row_count(const Geo& G, const Terms& T, long long row) {
     int q[3], c;
     long long node;
     row_to_cell(G, row, q, &c, &node);
-    int cols[kMaxEntries];
-    return row_entries<kRowStructure, true>(G, T, q, c, node, cols, nullptr, nullptr, nullptr);
+    return row_entries<kRowStructure, true>(G, T, q, c, node, nullptr, nullptr);
 }
 
 // block-wide inclusive scan of one int per thread (wave64 shuffles + LDS)
@@ -384,31 +388,31 @@ __global__ __launch_bounds__(kScanThreads) void k_write_structure(Geo G, Terms T
                                                                   int* __restrict__ col) {
     __shared__ int lds[kScanThreads / 64];
     const long long base = static_cast<long long>(blockIdx.x) * kScanTile;
-    // each thread owns kScanItems consecutive rows so that a block scan gives row offsets
-    int cnt[kScanItems];
-    int s = 0;
+    long long off = tile_off[blockIdx.x];
     for (int i = 0; i < kScanItems; i++) {
-        const long long row = base + static_cast<long long>(threadIdx.x) * kScanItems + i;
-        cnt[i] = row < nrows ? row_count(G, T, row) : 0;
-        s += cnt[i];
-    }
-    const int incl = block_scan_incl(s, lds);
-    long long off = tile_off[blockIdx.x] + incl - s;
-    for (int i = 0; i < kScanItems; i++) {
-        const long long row = base + static_cast<long long>(threadIdx.x) * kScanItems + i;
-        if (row >= nrows) break;
-        row_ptr[row] = static_cast<int>(off);
-        int q[3], c;
-        long long node;
-        row_to_cell(G, row, q, &c, &node);
-        int cols[kMaxEntries];
-        const int k = row_entries<kRowStructure, true>(G, T, q, c, node, cols, nullptr, nullptr, nullptr);
-        for (int j = 0; j < k; j++) col[off + j] = cols[j];
-        off += k;
+        const long long row = base + static_cast<long long>(i) * kScanThreads + threadIdx.x;
+        const int cnt = row < nrows ? row_count(G, T, row) : 0;
+        const int incl = block_scan_incl(cnt, lds);
+        int total = 0;
+        for (int w = 0; w < kScanThreads / 64; w++) total += lds[w];
+        if (row < nrows) {
+            const long long o = off + incl - cnt;
+            row_ptr[row] = static_cast<int>(o);
+            int q[3], c;
+            long long node;
+            row_to_cell(G, row, q, &c, &node);
+            row_entries<kRowStructure, true>(G, T, q, c, node, nullptr, nullptr, nullptr, nullptr,
+                                             [&](int j, int cl, double) { col[o + j] = cl; });
+        }
+        off += total;
+        __syncthreads();
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) row_ptr[nrows] = static_cast<int>(tile_off[gridDim.x]);
 }
 
+// CSR fill, one lane per row. DIM and FEAT as k_fill_dia's masks: the common operators' kernels
+// hold only their terms.
+template <int DIM, int FEAT>
 __global__ __launch_bounds__(256) void k_fill_values(Geo G, Terms T, long long nrows,
                                                      const int* __restrict__ row_ptr,
                                                      double* __restrict__ val, double* __restrict__ rhs,
@@ -418,12 +422,10 @@ __global__ __launch_bounds__(256) void k_fill_values(Geo G, Terms T, long long n
     int q[3], c;
     long long node;
     row_to_cell(G, row, q, &c, &node);
-    int cols[kMaxEntries];
-    double vals[kMaxEntries];
-    double r = 0., x = 0.;
-    const int k = row_entries<kRowValues, true>(G, T, q, c, node, cols, vals, &r, &x);
     const int o = row_ptr[row];
-    for (int j = 0; j < k; j++) val[o + j] = vals[j];
+    double r = 0., x = 0.;
+    row_entries<kRowValues, true, DIM, FEAT>(G, T, q, c, node, &r, &x, nullptr, nullptr,
+                                             [&](int j, int, double v) { val[o + j] = v; });
     rhs[row] = r;
     if (x0) x0[row] = x;
 }
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(256) void k_fill_dia(Geo G, Terms T, double* __rest
     const long long row = node * N + c;
     double slotv[kDiaSlots];
     double r = 0., x = 0.;
-    row_entries<kRowValues, false, 3, FEAT>(G, T, q, c, node, nullptr, nullptr, &r, &x, slotv);
+    row_entries<kRowValues, false, 3, FEAT>(G, T, q, c, node, &r, &x, slotv);
     if constexpr (HALF) {                           // W, S, B, C
 #pragma unroll
         for (int sl = 0; sl < 4; sl++) put<NT>(dia + sl * nrows + row, slotv[sl]);
@@ -512,11 +514,9 @@ __global__ __launch_bounds__(256) void k_materialize_csr(Geo G, Terms T, long lo
     row_to_cell(G, row, q, &c, &node);
     double sl_in[kDiaSlots];
     for (int sl = 0; sl < kDiaSlots; sl++) sl_in[sl] = sl < slots ? dia[sl * nrows + row] : 0.;
-    double vals[kMaxEntries];
-    const int k = row_entries<kRowFromSlots, true>(G, T, q, c, node, nullptr, vals, nullptr, nullptr, nullptr,
-                                                   sl_in);
     const int o = row_ptr[row];
-    for (int jj = 0; jj < k; jj++) val[o + jj] = vals[jj];
+    row_entries<kRowFromSlots, true, 3>(G, T, q, c, node, nullptr, nullptr, nullptr, sl_in,
+                                        [&](int j, int, double v) { val[o + j] = v; });
 }
 
 int make_terms(const Geo& G, const dare_terms* t, const double* phi, Terms* T) {
@@ -793,18 +793,19 @@ int dare_csr_fill_values(dare_ctx* ctx, dare_csr* A, const dare_grid* g, const d
     DARE_CHECK_ARG(T.cross == A->cross, "reaction terms differ from the ones the structure was built with");
     for (int f = 0; f < 6; f++)
         DARE_CHECK_ARG(T.bc_type[f] == A->bc_type[f], "boundary edits differ from the structure's");
+    // the terms of this operator beyond DDT, constant / per-component diffusion and
+    // Dirichlet / Neumann edits; the instantiation is the first whose mask covers them
+    int feat = (T.conv_limiter >= 0 ? kFeatConv : 0) | (T.diff_cell ? kFeatDiffCell : 0) |
+               (T.source ? kFeatSource : 0) | (T.cross ? kFeatCross : 0);
+    for (int f = 0; f < 6; f++)
+        if (T.bc_type[f] == DARE_BC_FIXED) feat |= kFeatFixed;
+    constexpr int kVar = kFeatDiffCell | kFeatSource;
     if (A->has_dia) {
         const dim3 grid(ceil_div(static_cast<long long>(G.n[2]) * G.N, 64), ceil_div(G.n[1], 4), G.n[0]);
         const int slots = A->cross ? 8 : 7;
         // the FP32 copy rides along once a mixed solve has used this matrix
         const bool f32 = A->dia32_mode && A->dia32 && A->cap_dia32 >= static_cast<int64_t>(slots) * nrows;
         const bool nt = A->nrows >= kStreamRows;
-        // the terms of this operator beyond DDT, constant / per-component diffusion and
-        // Dirichlet / Neumann edits; the instantiation is the first whose mask covers them
-        int feat = (T.conv_limiter >= 0 ? kFeatConv : 0) | (T.diff_cell ? kFeatDiffCell : 0) |
-                   (T.source ? kFeatSource : 0) | (T.cross ? kFeatCross : 0);
-        for (int f = 0; f < 6; f++)
-            if (T.bc_type[f] == DARE_BC_FIXED) feat |= kFeatFixed;
         // Symmetric by construction: a face coefficient is A_d * (dnr_d * D_f) in both rows it
         // couples (with the signs exchanged twice), and the per-cell harmonic mean takes its two
         // diffusivities in face order (low cell first) from either side. Not claimed for fixed
@@ -826,7 +827,6 @@ int dare_csr_fill_values(dare_ctx* ctx, dare_csr* A, const dare_grid* g, const d
                 hipLaunchKernelGGL((k_fill_dia<NTV, F32V, decltype(fc)::value, HV>), grid, dim3(256), 0, ctx->stream, G,
                                    T, A->dia, F32V ? A->dia32 : nullptr, slots, rhs, x0);
             };
-            constexpr int kVar = kFeatDiffCell | kFeatSource;
             if (feat == 0) run(std::integral_constant<int, 0>{});
             else if ((feat & ~kVar) == 0) run(std::integral_constant<int, kVar>{});
             else if constexpr (!HV) {       // a symmetric operator has none of the other terms
@@ -859,8 +859,17 @@ int dare_csr_fill_values(dare_ctx* ctx, dare_csr* A, const dare_grid* g, const d
         A->sym64 = -1;
         return DARE_OK;
     }
-    hipLaunchKernelGGL(k_fill_values, dim3(ceil_div(nrows, 256)), dim3(256), 0, ctx->stream, G, T, nrows,
-                       A->row_ptr, A->val, rhs, x0);
+    auto fill = [&](auto dc, auto fc) {
+        hipLaunchKernelGGL((k_fill_values<decltype(dc)::value, decltype(fc)::value>), dim3(ceil_div(nrows, 256)),
+                           dim3(256), 0, ctx->stream, G, T, nrows, A->row_ptr, A->val, rhs, x0);
+    };
+    using Two = std::integral_constant<int, 2>;
+    if (G.dim != 2) fill(std::integral_constant<int, 0>{}, std::integral_constant<int, kFeatAll>{});
+    else if (feat == 0) fill(Two{}, std::integral_constant<int, 0>{});
+    else if ((feat & ~kVar) == 0) fill(Two{}, std::integral_constant<int, kVar>{});
+    else if (feat == kFeatConv) fill(Two{}, std::integral_constant<int, kFeatConv>{});
+    else if (feat == kFeatCross) fill(Two{}, std::integral_constant<int, kFeatCross>{});
+    else fill(Two{}, std::integral_constant<int, kFeatAll>{});
     DARE_LAUNCH_CHECK();
     A->vals_stale = 0;
     return DARE_OK;
