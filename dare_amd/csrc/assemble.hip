@@ -816,11 +816,9 @@ int dare_csr_fill_values(dare_ctx* ctx, dare_csr* A, const dare_grid* g, const d
         bool sym = G.N == 1 && t->conv_limiter < 0 && t->react == nullptr;
         for (int f = 0; f < 6; f++) sym = sym && t->bc_type[f] != DARE_BC_FIXED;
         for (int d = 0; d < G.dim; d++) sym = sym && G.n[d] > 1 && !(t->diff_cell && G.per[d]);
-        // E, N, T are left out when the solvers will take the symmetric traversals (an even k
-        // extent for the FP64 pairs, a multiple of four for the FP32 quads) and no consumer of
-        // this matrix has needed the seven slots yet
-        const bool half = sym && !A->cross && A->sym_traversal && !A->ent_full && G.n[2] % 2 == 0 &&
-                          (!f32 || G.n[2] % 4 == 0);
+        // E, N, T are left out when the solvers will take the symmetric traversals and no consumer
+        // of this matrix has needed the seven slots yet
+        const bool half = sym && !A->cross && A->sym_traversal && !A->ent_full;
         auto launch = [&](auto ntc, auto f32c, auto halfc) {
             constexpr bool NTV = decltype(ntc)::value, F32V = decltype(f32c)::value, HV = decltype(halfc)::value;
             auto run = [&](auto fc) {

@@ -54,11 +54,13 @@ struct SolveOp {
                         hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4>), dim3(grid), dim3(kThreads), 0, sm, d, x,
                                            epi, ws, st, tail, check);
                 }
-            } else if (d.pair == 2 && d.sym) {   // FP64 operators only (op64)
-                if constexpr (std::is_same_v<VT, double>)
-                    hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 2, true>), dim3(grid), dim3(kThreads), 0, sm, d, x,
-                                       epi, ws, st, tail, check);
-            } else if (d.pair == 2)
+            } else if (d.pair == 2 && d.sym)
+                hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 2, true>), dim3(grid), dim3(kThreads), 0, sm, d, x, epi,
+                                   ws, st, tail, check);
+            else if (d.sym)
+                hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 1, true>), dim3(grid), dim3(kThreads), 0, sm, d, x, epi,
+                                   ws, st, tail, check);
+            else if (d.pair == 2)
                 hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 2>), dim3(grid), dim3(kThreads), 0, sm, d, x, epi, ws,
                                    st, tail, check);
             else
@@ -88,8 +90,9 @@ struct SolveOp {
                 else hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 4, false>), g, b, 0, sm, d, S, R);
             }
         } else if (d.pair == 2 && d.sym) {
-            if constexpr (std::is_same_v<VT, double>)
-                hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 2, true>), g, b, 0, sm, d, S, R);
+            hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 2, true>), g, b, 0, sm, d, S, R);
+        } else if (d.sym) {
+            hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 1, true>), g, b, 0, sm, d, S, R);
         } else if (d.pair == 2) {
             hipLaunchKernelGGL((k_step_dia<1, VT, XT, GCR, 2, false>), g, b, 0, sm, d, S, R);
         } else {
@@ -579,7 +582,13 @@ static int sym64_prepare(dare_ctx* ctx, dare_csr* A) {
     return DARE_OK;
 }
 
-// The FP64 operator of A: the diagonal view (its symmetric pair traversal when the view is
+// Whether to look for the symmetric traversal of `pair` cells a lane. The scalar one (odd k
+// extents) takes a view that is symmetric by construction, but does not pay the device's check.
+static bool sym_wanted(const dare_csr* A, int pair) {
+    return A->sym_traversal && (pair > 1 || A->sym_fill || A->sym64 == 1);
+}
+
+// The FP64 operator of A: the diagonal view (its symmetric traversals when the view is
 // exactly symmetric) or the CSR values.
 // vecs: the caller's vectors the traversal reads or writes. The paired, quad and two-component
 // traversals move 16-byte vectors, so those must start on 16-byte boundaries (any allocation
@@ -595,7 +604,7 @@ static int op64(dare_ctx* ctx, const dare_csr* A, bool allow_dia, SolveOp<double
         op.d = make_dia<double>(A->dia_view, A->dia, true);
         op.dia = kXcd * op.d.per_xcd <= kReduceBlocks;   // else the CSR traversal
     }
-    if (op.dia && op.d.pair == 2 && A->sym_traversal) {
+    if (op.dia && sym_wanted(A, op.d.pair)) {
         const int rc = sym64_prepare(ctx, const_cast<dare_csr*>(A));
         if (rc) return rc;
         op.d.sym = A->sym64 == 1;
@@ -974,9 +983,9 @@ int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* Ac, const double* b, 
         op32.d = make_dia<float>(A->dia_view, A->dia32, true);
         op32.d.unit_c = unit_c;
         op32.dia = kXcd * op32.d.per_xcd <= kReduceBlocks;
-        if (op32.dia && op32.d.pair == 4 && !pre && A->sym_traversal) {
+        if (op32.dia && !pre && sym_wanted(A, op32.d.pair)) {
             // the FP32 copy of an exactly symmetric FP64 view is exactly symmetric (Jacobi
-            // column scaling off): the quad traversal then reads E, N, T from the neighbours'
+            // column scaling off): the traversal then reads E, N, T from the neighbours'
             // W, S, B slots. The FP64 view's symmetry is known on the host (sym64_prepare).
             const int src = sym64_prepare(ctx, A);
             if (src) return src;

@@ -669,7 +669,10 @@ __global__ __launch_bounds__(kThreads) void k_apply_csr(CsrOp<VT> A, const XT* _
 // values of x rolled through registers. x and D belong to one system; row0 is that system's
 // first row in the epilogue's vectors (0 for a single system).
 // COPY: each slot value is also written to D32 in FP32 (every row is visited once per sweep).
-template <int NC, typename VT, bool COPY = false, class Src, class Epi>
+// SYM (one component): the view is exactly symmetric, and a row's E, N and T are read as the W, S
+// and B of its east, north and top neighbours, as in dia_column_pair_sym: four slots' bytes instead
+// of seven where an odd k extent keeps the pairs out (145 x 128 x 121, FP64: 28.7 -> 22.5 us).
+template <int NC, typename VT, bool COPY = false, bool SYM = false, class Src, class Epi>
 __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, const Src x,
                                   long long row0, int k, int j, int i0, int i1, const Epi& epi, double* acc,
                                   float* __restrict__ D32 = nullptr) {
@@ -688,6 +691,13 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
     const Ix dT = !hasT ? 0 : (k == n2 - 1) ? one - sJ : one;
     Ix node = (static_cast<Ix>(i0) * n1 + j) * n2 + k;
     double xp[NC], xc[NC];
+    static_assert(!SYM || (NC == 1 && !COPY), "symmetric views have one component");
+    const auto ldnt = [](const VT* p) {
+        if constexpr (Epi::kNT) return ld_nt(p);
+        else return *p;
+    };
+    VT wv = VT(0);             // SYM: W of this plane's row, the E of the plane before
+    if constexpr (SYM) wv = ldnt(at_off(D, node));
     {
         const bool need = !(i0 == 0 && V.rm_lo[0]);
         const Ix nprev = !need ? node : (i0 == 0) ? node + (n0 - 1) * sI : node - sI;
@@ -741,10 +751,18 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
                 xnn[c] = static_cast<double>(src1(x, (node + dN) * NC + c));
                 xb[c] = static_cast<double>(src1(x, (node + dB) * NC + c));
                 xt[c] = static_cast<double>(src1(x, (node + dT) * NC + c));
+                if constexpr (SYM) {      // S and B are read again as partners: no hint
+                    dv[c][0] = wv;
+                    dv[c][1] = *at_off(D + nr, row);
+                    dv[c][2] = *at_off(D + 2 * nr, row);
+                    dv[c][3] = ldnt(at_off(D + 3 * nr, row));
+                    dv[c][4] = *at_off(D + 2 * nr, row + dT);
+                    dv[c][5] = *at_off(D + nr, row + dN);
+                    dv[c][6] = wv = ldnt(at_off(D, nnext));
+                }
 #pragma unroll
-                for (int sl = 0; sl < 7; sl++) {
-                    if constexpr (Epi::kNT) dv[c][sl] = ld_nt(at_off(D + sl * nr, row));
-                    else dv[c][sl] = *at_off(D + sl * nr, row);
+                for (int sl = 0; sl < (SYM ? 0 : 7); sl++) {
+                    dv[c][sl] = ldnt(at_off(D + sl * nr, row));
                     if constexpr (COPY) D32[sl * nr + row] = static_cast<float>(dv[c][sl]);
                 }
                 dv[c][7] = VT(0);
@@ -1179,7 +1197,7 @@ __device__ inline void dia_tile(const DiaOp<VT>& A, const Src x, const Epi& epi,
     } else if constexpr (PAIR == 2) {
         dia_column_pair<VT>(A.V, A.D, x, k, j, i0, i1, epi, acc);
     } else {
-        dia_column<NC, VT>(A.V, A.D, x, 0, k, j, i0, i1, epi, acc);
+        dia_column<NC, VT, false, SYM>(A.V, A.D, x, 0, k, j, i0, i1, epi, acc);
     }
 }
 
