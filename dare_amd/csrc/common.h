@@ -129,9 +129,9 @@ struct dare_csr {
     // ent_lazy 1: the last fill left the E, N, T slots (4-6) of the view -- and of the FP32 copy
     // while dia32_fresh -- unwritten: the operator is symmetric by construction and the symmetric
     // traversals read those coefficients as the W, S, B slots of the east, north and top
-    // neighbours. dia_ensure_full writes them for any other consumer (seven-slot traversals,
-    // Jacobi scaling, multigrid, CSR values, batches) and sets ent_full, after which the fills
-    // of this matrix write every slot.
+    // neighbours (so do right Jacobi scaling and the multigrid). dia_ensure_full writes them for
+    // any other consumer (seven-slot traversals, left Jacobi scaling, CSR values, batches) and
+    // sets ent_full, after which the fills of this matrix write every slot.
     int ent_lazy = 0, ent_full = 0;
     // Jacobi right preconditioning: 1 / diag(A) and the column-scaled FP64 operator A diag(A)^-1
     // (diagonal-view slots, or CSR values for a matrix without a diagonal view)

@@ -116,8 +116,8 @@ __global__ __launch_bounds__(kThreads) void k_mg_weight(long long n, const VT* _
 // What bounds the fine level is the slots' and vectors' bytes; before, with a lane per cell, 28
 // (up) and 21 (down) loads a cell in runs of 16 k cells kept it above that. Here a run is up to 64
 // cells, the four cells share their neighbours, and the seven values of zc serve all four (18 and
-// 16 loads a cell). 145 x 128 x 121, FP64, four slots: down 28.8 -> 25.7 us, up 34.3 -> 27.5 (seven slots and 64-bit
-// rows: down 35, up 38).
+// 16 loads a cell). 145 x 128 x 121, FP64, four slots: down 28.8 -> 25.7 us, up 34.3 -> 27.5 (seven
+// slots and 64-bit rows: down 35, up 38).
 struct MgTiles {
     int lk;                    // log2 of the lanes along k
     unsigned tk, tj;           // tiles along k and along j

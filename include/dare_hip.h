@@ -232,11 +232,11 @@ int dare_axpby(dare_ctx* ctx, int64_t n, double a, const double* x, double b, do
 /* r = b - A x (the operator the solver uses) and, if norm_host != NULL, ||r|| (BiCGStab2.inl:265-266). */
 int dare_residual(dare_ctx* ctx, const dare_csr* csr, const double* b, const double* x, double* r, double* norm_host);
 /* *out = 1 when the FP64 solves, dare_residual, dare_spmv_dot (and dare_spmv without a
- * periodic axis) apply A through the symmetric traversal of its diagonal view (E, N, T of each
- * row read as W, S, B of its neighbours, with results bit-identical to the seven-slot one: the
- * view is exactly symmetric, by construction of the last fill or by the device's slot-by-slot
- * check), 0 otherwise (no diagonal view, two components, an odd k extent, convection, a failed
- * check). No counterpart in the reference; waits for the context stream. */
+ * periodic axis) apply A through the paired symmetric traversal of its diagonal view (E, N, T of
+ * each row read as W, S, B of its neighbours, with results bit-identical to the seven-slot one:
+ * the view is exactly symmetric, by construction of the last fill or by the device's slot-by-slot
+ * check), 0 otherwise (no diagonal view, two components, convection, a failed check, an odd k
+ * extent: a view that is symmetric by construction takes the one-row form there). No counterpart in the reference; waits for the context stream. */
 int dare_csr_symmetric(dare_ctx* ctx, const dare_csr* csr, int32_t* out);
 /* enable = 0: every FP64 and FP32 traversal of this matrix reads its seven slots (the results
  * are the same bits either way); 1 (the default): symmetric views take the four-slot
