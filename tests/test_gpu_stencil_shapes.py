@@ -55,3 +55,24 @@ def test_stencils_match_oracle(ctx, rng, n, ncomp, lim):
         f2 = pd.clone()
         da.copy_to_field(ctx, g, dev(x), f2)
         assert bits_equal(host(f2), orc.copy_to_field(go, x, filled))
+
+
+@pytest.mark.parametrize("n,ncomp", [([61, 67, 87], 3), ([64, 65, 127], 2), ([1025, 1027], 1), ([513, 700], 3),
+                                     ([1048577], 1), ([700001], 2), ([1, 1, 1], 1), ([2, 1, 1], 3), ([3, 2], 2)])
+def test_paired_gradient_and_divergence_match_oracle(ctx, rng, n, ncomp):
+    """A lane takes two neighbours of a line of cells and components: odd and even lines, the pair that
+    ends one cell and starts the next, and the last cell's far faces."""
+    import torch
+    go = orc.grid(n, size=[0.7 + 0.2 * d for d in range(len(n))], ghost=2, ncomp=ncomp)
+    g = da.Grid()
+    ctypes.memmove(ctypes.byref(g), ctypes.byref(go), ctypes.sizeof(g))
+    phi = rng.normal(size=orc.lib().orc_num_cells_padded(ctypes.byref(go)) * ncomp)
+    pd = torch.from_numpy(phi).cuda()
+    exp = orc.grad_faces(go, phi)
+    fd = [torch.full((e.size,), np.nan, dtype=torch.float64, device="cuda") for e in exp]
+    da.grad_faces(ctx, g, pd, fd)
+    for d in range(len(n)):
+        assert bits_equal(fd[d].cpu().numpy(), exp[d]), d
+    div = torch.zeros_like(pd)
+    da.div_faces(ctx, g, fd, div)
+    assert bits_equal(div.cpu().numpy(), orc.div_faces(go, exp))
