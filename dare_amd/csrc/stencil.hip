@@ -55,6 +55,15 @@ static Launch cell_launch(const Geo& G, int each = 1) {
     return L;
 }
 
+constexpr unsigned kGridYZ = 65535;      // work-groups along y and z that a launch takes
+// the same for line_pairs: two entries a lane, any number of rows and planes
+static Launch pair_launch(const Geo& G) {
+    Launch L = cell_launch(G, 2);
+    L.grid.y = L.grid.y < kGridYZ ? L.grid.y : kGridYZ;
+    L.grid.z = L.grid.z < kGridYZ ? L.grid.z : kGridYZ;
+    return L;
+}
+
 template <int DIM>
 __device__ inline bool cell_coord(const Geo& G, int q[3], int& c) {
     q[0] = q[1] = q[2] = 0;
@@ -196,84 +205,99 @@ struct LinePair {
     int e;             // first entry
     bool two, high0, high1;   // a second entry; entries in the line's last cell
 };
-template <int DIM>
-__device__ inline bool line_pair(const Geo& G, LinePair<DIM>& L) {
+// f(LinePair) for this lane's entries of every line it owns: one, but for grids of more than 65535
+// planes or work-groups of rows
+template <int DIM, class F>
+__device__ __forceinline__ void line_pairs(const Geo& G, F&& f) {
     const int len = G.n[DIM - 1] * G.N;
-    L.e = 2 * static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    L.q[0] = L.q[1] = L.q[2] = 0;
-    if (DIM >= 2) L.q[DIM - 2] = blockIdx.y * blockDim.y + threadIdx.y;
-    if (DIM == 3) L.q[0] = blockIdx.z;
+    const unsigned e = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
+    if (e >= static_cast<unsigned>(len)) return;
+    LinePair<DIM> L;
+    L.e = static_cast<int>(e);
     L.two = L.e + 1 < len;
     L.high0 = L.e >= len - G.N;
     L.high1 = L.two && L.e + 1 >= len - G.N;
-    return L.e < len && (DIM < 2 || L.q[DIM - 2] < G.n[DIM - 2]);
+    const int n0 = DIM == 3 ? G.n[0] : 1, n1 = DIM >= 2 ? G.n[DIM - 2] : 1;
+    for (int i = blockIdx.z; i < n0; i += gridDim.z)
+        for (int j = blockIdx.y * blockDim.y + threadIdx.y; j < n1; j += gridDim.y * blockDim.y) {
+            L.q[0] = L.q[1] = L.q[2] = 0;
+            if (DIM >= 2) L.q[DIM - 2] = j;
+            if (DIM == 3) L.q[0] = i;
+            f(L);
+        }
 }
 __device__ inline pair2 ld_pair(const double* p, bool two) {
     if (two) return *reinterpret_cast<const pair2*>(p);
     return pair2{p[0], 0.};
 }
+template <bool NT>
 __device__ inline void st_pair(double* p, pair2 v, bool two) {
-    if (two) *reinterpret_cast<pair2*>(p) = v;
-    else p[0] = v.x;
+    if (!two) p[0] = v.x;
+    else if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<pair2*>(p));
+    else *reinterpret_cast<pair2*>(p) = v;
 }
 
 // --------------------------------------------------------------------------- face gradient
-// Gradient_Cartesian.inl:62-96: W = (phiC - phiW) dn_r, E = (phiE - phiC) dn_r, ... Bytes bound it,
-// and 16-byte accesses move more per instruction than one entry a lane: 97 x 131 x 115 cells of
-// three components 37.9 -> 34.4 us (divergence 32.7 -> 29.5), 64^3 of three 7.5 -> 6.5 (5.5 ->
-// 4.4), 1024^2 6.6 -> 5.8 (5.2 -> 4.3), level at 10^5 entries.
-template <int DIM>
+// Gradient_Cartesian.inl:62-96: W = (phiC - phiW) dn_r, E = (phiE - phiC) dn_r, ... Bytes bound it.
+// 16-byte accesses move more per instruction than one entry a lane: 97 x 131 x 115 cells of three
+// components 37.9 -> 34.4 us (divergence 32.7 -> 29.5), 64^3 of three 7.5 -> 6.5 (5.5 -> 4.4),
+// 1024^2 6.6 -> 5.8 (5.2 -> 4.3), level at 10^5 entries. And entries in the order of memory keep
+// the pages of the four arrays few: a march along i in persistent work-groups, which re-reads
+// nothing, took 277 us for gradient and divergence of 256^3 on arrays in turn, this form 201 (128^3
+// 33.7 and 28.5; on one set of arrays over and over 270 and 200, 161^3 54 and 61). NT: stores past
+// the caches from kStreamRows entries on (256^3 without 230; 128^3 with 26.9 against 26.7).
+template <int DIM, bool NT>
 __global__ __launch_bounds__(256) void k_grad_faces(Geo G, FaceGeo F, const double* __restrict__ phi,
                                                     double* __restrict__ f0, double* __restrict__ f1,
                                                     double* __restrict__ f2) {
-    LinePair<DIM> L;
-    if (!line_pair(G, L)) return;
     double* out[3] = {f0, f1, f2};
     const int N = G.N;
-    const double* b = phi + pad_ord<DIM>(G, L.q) * N + L.e;
-    const pair2 pc = ld_pair(b, L.two);
-    pair2 lo[DIM];
+    line_pairs<DIM>(G, [&](const LinePair<DIM>& L) {
+        const double* b = phi + pad_ord<DIM>(G, L.q) * N + L.e;
+        const pair2 pc = ld_pair(b, L.two);
+        pair2 lo[DIM];
 #pragma unroll
-    for (int d = 0; d < DIM; d++) lo[d] = ld_pair(b - G.sl[d] * N, L.two);
+        for (int d = 0; d < DIM; d++) lo[d] = ld_pair(b - G.sl[d] * N, L.two);
 #pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        double* o = out[d] + face_ord<DIM>(F, d, L.q) * N + L.e;
-        st_pair(o, (pc - lo[d]) * G.dnr[d], L.two);
-        if (d < DIM - 1) {
-            if (L.q[d] == G.n[d] - 1)
-                st_pair(o + F.fs[d][d] * N, (ld_pair(b + G.sl[d] * N, L.two) - pc) * G.dnr[d], L.two);
-        } else {
-            if (L.high0) o[N] = (b[N] - pc.x) * G.dnr[d];
-            if (L.high1) o[N + 1] = (b[N + 1] - pc.y) * G.dnr[d];
+        for (int d = 0; d < DIM; d++) {
+            double* o = out[d] + face_ord<DIM>(F, d, L.q) * N + L.e;
+            st_pair<NT>(o, (pc - lo[d]) * G.dnr[d], L.two);
+            if (d < DIM - 1) {
+                if (L.q[d] == G.n[d] - 1)
+                    st_pair<NT>(o + F.fs[d][d] * N, (ld_pair(b + G.sl[d] * N, L.two) - pc) * G.dnr[d], L.two);
+            } else {
+                if (L.high0) o[N] = (b[N] - pc.x) * G.dnr[d];
+                if (L.high1) o[N + 1] = (b[N + 1] - pc.y) * G.dnr[d];
+            }
         }
-    }
+    });
 }
 
 // ---------------------------------------------------------------------- value divergence
 // Divergence_Cartesian.inl:211-235: A0 E - A0 W + A1 N - A1 S + A2 T - A2 B, in that order.
-template <int DIM>
+template <int DIM, bool NT>
 __global__ __launch_bounds__(256) void k_div_faces(Geo G, FaceGeo F, const double* __restrict__ f0,
                                                    const double* __restrict__ f1, const double* __restrict__ f2,
                                                    double* __restrict__ out) {
-    LinePair<DIM> L;
-    if (!line_pair(G, L)) return;
     const double* in[3] = {f0, f1, f2};
     const int N = G.N;
-    pair2 lo[DIM], hi[DIM];
+    line_pairs<DIM>(G, [&](const LinePair<DIM>& L) {
+        pair2 lo[DIM], hi[DIM];
 #pragma unroll
-    for (int d = 0; d < DIM; d++) {
-        const double* f = in[d] + face_ord<DIM>(F, d, L.q) * N + L.e;
-        lo[d] = ld_pair(f, L.two);
-        hi[d] = ld_pair(f + F.fs[d][d] * N, L.two);
-    }
-    pair2 v = G.A[0] * hi[0];
-    v -= G.A[0] * lo[0];
+        for (int d = 0; d < DIM; d++) {
+            const double* f = in[d] + face_ord<DIM>(F, d, L.q) * N + L.e;
+            lo[d] = ld_pair(f, L.two);
+            hi[d] = ld_pair(f + F.fs[d][d] * N, L.two);
+        }
+        pair2 v = G.A[0] * hi[0];
+        v -= G.A[0] * lo[0];
 #pragma unroll
-    for (int d = 1; d < DIM; d++) {
-        v += G.A[d] * hi[d];
-        v -= G.A[d] * lo[d];
-    }
-    st_pair(out + pad_ord<DIM>(G, L.q) * N + L.e, v, L.two);
+        for (int d = 1; d < DIM; d++) {
+            v += G.A[d] * hi[d];
+            v -= G.A[d] * lo[d];
+        }
+        st_pair<NT>(out + pad_ord<DIM>(G, L.q) * N + L.e, v, L.two);
+    });
 }
 
 // ------------------------------------------------------------ cell-centred velocity -> faces
@@ -373,29 +397,7 @@ __global__ __launch_bounds__(256) void k_tvd_step(Geo G, FaceGeo F, int lim, con
     phi_out[at] = p[0][2] - fac * v;
 }
 
-constexpr int kStepTileK = 64, kStepTileJ = 4, kStepXcd = 8, kStepMinPlanes = 8;
-
-// Walks logical block L's column-plane range [L*chunk, (L+1)*chunk) (columns of 64 PW (k) x 4
-// (j) cells ordered k-tile fastest, planes along i; lane l takes cells PW l .. PW l + PW - 1 of
-// its column) and calls march(k, j, i0, i1) for each column piece with k its first cell; blocks
-// are dealt XCD by XCD (blocks b = x mod 8 own a contiguous run).
-template <int PW = 1, class F>
-__device__ __forceinline__ void march_columns(const Geo& G, int tiles_k, long long total, long long chunk,
-                                              int per_xcd, F&& march) {
-    const long long L = static_cast<long long>(blockIdx.x % kStepXcd) * per_xcd + blockIdx.x / kStepXcd;
-    const int n0 = G.n[0];
-    long long c = L * chunk;
-    const long long cend = (c + chunk < total) ? c + chunk : total;
-    while (c < cend) {
-        const long long col = c / n0;
-        const int i0 = static_cast<int>(c - col * n0);
-        const int i1 = (cend - c < n0 - i0) ? i0 + static_cast<int>(cend - c) : n0;
-        const int k = (static_cast<int>(col % tiles_k) * kStepTileK + (threadIdx.x & 63)) * PW;   // PW cells per lane
-        const int j = static_cast<int>(col / tiles_k) * kStepTileJ + (threadIdx.x >> 6);
-        if (k < G.n[2] && j < G.n[1]) march(k, j, i0, i1);
-        c += i1 - i0;
-    }
-}
+constexpr int kStepTileK = 64, kStepXcd = 8, kStepMinPlanes = 8;
 
 // LDS-staged march of a 64 (k) x TJ (j) tile over the planes [i0, i1) (all 64 TJ threads active,
 // so the block can synchronise). The planes i-2..i+2 of phi at a cell stay in registers and the
@@ -525,8 +527,8 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
 }
 
 // 3-D, one component, persistent and balanced TVD step over 64 (k) x kStepTvdJ (j) tiles.
-// Logical block L takes the column-plane range [L*chunk, (L+1)*chunk) (the walk of
-// march_columns). The limiter is a template parameter so that each instantiation carries only its
+// Logical block L takes the column-plane range [L*chunk, (L+1)*chunk): columns ordered k-tile
+// fastest, planes along i; blocks are dealt XCD by XCD (blocks b = x mod 8 own a contiguous run). The limiter is a template parameter so that each instantiation carries only its
 // own branch.
 constexpr int kStepTvdJ = 8;
 template <bool NT, int LIM>
@@ -552,144 +554,6 @@ __global__ __launch_bounds__(64 * kStepTvdJ) void k_tvd_step3(Geo G, const doubl
         tvd_march3_lds<NT, kStepTvdJ>(G, LIM, phi, ux, uy, uz, fac, out, k0, j0, i0, i1, T, Fy, Fz);
         c += i1 - i0;
     }
-}
-
-// 3-D, one component: face gradient (same expressions as k_grad_faces) marching along i with
-// phi(i-1) in a register; face i of an axis is (phi(i) - phi(i-1)) dn_r, the high boundary face
-// (phi(n) - phi(n-1)) dn_r is written by the last cell.
-template <bool NT>
-__global__ __launch_bounds__(256) void k_grad3(Geo G, const double* __restrict__ phi, double* __restrict__ fx,
-                                               double* __restrict__ fy, double* __restrict__ fz, int tiles_k,
-                                               long long total, long long chunk, int per_xcd) {
-    march_columns(G, tiles_k, total, chunk, per_xcd, [&](int k, int j, int i0, int i1) {
-        const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
-        const long long sI = G.sl[0], sJ = G.sl[1];
-        const double d0 = G.dnr[0], d1 = G.dnr[1], d2 = G.dnr[2];
-        const bool lastj = j == n1 - 1, lastk = k == n2 - 1;
-        long long lp = (static_cast<long long>(i0 + G.g) * G.np[1] + (j + G.g)) * G.np[2] + (k + G.g);
-        const long long fxs = static_cast<long long>(n1) * n2;
-        long long ox = static_cast<long long>(i0) * fxs + static_cast<long long>(j) * n2 + k;
-        long long oy = (static_cast<long long>(i0) * (n1 + 1) + j) * n2 + k;
-        const long long fys = static_cast<long long>(n1 + 1) * n2;
-        long long oz = (static_cast<long long>(i0) * n1 + j) * (n2 + 1) + k;
-        const long long fzs = static_cast<long long>(n1) * (n2 + 1);
-        double pm = phi[lp - sI];
-        for (int i = i0; i < i1; i++) {
-            const double p0 = phi[lp], pS = phi[lp - sJ], pB = phi[lp - 1];
-            const double pN = phi[lastj ? lp + sJ : lp], pT = phi[lastk ? lp + 1 : lp];
-            put<NT>(fx + ox, (p0 - pm) * d0);
-            put<NT>(fy + oy, (p0 - pS) * d1);
-            if (lastj) put<NT>(fy + oy + n2, (pN - p0) * d1);
-            put<NT>(fz + oz, (p0 - pB) * d2);
-            if (lastk) put<NT>(fz + oz + 1, (pT - p0) * d2);
-            pm = p0;
-            lp += sI;
-            ox += fxs;
-            oy += fys;
-            oz += fzs;
-        }
-        if (i1 == n0) put<NT>(fx + ox, (phi[lp] - pm) * d0);   // lp is now the ghost plane n0
-    });
-}
-
-// k_grad3 with two k-adjacent cells per lane (n2 even, 16-byte aligned arrays): phi and the x,
-// y and z faces move as 16-byte vectors (z-face rows hold n2 + 1 faces, so a row starting on an
-// odd face pairs each lane's second face with the next lane's first). Each face is the same
-// difference times the same factor as in k_grad3, so the results are bit-identical.
-template <bool NT>
-__global__ __launch_bounds__(256) void k_grad3_pair(Geo G, const double* __restrict__ phi, double* __restrict__ fx,
-                                                    double* __restrict__ fy, double* __restrict__ fz, int tiles_k,
-                                                    long long total, long long chunk, int per_xcd) {
-    typedef double d2 __attribute__((ext_vector_type(2)));
-    auto ld2 = [](const double* p) { return *reinterpret_cast<const d2*>(p); };
-    auto st2 = [](double* p, d2 v) {
-        if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<d2*>(p));
-        else *reinterpret_cast<d2*>(p) = v;
-    };
-    march_columns<2>(G, tiles_k, total, chunk, per_xcd, [&](int k, int j, int i0, int i1) {
-        const int n0 = G.n[0], n1 = G.n[1], n2 = G.n[2];
-        const long long sI = G.sl[0], sJ = G.sl[1];
-        const double d0 = G.dnr[0], d1 = G.dnr[1], dz2 = G.dnr[2];
-        const bool lastj = j == n1 - 1, lastk = k == n2 - 2;     // cell k + 1 is the last one
-        long long lp = (static_cast<long long>(i0 + G.g) * G.np[1] + (j + G.g)) * G.np[2] + (k + G.g);
-        const long long fxs = static_cast<long long>(n1) * n2;
-        long long ox = static_cast<long long>(i0) * fxs + static_cast<long long>(j) * n2 + k;
-        long long oy = (static_cast<long long>(i0) * (n1 + 1) + j) * n2 + k;
-        const long long fys = static_cast<long long>(n1 + 1) * n2;
-        long long oz = (static_cast<long long>(i0) * n1 + j) * (n2 + 1) + k;
-        const long long fzs = static_cast<long long>(n1) * (n2 + 1);
-        d2 pm = ld2(phi + lp - sI);
-        for (int i = i0; i < i1; i++) {
-            const d2 p0 = ld2(phi + lp), pS = ld2(phi + lp - sJ);
-            const double pB = phi[lp - 1];
-            const d2 pN = ld2(phi + (lastj ? lp + sJ : lp));
-            const double pT = phi[lastk ? lp + 2 : lp + 1];
-            st2(fx + ox, (p0 - pm) * d0);
-            st2(fy + oy, (p0 - pS) * d1);
-            if (lastj) st2(fy + oy + n2, (pN - p0) * d1);
-            const double z0 = (p0.x - pB) * dz2, z1 = (p0.y - p0.x) * dz2;
-            if ((oz & 1) == 0) {              // wave-uniform: k is even in every lane
-                st2(fz + oz, d2{z0, z1});
-                if (lastk) put<NT>(fz + oz + 2, (pT - p0.y) * dz2);
-            } else {
-                // a row starting on an odd face: the aligned pairs are (k + 1, k + 2), face k + 2
-                // coming from the next lane (active whenever this one is not the row's last
-                // pair); lane 0 writes its face k alone, lane 63 its face k + 1 alone (the next
-                // tile's lane 0 writes k + 2)
-                const int lane = threadIdx.x & 63;
-                const double zn = __shfl_down(z0, 1);
-                if (lane == 0) put<NT>(fz + oz, z0);
-                if (lastk) st2(fz + oz + 1, d2{z1, (pT - p0.y) * dz2});
-                else if (lane < 63) st2(fz + oz + 1, d2{z1, zn});
-                else put<NT>(fz + oz + 1, z1);
-            }
-            pm = p0;
-            lp += sI;
-            ox += fxs;
-            oy += fys;
-            oz += fzs;
-        }
-        if (i1 == n0) st2(fx + ox, (ld2(phi + lp) - pm) * d0);   // lp is now the ghost plane n0
-    });
-}
-
-// 3-D, one component: value divergence A0 E - A0 W + A1 N - A1 S + A2 T - A2 B (the order of
-// k_div_faces) marching along i with the x face shared by consecutive planes in a register.
-template <bool NT>
-__global__ __launch_bounds__(256) void k_div3(Geo G, const double* __restrict__ fx, const double* __restrict__ fy,
-                                              const double* __restrict__ fz, double* __restrict__ out, int tiles_k,
-                                              long long total, long long chunk, int per_xcd) {
-    march_columns(G, tiles_k, total, chunk, per_xcd, [&](int k, int j, int i0, int i1) {
-        const int n1 = G.n[1], n2 = G.n[2];
-        const double A0 = G.A[0], A1 = G.A[1], A2 = G.A[2];
-        long long lp = (static_cast<long long>(i0 + G.g) * G.np[1] + (j + G.g)) * G.np[2] + (k + G.g);
-        const long long sI = G.sl[0];
-        const long long fxs = static_cast<long long>(n1) * n2;
-        long long ox = static_cast<long long>(i0) * fxs + static_cast<long long>(j) * n2 + k;
-        long long oy = (static_cast<long long>(i0) * (n1 + 1) + j) * n2 + k;
-        const long long fys = static_cast<long long>(n1 + 1) * n2;
-        long long oz = (static_cast<long long>(i0) * n1 + j) * (n2 + 1) + k;
-        const long long fzs = static_cast<long long>(n1) * (n2 + 1);
-        double xlo = fx[ox];
-        for (int i = i0; i < i1; i++) {
-            double xhi;
-            if constexpr (NT) xhi = ld_nt(fx + ox + fxs);
-            else xhi = fx[ox + fxs];
-            const double ylo = fy[oy], yhi = fy[oy + n2], zlo = fz[oz], zhi = fz[oz + 1];
-            double v = A0 * xhi;
-            v -= A0 * xlo;
-            v += A1 * yhi;
-            v -= A1 * ylo;
-            v += A2 * zhi;
-            v -= A2 * zlo;
-            put<NT>(out + lp, v);
-            xlo = xhi;
-            lp += sI;
-            ox += fxs;
-            oy += fys;
-            oz += fzs;
-        }
-    });
 }
 
 __global__ void k_fill(double* __restrict__ p, long long n, double v) {
@@ -745,11 +609,10 @@ __global__ __launch_bounds__(256) void k_copy_to_field(Geo G, const double* __re
     phi[pad_ord<DIM>(G, q) * G.N + c] = x[nd * G.N + c];
 }
 
-// Cells from which the 3-D one-component stencils march along i in persistent work-groups. Below,
-// a launch of one lane per cell is over before a march of eight planes (its shortest): TVD van
-// Leer 24^3 10.6 us marched, 4.6 not; 64^3 14.6 and 6.7; 96^3 22.8 and 17.5; level at 1.3 M cells;
-// 150 x 161 x 173 50 and 66. Gradient 64^3 6.9 and 4.7, divergence level below 1 M, 8.6 and 11.0 at
-// 1.3 M.
+// Cells from which the 3-D one-component TVD step marches along i in persistent work-groups. Below,
+// a launch of one lane per cell is over before a march of eight planes (its shortest): van Leer
+// 24^3 10.6 us marched, 4.6 not; 64^3 14.6 and 6.7; 96^3 22.8 and 17.5; level at 1.3 M cells;
+// 150 x 161 x 173 50 and 66.
 constexpr long long kMarchCells = 1LL << 20;
 
 // Balanced persistent schedule of the 3-D marching kernels: as many 256-thread blocks as stay
@@ -760,10 +623,9 @@ struct MarchPlan {
     unsigned grid;
 };
 
-inline MarchPlan march_plan(const dare_ctx* ctx, const Geo& G, int per_cu, int tile_j = kStepTileJ,
-                            int tile_k = kStepTileK) {
+inline MarchPlan march_plan(const dare_ctx* ctx, const Geo& G, int per_cu, int tile_j) {
     MarchPlan P;
-    P.tiles_k = static_cast<int>(ceil_div(G.n[2], tile_k));
+    P.tiles_k = static_cast<int>(ceil_div(G.n[2], kStepTileK));
     P.total = static_cast<long long>(P.tiles_k) * ceil_div(G.n[1], tile_j) * G.n[0];
     long long nb = static_cast<long long>(ctx->num_cu) * per_cu;
     const long long by_work = ceil_div(P.total, kStepMinPlanes);
@@ -791,31 +653,6 @@ void launch_step3(dare_ctx* ctx, const Geo& G, const double* phi, const double* 
 }
 
 template <bool NT>
-void launch_grad3(dare_ctx* ctx, const Geo& G, const double* phi, double* fx, double* fy, double* fz) {
-    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    if (G.n[2] % 2 == 0 && G.np[2] % 2 == 0 && G.g % 2 == 0 && aligned(phi) && aligned(fx) && aligned(fy) &&
-        aligned(fz)) {
-        static const int per_cu2 = resident_per_cu(k_grad3_pair<NT>);
-        const MarchPlan P = march_plan(ctx, G, per_cu2, kStepTileJ, 2 * kStepTileK);
-        hipLaunchKernelGGL((k_grad3_pair<NT>), dim3(P.grid), dim3(256), 0, ctx->stream, G, phi, fx, fy, fz, P.tiles_k,
-                           P.total, P.chunk, P.per_xcd);
-        return;
-    }
-    static const int per_cu = resident_per_cu(k_grad3<NT>);
-    const MarchPlan P = march_plan(ctx, G, per_cu);
-    hipLaunchKernelGGL((k_grad3<NT>), dim3(P.grid), dim3(256), 0, ctx->stream, G, phi, fx, fy, fz, P.tiles_k, P.total,
-                       P.chunk, P.per_xcd);
-}
-
-template <bool NT>
-void launch_div3(dare_ctx* ctx, const Geo& G, const double* fx, const double* fy, const double* fz, double* out) {
-    static const int per_cu = resident_per_cu(k_div3<NT>);
-    const MarchPlan P = march_plan(ctx, G, per_cu);
-    hipLaunchKernelGGL((k_div3<NT>), dim3(P.grid), dim3(256), 0, ctx->stream, G, fx, fy, fz, out, P.tiles_k, P.total,
-                       P.chunk, P.per_xcd);
-}
-
-template <bool NT>
 void launch_step3_lim(dare_ctx* ctx, const Geo& G, int lim, const double* phi, const double* ux,
                       const double* uy, const double* uz, double fac, double* out) {
     switch (lim) {
@@ -833,6 +670,15 @@ void launch_step3_lim(dare_ctx* ctx, const Geo& G, int lim, const double* phi, c
         case 1: hipLaunchKernelGGL(KERNEL<1>, (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
         case 2: hipLaunchKernelGGL(KERNEL<2>, (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
         default: hipLaunchKernelGGL(KERNEL<3>, (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
+        }                                                                                        \
+    } while (0)
+
+#define DARE_DISPATCH_DIM_NT(G, KERNEL, NT, L, ...)                                                \
+    do {                                                                                         \
+        switch ((G).dim) {                                                                       \
+        case 1: hipLaunchKernelGGL((KERNEL<1, NT>), (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
+        case 2: hipLaunchKernelGGL((KERNEL<2, NT>), (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
+        default: hipLaunchKernelGGL((KERNEL<3, NT>), (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
         }                                                                                        \
     } while (0)
 
@@ -932,15 +778,10 @@ int dare_grad_faces(dare_ctx* ctx, const dare_grid* g, const double* phi, double
     DARE_CHECK_ARG(G.g >= 1, "face gradient needs >= 1 ghost layer");
     DARE_CHECK_ARG(G.dim < 2 || fy, "fy is NULL");
     DARE_CHECK_ARG(G.dim < 3 || fz, "fz is NULL");
-    if (G.dim == 3 && G.N == 1 && G.ncell_int >= kMarchCells) {
-        if (G.ncell_int >= kStreamRows) launch_grad3<true>(ctx, G, phi, fx, fy, fz);
-        else launch_grad3<false>(ctx, G, phi, fx, fy, fz);
-        DARE_LAUNCH_CHECK();
-        return DARE_OK;
-    }
     const FaceGeo F = make_face_geo(G);
-    const Launch L = cell_launch(G, 2);
-    DARE_DISPATCH_DIM(G, k_grad_faces, L, G, F, phi, fx, fy, fz);
+    const Launch L = pair_launch(G);
+    if (G.ncell_int * G.N >= kStreamRows) DARE_DISPATCH_DIM_NT(G, k_grad_faces, true, L, G, F, phi, fx, fy, fz);
+    else DARE_DISPATCH_DIM_NT(G, k_grad_faces, false, L, G, F, phi, fx, fy, fz);
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }
@@ -971,15 +812,10 @@ int dare_div_faces(dare_ctx* ctx, const dare_grid* g, const double* fx, const do
     if (rc) return rc;
     DARE_CHECK_ARG(G.dim < 2 || fy, "fy is NULL");
     DARE_CHECK_ARG(G.dim < 3 || fz, "fz is NULL");
-    if (G.dim == 3 && G.N == 1 && G.ncell_int >= kMarchCells) {
-        if (G.ncell_int >= kStreamRows) launch_div3<true>(ctx, G, fx, fy, fz, out);
-        else launch_div3<false>(ctx, G, fx, fy, fz, out);
-        DARE_LAUNCH_CHECK();
-        return DARE_OK;
-    }
     const FaceGeo F = make_face_geo(G);
-    const Launch L = cell_launch(G, 2);
-    DARE_DISPATCH_DIM(G, k_div_faces, L, G, F, fx, fy, fz, out);
+    const Launch L = pair_launch(G);
+    if (G.ncell_int * G.N >= kStreamRows) DARE_DISPATCH_DIM_NT(G, k_div_faces, true, L, G, F, fx, fy, fz, out);
+    else DARE_DISPATCH_DIM_NT(G, k_div_faces, false, L, G, F, fx, fy, fz, out);
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }
@@ -1016,7 +852,9 @@ int dare_tvd_explicit_step(dare_ctx* ctx, const dare_grid* g, int32_t limiter, c
     const FaceGeo F = make_face_geo(G);
     const Launch L = cell_launch(G);
     const double fac = dt / G.V;
-    if (G.dim == 3 && G.N == 1 && G.ncell_int >= kMarchCells) {
+    // (the march takes any number of rows and planes)
+    const bool march = G.ncell_int >= kMarchCells || L.grid.y > kGridYZ || L.grid.z > kGridYZ;
+    if (G.dim == 3 && G.N == 1 && march) {
         if (G.ncell_int >= kStreamRows) launch_step3_lim<true>(ctx, G, limiter, phi, ux, uy, uz, fac, phi_out);
         else launch_step3_lim<false>(ctx, G, limiter, phi, ux, uy, uz, fac, phi_out);
         DARE_LAUNCH_CHECK();

@@ -58,7 +58,8 @@ def test_stencils_match_oracle(ctx, rng, n, ncomp, lim):
 
 
 @pytest.mark.parametrize("n,ncomp", [([61, 67, 87], 3), ([64, 65, 127], 2), ([1025, 1027], 1), ([513, 700], 3),
-                                     ([1048577], 1), ([700001], 2), ([1, 1, 1], 1), ([2, 1, 1], 3), ([3, 2], 2)])
+                                     ([1048577], 1), ([700001], 2), ([1, 1, 1], 1), ([2, 1, 1], 3), ([3, 2], 2),
+                                     ([161, 162, 163], 1), ([66000, 4, 5], 1), ([3, 263000, 2], 1)])
 def test_paired_gradient_and_divergence_match_oracle(ctx, rng, n, ncomp):
     """A lane takes two neighbours of a line of cells and components: odd and even lines, the pair that
     ends one cell and starts the next, and the last cell's far faces."""
@@ -76,3 +77,18 @@ def test_paired_gradient_and_divergence_match_oracle(ctx, rng, n, ncomp):
     div = torch.zeros_like(pd)
     da.div_faces(ctx, g, fd, div)
     assert bits_equal(div.cpu().numpy(), orc.div_faces(go, exp))
+
+
+def test_tvd_step_of_more_planes_than_a_launch_takes(ctx, rng):
+    """Fewer cells than the march starts at, but more planes than a grid's third extent."""
+    import torch
+    n = [66000, 3, 5]
+    go = orc.grid(n, size=[66.0, 0.3, 0.5], ghost=2)
+    g = da.Grid()
+    ctypes.memmove(ctypes.byref(g), ctypes.byref(go), ctypes.sizeof(g))
+    phi = rng.normal(size=orc.lib().orc_num_cells_padded(ctypes.byref(go)))
+    vel = [rng.uniform(-1, 1, size=orc.lib().orc_num_faces(ctypes.byref(go), d)) for d in range(3)]
+    pd, vd = torch.from_numpy(phi).cuda(), [torch.from_numpy(v).cuda() for v in vel]
+    out = pd.clone()
+    da.tvd_explicit_step(ctx, g, da.VANLEER, pd, vd, 1e-3, out)
+    assert bits_equal(out.cpu().numpy(), orc.tvd_explicit_step(go, da.VANLEER, phi, vel, 1e-3))
