@@ -247,8 +247,8 @@ def main():
     stencils = {}
     csr_bytes = 12 * nnz + 4 * (nrows + 1) + 16 * nrows
     for name, kern, sec, nbytes in (("tvd_step", "k_tvd_step3", tvd_s, tvd_bytes),
-                                    ("gradient", "k_grad3_pair", grad_s, 8 * (ncell + nface)),
-                                    ("divergence", "k_div3", div_s, 8 * (nface + ncell)),
+                                    ("gradient", "k_grad_faces", grad_s, 8 * (ncell + nface)),
+                                    ("divergence", "k_div_faces", div_s, 8 * (nface + ncell)),
                                     ("csr_spmv", "k_apply_csr<double,double,EpiStore>", csr_s, csr_bytes)):
         gbs = nbytes / sec / 1e9
         stencils[name] = {"kernel": kern, "bytes_per_cell": round(nbytes / ncell, 3), "achieved": round(gbs, 1),
