@@ -499,17 +499,6 @@ struct dare_batch {
 
 namespace {
 
-// lanes along k for tile_k = 0: the split (64, 32 or 16) with the fewest idle lanes
-int tk_auto(int ny, int nz) {
-    int best = 6;
-    const auto tiles = [&](int lk) {
-        return static_cast<long long>((nz + (1 << lk) - 1) >> lk) * ((ny + (kThreads >> lk) - 1) / (kThreads >> lk));
-    };
-    for (int lk = 5; lk >= 4; lk--)
-        if (tiles(lk) < tiles(best)) best = lk;
-    return best;
-}
-
 void drop_graphs(dare_batch* B) {
     if (B->g64) hipGraphExecDestroy(B->g64);
     if (B->g32) hipGraphExecDestroy(B->g32);
@@ -548,7 +537,7 @@ int apply_config(dare_ctx* ctx, dare_batch* B, const dare_batch_config& cfg) {
         S.dia = B->sys[s]->dia;
         S.dia32 = B->dia32 ? B->dia32 + 8 * B->row0[s] : nullptr;
         S.row0 = B->row0[s];
-        S.tk_log2 = cfg.tile_k ? (cfg.tile_k == 16 ? 4 : cfg.tile_k == 32 ? 5 : 6) : tk_auto(V.n[1], V.n[2]);
+        S.tk_log2 = cfg.tile_k ? (cfg.tile_k == 16 ? 4 : cfg.tile_k == 32 ? 5 : 6) : lane_split(V, 1).lk_log2;
         S.tile_i = std::min(cfg.tile_i, V.n[0]);
         S.tiles_k = (V.n[2] + (1 << S.tk_log2) - 1) >> S.tk_log2;
         const int tj = kThreads >> S.tk_log2;

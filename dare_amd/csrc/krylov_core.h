@@ -258,16 +258,47 @@ struct DiaOp {
     bool unit_c = false;         // every C coefficient is 1 and not stored (FP32 quads, column-scaled view)
 };
 
-// Tile of a work-group: 2^lk lanes along k (pair cells each) x 256 / 2^lk rows along j, marched
-// over tile_i planes. The lane split with the fewest idle lanes is taken (the widest on a tie):
-// at n2 = 64 the paired traversal fills 32 lanes, and 64 x 4 tiles left half of every wave idle.
-// tile_i starts at 16, which reads x about once, and is halved while the launch has too few
-// work-groups. A march is a chain of dependent loads, so small systems need them spread out:
-// 512 below a million rows (64^3: 15.2 us per sweep as 64 work-groups of 16 planes, 4.9 as 256,
-// 4.5 as 512). Above, a sweep is bound by the bytes in flight: one cell per lane needs four
-// work-groups per CU (145 x 128 x 121: 32.8 us as 640, 29.3 as 1216), two or four cells per lane
-// one (128^3: 24.4 us as 256, 25.8 as 1024, whose shorter marches read more of x twice).
+// Lanes along k of a tile (2^lk, the other kThreads / 2^lk along j) for nk lanes' worth of k
+// extent. Small systems take the split with the fewest idle lanes (the widest on a tie): at n2 = 64
+// the paired traversal fills 32 lanes, and 64 x 4 tiles left half of every wave idle. Large ones
+// are bound by memory, not by lanes, and a row of a narrow tile is a short piece of every array, so
+// a narrower split must save a fifth of the tiles, and 16 lanes are for k extents of 16 only (seven
+// slots, FP64, us a sweep with 64, 32 and 16 lanes: pairs, 2 M rows, n2 = 66: 34, 40, 38; n2 =
+// 150, a quarter fewer tiles of 32: 33, 30, 33; one row, 6 M rows, n2 = 161: 110, 117, 164). The
+// line lies at 1.6 M rows, of one row a lane at 2.6 M (0.9 M rows, n2 = 97, two tiles against 1.75:
+// a four-pass solve 0.83 and 0.74 ms; 2 M, n2 = 33: 1.24 and 1.10).
+struct LaneSplit {
+    int lk_log2, tiles_k, tiles_j;
+    long long tiles() const { return static_cast<long long>(tiles_k) * tiles_j; }
+};
+inline LaneSplit lane_split(int nk, int nj, bool large) {
+    const auto split = [&](int lk) {
+        return LaneSplit{lk, (nk + (1 << lk) - 1) >> lk, (nj + (kThreads >> lk) - 1) / (kThreads >> lk)};
+    };
+    LaneSplit best = split(6);
+    for (int lk = 5; lk >= 4; lk--) {
+        const LaneSplit L = split(lk);
+        const bool fewer = lk == 5 && large ? 5 * L.tiles() <= 4 * best.tiles() : L.tiles() < best.tiles();
+        if (fewer && (lk == 5 || !large || nk <= 16)) best = L;
+    }
+    return best;
+}
+inline LaneSplit lane_split(const DiaView& V, int pair) {
+    return lane_split((V.n[2] + pair - 1) / pair, V.n[1], V.nrows >= (pair == 1 ? 5LL << 19 : 3LL << 19));
+}
+
+// Tile of a work-group: lane_split's lanes, pair cells each, marched over tile_i planes. 16 planes
+// read x about once; shorter marches make more work-groups of the launch. A march is a chain of
+// dependent loads, so small systems need them spread out: 512 work-groups below a million rows
+// (64^3: 15.2 us per sweep as 64 of 16 planes, 4.9 as 256, 4.5 as 512), of one row a lane 1024 up
+// to 2.6 M (206 x 207 x 33: 18.4 us as 507, 15.4 as 1014). Above, a work-group for each of the
+// kFullGrid CUs, and of the marches of 16, 8, 4 and 2 planes that give that, the one with the fewest
+// planes on the busiest CU, a march counting 0.7 of a plane for its start (seven slots, FP64: 128^3,
+// 256 work-groups of 16 planes 27.7 us, 512 of 8 28.8; 112^3, 196 of 16 17.5, 392 of 8 16.3; 134 x
+// 135 x 66, 306 of 16 21.9, 1156 of 4 19.8; four slots, one row a lane: 145 x 128 x 121, 640 of 16
+// 32.8, 1216 of 8 29.3).
 // tile_i grows past 16 only where the reduction slots would not hold the grid.
+constexpr int kFullGrid = 256;
 template <typename VT>
 DiaOp<VT> make_dia(const DiaView& V, const VT* D, bool allow_pair = false) {
     DiaOp<VT> A;
@@ -275,21 +306,21 @@ DiaOp<VT> make_dia(const DiaView& V, const VT* D, bool allow_pair = false) {
     A.D = D;
     A.pair = (allow_pair && V.N == 1 && V.n[2] % 2 == 0) ? 2 : 1;
     if (allow_pair && std::is_same_v<VT, float> && V.N == 1 && V.n[2] % 4 == 0) A.pair = 4;
-    long long best = 0;
-    for (int lk = 6; lk >= 4; lk--) {
-        const int lanes = 1 << lk, rows = kThreads >> lk;
-        const long long tk = (V.n[2] + lanes * A.pair - 1) / (lanes * A.pair), tj = (V.n[1] + rows - 1) / rows;
-        if (best == 0 || tk * tj < best) {
-            best = tk * tj;
-            A.lk_log2 = lk;
-            A.tiles_k = static_cast<int>(tk);
-            A.tiles_j = static_cast<int>(tj);
-        }
-    }
-    auto tiles = [&](int ti) { return best * ((V.n[0] + ti - 1) / ti); };
+    const LaneSplit L = lane_split(V, A.pair);
+    A.lk_log2 = L.lk_log2;
+    A.tiles_k = L.tiles_k;
+    A.tiles_j = L.tiles_j;
+    auto tiles = [&](int ti) { return L.tiles() * ((V.n[0] + ti - 1) / ti); };
     A.tile_i = kTileI;
-    const int want = V.nrows < (1LL << 20) ? 512 : A.pair == 1 ? 1024 : 256;
-    while (A.tile_i > 1 && tiles(A.tile_i) < want) A.tile_i /= 2;
+    if (V.nrows < (A.pair == 1 ? 5LL << 19 : 1LL << 20)) {
+        const int want = kFullGrid * (V.nrows < (1LL << 20) ? 2 : 4);
+        while (A.tile_i > 1 && tiles(A.tile_i) < want) A.tile_i /= 2;
+    } else {
+        const auto cost = [&](int ti) { return (tiles(ti) + kFullGrid - 1) / kFullGrid * (10 * ti + 7); };
+        while (A.tile_i > 2 && tiles(A.tile_i) < kFullGrid) A.tile_i /= 2;
+        for (int ti = A.tile_i / 2; ti >= 2; ti /= 2)
+            if (cost(ti) < cost(A.tile_i)) A.tile_i = ti;
+    }
     while (kXcd * ((tiles(A.tile_i) + kXcd - 1) / kXcd) > kReduceBlocks && A.tile_i < V.n[0]) A.tile_i *= 2;
     A.tiles_i = (V.n[0] + A.tile_i - 1) / A.tile_i;
     A.per_xcd = static_cast<int>((tiles(A.tile_i) + kXcd - 1) / kXcd);

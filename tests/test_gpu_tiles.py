@@ -81,6 +81,15 @@ def test_sweep_and_solves_on_tile_edges(ctx, rng, shape, op):
     A.close()
 
 
+@pytest.mark.parametrize("shape,op", [((20, 163, 161), "conv"), ((41, 160, 161), "diff"), ((100, 101, 104), "conv"),
+                                      ((112, 98, 96), "diff"), ((134, 135, 66), "conv"), ((71, 150, 150), "diff"),
+                                      ((103, 200, 128), "react"), ((60, 2000, 22), "diff")])
+def test_sweep_and_solves_on_both_sides_of_the_tile_rules_lines(ctx, rng, shape, op):
+    """Half a million to 2.7 M rows: narrow tiles below the line and wide ones above it, marches of 2 to
+    16 planes chosen by how evenly they fall on the CUs, with the last tile and the last march cut."""
+    test_sweep_and_solves_on_tile_edges(ctx, rng, shape, op)
+
+
 @pytest.mark.parametrize("n", [1, 257])
 def test_breakdown_after_the_first_x_update_keeps_it(ctx, n):
     """A multiple of the identity breaks the method down in its first pass after step 10 (r = 0,
