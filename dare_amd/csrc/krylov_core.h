@@ -486,14 +486,18 @@ __device__ __forceinline__ void epi_quad(const Epi& e, long long i, const double
     for (int m = 0; m < 4; m++) e(i + m, y[m], xc[m], pre[m], acc);
 }
 // ------------------------------------------------------------------------------ operands
-// Element offsets within one system's slot or vector. Where a sweep does not stream from memory
-// they are 32 bits, also in bytes (so up to kWideRows rows): a load then takes a scalar base and
-// one register of offset instead of a 64-bit address per access, which gives the fused steps a
-// wave more per SIMD (128^3, seven slots: 37.9 -> 31.1 us). The streaming sweeps, every single
-// solver's from kStreamRows rows on, keep 64 bits: with eight waves per SIMD instead of six the
-// symmetric pairs evict the partner slots they are about to read again (256^3: 179 -> 192 us). So
-// does the five-dot sweep of step 18, which reads two vectors more (128^3: 33.5 us, with 32 bits
-// 40.2), and a batch with a system of more rows than kWideRows (Wide).
+// Element offsets within one system's slot or vector, 32 or 64 bits. 32 (also in bytes, so up to
+// kWideRows rows): a load takes a scalar base and one register of offset instead of a 64-bit
+// address per access, which leaves room for another wave per SIMD. The traversal of one row a lane
+// takes them wherever it does not stream (odd extents, 0.7-1.3 M rows, FP64, five-slot start to end
+// 2-3 % faster), and so do the fused steps, whose operand reads two vectors (128^3, seven slots:
+// 37.9 -> 31.1 us; pairs in FP32 115 x 116 x 150: a four-pass solve 1.3 of 1.6 ms). The other
+// sweeps of pairs and quads keep 64 bits: their waves already fill the memory's queues, and one more
+// per SIMD evicts the lines that the next plane or the partner row is about to read again (FP64
+// pairs, 115 x 116 x 150: four slots 28.4 us with 32 bits, 19.2 with 64, seven 32.8 and 26.7; 256^3
+// 192 and 179; level at 128^3). So do the five-dot sweep of step 18, which reads two vectors more
+// (128^3: 33.5 us, with 32 bits 40.2), everything from kStreamRows rows on, and a batch with a
+// system of more rows than kWideRows (Wide).
 constexpr long long kWideRows = 1LL << 29;
 template <class Epi>
 struct Wide : Epi {};
@@ -507,6 +511,17 @@ struct SweepIndexOf<Wide<Epi>> {
 };
 template <class Epi>
 using SweepIndex = typename SweepIndexOf<Epi>::type;
+// of the pairs and quads: 32 bits in the epilogues of the fused steps (kStep) alone
+template <class Epi, class = void>
+struct PairIndexOf {
+    using type = long long;
+};
+template <class Epi>
+struct PairIndexOf<Epi, std::enable_if_t<Epi::kStep>> {
+    using type = SweepIndex<Epi>;
+};
+template <class Epi>
+using PairIndex = typename PairIndexOf<Epi>::type;
 template <typename T>
 __device__ __forceinline__ const T* at_off(const T* base, unsigned e) {
     return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + e * static_cast<unsigned>(sizeof(T)));
@@ -837,7 +852,7 @@ __device__ inline void dia_column(const DiaView& V, const VT* __restrict__ D, co
 template <typename VT, class Src, class Epi>
 __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ D, const Src x,
                                        int k, int j, int i0, int i1, const Epi& epi, double* acc) {
-    using Ix = SweepIndex<Epi>;
+    using Ix = PairIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
@@ -915,7 +930,7 @@ __device__ inline void dia_column_pair(const DiaView& V, const VT* __restrict__ 
 template <typename VT, class Src, class Epi>
 __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restrict__ D, const Src x,
                                            int k, int j, int i0, int i1, const Epi& epi, double* acc) {
-    using Ix = SweepIndex<Epi>;
+    using Ix = PairIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
@@ -1000,7 +1015,7 @@ __device__ inline void dia_column_pair_sym(const DiaView& V, const VT* __restric
 template <bool UNIT, class Src, class Epi>
 __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict__ D, const Src x,
                                        int k, int j, int i0, int i1, const Epi& epi, double* acc) {
-    using Ix = SweepIndex<Epi>;
+    using Ix = PairIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
@@ -1073,7 +1088,7 @@ __device__ inline void dia_column_quad(const DiaView& V, const float* __restrict
 template <class Src, class Epi>
 __device__ inline void dia_column_quad_sym(const DiaView& V, const float* __restrict__ D, const Src x,
                                            int k, int j, int i0, int i1, const Epi& epi, double* acc) {
-    using Ix = SweepIndex<Epi>;
+    using Ix = PairIndex<Epi>;
     const int n0 = V.n[0], n1 = V.n[1], n2 = V.n[2];
     const Ix sI = static_cast<Ix>(n1) * n2, sJ = n2, one = 1;
     const long long nr = V.nrows;
@@ -1325,6 +1340,7 @@ __device__ inline bool step_state(const StepRed& R, KState* st) {
 
 template <typename XT>
 struct EpiStepDot {      // the operand and out = A p; <out, w>
+    static constexpr bool kStep = true;
     static constexpr int NDOT = 1;
     static constexpr bool kNT = false;
     XT* xo;
