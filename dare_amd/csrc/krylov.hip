@@ -1,11 +1,11 @@
 // Krylov kernels and the BiCGStab(2) driver for gfx950.
 //
 // BiCGStab2::Solve (MatrixSystem/BiCGStab2.inl:167-582) is restated as nine launches per pass and
-// a one-work-group finish kernel after each of its five reductions; below 4 M rows as five
-// launches and one finish (k_step_*, k_step_end). All method scalars (alpha, beta, gamma, rho,
-// omega, mu, nu, tau) live in device memory and are updated there, so the host reads back only
-// one small status block per pass (the convergence test). Reductions are
-// deterministic: fixed grid, fixed per-thread order, block partials summed in block order.
+// a one-work-group finish kernel after each of its five reductions; without multigrid and up to 1
+// to 4 M rows (SolveOp::fused) as five launches and one finish (k_step_*, k_step_end). All method
+// scalars (alpha, beta, gamma, rho, omega, mu, nu, tau) live in device memory and are updated
+// there, so the host reads back only one small status block per pass (the convergence test).
+// Reductions are deterministic: fixed grid, fixed per-thread order, block partials summed in block order.
 //
 // Operators: a generic CSR traversal (grid-stride, one row per lane) and, for matrices
 // assembled from the 7-point structure, a tiled traversal of the slot-major diagonal view:
@@ -76,10 +76,37 @@ struct SolveOp {
 
     unsigned grid() const { return dia ? static_cast<unsigned>(kXcd * d.per_xcd) : grid_rows(n); }
 
+    unsigned step_grid() const { return dia || grid() < kStepCsrGrid ? grid() : kStepCsrGrid; }
+
+    // Whether a pass without multigrid runs as fused steps: up to the row count at which the two
+    // forms are level, which depends on the traversal. Four passes, time of the fused form over that
+    // of the separate kernels, mean over k extents of 24 to 258 (CSR: 2-D grids and a 3-D one), at
+    // 0.8, 1.2, 2.0, 3.0 and 4.0 M rows:
+    //   pairs, FP64, four slots     0.89 1.03 1.07 1.19 1.32     seven    0.84 0.92 0.95 1.11 1.08
+    //   pairs, FP32, four slots     0.93 0.98 1.04 1.11 1.12     seven    0.92 1.05 1.11 1.18 1.16
+    //   quads, four slots           0.96 0.94 1.03 1.09 1.11     seven    0.96 0.89 0.97 1.01 1.02
+    //   one row, FP64, four slots   0.85 0.89 0.95 1.03 1.08     seven    0.87 0.93 0.98 1.11 1.08
+    //   one row, FP32, four slots   0.90 0.87 0.96 0.96 0.97     seven    0.86 0.88 0.96 0.96 0.97
+    //   two components, FP64        0.82 0.90 0.93 1.03 1.03     FP32     0.90 0.89 0.96 0.99 1.01
+    //   CSR, FP64                   0.89 0.90 0.93 0.99 1.02     FP32     0.86 0.87 0.87 0.89 0.93-1.03
+    // (Four slots read the two operands for fewer bytes of matrix, so the gain ends earlier; at
+    // 128^3 itself quads gain 6 %.) Nor where most lanes of many tiles are idle: 30000 x 4 x 4 cells
+    // took 4.2 ms fused and 2.3 not, 70000 x 4 x 4 9.0 and 4.3.
+    bool fused() const {
+        constexpr bool f64 = std::is_same_v<VT, double>;
+        if (!dia) return n <= (f64 ? kFusedRows / 2 : kFusedRows * 11 / 16);
+        if (grid() > 1024 && n < 384LL * grid()) return false;
+        if (d.V.N == 2) return n <= kFusedRows * 11 / 16;
+        if (d.pair == 1) return n <= (!f64 ? kFusedRows : d.sym ? kFusedRows * 11 / 16 : kFusedRows / 2);
+        if (d.pair == 4) return n <= kFusedRows / 2;
+        if (f64) return n <= (d.sym ? kFusedRows / 4 : kFusedRows / 2);
+        return n <= (d.sym ? kFusedRows * 3 / 8 : kFusedRows / 4);
+    }
+
     // one fused step (k_step_dia / k_step_csr), the traversals as in launch
     template <bool GCR, typename XT>
     void step(hipStream_t sm, const StepVecs<XT>& S, const StepRed& R) const {
-        const dim3 g(grid()), b(kThreads);
+        const dim3 g(step_grid()), b(kThreads);
         if (!dia) {
             hipLaunchKernelGGL((k_step_csr<VT, XT, GCR>), g, b, 0, sm, csr, S, R);
         } else if (d.V.N == 2) {
@@ -201,7 +228,7 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, St
     XT* w = s + n;
     XT* t = w + n;
     XT *rr = w, *uu = t, *vv = t + n;
-    const bool fused = !NT && !mg && n < kFusedRows;
+    const bool fused = !NT && !mg && A.fused();
     const unsigned gr = grid_for(n);
     hipStream_t sm = ctx->stream;
     *out = Outcome{};
@@ -249,7 +276,7 @@ int bicgstab2_run_nt(dare_ctx* ctx, const SolveOp<VT>& A, const XT* b, XT* x, St
         pub = publish(ctx);
         if (fused) {
             double *p0 = ws.partial, *p1 = ws.partial + 2 * kReduceBlocks;     // two dots, five dots
-            const unsigned g = A.grid(), ge = gr < kFusedEndBlocks ? gr : kFusedEndBlocks;
+            const unsigned g = A.step_grid(), ge = gr < kFusedEndBlocks ? gr : kFusedEndBlocks;
             A.template step<false>(sm, StepVecs<XT>{ro, uo, uu, v, rhv, nullptr},
                                    StepRed{nullptr, 0, p0, st, nullptr, TAIL_NONE, 0});                   // (5)-(7)
             A.template step<false>(sm, StepVecs<XT>{ro, v, rr, s, rhv, nullptr},

@@ -1264,16 +1264,16 @@ __global__ __launch_bounds__(kThreads) void k_apply_dia(DiaOp<VT> A, const XT* _
 }
 
 // ------------------------------------------------------------------------------ fused steps
-// Passes below kFusedRows: five launches and a finish instead of thirteen. Each operator
-// application forms its operand a - c b where it reads it (steps 5, 8, 12, 17) and writes it out
-// once; and each kernel sums the previous one's partials itself and applies the scalar update
-// (every work-group alike; the first one stores the new state for the next kernel, which reads
-// another slot), so the four finish kernels between them are gone. A small kernel is a few
-// microseconds of latency whatever it does: the 64^3 implicit step went from 233 to 172 us (with
-// the readback through pinned memory), a 160 x 120 two-component one from 200 to 123. At 128^3
-// the two forms are level (a step 37.9 us; update, sweep and finish 9.0 + 24.3 + 4.5), and above
-// 4 M rows the sweep's streaming form is not given up. The vector operations round as the
-// separate kernels do.
+// Passes of SolveOp::fused: five launches and a finish instead of nine launches and five finish
+// kernels. Each operator application forms its operand a - c b where it reads it (steps 5, 8, 12,
+// 17) and writes it out once; and each kernel sums the previous one's partials itself and applies
+// the scalar update (every work-group alike; the first one stores the new state for the next
+// kernel, which reads another slot), so the four finish kernels between them are gone. A small
+// kernel is a few microseconds of latency whatever it does: a 64^3 implicit step went from 233 to
+// 156 us (with the readback through pinned memory), a 160 x 120 two-component one from 200 to 123.
+// At 128^3 a step of seven slots takes 31 us; update, sweep and finish took 9.0 + 24.3 + 4.5. Where
+// the two forms are level stands beside SolveOp::fused; where sweeps stream, the streaming form is
+// not given up. The vector operations round as the separate kernels do.
 template <typename XT>
 struct StepVecs {
     const XT *a, *b;     // the operand is a - c b
@@ -1593,8 +1593,10 @@ __global__ void k_clear_state(KState* st) {
     }
 }
 
-// Rows below which a solve runs the fused steps (figures there).
+// The fused steps: never from kFusedRows rows on, where sweeps stream; below by the traversal
+// (SolveOp::fused in krylov.hip).
 constexpr long long kFusedRows = kStreamRows;
+constexpr unsigned kStepCsrGrid = 1024;      // ... on CSR, whose waves loop over their rows
 constexpr unsigned kFusedEndBlocks = 512;    // k_step_end: every work-group sums all of step 18's partials
 constexpr int kStates = 5;                   // state slots of a solve, one per kernel of a fused pass
 constexpr int kPassVecs = 8;                 // work vectors of a pass (seven without the fused steps)

@@ -90,6 +90,14 @@ def test_sweep_and_solves_on_both_sides_of_the_tile_rules_lines(ctx, rng, shape,
     test_sweep_and_solves_on_tile_edges(ctx, rng, shape, op)
 
 
+@pytest.mark.parametrize("shape,op", [((600, 701), "conv"), ((1446, 1450), "conv"), ((1450, 1447), "diff"),
+                                      ((1698, 1699), "diff"), ((20000, 4, 4), "conv"), ((101, 102, 103), "diff")])
+def test_solves_on_both_sides_of_the_fused_steps_lines(ctx, rng, shape, op):
+    """CSR steps whose work-groups loop over their rows, CSR and view solves just below and just above
+    the row counts from which the separate kernels take over, and tiles that are mostly idle."""
+    test_sweep_and_solves_on_tile_edges(ctx, rng, shape, op)
+
+
 @pytest.mark.parametrize("n", [1, 257])
 def test_breakdown_after_the_first_x_update_keeps_it(ctx, n):
     """A multiple of the identity breaks the method down in its first pass after step 10 (r = 0,
