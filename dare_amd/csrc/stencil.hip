@@ -56,9 +56,32 @@ static Launch cell_launch(const Geo& G, int each = 1) {
 }
 
 constexpr unsigned kGridYZ = 65535;      // work-groups along y and z that a launch takes
-// the same for line_pairs: two entries a lane, any number of rows and planes
-static Launch pair_launch(const Geo& G) {
-    Launch L = cell_launch(G, 2);
+// The same for line_pairs: two entries a lane, any number of rows and planes. From kDieEntries
+// entries on, the tiles of a 3-D plane (at least 28) are dealt in eight runs, one for each die
+// (work-groups b = x mod 8, along the grid's x, per_xcd slots a run), so that what the next plane
+// reads again comes from the die's own L2; the planes follow one another, which keeps the pages of
+// the arrays few. The runs move on by a die every eight planes: their lengths differ by one tile,
+// and without it 57 tiles a plane left seven dies waiting for the eighth (152^3 on arrays in turn
+// 54.8 us with tiles in order, 59 with fixed runs, 53.0 now). Gradient and divergence, us, tiles in
+// order and dealt: 161^3 on the same arrays 61.4 and 46.2, on arrays in turn 66.0 and 62.0; 112^3
+// 21.5 and 18.6, 25.6 and 24.4; 224^3 154 and 137, 156 and 143; level from 256^3 on and below a
+// million entries; 300 x 100 x 101, 25 tiles a plane, in turn 49.2 and 55.1.
+constexpr long long kDieEntries = 1LL << 20;
+struct PairTiles {
+    unsigned tiles_x, tiles, per_xcd;
+};
+struct PairLaunch : Launch {
+    PairTiles P{1, 0, 0};
+};
+static PairLaunch pair_launch(const Geo& G) {
+    PairLaunch L;
+    static_cast<Launch&>(L) = cell_launch(G, 2);
+    const unsigned long long tiles = static_cast<unsigned long long>(L.grid.x) * L.grid.y, per = (tiles + 7) / 8;
+    if (G.dim == 3 && G.ncell_int * G.N >= kDieEntries && tiles >= 28 && tiles <= (1ULL << 20)) {
+        L.P = PairTiles{L.grid.x, static_cast<unsigned>(tiles), static_cast<unsigned>(per)};
+        L.grid.x = 8 * L.P.per_xcd;
+        L.grid.y = 1;
+    }
     L.grid.y = L.grid.y < kGridYZ ? L.grid.y : kGridYZ;
     L.grid.z = L.grid.z < kGridYZ ? L.grid.z : kGridYZ;
     return L;
@@ -207,10 +230,17 @@ struct LinePair {
 };
 // f(LinePair) for this lane's entries of every line it owns: one, but for grids of more than 65535
 // planes or work-groups of rows
-template <int DIM, class F>
-__device__ __forceinline__ void line_pairs(const Geo& G, F&& f) {
+template <int DIM, bool DIES, class F>
+__device__ __forceinline__ void line_pairs(const Geo& G, const PairTiles& P, F&& f) {
     const int len = G.n[DIM - 1] * G.N;
-    const unsigned e = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
+    unsigned bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (DIES) {
+        const unsigned d = (bx + (blockIdx.z >> 3)) & 7, t = (P.tiles * d >> 3) + (bx >> 3);
+        if (t >= P.tiles * (d + 1) >> 3) return;
+        by = t / P.tiles_x;
+        bx = t - by * P.tiles_x;
+    }
+    const unsigned e = 2 * (bx * blockDim.x + threadIdx.x);
     if (e >= static_cast<unsigned>(len)) return;
     LinePair<DIM> L;
     L.e = static_cast<int>(e);
@@ -219,11 +249,12 @@ __device__ __forceinline__ void line_pairs(const Geo& G, F&& f) {
     L.high1 = L.two && L.e + 1 >= len - G.N;
     const int n0 = DIM == 3 ? G.n[0] : 1, n1 = DIM >= 2 ? G.n[DIM - 2] : 1;
     for (int i = blockIdx.z; i < n0; i += gridDim.z)
-        for (int j = blockIdx.y * blockDim.y + threadIdx.y; j < n1; j += gridDim.y * blockDim.y) {
+        for (int j = by * blockDim.y + threadIdx.y; j < n1; j += gridDim.y * blockDim.y) {
             L.q[0] = L.q[1] = L.q[2] = 0;
             if (DIM >= 2) L.q[DIM - 2] = j;
             if (DIM == 3) L.q[0] = i;
             f(L);
+            if (DIES) break;
         }
 }
 __device__ inline pair2 ld_pair(const double* p, bool two) {
@@ -243,16 +274,16 @@ __device__ inline void st_pair(double* p, pair2 v, bool two) {
 // components 37.9 -> 34.4 us (divergence 32.7 -> 29.5), 64^3 of three 7.5 -> 6.5 (5.5 -> 4.4),
 // 1024^2 6.6 -> 5.8 (5.2 -> 4.3), level at 10^5 entries. And entries in the order of memory keep
 // the pages of the four arrays few: a march along i in persistent work-groups, which re-reads
-// nothing, took 277 us for gradient and divergence of 256^3 on arrays in turn, this form 201 (128^3
-// 33.7 and 28.5; on one set of arrays over and over 270 and 200, 161^3 54 and 61). NT: stores past
+// nothing, took 277 us for gradient and divergence of 256^3 on arrays in turn, this form 194 (128^3
+// 40.8 and 31.9; on one set of arrays over and over 268 and 194, 161^3 54 and 46). NT: stores past
 // the caches from kStreamRows entries on (256^3 without 230; 128^3 with 26.9 against 26.7).
-template <int DIM, bool NT>
-__global__ __launch_bounds__(256) void k_grad_faces(Geo G, FaceGeo F, const double* __restrict__ phi,
+template <int DIM, bool NT, bool DIES>
+__global__ __launch_bounds__(256) void k_grad_faces(Geo G, FaceGeo F, PairTiles P, const double* __restrict__ phi,
                                                     double* __restrict__ f0, double* __restrict__ f1,
                                                     double* __restrict__ f2) {
     double* out[3] = {f0, f1, f2};
     const int N = G.N;
-    line_pairs<DIM>(G, [&](const LinePair<DIM>& L) {
+    line_pairs<DIM, DIES>(G, P, [&](const LinePair<DIM>& L) {
         const double* b = phi + pad_ord<DIM>(G, L.q) * N + L.e;
         const pair2 pc = ld_pair(b, L.two);
         pair2 lo[DIM];
@@ -275,13 +306,13 @@ __global__ __launch_bounds__(256) void k_grad_faces(Geo G, FaceGeo F, const doub
 
 // ---------------------------------------------------------------------- value divergence
 // Divergence_Cartesian.inl:211-235: A0 E - A0 W + A1 N - A1 S + A2 T - A2 B, in that order.
-template <int DIM, bool NT>
-__global__ __launch_bounds__(256) void k_div_faces(Geo G, FaceGeo F, const double* __restrict__ f0,
+template <int DIM, bool NT, bool DIES>
+__global__ __launch_bounds__(256) void k_div_faces(Geo G, FaceGeo F, PairTiles P, const double* __restrict__ f0,
                                                    const double* __restrict__ f1, const double* __restrict__ f2,
                                                    double* __restrict__ out) {
     const double* in[3] = {f0, f1, f2};
     const int N = G.N;
-    line_pairs<DIM>(G, [&](const LinePair<DIM>& L) {
+    line_pairs<DIM, DIES>(G, P, [&](const LinePair<DIM>& L) {
         pair2 lo[DIM], hi[DIM];
 #pragma unroll
         for (int d = 0; d < DIM; d++) {
@@ -673,14 +704,23 @@ void launch_step3_lim(dare_ctx* ctx, const Geo& G, int lim, const double* phi, c
         }                                                                                        \
     } while (0)
 
-#define DARE_DISPATCH_DIM_NT(G, KERNEL, NT, L, ...)                                                \
-    do {                                                                                         \
-        switch ((G).dim) {                                                                       \
-        case 1: hipLaunchKernelGGL((KERNEL<1, NT>), (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
-        case 2: hipLaunchKernelGGL((KERNEL<2, NT>), (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
-        default: hipLaunchKernelGGL((KERNEL<3, NT>), (L).grid, (L).block, 0, ctx->stream, __VA_ARGS__); break; \
-        }                                                                                        \
-    } while (0)
+// a kernel over line pairs: by dimension, streaming stores, planes dealt to the dies
+template <class F>
+void dispatch_pairs(const Geo& G, const PairLaunch& L, F&& f) {
+    using D1 = std::integral_constant<int, 1>;
+    using D2 = std::integral_constant<int, 2>;
+    using D3 = std::integral_constant<int, 3>;
+    using Yes = std::true_type;
+    using No = std::false_type;
+    const auto nt = [&](auto dim, auto dies) {
+        if (G.ncell_int * G.N >= kStreamRows) f(dim, Yes{}, dies);
+        else f(dim, No{}, dies);
+    };
+    if (G.dim == 1) nt(D1{}, No{});
+    else if (G.dim == 2) nt(D2{}, No{});
+    else if (L.P.per_xcd) nt(D3{}, Yes{});
+    else nt(D3{}, No{});
+}
 
 }  // namespace dare_hip
 
@@ -779,9 +819,11 @@ int dare_grad_faces(dare_ctx* ctx, const dare_grid* g, const double* phi, double
     DARE_CHECK_ARG(G.dim < 2 || fy, "fy is NULL");
     DARE_CHECK_ARG(G.dim < 3 || fz, "fz is NULL");
     const FaceGeo F = make_face_geo(G);
-    const Launch L = pair_launch(G);
-    if (G.ncell_int * G.N >= kStreamRows) DARE_DISPATCH_DIM_NT(G, k_grad_faces, true, L, G, F, phi, fx, fy, fz);
-    else DARE_DISPATCH_DIM_NT(G, k_grad_faces, false, L, G, F, phi, fx, fy, fz);
+    const PairLaunch L = pair_launch(G);
+    dispatch_pairs(G, L, [&](auto dim, auto nt, auto dies) {
+        hipLaunchKernelGGL((k_grad_faces<decltype(dim)::value, decltype(nt)::value, decltype(dies)::value>), L.grid, L.block, 0,
+                           ctx->stream, G, F, L.P, phi, fx, fy, fz);
+    });
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }
@@ -813,9 +855,11 @@ int dare_div_faces(dare_ctx* ctx, const dare_grid* g, const double* fx, const do
     DARE_CHECK_ARG(G.dim < 2 || fy, "fy is NULL");
     DARE_CHECK_ARG(G.dim < 3 || fz, "fz is NULL");
     const FaceGeo F = make_face_geo(G);
-    const Launch L = pair_launch(G);
-    if (G.ncell_int * G.N >= kStreamRows) DARE_DISPATCH_DIM_NT(G, k_div_faces, true, L, G, F, fx, fy, fz, out);
-    else DARE_DISPATCH_DIM_NT(G, k_div_faces, false, L, G, F, fx, fy, fz, out);
+    const PairLaunch L = pair_launch(G);
+    dispatch_pairs(G, L, [&](auto dim, auto nt, auto dies) {
+        hipLaunchKernelGGL((k_div_faces<decltype(dim)::value, decltype(nt)::value, decltype(dies)::value>), L.grid, L.block, 0,
+                           ctx->stream, G, F, L.P, fx, fy, fz, out);
+    });
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }

@@ -79,6 +79,14 @@ def test_paired_gradient_and_divergence_match_oracle(ctx, rng, n, ncomp):
     assert bits_equal(div.cpu().numpy(), orc.div_faces(go, exp))
 
 
+@pytest.mark.parametrize("n,ncomp", [([40, 112, 240], 1), ([11, 333, 301], 1), ([21, 161, 163], 2), ([13, 167, 173], 3),
+                                     ([9, 113, 1031], 1)])
+def test_gradient_and_divergence_dealt_to_the_dies_match_oracle(ctx, rng, n, ncomp):
+    """From 2^20 entries a plane's tiles go to the dies in runs that move on every eight planes: 28 tiles
+    and more, run lengths that differ by one tile, a last group of planes cut short."""
+    test_paired_gradient_and_divergence_match_oracle(ctx, rng, n, ncomp)
+
+
 def test_tvd_step_of_more_planes_than_a_launch_takes(ctx, rng):
     """Fewer cells than the march starts at, but more planes than a grid's third extent."""
     import torch
