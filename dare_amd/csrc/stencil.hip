@@ -26,13 +26,12 @@ static FaceGeo make_face_geo(const Geo& G) {
 }
 
 // Launch shape of the kernels for any dimension and component count: one lane per (cell,
-// component), or per two of them (`each`), x along axis dim-1 with the components innermost, y along axis dim-2, z along axis
-// dim-3; 64 x 4 lanes, or 32 x 8 or 16 x 16 where that saves an eighth of the work-groups (for
-// 5 % fewer, the shorter rows of writes cost more: the case below 83 us instead of 77).
-// A lane per cell that looped over its N components made every access of a wave N doubles apart:
-// three components on 97 x 131 x 115 cells, gradient and divergence 119 us a pair with the ghost
-// fill, then 77 (a contiguous run of tiles per die instead of tiles in order: 82, the face arrays'
-// writes then go to eight places at once).
+// component), or per two of them (`each`), x along axis dim-1 with the components innermost, y along
+// axis dim-2, z along axis dim-3; 64 x 4 lanes, or 32 x 8 where that saves an eighth of the
+// work-groups, or 16 x 16 where that saves a quarter more (the shorter rows cost otherwise: 112^3,
+// an eighth fewer of 16 lanes, face interpolation 11.2 -> 13.6 us, flux 20.9 -> 24.8). A lane per
+// cell that looped over its N components made every access of a wave N doubles apart: TVD step,
+// two components on 130 x 131 x 90 cells, 74 -> 47 us.
 struct Launch {
     dim3 grid, block;
 };
@@ -49,7 +48,7 @@ static Launch cell_launch(const Geo& G, int each = 1) {
     unsigned lanes = 64;
     const auto tiles = [&](unsigned l) { return static_cast<long long>(ceil_div(nx, l)) * ceil_div(G.n[ax_y], 256 / l); };
     for (unsigned l = 32; l >= 16; l /= 2)
-        if (8 * tiles(l) <= 7 * tiles(lanes)) lanes = l;
+        if (l == 32 ? 8 * tiles(l) <= 7 * tiles(lanes) : 4 * tiles(l) <= 3 * tiles(lanes)) lanes = l;
     L.block = dim3(lanes, 256 / lanes);
     L.grid = dim3(ceil_div(nx, lanes), ceil_div(G.n[ax_y], 256 / lanes), ax_z >= 0 ? G.n[ax_z] : 1);
     return L;
