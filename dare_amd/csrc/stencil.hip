@@ -167,6 +167,14 @@ __device__ inline double tvd_flux4(double a, double b, double c, double d, int l
     return (pU + (psi * 0.5) * (pD - pU)) * u;
 }
 
+// The same for a limiter of one value psi (CDS, UPWIND), which needs L and L+1 alone.
+__device__ inline double tvd_flux2(double b, double c, double psi, double u) {
+    const bool up = u >= 0.;
+    const double pU = up ? b : c, pD = up ? c : b;
+    return (pU + (psi * 0.5) * (pD - pU)) * u;
+}
+constexpr bool one_psi(int lim) { return lim == DARE_LIMITER_CDS || lim == DARE_LIMITER_UPWIND; }
+
 // ------------------------------------------------------------------------------ ghost fill
 struct GhostSlabs {
     long long start[7];      // prefix offsets of the 6 slabs (W,E,S,N,B,T)
@@ -394,7 +402,9 @@ __global__ __launch_bounds__(256) void k_tvd_flux(Geo G, FaceGeo F, int lim, con
 // ------------------------------------------------------------------ fused explicit TVD step
 // phi_out = phi - (dt/V) * div(phi_f * u_f); reads phi (13-point star) + 2 face velocities per
 // axis, writes one value per cell.
-template <int DIM>
+// ONE: a limiter of one value: neither the second neighbours nor the ratio (88^3, upwind: 12.8 us
+// with them).
+template <int DIM, bool ONE>
 __global__ __launch_bounds__(256) void k_tvd_step(Geo G, FaceGeo F, int lim, const double* __restrict__ phi,
                                                   const double* __restrict__ u0,
                                                   const double* __restrict__ u1,
@@ -411,15 +421,22 @@ __global__ __launch_bounds__(256) void k_tvd_step(Geo G, FaceGeo F, int lim, con
     for (int d = 0; d < DIM; d++) {
         const long long s = G.sl[d] * N, fi = face_ord<DIM>(F, d, q);
 #pragma unroll
-        for (int m = 0; m < 5; m++) p[d][m] = b[(m - 2) * s];
+        for (int m = ONE; m < 5 - ONE; m++) p[d][m] = b[(m - 2) * s];
         ulo[d] = vel[d][fi];
         uhi[d] = vel[d][fi + F.fs[d][d]];
     }
+    const double psi = ONE && lim == DARE_LIMITER_CDS ? 1. : 0.;      // of ONE
     double v = 0.;
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-        const double flo = tvd_flux4(p[d][0], p[d][1], p[d][2], p[d][3], lim, ulo[d]);
-        const double fhi = tvd_flux4(p[d][1], p[d][2], p[d][3], p[d][4], lim, uhi[d]);
+        double flo, fhi;
+        if constexpr (ONE) {
+            flo = tvd_flux2(p[d][1], p[d][2], psi, ulo[d]);
+            fhi = tvd_flux2(p[d][2], p[d][3], psi, uhi[d]);
+        } else {
+            flo = tvd_flux4(p[d][0], p[d][1], p[d][2], p[d][3], lim, ulo[d]);
+            fhi = tvd_flux4(p[d][1], p[d][2], p[d][3], p[d][4], lim, uhi[d]);
+        }
         if (d == 0) v = G.A[0] * fhi;
         else v += G.A[d] * fhi;
         v -= G.A[d] * flo;
@@ -444,7 +461,7 @@ constexpr int kStepTileK = 64, kStepXcd = 8, kStepMinPlanes = 8;
 // without LDS, five fluxes and fourteen loads per cell: 150 x 161 x 173, a third of whose tiles
 // are cut, 57.5 -> 54.3 us.)
 constexpr int kTvdRow = 68;   // staged row: 2 + 64 + 2 doubles
-template <bool NT, int TJ>
+template <bool NT, int TJ, bool AHEAD>
 __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const double* __restrict__ phi,
                                                const double* __restrict__ ux, const double* __restrict__ uy,
                                                const double* __restrict__ uz, double fac, double* __restrict__ out,
@@ -482,7 +499,7 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
     const long long ty_off = static_cast<long long>(upto(j0 + TJ, n1) - jy) * n2;
     const long long zx_off = static_cast<long long>(upto(j0 + lane, n1 - 1) - jx) * (n2 + 1) + (upto(k0 + 64, n2) - kz);
     double pm2 = phi[lp - 2 * sI], pm1 = phi[lp - sI], p0 = phi[lp], pp1 = phi[lp + sI];
-    double f_lo = tvd_flux4(pm2, pm1, p0, pp1, lim, ux[fx]);
+    const double u_lo = ux[fx], row0 = hload ? phi[lp + hoff] : 0., col0 = gload ? phi[lp + goff] : 0.;
     const double A0 = G.A[0], A1 = G.A[1], A2 = G.A[2];
     // Plane i + 1 is staged while plane i is computed from the other buffer, and the fluxes are shared
     // through two buffers too, so a plane has one barrier. nx: what the next plane reads, and the
@@ -503,19 +520,21 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
         nx[6] = hload ? phi[at + sI + hoff] : 0.;
         nx[7] = gload ? phi[at + sI + goff] : 0.;
     };
-    load(lp, fx, fy, fz);
+    if constexpr (AHEAD) load(lp, fx, fy, fz);
     T[own_slot] = p0;
-    if (hload) T[row_slot] = phi[lp + hoff];
-    if (gload) T[gslot] = phi[lp + goff];
+    if (hload) T[row_slot] = row0;
+    if (gload) T[gslot] = col0;
+    double f_lo = tvd_flux4(pm2, pm1, p0, pp1, lim, u_lo);
     __syncthreads();
     for (int i = i0; i < i1; i++) {
         const int buf = (i - i0) & 1;
+        if constexpr (!AHEAD) load(lp, fx, fy, fz);
         const double pp2 = nx[0], u_hi = nx[1], vy = nx[2], wz = nx[3], vyt = nx[4], wzr = nx[5];
         double* Tn = T + (buf ? 0 : kT);
         Tn[own_slot] = pp1;
         if (hload) Tn[row_slot] = nx[6];
         if (gload) Tn[gslot] = nx[7];
-        if (i + 1 < i1) load(lp + sI, fx + fxs, fy + fys, fz + fzs);
+        if (AHEAD && i + 1 < i1) load(lp + sI, fx + fxs, fy + fys, fz + fzs);
         const double* Ti = T + (buf ? kT : 0);
         double* Y = Fy + (buf ? kY : 0);
         double* Z = Fz + (buf ? kZ : 0);
@@ -561,7 +580,7 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
 // fastest, planes along i; blocks are dealt XCD by XCD (blocks b = x mod 8 own a contiguous run). The limiter is a template parameter so that each instantiation carries only its
 // own branch.
 constexpr int kStepTvdJ = 8;
-template <bool NT, int LIM>
+template <bool NT, int LIM, bool AHEAD>
 __global__ __launch_bounds__(64 * kStepTvdJ) void k_tvd_step3(Geo G, const double* __restrict__ phi,
                                                               const double* __restrict__ ux,
                                                               const double* __restrict__ uy,
@@ -581,7 +600,7 @@ __global__ __launch_bounds__(64 * kStepTvdJ) void k_tvd_step3(Geo G, const doubl
         const int i1 = (cend - c < n0 - i0) ? i0 + static_cast<int>(cend - c) : n0;
         const int k0 = static_cast<int>(col % tiles_k) * kStepTileK;
         const int j0 = static_cast<int>(col / tiles_k) * kStepTvdJ;
-        tvd_march3_lds<NT, kStepTvdJ>(G, LIM, phi, ux, uy, uz, fac, out, k0, j0, i0, i1, T, Fy, Fz);
+        tvd_march3_lds<NT, kStepTvdJ, AHEAD>(G, LIM, phi, ux, uy, uz, fac, out, k0, j0, i0, i1, T, Fy, Fz);
         c += i1 - i0;
     }
 }
@@ -673,13 +692,26 @@ int resident_per_cu(K kernel, int threads = 256) {
     return (e == hipSuccess && n > 0) ? n : 2;
 }
 
+// A short march of a limiter without divisions has nothing to hide the loads of the next plane
+// behind, and the extra ones before its first plane cost it: 128^3, upwind, 8 planes 16.9 us with
+// them, 16.2 without; 200^3, 32 planes 70.9 and 74.0.
+constexpr long long kShortMarch = 12;
 template <bool NT, int LIM>
 void launch_step3(dare_ctx* ctx, const Geo& G, const double* phi, const double* ux, const double* uy,
                   const double* uz, double fac, double* out) {
-    static const int per_cu = resident_per_cu(k_tvd_step3<NT, LIM>, 64 * kStepTvdJ);
+    const auto run = [&](auto ahead, const MarchPlan& P) {
+        hipLaunchKernelGGL((k_tvd_step3<NT, LIM, decltype(ahead)::value>), dim3(P.grid), dim3(64 * kStepTvdJ), 0,
+                           ctx->stream, G, phi, ux, uy, uz, fac, out, P.tiles_k, P.total, P.chunk, P.per_xcd);
+    };
+    static const int per_cu = resident_per_cu(k_tvd_step3<NT, LIM, true>, 64 * kStepTvdJ);
     const MarchPlan P = march_plan(ctx, G, per_cu, kStepTvdJ);
-    hipLaunchKernelGGL((k_tvd_step3<NT, LIM>), dim3(P.grid), dim3(64 * kStepTvdJ), 0, ctx->stream, G, phi, ux, uy, uz,
-                       fac, out, P.tiles_k, P.total, P.chunk, P.per_xcd);
+    if constexpr (!NT && one_psi(LIM)) {
+        if (P.chunk <= kShortMarch) {
+            run(std::false_type{}, P);
+            return;
+        }
+    }
+    run(std::true_type{}, P);
 }
 
 template <bool NT>
@@ -903,7 +935,17 @@ int dare_tvd_explicit_step(dare_ctx* ctx, const dare_grid* g, int32_t limiter, c
         DARE_LAUNCH_CHECK();
         return DARE_OK;
     }
-    DARE_DISPATCH_DIM(G, k_tvd_step, L, G, F, limiter, phi, ux, uy, uz, fac, phi_out);
+    const auto step = [&](auto dim, auto one) {
+        hipLaunchKernelGGL((k_tvd_step<decltype(dim)::value, decltype(one)::value>), L.grid, L.block, 0, ctx->stream, G, F,
+                           limiter, phi, ux, uy, uz, fac, phi_out);
+    };
+    const auto by_dim = [&](auto one) {
+        if (G.dim == 1) step(std::integral_constant<int, 1>{}, one);
+        else if (G.dim == 2) step(std::integral_constant<int, 2>{}, one);
+        else step(std::integral_constant<int, 3>{}, one);
+    };
+    if (one_psi(limiter)) by_dim(std::true_type{});
+    else by_dim(std::false_type{});
     DARE_LAUNCH_CHECK();
     return DARE_OK;
 }

@@ -87,6 +87,15 @@ def test_gradient_and_divergence_dealt_to_the_dies_match_oracle(ctx, rng, n, nco
     test_paired_gradient_and_divergence_match_oracle(ctx, rng, n, ncomp)
 
 
+@pytest.mark.parametrize("lim", [da.CDS, da.UPWIND])
+@pytest.mark.parametrize("n,ncomp", [([5, 7, 65], 1), ([3, 6, 22], 3), ([33, 65], 2), ([67], 1), ([130, 90, 97], 1),
+                                     ([200, 121, 150], 1)])
+def test_limiters_of_one_value_match_oracle(ctx, rng, n, ncomp, lim):
+    """The step of CDS and UPWIND reads the next neighbours alone; on the march (the last two shapes, 8 and
+    19 planes a work-group) it loads the next plane ahead only where the march is long."""
+    test_stencils_match_oracle(ctx, rng, n, ncomp, lim)
+
+
 def test_tvd_step_of_more_planes_than_a_launch_takes(ctx, rng):
     """Fewer cells than the march starts at, but more planes than a grid's third extent."""
     import torch
