@@ -122,15 +122,16 @@ __device__ __forceinline__ int row_entries(const Geo& G, const Terms& T, const i
         else if (q[d] == G.n[d] - 1 && T.bc_type[2 * d + 1] == DARE_BC_FIXED) fixed_face = 2 * d + 1;
     }
     const bool fixed = fixed_face >= 0;
-    // boundary faces hit by an edit (they only depend on the structure)
-    int bc_face[3] = {-1, -1, -1};
+    // boundary faces hit by an edit (they only depend on the structure). Without short circuits:
+    // the types behind a branch each were loaded one after the other (a fill of 64^3 5.9 us, 5.6
+    // with every load at the start)
+    bool at_lo[3] = {false, false, false}, at_hi[3] = {false, false, false};
 #pragma unroll
     for (int d = 0; d < kD && (DIM || d < dim); d++) {
-        if (q[d] == 0 && T.bc_type[2 * d] != 0) bc_face[d] = 2 * d;
-        else if (q[d] == G.n[d] - 1 && T.bc_type[2 * d + 1] != 0) bc_face[d] = 2 * d + 1;
-        // position bc_face + 1, written with constant indices
-        if (bc_face[d] == 2 * d) removed[2 * d + 1] = true;
-        else if (bc_face[d] == 2 * d + 1) removed[2 * d + 2] = true;
+        at_lo[d] = (q[d] == 0) & (T.bc_type[2 * d] != 0);
+        at_hi[d] = !at_lo[d] & (q[d] == G.n[d] - 1) & (T.bc_type[2 * d + 1] != 0);
+        removed[2 * d + 1] = at_lo[d];
+        removed[2 * d + 2] = at_hi[d];
     }
     if (fixed)
         for (int pos = 1; pos < 7; pos++) removed[pos] = true;
@@ -231,12 +232,13 @@ __device__ __forceinline__ int row_entries(const Geo& G, const Terms& T, const i
         }
 #pragma unroll
         for (int d = 0; d < kD && (DIM || d < dim); d++) {                  // boundary edits
-            const int f = bc_face[d];
-            if (f < 0) continue;
-            const double nbf = (f == 2 * d) ? nbv[2 * d + 1] : nbv[2 * d + 2];   // nbv[f + 1]
-            if (T.bc_type[f] == DARE_BC_DIRICHLET) {
+            const bool dirichlet = (at_lo[d] ? T.bc_type[2 * d] : T.bc_type[2 * d + 1]) == DARE_BC_DIRICHLET;
+            const double value = at_lo[d] ? T.bc_value[2 * d] : T.bc_value[2 * d + 1];
+            if (!(at_lo[d] | at_hi[d])) continue;
+            const double nbf = at_lo[d] ? nbv[2 * d + 1] : nbv[2 * d + 2];
+            if (dirichlet) {
                 nbv[0] -= nbf;
-                rhs -= (2. * T.bc_value[f]) * nbf;
+                rhs -= (2. * value) * nbf;
             } else {
                 nbv[0] += nbf;
             }
