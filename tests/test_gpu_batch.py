@@ -177,3 +177,52 @@ def test_batch_rejects_mixed_components_and_unstructured(ctx, rng):
     da.upload_host_csr(ctx, A, np.array([0, 1]), np.array([0]), np.array([2.0]))
     with pytest.raises(da.DareError):
         da.Batch(ctx, [A])
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("ncomp", [1, 2])
+def test_batch_system_that_breaks_down_among_others(ctx, rng, ncomp, mixed):
+    """Systems without diffusion (cells of volume 1: 0 I and 2 I) break down in their first pass, before
+    and after step 10, where x stays and where it has moved to the solution (whole numbers: exactly).
+    The others keep the bits that they have when those systems are solved at entry."""
+    import torch
+    systems = make_systems(ctx, rng, DIMS[:8], ncomp)
+    for s, c in ((1, 2.0), (3, 0.0), (7, 2.0)):
+        n = DIMS[s]
+        g = da.Grid.make(list(n), size=list(map(float, n)), ghost=1, ncomp=ncomp)
+        t = da.Terms.make(dt=1 / c if c else 0.0, bc_type=[da.BC_DIRICHLET] * 6, bc_value=[0.0] * 6,
+                          **({"diff_comp": [0.0, 0.0]} if ncomp == 2 else {"diff": 0.0}))
+        A = da.Csr(ctx)
+        da.build_structure(ctx, A, g, t)
+        phi = torch.zeros(int(np.prod([v + 2 for v in n])) * ncomp, dtype=torch.float64, device="cuda")
+        rows = int(np.prod(n)) * ncomp
+        b, x = (rng.integers(-8, 9, size=rows).astype(np.float64) for _ in range(2))
+        systems[s] = dict(g=g, t=t, A=A, phi=phi, rows=rows, c=c, b=b, x=x)
+    B = da.Batch(ctx, [S["A"] for S in systems])
+    got = {}
+    for broken in (True, False):
+        for passes in (0, 3):
+            fill_batch(ctx, B, systems)
+            for s, S in enumerate(systems):
+                if "c" in S:
+                    b = S["b"] if broken else S["c"] * S["x"]
+                    da.check(da.lib().dare_memcpy_h2d(ctx.h, B.rhs_ptr(s), b.ctypes.data, 8 * S["rows"]), "h2d")
+                    da.check(da.lib().dare_memcpy_h2d(ctx.h, B.x_ptr(s), S["x"].ctypes.data, 8 * S["rows"]), "h2d")
+            res = B.solve(tol=1e-10, tol_kind=1, max_it=300, mixed=mixed, graph_passes=passes)
+            got[broken, passes] = [(d2h(ctx, B.x_ptr(s), S["rows"]), r["iterations"]) for s, (S, r) in
+                                   enumerate(zip(systems, res))]
+            for s, (S, r) in enumerate(zip(systems, res)):
+                x = got[broken, passes][s][0]
+                if "c" not in S:
+                    assert r["converged"] == 1 and r["status"] == 0, s
+                elif broken:
+                    assert r["converged"] == 0 and r["status"] == da.DARE_ERR_BREAKDOWN and r["iterations"] == 1, s
+                    assert np.array_equal(x, S["b"] / 2 if S["c"] else S["x"]), s
+                else:
+                    assert r["converged"] == 1 and np.array_equal(x, S["x"]), s
+    for s, S in enumerate(systems):
+        if "c" not in S:
+            x, it = got[True, 0][s]
+            for k in ((True, 3), (False, 0), (False, 3)):
+                assert it == got[k][s][1] and np.array_equal(x.view(np.int64), got[k][s][0].view(np.int64)), (s, k)
+    B.close()

@@ -286,3 +286,68 @@ def test_symmetric_sweeps_of_every_extent_give_the_same_bits(ctx, rng, shape):
         got.append(([a.cpu().numpy() for a in [y] + xs], [q["iterations"] for q in r]))
     assert all(bits_equal(p, q) for p, q in zip(got[0][0], got[1][0])) and got[0][1] == got[1][1]
     A.close()
+
+
+@pytest.mark.parametrize("c", [0.0, 2.0])
+@pytest.mark.parametrize("shape", [(4, 6), (5, 7, 9), (6, 7, 10), (9, 8, 12), (128, 128, 256), (161, 163, 161),
+                                   (161, 163, 163)])
+def test_views_that_are_multiples_of_the_identity(ctx, rng, shape, c):
+    """Cells of volume 1 without diffusion: the operator is (1 / dt) I with explicit zeros beside its
+    diagonal, whose solves break down in their first pass, before step 10 (0 I, x stays) and after it
+    (2 I, x has moved to the solution), in the fused steps and in the separate kernels, on four slots
+    and on seven. Whole numbers make every sum exact, so x is the oracle's to the bit."""
+    import torch
+    go = orc.grid(list(shape), size=list(map(float, shape)), ghost=1)
+    g = da.Grid.make(list(shape), size=list(map(float, shape)), ghost=1)
+    kw = dict(dt=1 / c if c else 0.0, diff=0.0, bc_type=[1] * 6, bc_value=[0.0] * 6)
+    rp, col, val, *_ = orc.assemble(go, orc.terms(**kw), np.zeros(int(np.prod([m + 2 for m in shape]))))
+    n = len(rp) - 1
+    b, x0 = (rng.integers(-8, 9, size=n).astype(np.float64) for _ in range(2))
+    xo, ok, it, *_ = orc.bicgstab2(rp, col, val, b, x0, 1e-30, 10)
+    assert not ok and it == 1 and np.array_equal(xo, b / 2 if c else x0)
+    bd, phi = torch.from_numpy(b).cuda(), torch.zeros(g.num_padded, dtype=torch.float64, device="cuda")
+    A = da.Csr(ctx)
+    t = da.Terms.make(**kw)
+    da.build_structure(ctx, A, g, t)
+    x = torch.zeros_like(bd)
+    for symmetric in (True, False):
+        if len(shape) == 3:
+            da.set_symmetric_traversal(A, symmetric)
+        da.fill_values(ctx, A, g, t, phi, torch.zeros_like(bd), x)
+        for precond in (0, 1) if c else (0,):
+            x.copy_(torch.from_numpy(x0))
+            r = da.bicgstab2(ctx, A, bd, x, tol=1e-30, tol_kind=0, max_it=10, precond=precond)
+            assert r["status"] == da.DARE_ERR_BREAKDOWN and r["converged"] == 0 and r["iterations"] == 1
+            assert bits_equal(x.cpu().numpy(), xo)
+            x.copy_(torch.from_numpy(x0))
+            r = da.refine_mixed(ctx, A, bd, x, tol=1e-30, tol_kind=0, precond=precond)
+            assert r["status"] == da.DARE_ERR_BREAKDOWN and r["converged"] == 0 and r["refinements"] == 1
+            assert np.array_equal(x.cpu().numpy(), xo)
+    A.close()
+
+
+@pytest.mark.parametrize("copies", [1, 128])
+@pytest.mark.parametrize("M,b,loose", [([[-1, 2], [-1, 0]], [1, 0], 0), ([[-2, -2], [2, 1]], [2, 0], 0),
+                                       ([[-2, 2, -1], [0, -1, -2], [0, 1, 0]], [0, 1, 0], 0),
+                                       ([[-2, 1, 0], [2, 2, 2], [1, 0, -1]], [0, 2, 0], 0),
+                                       ([[-2, 1, 0], [2, 2, 2], [1, 0, -1]], [0, 2, 0], 1.5)])
+def test_breakdown_at_mu_and_tau(ctx, M, b, loose, copies):
+    """Blocks whose first pass ends at mu == 0 (s = 0) or at tau == 0 (t parallel to s) in exact binary
+    fractions: x keeps step 10 alone, and at tau == 0 the true residual decides on convergence."""
+    import scipy.sparse as sp
+    import torch
+    S = sp.kron(sp.eye(copies), sp.csr_matrix(np.ones_like(M))).tocsr()
+    S.sort_indices()
+    rp, col = S.indptr.astype(np.int32), S.indices.astype(np.int32)
+    val, b = np.tile(np.asarray(M, np.float64).ravel(), copies), np.tile(np.asarray(b, np.float64), copies)
+    tol = loose * np.sqrt(copies) if loose else 1e-30
+    xo, ok, it, res, _ = orc.bicgstab2(rp, col, val, b, np.zeros(len(b)), tol, 10)
+    assert ok == bool(loose) and it == 1 and np.any(xo)
+    A = da.Csr(ctx)
+    da.upload_host_csr(ctx, A, rp, col, val)
+    x = torch.zeros(len(b), dtype=torch.float64, device="cuda")
+    r = da.bicgstab2(ctx, A, torch.from_numpy(b).cuda(), x, tol=tol, tol_kind=0, max_it=10)
+    assert r["status"] == (0 if ok else da.DARE_ERR_BREAKDOWN)
+    assert r["converged"] == ok and r["iterations"] == it and r["residual"] == res
+    assert bits_equal(x.cpu().numpy(), xo)
+    A.close()
