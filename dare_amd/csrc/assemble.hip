@@ -812,12 +812,16 @@ int dare_csr_fill_values(dare_ctx* ctx, dare_csr* A, const dare_grid* g, const d
         // couples (with the signs exchanged twice), and the per-cell harmonic mean takes its two
         // diffusivities in face order (low cell first) from either side. Not claimed for fixed
         // faces (identity rows), for per-cell diffusivity across a periodic wrap (the wrapped
-        // face reads the caller's ghost values, which need not be the periodic images) or for a
+        // face reads the caller's ghost values, which need not be the periodic images), for a
         // single-cell axis (a cell coupled to itself through both faces; the structure refuses
-        // it unless periodic).
+        // it unless periodic) or for an axis edited at its low face alone, which wraps on any
+        // grid with a periodic axis: the last cell's high neighbour, the first cell, has had the
+        // low entry taken out that the traversals would read for it.
         bool sym = G.N == 1 && t->conv_limiter < 0 && t->react == nullptr;
         for (int f = 0; f < 6; f++) sym = sym && t->bc_type[f] != DARE_BC_FIXED;
-        for (int d = 0; d < G.dim; d++) sym = sym && G.n[d] > 1 && !(t->diff_cell && G.per[d]);
+        for (int d = 0; d < G.dim; d++)
+            sym = sym && G.n[d] > 1 && !(t->diff_cell && G.per[d]) &&
+                  !(t->bc_type[2 * d] != DARE_BC_NONE && t->bc_type[2 * d + 1] == DARE_BC_NONE);
         // E, N, T are left out when the solvers will take the symmetric traversals and no consumer
         // of this matrix has needed the seven slots yet
         const bool half = sym && !A->cross && A->sym_traversal && !A->ent_full;
