@@ -438,8 +438,10 @@ __global__ __launch_bounds__(kThreads) void k_dia_colscale(DiaView V, const doub
         for (int d = 0; d < 3; d++) {
             const int n = V.n[d];
             long long lo = node - stride[d], hi = node + stride[d];
-            if (pos[d] == 0) lo = V.per[d] ? node + static_cast<long long>(n - 1) * stride[d] : node;
-            if (pos[d] == n - 1) hi = V.per[d] ? node - static_cast<long long>(n - 1) * stride[d] : node;
+            // the wrapped neighbour unless an edit removed the entry: beside a periodic axis the
+            // others wrap too
+            if (pos[d] == 0) lo = V.rm_lo[d] ? node : node + static_cast<long long>(n - 1) * stride[d];
+            if (pos[d] == n - 1) hi = V.rm_hi[d] ? node : node - static_cast<long long>(n - 1) * stride[d];
             nb[d] = lo;
             nb[6 - d] = hi;
             hi_gone[d] = pos[d] == n - 1 && V.rm_hi[d];

@@ -75,7 +75,7 @@ def test_products_and_solves_of_wrapped_views_match_oracle(ctx, rng, shape, wrap
         # at most eight products a row, in another order than the oracle's at the wraps
         assert np.all(np.abs(y.cpu().numpy() - M @ v) <= 16 * 2.0 ** -53 * (abs(M) @ np.abs(v)))
         out = [y.cpu().numpy().copy()]
-        for precond in (0, da.PRECOND_MG):
+        for precond in (0, 1, da.PRECOND_MG):
             for mixed in (False, True):
                 x = x0.clone()
                 if mixed:
