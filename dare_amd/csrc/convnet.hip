@@ -91,15 +91,10 @@ __device__ inline uint2 relu_mask(uint2 g, const uint16_t* y) {
 template <int COUT>
 constexpr int conv_nbb() { return COUT / 16 < 2 ? COUT / 16 : 2; }
 
-// Fusions of k_conv (MODE bits): kConvUp -- the input is the half-resolution tensor and the
-// conv reads its nearest-neighbour upsampling (staging fetches each voxel's parent); kConvAdd --
-// the epilogue also writes Y2 = bf16(Y + E) (the decoder's skip connection, as k_add); kConvMask
-// -- the ReLU backward of the layer below: Y2 = Y where E > 0, else 0, and Y itself only if it is
-// not NULL (the skip gradients, which two consumers read). The mask as a pass of its own over the
-// written gradient took 3-8 us per layer at 64^3.
-constexpr int kConvUp = 1, kConvAdd = 2, kConvMask = 4;
-
-template <int CIN, int COUT, bool RELU, int OUT, int NSEG, int MODE = 0>
+// MASK: the epilogue also applies the ReLU backward of the layer below: Y2 = Y where E > 0, else
+// 0, and Y itself is written only if it is not NULL (the skip gradients, which two consumers
+// read). The mask as a pass of its own over the written gradient took 3-8 us per layer at 64^3.
+template <int CIN, int COUT, bool RELU, int OUT, int NSEG, bool MASK = false>
 __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Wt,
                                                      uint16_t* __restrict__ Y, float* __restrict__ Yf, int D, int H,
                                                      int W, const uint16_t* __restrict__ E, uint16_t* __restrict__ Y2) {
@@ -145,9 +140,7 @@ __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict
                 const int xl = v % SX, yl = (v / SX) % SY, zl = v / (SX * SY);
                 const int gx = x0 - 1 + xl, gy = y0 - 1 + yl, gz = z - 1 + zl;
                 if (gx >= 0 && gx < W && gy >= 0 && gy < H && gz >= 0 && gz < D) {
-                    const long long src = (MODE & kConvUp)
-                        ? (static_cast<long long>(gz >> 1) * (H >> 1) + (gy >> 1)) * (W >> 1) + (gx >> 1)
-                        : (static_cast<long long>(gz) * H + gy) * W + gx;
+                    const long long src = (static_cast<long long>(gz) * H + gy) * W + gx;
                     u[r] = *reinterpret_cast<const uint4*>(X + src * CIN + 16 * cc + 8 * h);
                 }
             } else if (t < NPIECE) { // weight piece (half, tap, co), co fastest
@@ -228,20 +221,8 @@ __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict
                 uint2 pk;
                 pk.x = static_cast<uint32_t>(b[0]) | (static_cast<uint32_t>(b[1]) << 16);
                 pk.y = static_cast<uint32_t>(b[2]) | (static_cast<uint32_t>(b[3]) << 16);
-                if (!(MODE & kConvMask) || Y) *reinterpret_cast<uint2*>(Y + at) = pk;
-                if constexpr ((MODE & kConvMask) != 0) *reinterpret_cast<uint2*>(Y2 + at) = relu_mask(pk, E + at);
-                if constexpr ((MODE & kConvAdd) != 0) {
-                    const uint2 ev = *reinterpret_cast<const uint2*>(E + at);
-                    const uint16_t e[4] = {static_cast<uint16_t>(ev.x & 0xffffu), static_cast<uint16_t>(ev.x >> 16),
-                                           static_cast<uint16_t>(ev.y & 0xffffu), static_cast<uint16_t>(ev.y >> 16)};
-                    uint16_t t[4];
-#pragma unroll
-                    for (int j = 0; j < 4; j++) t[j] = f2bf(bf2f(b[j]) + bf2f(e[j]));
-                    uint2 sk;
-                    sk.x = static_cast<uint32_t>(t[0]) | (static_cast<uint32_t>(t[1]) << 16);
-                    sk.y = static_cast<uint32_t>(t[2]) | (static_cast<uint32_t>(t[3]) << 16);
-                    *reinterpret_cast<uint2*>(Y2 + at) = sk;
-                }
+                if (!MASK || Y) *reinterpret_cast<uint2*>(Y + at) = pk;
+                if constexpr (MASK) *reinterpret_cast<uint2*>(Y2 + at) = relu_mask(pk, E + at);
             } else if (cob == 0 && kq == 0) {
                 Yf[vrow + v] = o[0];
             }
@@ -257,10 +238,9 @@ __global__ __launch_bounds__(kNetThreads) void k_conv(const uint16_t* __restrict
 // registers they would cost a wave per SIMD, which loses more than the LDS reads they save).
 // The input planes live in a ring of three LDS slots: plane z+2 is loaded into registers while plane z is computed and
 // written into the slot of plane z-1 afterwards, so each input plane is staged once per block
-// instead of three times and its loads overlap the MFMAs. MODE as k_conv (upsampled input,
-// skip-sum epilogue). Same operand layout, K order and accumulation order as k_conv
-// (bit-identical results).
-template <int CIN, int COUT, bool RELU, int OUT, int NSEG, int MODE = 0>
+// instead of three times and its loads overlap the MFMAs. MASK, operand layout, K order and
+// accumulation order as k_conv (bit-identical results).
+template <int CIN, int COUT, bool RELU, int OUT, int NSEG, bool MASK = false>
 __global__ __launch_bounds__(kNetThreads) void k_conv_zm(const uint16_t* __restrict__ X, const uint16_t* __restrict__ Wt,
                                                         uint16_t* __restrict__ Y, float* __restrict__ Yf, int D, int H,
                                                         int W, int ZB, const uint16_t* __restrict__ E,
@@ -299,9 +279,7 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_zm(const uint16_t* __restr
             if (t < PPL && gz >= 0 && gz < D) {
                 const int gx = x0 - 1 + v % SX, gy = y0 - 1 + v / SX;
                 if (gx >= 0 && gx < W && gy >= 0 && gy < H) {
-                    const long long src = (MODE & kConvUp)
-                        ? (static_cast<long long>(gz >> 1) * (H >> 1) + (gy >> 1)) * (W >> 1) + (gx >> 1)
-                        : (static_cast<long long>(gz) * H + gy) * W + gx;
+                    const long long src = (static_cast<long long>(gz) * H + gy) * W + gx;
                     u[r] = *reinterpret_cast<const uint4*>(X + src * CIN + 8 * p8);
                 }
             }
@@ -412,20 +390,8 @@ __global__ __launch_bounds__(kNetThreads) void k_conv_zm(const uint16_t* __restr
                     uint2 pk;
                     pk.x = static_cast<uint32_t>(b[0]) | (static_cast<uint32_t>(b[1]) << 16);
                     pk.y = static_cast<uint32_t>(b[2]) | (static_cast<uint32_t>(b[3]) << 16);
-                    if (!(MODE & kConvMask) || Y) *reinterpret_cast<uint2*>(Y + at) = pk;
-                    if constexpr ((MODE & kConvMask) != 0) *reinterpret_cast<uint2*>(Y2 + at) = relu_mask(pk, E + at);
-                    if constexpr ((MODE & kConvAdd) != 0) {
-                        const uint2 ev = *reinterpret_cast<const uint2*>(E + at);
-                        const uint16_t e[4] = {static_cast<uint16_t>(ev.x & 0xffffu), static_cast<uint16_t>(ev.x >> 16),
-                                               static_cast<uint16_t>(ev.y & 0xffffu), static_cast<uint16_t>(ev.y >> 16)};
-                        uint16_t t[4];
-#pragma unroll
-                        for (int j = 0; j < 4; j++) t[j] = f2bf(bf2f(b[j]) + bf2f(e[j]));
-                        uint2 sk;
-                        sk.x = static_cast<uint32_t>(t[0]) | (static_cast<uint32_t>(t[1]) << 16);
-                        sk.y = static_cast<uint32_t>(t[2]) | (static_cast<uint32_t>(t[3]) << 16);
-                        *reinterpret_cast<uint2*>(Y2 + at) = sk;
-                    }
+                    if (!MASK || Y) *reinterpret_cast<uint2*>(Y + at) = pk;
+                    if constexpr (MASK) *reinterpret_cast<uint2*>(Y2 + at) = relu_mask(pk, E + at);
                 } else if (grp == 0 && kq == 0) {
                     Yf[vrow + v] = o[0];
                 }
@@ -960,18 +926,6 @@ __global__ __launch_bounds__(kNetThreads) void k_pool_bwd_add_mask(const uint16_
     }
 }
 
-// n: elements (a multiple of 8)
-__global__ __launch_bounds__(kNetThreads) void k_add(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
-                                                    uint16_t* __restrict__ out, long long n) {
-    DARE_EW8_LOOP(n / 8) {
-        const Bf8 x = ld8(a, q), z = ld8(b, q);
-        Bf8 o;
-#pragma unroll
-        for (int e = 0; e < 8; e++) o.h[e] = f2bf(bf2f(x.h[e]) + bf2f(z.h[e]));
-        st8(out, q, o);
-    }
-}
-
 // ------------------------------------------------------------------------------ solver side
 // Normalisation scales: s[0] = max|phi^n|, s[1] = max|phi^n - phi^{n-1}|,
 // s[2] = max|resid * resid_scale| over the cells of the box (block maxima, then one block);
@@ -1359,7 +1313,7 @@ int resident_blocks() {
     return n;
 }
 
-template <int CIN, int COUT, bool RELU, int OUT, int MODE = 0>
+template <int CIN, int COUT, bool RELU, int OUT, bool MASK = false>
 void conv(hipStream_t sm, const uint16_t* X, const uint16_t* Wt, uint16_t* Y, float* Yf, const int* d, int level,
           const uint16_t* E = nullptr, uint16_t* Y2 = nullptr) {
     const int D = d[0] >> level, H = d[1] >> level, W = d[2] >> level;
@@ -1373,31 +1327,31 @@ void conv(hipStream_t sm, const uint16_t* X, const uint16_t* Wt, uint16_t* Y, fl
         const unsigned gx = static_cast<unsigned>((W + 16 * nseg - 1) / (16 * nseg));
         const unsigned gzm = static_cast<unsigned>((H + 3) / 4) * (COUT / 16);
         int per_cu = 1;
-        if (nseg == 4) per_cu = resident_blocks<k_conv_zm<CIN, COUT, RELU, OUT, (CIN <= 16 ? 4 : 2), MODE>>();
-        else if (nseg == 2) per_cu = resident_blocks<k_conv_zm<CIN, COUT, RELU, OUT, 2, MODE>>();
-        else per_cu = resident_blocks<k_conv_zm<CIN, COUT, RELU, OUT, 1, MODE>>();
+        if (nseg == 4) per_cu = resident_blocks<k_conv_zm<CIN, COUT, RELU, OUT, (CIN <= 16 ? 4 : 2), MASK>>();
+        else if (nseg == 2) per_cu = resident_blocks<k_conv_zm<CIN, COUT, RELU, OUT, 2, MASK>>();
+        else per_cu = resident_blocks<k_conv_zm<CIN, COUT, RELU, OUT, 1, MASK>>();
         const long long cols = static_cast<long long>(gx) * gzm;
         const long long nzb = std::max<long long>(1, static_cast<long long>(device_cus()) * per_cu / cols);
         const int zb = static_cast<int>((D + nzb - 1) / nzb);
         const dim3 grid(gx, gzm, static_cast<unsigned>((D + zb - 1) / zb));
         if (nseg == 4)
-            hipLaunchKernelGGL((k_conv_zm<CIN, COUT, RELU, OUT, (CIN <= 16 ? 4 : 2), MODE>), grid, blk, 0, sm, X, Wt, Y,
+            hipLaunchKernelGGL((k_conv_zm<CIN, COUT, RELU, OUT, (CIN <= 16 ? 4 : 2), MASK>), grid, blk, 0, sm, X, Wt, Y,
                                Yf, D, H, W, zb, E, Y2);
         else if (nseg == 2)
-            hipLaunchKernelGGL((k_conv_zm<CIN, COUT, RELU, OUT, 2, MODE>), grid, blk, 0, sm, X, Wt, Y, Yf, D, H, W, zb,
+            hipLaunchKernelGGL((k_conv_zm<CIN, COUT, RELU, OUT, 2, MASK>), grid, blk, 0, sm, X, Wt, Y, Yf, D, H, W, zb,
                                E, Y2);
         else
-            hipLaunchKernelGGL((k_conv_zm<CIN, COUT, RELU, OUT, 1, MODE>), grid, blk, 0, sm, X, Wt, Y, Yf, D, H, W, zb,
+            hipLaunchKernelGGL((k_conv_zm<CIN, COUT, RELU, OUT, 1, MASK>), grid, blk, 0, sm, X, Wt, Y, Yf, D, H, W, zb,
                                E, Y2);
     } else {
         if (W >= 64) {
-            hipLaunchKernelGGL((k_conv<CIN, COUT, RELU, OUT, 4, MODE>), dim3((W + 63) / 64, gy, D), blk, 0, sm, X, Wt,
+            hipLaunchKernelGGL((k_conv<CIN, COUT, RELU, OUT, 4, MASK>), dim3((W + 63) / 64, gy, D), blk, 0, sm, X, Wt,
                                Y, Yf, D, H, W, E, Y2);
         } else if (W >= 32) {
-            hipLaunchKernelGGL((k_conv<CIN, COUT, RELU, OUT, 2, MODE>), dim3((W + 31) / 32, gy, D), blk, 0, sm, X, Wt,
+            hipLaunchKernelGGL((k_conv<CIN, COUT, RELU, OUT, 2, MASK>), dim3((W + 31) / 32, gy, D), blk, 0, sm, X, Wt,
                                Y, Yf, D, H, W, E, Y2);
         } else {
-            hipLaunchKernelGGL((k_conv<CIN, COUT, RELU, OUT, 1, MODE>), dim3((W + 15) / 16, gy, D), blk, 0, sm, X, Wt,
+            hipLaunchKernelGGL((k_conv<CIN, COUT, RELU, OUT, 1, MASK>), dim3((W + 15) / 16, gy, D), blk, 0, sm, X, Wt,
                                Y, Yf, D, H, W, E, Y2);
         }
     }
@@ -1465,9 +1419,9 @@ void conv_bwd(hipStream_t sm, int cin, int cout, const uint16_t* X, const uint16
 // (may be NULL) receives the unmasked gradient
 void conv_bwd_mask(hipStream_t sm, int ch, const uint16_t* X, const uint16_t* Wt, uint16_t* raw, const uint16_t* act,
                    uint16_t* masked, const int* d, int level) {
-    if (ch == 16) conv<16, 16, false, 0, kConvMask>(sm, X, Wt, raw, nullptr, d, level, act, masked);
-    else if (ch == 32) conv<32, 32, false, 0, kConvMask>(sm, X, Wt, raw, nullptr, d, level, act, masked);
-    else conv<64, 64, false, 0, kConvMask>(sm, X, Wt, raw, nullptr, d, level, act, masked);
+    if (ch == 16) conv<16, 16, false, 0, true>(sm, X, Wt, raw, nullptr, d, level, act, masked);
+    else if (ch == 32) conv<32, 32, false, 0, true>(sm, X, Wt, raw, nullptr, d, level, act, masked);
+    else conv<64, 64, false, 0, true>(sm, X, Wt, raw, nullptr, d, level, act, masked);
 }
 
 // Partials of several layers share the buffer until k_chunk_sum runs over them.

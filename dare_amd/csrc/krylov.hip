@@ -47,10 +47,11 @@ struct SolveOp {
                     if (d.sym)
                         hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4, true>), dim3(grid), dim3(kThreads), 0, sm, d,
                                            x, epi, ws, st, tail, check);
-                    else if (d.unit_c)
-                        hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4, false, true>), dim3(grid), dim3(kThreads), 0,
-                                           sm, d, x, epi, ws, st, tail, check);
-                    else
+                    else if (d.unit_c) {      // only from kStreamRows (streaming epilogues)
+                        if constexpr (Epi::kNT)
+                            hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4, false, true>), dim3(grid),
+                                               dim3(kThreads), 0, sm, d, x, epi, ws, st, tail, check);
+                    } else
                         hipLaunchKernelGGL((k_apply_dia<1, VT, XT, Epi, 4>), dim3(grid), dim3(kThreads), 0, sm, d, x,
                                            epi, ws, st, tail, check);
                 }

@@ -93,6 +93,12 @@ def test_products_and_solves_of_wrapped_views_match_oracle(ctx, rng, shape, wrap
     A.close()
 
 
+@pytest.mark.parametrize("shape,wrap,op", [((162, 163, 162), "all", "diff"), ((161, 163, 163), "axis0", "diff"),
+                                           ((128, 128, 260), "no_edits_beside", "conv")])
+def test_products_and_solves_of_wrapped_views_above_four_million_rows(ctx, rng, shape, wrap, op):
+    test_products_and_solves_of_wrapped_views_match_oracle(ctx, rng, shape, wrap, op)
+
+
 @pytest.mark.parametrize("op", ["diff", "var", "conv"])
 @pytest.mark.parametrize("shape", [(1, 6, 8), (6, 1, 4), (5, 4, 1), (1, 1, 6), (1, 5, 64)])
 def test_products_and_solves_of_views_with_a_periodic_axis_of_one_cell(ctx, rng, shape, op):
