@@ -498,6 +498,7 @@ class Batch:
         check(lib().dare_batch_vectors(self.h, ctypes.byref(b), ctypes.byref(x), offs), "dare_batch_vectors")
         self.b_addr, self.x_addr = b.value, x.value
         self.offsets = np.array(offs[:], dtype=np.int64)
+        self._created = self.config()
 
     @property
     def rows(self):
@@ -514,8 +515,10 @@ class Batch:
         check(lib().dare_batch_get_config(self.h, ctypes.byref(c)), "dare_batch_get_config")
         return c.as_dict()
 
-    def set_config(self, tile_k=0, tile_i=16, grid=2048, order=1):
-        c = BatchConfig(tile_k, tile_i, grid, order)
+    def set_config(self, tile_k=None, tile_i=None, grid=None, order=None):
+        """Fields left out take the values that the batch was created with."""
+        new = dict(tile_k=tile_k, tile_i=tile_i, grid=grid, order=order)
+        c = BatchConfig(**{k: self._created[k] if v is None else v for k, v in new.items()})
         check(lib().dare_batch_set_config(self.ctx.h, self.h, ctypes.byref(c)), "dare_batch_set_config")
 
     def autotune(self, reps=5):

@@ -1,7 +1,7 @@
 """Autotuner cache for batched solves.
 
 dare_batch_autotune (C-ABI) times every candidate configuration — lanes per tile along k
-(16/32/64 or by each system's nz), planes per tile, persistent grid size and the order of the
+(16/32/64 or by each system's extents), planes per tile, persistent grid size and the order of the
 work list — on the batch itself and keeps the fastest. This module keys the result by the
 batch's shape (system sizes, components) and the device, and stores it in a JSON file so a
 later run with the same batch skips the search.

@@ -523,7 +523,7 @@ std::vector<BItem> make_items(const std::vector<int>& counts, const std::vector<
 
 int apply_config(dare_ctx* ctx, dare_batch* B, const dare_batch_config& cfg) {
     DARE_CHECK_ARG(cfg.tile_k == 0 || cfg.tile_k == 16 || cfg.tile_k == 32 || cfg.tile_k == 64,
-                   "tile_k must be 0 (by nz), 16, 32 or 64");
+                   "tile_k must be 0 (by the extents), 16, 32 or 64");
     DARE_CHECK_ARG(cfg.tile_i >= 1 && cfg.tile_i <= 4096, "tile_i out of range");
     DARE_CHECK_ARG(cfg.grid >= kXcd && cfg.grid <= 65536 && cfg.grid % kXcd == 0,
                    "grid must be a multiple of 8 in [8, 65536]");

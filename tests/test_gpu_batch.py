@@ -226,3 +226,15 @@ def test_batch_system_that_breaks_down_among_others(ctx, rng, ncomp, mixed):
             for k in ((True, 3), (False, 0), (False, 3)):
                 assert it == got[k][s][1] and np.array_equal(x.view(np.int64), got[k][s][0].view(np.int64)), (s, k)
     B.close()
+
+
+def test_batch_config_fields_left_out_are_the_created_ones(ctx, rng):
+    systems = make_systems(ctx, rng, DIMS[:3], 1)
+    B = da.Batch(ctx, [S["A"] for S in systems])
+    created = B.config()
+    B.set_config(tile_k=16, tile_i=2, grid=1024, order=2)
+    B.set_config(order=1)
+    assert B.config() == dict(created, order=1)
+    B.set_config()
+    assert B.config() == created
+    B.close()
