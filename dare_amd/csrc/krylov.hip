@@ -469,7 +469,8 @@ __global__ __launch_bounds__(kThreads) void k_dia_colscale(DiaView V, const doub
 template <typename OT>
 void launch_colscale(hipStream_t sm, const dare_csr* A, OT* out, bool skip_c = false) {
     const DiaView& V = A->dia_view;
-    const dim3 g(ceil_div(static_cast<long long>(V.n[2]) * V.N, 64), ceil_div(V.n[1], 4), V.n[0]), b(kThreads);
+    const int gz = V.n[0] < 65535 ? V.n[0] : 65535;      // longer grids take the kernel's loop
+    const dim3 g(ceil_div(static_cast<long long>(V.n[2]) * V.N, 64), ceil_div(V.n[1], 4), gz), b(kThreads);
     if (A->ent_lazy)
         hipLaunchKernelGGL((k_dia_colscale<OT, true>), g, b, 0, sm, A->dia_view, A->dia, A->dinv, out, skip_c);
     else

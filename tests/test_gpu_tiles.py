@@ -351,3 +351,8 @@ def test_breakdown_at_mu_and_tau(ctx, M, b, loose, copies):
     assert r["converged"] == ok and r["iterations"] == it and r["residual"] == res
     assert bits_equal(x.cpu().numpy(), xo)
     A.close()
+
+
+@pytest.mark.parametrize("op", ["diff", "conv"])
+def test_solves_of_more_planes_than_a_launch_has_along_z(ctx, rng, op):
+    test_sweep_and_solves_on_tile_edges(ctx, rng, (66000, 2, 3), op)
