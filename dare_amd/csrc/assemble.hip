@@ -123,8 +123,8 @@ __device__ __forceinline__ int row_entries(const Geo& G, const Terms& T, const i
     }
     const bool fixed = fixed_face >= 0;
     // boundary faces hit by an edit (they only depend on the structure). Without short circuits:
-    // the types behind a branch each were loaded one after the other (a fill of 64^3 5.9 us, 5.6
-    // with every load at the start)
+    // the types behind a branch each were loaded one after the other (a fill of 64^3 5.9 us, 4.9
+    // with every load at the start; 256^3, cell diffusivity, four slots 355 and 325)
     bool at_lo[3] = {false, false, false}, at_hi[3] = {false, false, false};
 #pragma unroll
     for (int d = 0; d < kD && (DIM || d < dim); d++) {
@@ -439,10 +439,10 @@ __global__ __launch_bounds__(256) void k_fill_values(Geo G, Terms T, long long n
 // N, T equal the W, S, B of the east, north and top neighbours, bit for bit (k_dia_mirror writes
 // them on demand).
 // With every term's code the kernel is bound by issue (arguments spilled to lanes, branches
-// around absent terms), hence one instantiation per common operator, before and after: cell
-// diffusivity and source, 256^3, W, S, B, C only 552 -> 366 us; TVD convection, 128^3 96 -> 75;
-// two components with a reaction, 16^3 to 64^3 cells 10.3 -> 6.7 each (a lane per cell looped over
-// its two rows before).
+// around absent terms), hence one instantiation per common operator. A call with every term's code
+// and now: cell diffusivity, W, S, B, C only, 128^3 48 and 32 us, 256^3 499 and 325; TVD convection,
+// 128^3 70 and 47; two components with a reaction, 64^3 cells 24.9 and 11.5 (a lane per cell looped
+// over its two rows).
 template <bool NT, bool F32, int FEAT, bool HALF>
 __global__ __launch_bounds__(256) void k_fill_dia(Geo G, Terms T, double* __restrict__ dia, float* __restrict__ dia32,
                                                   int slots, double* __restrict__ rhs, double* __restrict__ x0) {

@@ -159,8 +159,8 @@ struct BVec {
 // The vector part of a pass is the single solver's (k_comb, k_pass_end): steps 5, 8, 12 and 17
 // write the next operand, everything else waits for V_END, and a system in its first pass reads
 // the shadow residual where r and u would be. (FP32, all of 96 two-component systems with 7.9 M
-// rows active: the separate updates of r and x, and of u, r and s, took 28 + 37 us a pass, now
-// VRUS + VSUS; the initial operator sweep on a zero guess, 99 us, is gone.)
+// rows active: the separate updates of r and x, and of u, r and s, took 28 + 37 us a pass, and the
+// initial operator sweep on a zero guess 99 us a solve; a whole mixed solve 6.47 -> 5.40 ms.)
 template <typename XT, int OP>
 __global__ __launch_bounds__(kThreads) void kb_vec(const BSys* __restrict__ sys, const BItem* __restrict__ items,
                                                   int nitems, BVec<XT> a, double* partial, long long pstride,

@@ -664,8 +664,9 @@ __global__ __launch_bounds__(256) void k_copy_to_field(Geo G, const double* __re
 // 150 x 161 x 173 50 and 66.
 constexpr long long kMarchCells = 1LL << 20;
 
-// Balanced persistent schedule of the 3-D marching kernels: as many 256-thread blocks as stay
-// resident at once (per_cu, queried once per kernel), each with at least kStepMinPlanes planes.
+// Balanced persistent schedule of the 3-D marching kernels: as many of their work-groups (512
+// threads for the TVD step) as stay resident at once (per_cu, queried once per kernel), each with at
+// least kStepMinPlanes planes.
 struct MarchPlan {
     int tiles_k, per_xcd;
     long long total, chunk;

@@ -260,7 +260,7 @@ int dare_bicgstab2_solve(dare_ctx* ctx, const dare_csr* csr, const double* b, do
 int dare_bicgstab2_solve_noalloc(dare_ctx* ctx, const dare_csr* csr, const double* b, double* x,
                                  const dare_solver_params* p, dare_solver_result* res);
 /* FP32 inner BiCGStab(2) inside FP64 iterative refinement; r = b - A x, the update of x and
- * the stopping test in FP64. No reference counterpart (north-star precision form). */
+ * the stopping test in FP64. No reference counterpart. */
 int dare_refine_solve_mixed(dare_ctx* ctx, const dare_csr* csr, const double* b, double* x,
                             const dare_solver_params* p, dare_solver_result* res);
 
