@@ -695,7 +695,10 @@ int resident_per_cu(K kernel, int threads = 256) {
 
 // A short march of a limiter without divisions has nothing to hide the loads of the next plane
 // behind, and the extra ones before its first plane cost it: 128^3, upwind, 8 planes 16.9 us with
-// them, 16.2 without; 200^3, 32 planes 70.9 and 74.0.
+// them, 16.2 without; 200^3, 32 planes 70.9 and 74.0. Minmod has one division and no special cases:
+// where it streams, loads ahead only fill the memory's queues (arrays in turn, 256^3 150-154 us with
+// them, 147-150 without; 200^3 88.5 and 87; level below), and so does the third work-group a CU that
+// fits without them (256^3 174).
 constexpr long long kShortMarch = 12;
 template <bool NT, int LIM>
 void launch_step3(dare_ctx* ctx, const Geo& G, const double* phi, const double* ux, const double* uy,
@@ -704,7 +707,9 @@ void launch_step3(dare_ctx* ctx, const Geo& G, const double* phi, const double* 
         hipLaunchKernelGGL((k_tvd_step3<NT, LIM, decltype(ahead)::value>), dim3(P.grid), dim3(64 * kStepTvdJ), 0,
                            ctx->stream, G, phi, ux, uy, uz, fac, out, P.tiles_k, P.total, P.chunk, P.per_xcd);
     };
-    static const int per_cu = resident_per_cu(k_tvd_step3<NT, LIM, true>, 64 * kStepTvdJ);
+    constexpr bool kAhead = !(NT && LIM == DARE_LIMITER_MINMOD);
+    static const int fit = resident_per_cu(k_tvd_step3<NT, LIM, kAhead>, 64 * kStepTvdJ);
+    const int per_cu = kAhead || fit < 2 ? fit : 2;
     const MarchPlan P = march_plan(ctx, G, per_cu, kStepTvdJ);
     if constexpr (!NT && one_psi(LIM)) {
         if (P.chunk <= kShortMarch) {
@@ -712,7 +717,7 @@ void launch_step3(dare_ctx* ctx, const Geo& G, const double* phi, const double* 
             return;
         }
     }
-    run(std::true_type{}, P);
+    run(std::integral_constant<bool, kAhead>{}, P);
 }
 
 template <bool NT>

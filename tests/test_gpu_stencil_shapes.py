@@ -109,3 +109,9 @@ def test_tvd_step_of_more_planes_than_a_launch_takes(ctx, rng):
     out = pd.clone()
     da.tvd_explicit_step(ctx, g, da.VANLEER, pd, vd, 1e-3, out)
     assert bits_equal(out.cpu().numpy(), orc.tvd_explicit_step(go, da.VANLEER, phi, vel, 1e-3))
+
+
+@pytest.mark.parametrize("lim", [da.MINMOD, da.VANLEER, da.UPWIND])
+def test_streaming_tvd_march_matches_oracle(ctx, rng, lim):
+    """From 4 M cells on the march streams, without loads a plane ahead for minmod; tiles cut along k and j."""
+    test_stencils_match_oracle(ctx, rng, [131, 165, 195], 1, lim)
