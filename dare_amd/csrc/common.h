@@ -112,8 +112,9 @@ struct dare_csr {
     // fill writes it next to the FP64 slots; dia32_fresh says it holds float(dia) of the last fill
     int dia32_mode = 0, dia32_fresh = 0;
     // 1: the last device fill's operator is exactly symmetric by construction (one component,
-    // no convection, reaction or fixed faces, per-cell diffusivity only without a periodic axis:
-    // every face coefficient is the same expression for both rows it couples)
+    // no convection, reaction or fixed faces, per-cell diffusivity only without a periodic axis, no
+    // axis edited at its low face alone: every face coefficient is the same expression for both rows
+    // it couples)
     int sym_fill = 0;
     // 1: the last device fill may be exactly symmetric (one component, no convection or
     // reaction): the FP64 view is then checked on the device unless sym_fill holds (the FP32
