@@ -499,7 +499,13 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
     const long long ty_off = static_cast<long long>(upto(j0 + TJ, n1) - jy) * n2;
     const long long zx_off = static_cast<long long>(upto(j0 + lane, n1 - 1) - jx) * (n2 + 1) + (upto(k0 + 64, n2) - kz);
     double pm2 = phi[lp - 2 * sI], pm1 = phi[lp - sI], p0 = phi[lp], pp1 = phi[lp + sI];
-    const double u_lo = ux[fx], row0 = hload ? phi[lp + hoff] : 0., col0 = gload ? phi[lp + goff] : 0.;
+    // the march's first flux: before the loads of its first plane for van Leer (150 x 161 x 173 53.7 us
+    // after them, 52.9 before; 128^3 23.6 and 23.1), after them for the others (minmod 128^3 19.3, 19.6
+    // before)
+    const bool flux_first = lim == DARE_LIMITER_VANLEER;
+    const double u_lo = ux[fx];
+    double f_lo = flux_first ? tvd_flux4(pm2, pm1, p0, pp1, lim, u_lo) : 0.;
+    const double row0 = hload ? phi[lp + hoff] : 0., col0 = gload ? phi[lp + goff] : 0.;
     const double A0 = G.A[0], A1 = G.A[1], A2 = G.A[2];
     // Plane i + 1 is staged while plane i is computed from the other buffer, and the fluxes are shared
     // through two buffers too, so a plane has one barrier. nx: what the next plane reads, and the
@@ -524,7 +530,7 @@ __device__ __forceinline__ void tvd_march3_lds(const Geo& G, int lim, const doub
     T[own_slot] = p0;
     if (hload) T[row_slot] = row0;
     if (gload) T[gslot] = col0;
-    double f_lo = tvd_flux4(pm2, pm1, p0, pp1, lim, u_lo);
+    if (!flux_first) f_lo = tvd_flux4(pm2, pm1, p0, pp1, lim, u_lo);
     __syncthreads();
     for (int i = i0; i < i1; i++) {
         const int buf = (i - i0) & 1;
